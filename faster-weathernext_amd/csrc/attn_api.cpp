@@ -134,6 +134,15 @@ int check_tiles(const fwn_attn_desc* d, const fwn_tiles* t, const char* name) {
   if (t->n_parts < 0 || t->n_split < 0 || (t->n_split > 0 && !t->split) || (t->n_split > 0) != (t->n_parts > 0))
     return fail(FWN_ERR_TILES, "%s: inconsistent split schedule (%d parts, %d split blocks)", name, t->n_parts,
                 t->n_split);
+  if (t->flags & ~FWN_TILES_NODES) return fail(FWN_ERR_INVALID_ARG, "%s: unknown flags 0x%x", name, t->flags);
+  if (t->flags & FWN_TILES_NODES) {
+    if (!t->node) return fail(FWN_ERR_TILES, "%s: null node table", name);
+    // The kernels form row offsets as 24-bit products of the node and the row stride. The stride
+    // is below 2^24 bytes for lists of two or more blocks (a slice spans less than 2 GiB).
+    const int64_t elem = d->dtype == FWN_BF16 ? 2 : 4;
+    if (d->n >= 1 << 24 || d->stride_n * elem >= 1 << 24 || d->ostride_n * elem >= 1 << 24)
+      return fail(FWN_ERR_INVALID_ARG, "%s: rows or row stride of 2^24 or more with a node table", name);
+  }
   if (t->work) {
     // An order table serves the (batch, head) count it was built for and holds every job.
     if (t->work_pairs != d->batch * d->heads)
@@ -228,6 +237,7 @@ void set_tiles(KArgs& a, const fwn_tiles* t, void* ws) {
   a.lanes = t->lanes;
   a.groups = t->groups;
   a.halves = t->halves;
+  a.node = t->flags & FWN_TILES_NODES ? t->node : nullptr;
   a.items = (const int32_t*)t->items;
   a.split = t->split;
   a.n_tiles = t->n_tiles;

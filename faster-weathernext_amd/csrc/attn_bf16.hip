@@ -18,6 +18,17 @@
 // logical chunk, and the 32 lanes of a transpose read hit 4 consecutive rows x 4 consecutive
 // chunks.
 //
+// Node tables (G): a list laid out in a node order of its own walks fewer tiles and live groups than
+// one in the caller's order, and the kernels then address rows through the list's node table: the
+// LDS DMA takes any per-lane source address, so a gathered tile copy costs one LDS read and one
+// multiply-add per 1 KB instruction, the nodes of the next tile having been copied into LDS (512
+// bytes, one instruction of one wave) a tile ahead. Forward + backward, refinement-6 mesh, order
+// given by the caller -> the list's own: 16 hops, 4 heads, mesh order 1.269 -> 0.682 ms (17,183 ->
+// 7,047 tiles; 0.742 with the tensors themselves in such an order, events between the kernels); 8
+// hops, 8 members 6.64 -> 2.93 ms; 32 hops, 6 heads, Hilbert order 2.745 -> 2.54 ms. The variants
+// without G stay for lists whose order is good already (hip_attn.ORDERED_GAIN) and for callers of
+// the C ABI that pass no table.
+//
 // Reference: pallas_attn.py:112-141 (forward), 161-215 (dQ, dK/dV), 274-311 (VJP driver).
 #include "attn_bf16_tiles.h"
 
@@ -33,11 +44,12 @@ using namespace dev;
 // Two workgroups per CU: one K buffer and one V buffer (64 KB at D = 128) and at most 256 VGPRs
 // per wave, so the two resident workgroups overlap one's softmax (VALU) with the other's MFMAs.
 // K(t+1) streams in during softmax(t) and PV(t), V(t+1) during S(t+1).
-template <int D>
+template <int D, bool G>
 __global__ void __launch_bounds__(NT, 2) fwd_kernel(KArgs a) {
   constexpr int TB = Tile<D>::BYTES;
   __shared__ __attribute__((aligned(1024))) char lk[TB];
   __shared__ __attribute__((aligned(1024))) char lv[TB];
+  __shared__ __attribute__((aligned(16))) char lnode[G ? 2 * 4 * BLK : 16];
   lds_char* K = (lds_char*)lk;
   lds_char* V = (lds_char*)lv;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -49,13 +61,15 @@ __global__ void __launch_bounds__(NT, 2) fwd_kernel(KArgs a) {
   const rsrc_t rK = make_rsrc((const uint16_t*)a.k + j.base, a.slice_bytes);
   const rsrc_t rV = make_rsrc((const uint16_t*)a.v + j.base, a.slice_bytes);
 
-  const int qrow = j.blk * BLK + 32 * w + i;
+  const int qrow = node_at<G>(a, j.blk * BLK + 32 * w + i);
   u32x4 qf[D / 16];
   load_frag<D>(qf, make_rsrc((const uint16_t*)a.q + j.base, a.slice_bytes), qrow, snb, g);
   Off<D> off;
   off.init(lane);
   TileDma<D> dma;
   dma.init(w, lane, snb);
+  NodeTab tab;
+  if constexpr (G) tab.init(a, (lds_char*)lnode);
   f32x16 o[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) o[db] = zero16();
@@ -69,9 +83,18 @@ __global__ void __launch_bounds__(NT, 2) fwd_kernel(KArgs a) {
     const int kb = ((ci32_ptr)a.col)[t0];
     mbits = tile_bits(a, t0, w, lane);
     gnext = tile_groups(a, t0);
-    dma.issue(rK, K, w, kb * BLK, snb);
-    wait_vmem();  // K(t0), its mask and group bits and the Q fragment
-    dma.issue(rV, V, w, kb * BLK, snb);
+    if constexpr (G) {
+      uint32_t nd[TileDma<D>::OPS];
+      dma.nodes(nd, a.node, kb);
+      dma.gather(rK, K, w, nd, snb);
+      if (w == 0 && t0 + 1 < t1) tab.load((t0 + 1) & 1, ((ci32_ptr)a.col)[t0 + 1], lane);
+      wait_vmem();  // K(t0), its mask and group bits, the Q fragment and the nodes of tile t0 + 1
+      dma.gather(rV, V, w, nd, snb);
+    } else {
+      dma.issue(rK, K, w, kb * BLK, snb);
+      wait_vmem();  // K(t0), its mask and group bits and the Q fragment
+      dma.issue(rV, V, w, kb * BLK, snb);
+    }
   }
   __syncthreads();
   for (int tt = t0; tt < t1; ++tt) {
@@ -112,7 +135,18 @@ __global__ void __launch_bounds__(NT, 2) fwd_kernel(KArgs a) {
     wait_vmem();      // this wave's part of V(t); the next tile's group bits
     __syncthreads();  // all of V(t) landed; every wave is done reading K(t)
     const uint32_t copy_next = any_rows(gnext);
-    if (t + 1 < t1) dma.issue(rK, K, w, ((ci32_ptr)a.col)[t + 1] * BLK, snb, copy_next);
+    if (t + 1 < t1) {
+      if constexpr (G) {
+        // The nodes of tile t + 1 landed by the last barrier; those of tile t + 2 go where tile
+        // t's were (read by every wave before this barrier).
+        uint32_t nd[TileDma<D>::OPS];
+        dma.nodes(nd, tab.block((t + 1) & 1));
+        dma.gather(rK, K, w, nd, snb, copy_next);
+        if (w == 0 && t + 2 < t1) tab.load(t & 1, ((ci32_ptr)a.col)[t + 2], lane);
+      } else {
+        dma.issue(rK, K, w, ((ci32_ptr)a.col)[t + 1] * BLK, snb, copy_next);
+      }
+    }
     float corr;
     // The row max and the lazy rescale first; then per group the exponentials and its PV MFMAs,
     // so one group's VALU work overlaps the previous group's MFMAs.
@@ -148,7 +182,15 @@ __global__ void __launch_bounds__(NT, 2) fwd_kernel(KArgs a) {
     st.l += sum;
     wait_vmem();      // this wave's part of K(t+1)
     __syncthreads();  // all of K(t+1) landed; every wave is done reading V(t)
-    if (t + 1 < t1) dma.issue(rV, V, w, ((ci32_ptr)a.col)[t + 1] * BLK, snb, copy_next);
+    if (t + 1 < t1) {
+      if constexpr (G) {
+        uint32_t nd[TileDma<D>::OPS];
+        dma.nodes(nd, tab.block((t + 1) & 1));
+        dma.gather(rV, V, w, nd, snb, copy_next);
+      } else {
+        dma.issue(rV, V, w, ((ci32_ptr)a.col)[t + 1] * BLK, snb, copy_next);
+      }
+    }
   }
   const float ltot = st.l + __shfl_xor(st.l, 32);
   if (j.part >= 0) {
@@ -167,11 +209,12 @@ __global__ void __launch_bounds__(NT, 2) fwd_kernel(KArgs a) {
 // Two workgroups per CU: single K and V buffers (64 KB at D = 128), refilled once every wave is
 // done with the tile, and at most 256 VGPRs per wave; the other resident workgroup computes while
 // the copy is in flight.
-template <int D>
+template <int D, bool G>
 __global__ void __launch_bounds__(NT, 2) dq_kernel(KArgs a) {
   constexpr int TB = Tile<D>::BYTES;
   __shared__ __attribute__((aligned(1024))) char lk[TB];
   __shared__ __attribute__((aligned(1024))) char lv[TB];
+  __shared__ __attribute__((aligned(16))) char lnode[G ? 2 * 4 * BLK : 16];
   lds_char* K = (lds_char*)lk;
   lds_char* V = (lds_char*)lv;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -183,12 +226,12 @@ __global__ void __launch_bounds__(NT, 2) dq_kernel(KArgs a) {
   const rsrc_t rK = make_rsrc((const uint16_t*)a.k + j.base, a.slice_bytes);
   const rsrc_t rV = make_rsrc((const uint16_t*)a.v + j.base, a.slice_bytes);
 
-  const int qrow = j.blk * BLK + 32 * w + i;
+  const int qrow = node_at<G>(a, j.blk * BLK + 32 * w + i);
   u32x4 qf[D / 16], df[D / 16];
   load_frag<D>(qf, make_rsrc((const uint16_t*)a.q + j.base, a.slice_bytes), qrow, snb, g);
   load_frag<D>(df, make_rsrc((const uint16_t*)a.dout + j.obase, a.oslice_bytes), qrow, (uint32_t)a.osn * 2, g);
   float lse_t = 0.f, delta = 0.f;
-  if (qrow < a.n) {
+  if ((unsigned)qrow < (unsigned)a.n) {
     lse_t = a.lse[stat_index(a, j, qrow)] * LOG2E;
     delta = a.delta[stat_index(a, j, qrow)];
   }
@@ -196,6 +239,8 @@ __global__ void __launch_bounds__(NT, 2) dq_kernel(KArgs a) {
   off.init(lane);
   TileDma<D> dma;
   dma.init(w, lane, snb);
+  NodeTab tab;
+  if constexpr (G) tab.init(a, (lds_char*)lnode);
   f32x16 acc[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) acc[db] = zero16();
@@ -213,8 +258,16 @@ __global__ void __launch_bounds__(NT, 2) dq_kernel(KArgs a) {
     mbits = tile_bits(a, t0, w, lane);
     gcur = tile_groups(a, t0);
     hcur = tile_halves(a, t0);
-    dma.issue(rK, K, w, kb * BLK, snb, 3u);
-    dma.issue(rV, V, w, kb * BLK, snb, 3u);
+    if constexpr (G) {
+      uint32_t nd[TileDma<D>::OPS];
+      dma.nodes(nd, a.node, kb);
+      dma.gather(rK, K, w, nd, snb, 3u);
+      dma.gather(rV, V, w, nd, snb, 3u);
+      if (w == 0) tab.load(t0 & 1, kb, lane);
+    } else {
+      dma.issue(rK, K, w, kb * BLK, snb, 3u);
+      dma.issue(rV, V, w, kb * BLK, snb, 3u);
+    }
   }
   // hv: this wave's live 16-key halves of the group (bit h); a clear half gets no dS work and
   // no dQ MFMAs (its dS is zero).
@@ -267,8 +320,18 @@ __global__ void __launch_bounds__(NT, 2) dq_kernel(KArgs a) {
       hnext = tile_halves(a, t + 1);
     }
     const uint32_t copy = any_rows(gt);
-    dma.issue(rK, K, w, kb * BLK, snb, copy & 12u);
-    dma.issue(rV, V, w, kb * BLK, snb, copy & 12u);
+    if constexpr (G) {
+      // The nodes of tile t landed by this barrier; those of tile t + 1 go where tile t - 1's were
+      // (last read before it).
+      uint32_t nd[TileDma<D>::OPS];
+      dma.nodes(nd, tab.block(t & 1));
+      dma.gather(rK, K, w, nd, snb, copy & 12u);
+      dma.gather(rV, V, w, nd, snb, copy & 12u);
+      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, ((ci32_ptr)a.col)[t + 1], lane);
+    } else {
+      dma.issue(rK, K, w, kb * BLK, snb, copy & 12u);
+      dma.issue(rV, V, w, kb * BLK, snb, copy & 12u);
+    }
     // Key groups with no valid element for this wave are skipped (p = 0 throughout); key groups
     // with none for any wave are not copied either.
     const uint32_t live = gt >> (4 * w) & 15u;
@@ -281,8 +344,15 @@ __global__ void __launch_bounds__(NT, 2) dq_kernel(KArgs a) {
       const int kb1 = ((ci32_ptr)a.col)[t + 1];
       const uint32_t copy1 = any_rows(gnext);
       mbits = tile_bits(a, t + 1, w, lane);
-      dma.issue(rK, K, w, kb1 * BLK, snb, copy1 & 3u);
-      dma.issue(rV, V, w, kb1 * BLK, snb, copy1 & 3u);
+      if constexpr (G) {
+        uint32_t nd[TileDma<D>::OPS];
+        dma.nodes(nd, tab.block((t + 1) & 1));
+        dma.gather(rK, K, w, nd, snb, copy1 & 3u);
+        dma.gather(rV, V, w, nd, snb, copy1 & 3u);
+      } else {
+        dma.issue(rK, K, w, kb1 * BLK, snb, copy1 & 3u);
+        dma.issue(rV, V, w, kb1 * BLK, snb, copy1 & 3u);
+      }
     }
     if (live & 4u) group(2, mb, full & 4u, hw >> 4 & 3u);
     if (live & 8u) group(3, mb, full & 8u, hw >> 6 & 3u);
@@ -347,12 +417,13 @@ struct DsUnit {
 // the wave's live halves run as a two-stage pipeline: half k + 1's unit goes through the other
 // 1 KB stage slot and its LDS reads are in flight while half k's MFMAs issue (C3 dQ -2% against
 // one key group at a time, whose MFMAs waited for all of the group's reads).
-template <int D>
+template <int D, bool G>
 __global__ void __launch_bounds__(NT, 2) dq_ds_kernel(KArgs a) {
   constexpr int TB = Tile<D>::BYTES;
   __shared__ __attribute__((aligned(1024))) char lk0[TB];
   __shared__ __attribute__((aligned(1024))) char lk1[TB];
   __shared__ __attribute__((aligned(1024))) char lstage[4 * 2048];  // per wave: two unit slots
+  __shared__ __attribute__((aligned(16))) char lnode[G ? 2 * 4 * BLK : 16];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 31, g = lane >> 5;
@@ -364,11 +435,13 @@ __global__ void __launch_bounds__(NT, 2) dq_ds_kernel(KArgs a) {
   lds_char* st = (lds_char*)lstage + 2048 * w;
   DsUnit du;
   du.init(lane);
-  const int qrow = j.blk * BLK + 32 * w + i;
+  const int qrow = node_at<G>(a, j.blk * BLK + 32 * w + i);
   Off<D> off;
   off.init(lane);
   TileDma<D> dma;
   dma.init(w, lane, snb);
+  NodeTab tab;
+  if constexpr (G) tab.init(a, (lds_char*)lnode);
   f32x16 acc[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) acc[db] = zero16();
@@ -415,14 +488,23 @@ __global__ void __launch_bounds__(NT, 2) dq_ds_kernel(KArgs a) {
   // read (live16 bit x: rows 16x .. 16x + 15), so the others are not copied (12% of the rows of
   // live 32-row groups at C3, 6% at the C5 shape; dQ -2% and -1.3%). Op `op` of this wave fills
   // rows 4 RPO op + RPO w .. + RPO - 1, inside one 16-row chunk.
-  auto copy16 = [&](lds_char* tile, int row0, uint32_t live16) {
+  // With a node table the rows are the nodes in LDS block `slot`, or (slot < 0, the first tile)
+  // in global memory.
+  auto copy16 = [&](lds_char* tile, int kb, int slot, uint32_t live16) {
     constexpr int RPO = Tile<D>::ROWS_PER_OP;
+    uint32_t nd[TileDma<D>::OPS];
+    if constexpr (G) {
+      if (slot < 0)
+        dma.nodes(nd, a.node, kb);
+      else
+        dma.nodes(nd, tab.block(slot));
+    }
     uint32_t base = (uint32_t)(uintptr_t)tile + (uint32_t)w * 1024u;
     asm volatile("" : "+s"(base));
 #pragma unroll
     for (int op = 0; op < Tile<D>::OPS_PER_WAVE; ++op) {
       if (!(live16 >> ((op * 4 * RPO + w * RPO) >> 4) & 1u)) continue;
-      const uint32_t vo = dma.voff + (uint32_t)(row0 + op * 4 * RPO) * snb;
+      const uint32_t vo = G ? row_bytes(nd[op], snb) + dma.chunk : dma.voff + (uint32_t)(kb * BLK + op * 4 * RPO) * snb;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rK, (__attribute__((address_space(3))) void*)(uintptr_t)(base + op * 4096u),
                                                16, (int)vo, 0, 0, 0);
     }
@@ -446,7 +528,11 @@ __global__ void __launch_bounds__(NT, 2) dq_ds_kernel(KArgs a) {
     const uint32_t ht = hcur;
     const bool more = t + 1 < t1;
     const uint32_t hl = h1, ul = u1;
-    if (more) copy16(nxt, c1 * BLK, live16(h1));
+    if (more) copy16(nxt, c1, (t + 1) & 1, live16(h1));
+    // The nodes of tile t + 2 go where tile t's were (read before this barrier).
+    if constexpr (G) {
+      if (w == 0 && t + 2 < t1) tab.load(t & 1, c2, lane);
+    }
     hcur = h1;
     c1 = c2;
     h1 = h2;
@@ -493,13 +579,16 @@ __global__ void __launch_bounds__(NT, 2) dq_ds_kernel(KArgs a) {
   lds_char* K1 = (lds_char*)lk1;
   if (t0 < t1) {
     const uint32_t hf0 = tile_halves(a, t0);
-    copy16(K0, ((ci32_ptr)a.col)[t0] * BLK, live16(hf0));
+    copy16(K0, ((ci32_ptr)a.col)[t0], -1, live16(hf0));
     load_units(dsA, hf0, (uint32_t)((cmap_ptr)a.ubase)[t0]);
     hcur = hf0;
     if (t0 + 1 < t1) {
       c1 = ((ci32_ptr)a.col)[t0 + 1];
       h1 = tile_halves(a, t0 + 1);
       u1 = (uint32_t)((cmap_ptr)a.ubase)[t0 + 1];
+      if constexpr (G) {
+        if (w == 0) tab.load((t0 + 1) & 1, c1, lane);
+      }
     }
     if (t0 + 2 < t1) {
       c2 = ((ci32_ptr)a.col)[t0 + 2];
@@ -739,11 +828,12 @@ struct KeyWave {
 // A unit's store is issued at the start of the wave's next unit (or after its final tile), so the
 // vmcnt(0) before each tile barrier never waits for a store issued just before it; the stores are
 // non-temporal (nothing in this kernel reads them; allocating them in L2 would evict Q/dO tiles).
-template <int D, bool DS = false>
+template <int D, bool DS, bool G>
 __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
   constexpr int TB = Tile<D>::BYTES;
   __shared__ __attribute__((aligned(1024))) char lds0[2 * TB + 1536];  // Q | dO | lse[128] | gap | delta[128]
   __shared__ __attribute__((aligned(1024))) char lds1[2 * TB + 1536];
+  __shared__ __attribute__((aligned(16))) char lnode[G ? 2 * 4 * BLK : 16];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);  // keys 16 wid .. 16 wid + 15 of the block
   const int g = lane >> 4, t16 = lane & 15;
@@ -754,7 +844,7 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
   const rsrc_t rO = make_rsrc((const uint16_t*)a.dout + j.obase, a.oslice_bytes);
   const rsrc_t rL = make_rsrc(a.lse + stat_index(a, j, 0), (uint32_t)a.n * 4);
   const rsrc_t rD = make_rsrc(a.delta + stat_index(a, j, 0), (uint32_t)a.n * 4);
-  const int krow = j.blk * BLK + 16 * wid + t16;
+  const int krow = node_at<G>(a, j.blk * BLK + 16 * wid + t16);
   KeyWave<D> kw;
   kw.init(a, j, krow, g, t16);
 
@@ -770,9 +860,46 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
   dmaQ.init(wid & 3, lane, snb);
   dmaO.init(wid & 3, lane, osnb);
   constexpr uint32_t kPastEnd = 0x7FFFFFF0u;
+  NodeTab tab;
+  if constexpr (G) tab.init(a, (lds_char*)lnode);
   auto stats_wave = [&](int mode) { return mode == 0 ? wid == 0 : (mode == 1 && (wid & 3) == 0); };
   bool stats_cur = false;  // this wave copied the current tile's lse and delta (it rescales them)
-  auto issue = [&](int qb, lds_char* buf, uint32_t copy, int mode) {
+  // With a node table, slot is the LDS block of query block qb's nodes (< 0: read from global
+  // memory, the first tile).
+  auto issue = [&](int qb, lds_char* buf, uint32_t copy, int mode, int slot) {
+    if constexpr (G) {
+      uint32_t nd[TileDma<D, true>::OPS];
+      if (mode != 2) {
+        if (slot < 0)
+          dmaQ.nodes(nd, a.node, qb);
+        else
+          dmaQ.nodes(nd, tab.block(slot));
+      }
+      if (mode == 0) {
+        if (wid < 4) {
+          dmaQ.gather(rQ, buf, wid, nd, snb, copy);
+        } else {
+          dmaO.gather(rO, buf + TB, wid - 4, nd, osnb, copy);
+        }
+      } else if (mode == 1) {
+        dmaQ.gather(rQ, buf, wid & 3, nd, snb, copy);
+        dmaO.gather(rO, buf + TB, wid & 3, nd, osnb, copy);
+      }
+      if (stats_wave(mode)) {
+        // Rows `lane` and 64 + lane, 4 bytes each (rows past n read zeros).
+        lds_char* stats = buf + 2 * TB;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const uint32_t at = 64u * h + lane;
+          const uint32_t vo = 4u * (slot < 0 ? (uint32_t)a.node[(int64_t)qb * BLK + at] : tab.block(slot)[at]);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rL, (__attribute__((address_space(3))) void*)(stats + 256 * h), 4,
+                                                   (int)vo, 0, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rD, (__attribute__((address_space(3))) void*)(stats + 1024 + 256 * h),
+                                                   4, (int)vo, 0, 0, 0);
+        }
+      }
+      return;
+    }
     if (mode == 0) {
       if (wid < 4) {
         dma.issue(rQ, buf, wid, qb * BLK, snb, copy);
@@ -848,12 +975,16 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
         const uint32_t ns4 = (uint32_t)__builtin_popcount(hfc >> (s + 4) & 0x01010101u);
         mode = ((wid < 4) == (ns <= ns4)) ? 1 : 2;
       }
-      issue(cnext, nxt, any_rows(gnext), mode);
+      issue(cnext, nxt, any_rows(gnext), mode, (t + 1) & 1);
       stats_nxt = stats_wave(mode);
     }
     if (t + 2 < t1) {
       gnext = tile_groups(a, t + 2);
       cnext = ((ci32_ptr)a.col)[t + 2];
+      // The nodes of tile t + 2 go where tile t's were (read before this barrier).
+      if constexpr (G) {
+        if (wid == 0) tab.load(t & 1, cnext, lane);
+      }
     }
     uint32_t live, full;
     KeyWave<D>::live_units(mw, live, full);
@@ -896,7 +1027,10 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
       ubc = ((cmap_ptr)a.tmap)[2 * t0];
       hfc = ((cmap_ptr)a.tmap)[2 * t0 + 1];
     }
-    issue(((ci32_ptr)a.col)[t0], b0, any_rows(tile_groups(a, t0)), 0);
+    issue(((ci32_ptr)a.col)[t0], b0, any_rows(tile_groups(a, t0)), 0, -1);
+    if constexpr (G) {
+      if (wid == 0 && t0 + 1 < t1) tab.load((t0 + 1) & 1, cnext, lane);
+    }
     stats_cur = wid == 0;
   }
   for (int tt = t0; tt < t1; tt += 2) {
@@ -907,18 +1041,23 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
   kw.store(a, j, krow, 16 * wid + t16, g);
 }
 
-template <int D>
-hipError_t launch_d(Kind kind, const KArgs& a, hipStream_t stream) {
+template <int D, bool G>
+hipError_t launch_dg(Kind kind, const KArgs& a, hipStream_t stream) {
   const dim3 grid((unsigned)job_count(a)), block(NT);
   switch (kind) {
-    case Kind::kFwd: hipLaunchKernelGGL(fwd_kernel<D>, grid, block, 0, stream, a); break;
-    case Kind::kDq: hipLaunchKernelGGL(dq_kernel<D>, grid, block, 0, stream, a); break;
-    case Kind::kDkv: hipLaunchKernelGGL((dkv16_kernel<D, false>), grid, dim3(NT8), 0, stream, a); break;
-    case Kind::kDkvDs: hipLaunchKernelGGL((dkv16_kernel<D, true>), grid, dim3(NT8), 0, stream, a); break;
-    case Kind::kDqDs: hipLaunchKernelGGL(dq_ds_kernel<D>, grid, block, 0, stream, a); break;
+    case Kind::kFwd: hipLaunchKernelGGL((fwd_kernel<D, G>), grid, block, 0, stream, a); break;
+    case Kind::kDq: hipLaunchKernelGGL((dq_kernel<D, G>), grid, block, 0, stream, a); break;
+    case Kind::kDkv: hipLaunchKernelGGL((dkv16_kernel<D, false, G>), grid, dim3(NT8), 0, stream, a); break;
+    case Kind::kDkvDs: hipLaunchKernelGGL((dkv16_kernel<D, true, G>), grid, dim3(NT8), 0, stream, a); break;
+    case Kind::kDqDs: hipLaunchKernelGGL((dq_ds_kernel<D, G>), grid, block, 0, stream, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
+}
+
+template <int D>
+hipError_t launch_d(Kind kind, const KArgs& a, hipStream_t stream) {
+  return a.node ? launch_dg<D, true>(kind, a, stream) : launch_dg<D, false>(kind, a, stream);
 }
 
 }  // namespace

@@ -65,11 +65,41 @@ template <int D, bool K16 = false>
 struct TileDma {
   static constexpr int C = Tile<D>::C;
   static constexpr int RPO = Tile<D>::ROWS_PER_OP;
-  uint32_t voff;
+  static constexpr int OPS = Tile<D>::OPS_PER_WAVE;
+  uint32_t voff;   // source offset of this lane in the tile: its row of op 0, and its chunk
+  uint32_t chunk;  // the chunk alone (node tables)
+  uint32_t first;  // this lane's row of op 0 (op: + 4 RPO op)
 
   __device__ __forceinline__ void init(int w, int lane, uint32_t snb) {
     const int row = w * RPO + lane / C;
-    voff = (uint32_t)row * snb + (uint32_t)((((lane % C) ^ tile_swz<C, K16>(row))) << 4);
+    first = (uint32_t)row;
+    chunk = (uint32_t)((((lane % C) ^ tile_swz<C, K16>(row))) << 4);
+    voff = (uint32_t)row * snb + chunk;
+  }
+
+  // With a node table: the nodes of this lane's rows of tile column block kb, from the table in
+  // global memory or from its 128 entries for the block in LDS.
+  __device__ __forceinline__ void nodes(uint32_t (&nd)[OPS], const int32_t* node, int kb) const {
+#pragma unroll
+    for (int op = 0; op < OPS; ++op) nd[op] = (uint32_t)node[(int64_t)kb * BLK + first + op * 4 * RPO];
+  }
+  __device__ __forceinline__ void nodes(uint32_t (&nd)[OPS], const __attribute__((address_space(3))) uint32_t* tab) const {
+#pragma unroll
+    for (int op = 0; op < OPS; ++op) nd[op] = tab[first + op * 4 * RPO];
+  }
+
+  // issue() of a tile whose rows are the given nodes.
+  __device__ __forceinline__ void gather(rsrc_t r, lds_char* tile, int w, const uint32_t (&nd)[OPS], uint32_t snb,
+                                         uint32_t live = 15u) const {
+    uint32_t base = (uint32_t)(uintptr_t)tile + (uint32_t)w * 1024u;
+    asm volatile("" : "+s"(base));
+#pragma unroll
+    for (int op = 0; op < OPS; ++op) {
+      if (!(live >> ((op * 4 * RPO + w * RPO) >> 5) & 1u)) continue;
+      const uint32_t vo = row_bytes(nd[op], snb) + chunk;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(uintptr_t)(base + op * 4096u),
+                                               16, (int)vo, 0, 0, 0);
+    }
   }
 
   // Copies the rows of the tile's 32-row groups in `live` (bit c: rows 32c..32c+31, a
@@ -89,6 +119,25 @@ struct TileDma {
                                                16, (int)vo, 0, 0, 0);
     }
   }
+};
+
+// The node table of the tiles being copied, two blocks of 128 entries in LDS: block `slot` is
+// loaded by one wave (lanes 0-31, 16 bytes each) a tile before the copies that read it.
+struct NodeTab {
+  typedef const __attribute__((address_space(3))) uint32_t* ptr;
+  lds_char* base;
+  rsrc_t r;
+
+  __device__ __forceinline__ void init(const KArgs& a, lds_char* lds) {
+    base = lds;
+    r = make_rsrc(a.node, (uint32_t)a.n_blocks * (BLK * 4));
+  }
+  __device__ __forceinline__ void load(int slot, int kb, int lane) const {
+    if (lane < 32)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(base + slot * (BLK * 4)), 16,
+                                               (kb * BLK + 4 * lane) * 4, 0, 0, 0);
+  }
+  __device__ __forceinline__ ptr block(int slot) const { return (ptr)(base + slot * (BLK * 4)); }
 };
 
 // Per-lane LDS byte offsets of the MFMA A operands.

@@ -78,8 +78,10 @@ __global__ void __launch_bounds__(kThreads) fwd_combine_kernel(KArgs a) {
   const Cell<D> cell;
   const Split s = decode_split(a, cell.job);
   const int r = cell.r, d = cell.d;
-  const int row = s.blk * BLK + r;
-  if (!s.ok || row >= a.n) return;
+  const int pos = s.blk * BLK + r;
+  if (!s.ok) return;
+  const int row = a.node ? a.node[pos] : pos;  // the node table covers every block
+  if ((unsigned)row >= (unsigned)a.n) return;
   float M = -__builtin_inff();
   for (int c = 0; c < s.np; ++c) M = fmaxf(M, slot_ptr<D>(a, s, c)[128 * D + r]);
   const float base = M == -__builtin_inff() ? 0.f : M;
@@ -106,8 +108,10 @@ __global__ void __launch_bounds__(kThreads) bwd_combine_kernel(KArgs a) {
   const Cell<D> cell;
   const Split s = decode_split(a, cell.job);
   const int r = cell.r, d = cell.d;
-  const int row = s.blk * BLK + r;
-  if (!s.ok || row >= a.n) return;
+  const int pos = s.blk * BLK + r;
+  if (!s.ok) return;
+  const int row = a.node ? a.node[pos] : pos;  // the node table covers every block
+  if ((unsigned)row >= (unsigned)a.n) return;
   const int64_t out_off = (int64_t)s.b * a.sb + (int64_t)s.h * a.sh + (int64_t)row * a.sn + d;
 #pragma unroll
   for (int o = 0; o < OUTS; ++o) {

@@ -118,6 +118,19 @@ struct Job {
   bool skip;     // an empty entry of the order table: the workgroup does nothing
 };
 
+// The node (row of the tensors) at position `pos` of the list's order: the position itself, or
+// with a node table (G) its entry. Positions past the last block (a malformed item) are past the
+// tensors' rows, whose loads read zeros and whose stores drop.
+template <bool G>
+__device__ __forceinline__ int node_at(const KArgs& a, int pos) {
+  if constexpr (G) return pos < a.n_blocks * BLK ? a.node[pos] : a.n;
+  return pos;
+}
+
+// Byte offset of a row from a node table: node * stride, both below 2^24 (one v_mul_u32_u24 or
+// v_mad_u32_u24; a 32-bit product takes four times as long).
+__device__ __forceinline__ uint32_t row_bytes(uint32_t node, uint32_t stride) { return __umul24(node, stride); }
+
 // Without an order table, workgroups are dealt round-robin over the 8 XCDs, each with its own
 // L2. Jobs are ordered (batch, head) major, then work items in block order, and XCD x gets a
 // contiguous range of them, so the workgroups resident on one XCD work on neighbouring blocks of
@@ -351,7 +364,7 @@ __device__ __forceinline__ bool softmax_live(f32x16 (&s)[N], uint32_t live, Soft
 
 // Natural log-sum-exp of the scaled logits: (m + log2 l) * ln 2 (pallas_attn.py:140-141).
 __device__ __forceinline__ void write_lse(const KArgs& a, const Job& j, int row, const SoftmaxState& st, float ltot) {
-  if (a.lse_out && row < a.n) {
+  if (a.lse_out && (unsigned)row < (unsigned)a.n) {
     const float lse = (st.m + __builtin_amdgcn_logf(fmaxf(ltot, 1e-30f))) * LN2;
     a.lse_out[stat_index(a, j, row)] = lse;
   }

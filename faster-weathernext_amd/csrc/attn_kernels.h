@@ -24,6 +24,8 @@ struct KArgs {
   const uint32_t* halves;  // per tile: bit 8r + 2c + h = ... in columns 32c + 16h..; NULL = all live
   const int32_t* items;   // fwn_item[n_items] as int32 quadruples (block, t0, t1, part)
   const int32_t* split;   // [n_split * 3] block, first partial slot, slot count (combine pass)
+  const int32_t* node;    // [n_blocks * 128] node at each position of the list's own order (n past the last),
+                          //   or NULL: positions are nodes
   const int32_t* order;   // order table: [n_order][2] (pair b * heads + h, item) per workgroup, or NULL
   float* work;            // partial slots: [n_parts][batch * heads][128][2 * head_dim + 2] float32
   uint16_t* ds;           // dS units (bf16 backward with the dS exchange): [batch * heads][n_units][512]

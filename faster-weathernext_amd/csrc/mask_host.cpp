@@ -16,36 +16,11 @@
 
 #include "fwn_attn.h"
 #include "fwn_internal.h"
+#include "host_parallel.h"
 
 namespace {
 
-int worker_count() {
-  unsigned hw = std::thread::hardware_concurrency();
-  if (hw == 0) hw = 4;
-  return (int)std::min<unsigned>(hw, 16);
-}
-
-// Runs fn(begin, end) over [0, n) split into chunks handed out dynamically to the workers.
-template <typename Fn>
-void parallel_for(int64_t n, int64_t grain, Fn fn) {
-  int workers = worker_count();
-  if (n <= grain || workers <= 1) {
-    fn((int64_t)0, n);
-    return;
-  }
-  std::atomic<int64_t> next(0);
-  std::vector<std::thread> pool;
-  for (int w = 0; w < workers; ++w) {
-    pool.emplace_back([&]() {
-      for (;;) {
-        int64_t b = next.fetch_add(grain);
-        if (b >= n) break;
-        fn(b, std::min(n, b + grain));
-      }
-    });
-  }
-  for (auto& t : pool) t.join();
-}
+using fwn::parallel_for;
 
 // Breadth-first ball of radius k around src; `stamp` marks visited nodes with `mark`.
 void bfs_ball(int32_t src, int32_t k, const int64_t* adj_ptr, const int32_t* adj_idx,

@@ -1,0 +1,334 @@
+// A locality order of a tile list's nodes, computed from its mask alone, and the list of the
+// permuted mask.
+//
+// The kernels compute whole 32 x 32 groups of a live tile, so their work depends on how compactly
+// each node's neighbourhood lies in the node numbering. The mask is the only description of the
+// geometry the op gets (the reference orders nodes along a Hilbert curve from their latitudes and
+// longitudes before building its list, patch.py:208-214), so the order is built from it: breadth-first
+// distances to a few far-apart landmark nodes, averaged over each node's neighbourhood (which
+// turns the coarse hop counts into smooth coordinates), then recursive bisection along the
+// principal axis of the coordinates, in runs of whole 128-row blocks. On the refinement-6
+// icosahedral mesh this leaves (live 32 x 32 groups / 16) 1,676 of 4,341 with the 8-hop mask in mesh
+// order (Hilbert order: 2,151), 3,955 of 7,576 with 16 hops (4,764) and 11,190 of 16,545 with 32
+// (12,528), within 1% of bisecting the nodes' true positions.
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <cstring>
+#include <new>
+#include <vector>
+
+#include "fwn_attn.h"
+#include "fwn_internal.h"
+#include "host_parallel.h"
+
+namespace {
+
+using fwn::parallel_for;
+
+constexpr int32_t kWords = FWN_BLOCK / 32;
+constexpr int64_t kTileWords = (int64_t)FWN_BLOCK * kWords;
+constexpr int kLandmarks = 6;
+constexpr int kSmooth = 3;      // neighbourhood averages of the distances
+constexpr int kDims = 8;        // coordinates per node (kLandmarks, padded for the vector units)
+constexpr int32_t kLeaf = 16;   // nodes of a bisection leaf: the finest width the kernels skip
+constexpr int kAxisSamples = 512;
+
+struct List {
+  int32_t n, n_blocks;
+  const int32_t* ptr;
+  const int32_t* col;
+  const uint32_t* bits;
+};
+
+// Breadth-first distances from `src`: a node is one step further than the nearest node its row
+// of the mask holds. Nodes not reached get the largest distance plus one. Each level reads the
+// tiles whose column block has a node of the last level, for rows not reached yet.
+void distances(const List& m, int32_t src, std::vector<int32_t>& dist) {
+  std::vector<uint32_t> front((size_t)m.n_blocks * kWords, 0u), next(front.size(), 0u);
+  std::vector<uint8_t> any(m.n_blocks, 0), next_any(m.n_blocks, 0);
+  dist.assign(m.n, -1);
+  dist[src] = 0;
+  front[src / 32] |= 1u << (src % 32);
+  any[src / FWN_BLOCK] = 1;
+  int32_t level = 0;
+  for (bool more = true; more;) {
+    ++level;
+    std::atomic<bool> found(false);
+    parallel_for(m.n_blocks, 16, [&](int64_t b, int64_t e) {
+      for (int64_t blk = b; blk < e; ++blk) {
+        uint32_t* out = &next[blk * kWords];
+        std::memset(out, 0, kWords * sizeof(uint32_t));
+        next_any[blk] = 0;
+        const int32_t r0 = (int32_t)blk * FWN_BLOCK, rows = std::min(FWN_BLOCK, m.n - r0);
+        for (int32_t t = m.ptr[blk]; t < m.ptr[blk + 1]; ++t) {
+          if (!any[m.col[t]]) continue;
+          const uint32_t* f = &front[(int64_t)m.col[t] * kWords];
+          const uint32_t* w = m.bits + t * kTileWords;
+          for (int32_t r = 0; r < rows; ++r, w += kWords) {
+            if (!((w[0] & f[0]) | (w[1] & f[1]) | (w[2] & f[2]) | (w[3] & f[3])) || dist[r0 + r] >= 0) continue;
+            dist[r0 + r] = level;
+            out[r / 32] |= 1u << (r % 32);
+            next_any[blk] = 1;
+          }
+        }
+        if (next_any[blk]) found = true;
+      }
+    });
+    front.swap(next);
+    any.swap(next_any);
+    more = found;
+  }
+  for (int32_t i = 0; i < m.n; ++i)
+    if (dist[i] < 0) dist[i] = level;
+}
+
+// One neighbourhood average of the coordinates: each node's are replaced by the mean over the
+// nodes its row holds (its own are kept when the row is empty).
+void average(const List& m, const std::vector<float>& x, std::vector<float>& y) {
+  parallel_for(m.n_blocks, 2, [&](int64_t b, int64_t e) {
+    for (int64_t blk = b; blk < e; ++blk) {
+      const int32_t r0 = (int32_t)blk * FWN_BLOCK, rows = std::min(FWN_BLOCK, m.n - r0);
+      for (int32_t r = 0; r < rows; ++r) {
+        float sum[kDims] = {};
+        int32_t count = 0;
+        for (int32_t t = m.ptr[blk]; t < m.ptr[blk + 1]; ++t) {
+          const uint32_t* w = m.bits + t * kTileWords + r * kWords;
+          for (int32_t q = 0; q < kWords; ++q) {
+            const float* base = &x[((int64_t)m.col[t] * FWN_BLOCK + 32 * q) * kDims];
+            for (uint32_t v = w[q]; v; v &= v - 1) {
+              const float* p = base + __builtin_ctz(v) * kDims;
+              for (int d = 0; d < kDims; ++d) sum[d] += p[d];
+              ++count;
+            }
+          }
+        }
+        float* o = &y[(int64_t)(r0 + r) * kDims];
+        if (count == 0) {
+          std::memcpy(o, &x[(int64_t)(r0 + r) * kDims], sizeof(sum));
+          continue;
+        }
+        const float inv = 1.f / (float)count;
+        for (int d = 0; d < kDims; ++d) o[d] = sum[d] * inv;
+      }
+    }
+  });
+}
+
+// Where a run of m nodes is cut: near its middle, at a whole number of blocks while it spans more
+// than one, then at a power of two of leaves (so that 64-, 32- and 16-row groups are compact too).
+int32_t cut(int32_t m) {
+  int32_t unit = FWN_BLOCK;
+  if (m <= FWN_BLOCK)
+    for (unit = kLeaf; unit * 4 <= m;) unit *= 2;
+  const int32_t k = std::max(unit, (m / 2 + unit / 2) / unit * unit);
+  return k < m ? k : unit;
+}
+
+struct Key {
+  float v;
+  int32_t node;
+  bool operator<(const Key& o) const { return v < o.v || (v == o.v && node < o.node); }
+};
+
+// Recursive bisection of keys[0, m) by their projection on the run's principal axis (power
+// iteration on the covariance of a sample, from its axis of largest variance).
+void bisect(const std::vector<float>& x, Key* keys, int32_t m) {
+  while (m > kLeaf) {
+    double mean[kDims] = {}, cov[kDims][kDims] = {};
+    const int32_t step = std::max(1, m / kAxisSamples);
+    int32_t count = 0;
+    for (int32_t i = 0; i < m; i += step, ++count)
+      for (int d = 0; d < kDims; ++d) mean[d] += x[(int64_t)keys[i].node * kDims + d];
+    for (int d = 0; d < kDims; ++d) mean[d] /= count;
+    for (int32_t i = 0; i < m; i += step) {
+      double c[kDims];
+      for (int d = 0; d < kDims; ++d) c[d] = x[(int64_t)keys[i].node * kDims + d] - mean[d];
+      for (int d = 0; d < kDims; ++d)
+        for (int f = 0; f < kDims; ++f) cov[d][f] += c[d] * c[f];
+    }
+    int top = 0;
+    for (int d = 1; d < kDims; ++d)
+      if (cov[d][d] > cov[top][top]) top = d;
+    double axis[kDims];
+    for (int d = 0; d < kDims; ++d) axis[d] = cov[top][d];
+    for (int it = 0; it < 24; ++it) {
+      double big = 0.0, y[kDims] = {};
+      for (int d = 0; d < kDims; ++d) big = std::max(big, std::fabs(axis[d]));
+      if (big == 0.0) break;  // every sampled node at one point: any cut will do
+      for (int d = 0; d < kDims; ++d)
+        for (int f = 0; f < kDims; ++f) y[d] += cov[d][f] * (axis[f] / big);
+      std::memcpy(axis, y, sizeof(y));
+    }
+    double norm = 0.0;
+    for (int d = 0; d < kDims; ++d) norm += axis[d] * axis[d];
+    norm = norm > 0.0 ? 1.0 / std::sqrt(norm) : 0.0;
+    for (int32_t i = 0; i < m; ++i) {
+      double v = 0.0;
+      for (int d = 0; d < kDims; ++d) v += axis[d] * norm * x[(int64_t)keys[i].node * kDims + d];
+      keys[i].v = (float)v;
+    }
+    const int32_t k = cut(m);
+    std::nth_element(keys, keys + k, keys + m);
+    bisect(x, keys, k);
+    keys += k;
+    m -= k;
+  }
+  std::sort(keys, keys + m, [](const Key& a, const Key& b) { return a.node < b.node; });
+}
+
+int make_list(List& m, const char* what, int32_t n, const int32_t* tile_ptr, const int32_t* tile_col,
+              const uint32_t* tile_bits) {
+  if (n <= 0 || !tile_ptr) return fwn::fail(FWN_ERR_INVALID_ARG, "%s: null or empty argument", what);
+  m = List{n, (n + FWN_BLOCK - 1) / FWN_BLOCK, tile_ptr, tile_col, tile_bits};
+  const int32_t n_tiles = tile_ptr[m.n_blocks];
+  if (n_tiles > 0 && (!tile_col || !tile_bits)) return fwn::fail(FWN_ERR_INVALID_ARG, "%s: null tile arrays", what);
+  return fwn::check_tile_list(m.n_blocks, n_tiles, n, tile_ptr, tile_col);
+}
+
+// Calls fn(row within the new block, new column) for every entry of rows [128 blk, + 128) of the
+// permuted mask. Bits past the last row or column are not part of the mask.
+template <typename Fn>
+void for_entries(const List& m, const int64_t* perm, const std::vector<int32_t>& inv, int64_t blk, Fn fn) {
+  const int32_t r0 = (int32_t)blk * FWN_BLOCK, rows = std::min(FWN_BLOCK, m.n - r0);
+  for (int32_t r = 0; r < rows; ++r) {
+    const int32_t o = (int32_t)perm[r0 + r], ob = o / FWN_BLOCK;
+    for (int32_t t = m.ptr[ob]; t < m.ptr[ob + 1]; ++t) {
+      const uint32_t* w = m.bits + t * kTileWords + (int64_t)(o % FWN_BLOCK) * kWords;
+      for (int32_t q = 0; q < kWords; ++q) {
+        const int32_t c0 = m.col[t] * FWN_BLOCK + 32 * q;
+        for (uint32_t v = w[q]; v; v &= v - 1) {
+          const int32_t c = c0 + __builtin_ctz(v);
+          if (c < m.n) fn(r, inv[c]);
+        }
+      }
+    }
+  }
+}
+
+int inverse(const char* what, int32_t n, const int64_t* perm, std::vector<int32_t>& inv) {
+  if (!perm) return fwn::fail(FWN_ERR_INVALID_ARG, "%s: null perm", what);
+  inv.assign(n, -1);
+  for (int32_t i = 0; i < n; ++i) {
+    if (perm[i] < 0 || perm[i] >= n || inv[perm[i]] >= 0)
+      return fwn::fail(FWN_ERR_INVALID_ARG, "%s: perm is not a permutation", what);
+    inv[perm[i]] = i;
+  }
+  return FWN_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int fwn_tiles_node_order(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
+                         int64_t* perm) {
+  fwn::clear_error();
+  List m;
+  if (int rc = make_list(m, "fwn_tiles_node_order", n, tile_ptr, tile_col, tile_bits)) return rc;
+  if (!perm) return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_node_order: null perm");
+  try {
+    // Landmarks: the node furthest from node 0, then each time the node furthest from all so far.
+    std::vector<int32_t> dist, nearest;
+    std::vector<float> x((size_t)m.n_blocks * FWN_BLOCK * kDims, 0.f), y(x.size(), 0.f);
+    distances(m, 0, dist);
+    int32_t src = (int32_t)(std::max_element(dist.begin(), dist.end()) - dist.begin());
+    for (int l = 0; l < kLandmarks; ++l) {
+      distances(m, src, dist);
+      for (int32_t i = 0; i < n; ++i) x[(int64_t)i * kDims + l] = (float)dist[i];
+      if (l == 0) nearest = dist;
+      for (int32_t i = 0; i < n; ++i) nearest[i] = std::min(nearest[i], dist[i]);
+      src = (int32_t)(std::max_element(nearest.begin(), nearest.end()) - nearest.begin());
+    }
+    for (int s = 0; s < kSmooth; ++s) {
+      average(m, x, y);
+      x.swap(y);
+    }
+    std::vector<Key> keys(n);
+    for (int32_t i = 0; i < n; ++i) keys[i] = Key{0.f, i};
+    bisect(x, keys.data(), n);
+    for (int32_t i = 0; i < n; ++i) perm[i] = keys[i].node;
+  } catch (const std::exception& e) {
+    return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_node_order: %s", e.what());
+  }
+  return FWN_OK;
+}
+
+int fwn_tiles_permute_count(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
+                            const int64_t* perm, int32_t* new_ptr) {
+  fwn::clear_error();
+  List m;
+  if (int rc = make_list(m, "fwn_tiles_permute_count", n, tile_ptr, tile_col, tile_bits)) return rc;
+  if (!new_ptr) return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_permute_count: null output");
+  try {
+    std::vector<int32_t> inv;
+    if (int rc = inverse("fwn_tiles_permute_count", n, perm, inv)) return rc;
+    std::vector<int32_t> count(m.n_blocks);
+    parallel_for(m.n_blocks, 2, [&](int64_t b, int64_t e) {
+      std::vector<uint8_t> seen(m.n_blocks);
+      for (int64_t blk = b; blk < e; ++blk) {
+        std::fill(seen.begin(), seen.end(), (uint8_t)0);
+        for_entries(m, perm, inv, blk, [&](int32_t, int32_t c) { seen[c / FWN_BLOCK] = 1; });
+        count[blk] = (int32_t)std::count(seen.begin(), seen.end(), (uint8_t)1);
+      }
+    });
+    int64_t total = 0;
+    new_ptr[0] = 0;
+    for (int32_t blk = 0; blk < m.n_blocks; ++blk) {
+      total += count[blk];
+      if (total > INT32_MAX) return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_permute_count: too many tiles");
+      new_ptr[blk + 1] = (int32_t)total;
+    }
+  } catch (const std::exception& e) {
+    return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_permute_count: %s", e.what());
+  }
+  return FWN_OK;
+}
+
+int fwn_tiles_permute_fill(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
+                           const int64_t* perm, const int32_t* new_ptr, int32_t* new_col, uint32_t* new_bits) {
+  fwn::clear_error();
+  List m;
+  if (int rc = make_list(m, "fwn_tiles_permute_fill", n, tile_ptr, tile_col, tile_bits)) return rc;
+  if (!new_ptr || (new_ptr[m.n_blocks] > 0 && (!new_col || !new_bits)))
+    return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_permute_fill: null output");
+  std::atomic<bool> bad(false);
+  try {
+    std::vector<int32_t> inv;
+    if (int rc = inverse("fwn_tiles_permute_fill", n, perm, inv)) return rc;
+    parallel_for(m.n_blocks, 2, [&](int64_t b, int64_t e) {
+      // One block's rows as a dense bitmap by column block, then its blocks with a bit in order.
+      std::vector<uint32_t> dense((size_t)m.n_blocks * kTileWords);
+      std::vector<uint8_t> seen(m.n_blocks);
+      for (int64_t blk = b; blk < e; ++blk) {
+        std::fill(seen.begin(), seen.end(), (uint8_t)0);
+        for_entries(m, perm, inv, blk, [&](int32_t r, int32_t c) {
+          const int32_t kb = c / FWN_BLOCK, within = c % FWN_BLOCK;
+          uint32_t* tile = &dense[kb * kTileWords];
+          if (!seen[kb]) {
+            seen[kb] = 1;
+            std::memset(tile, 0, kTileWords * sizeof(uint32_t));
+          }
+          tile[r * kWords + within / 32] |= 1u << (within % 32);
+        });
+        int64_t t = new_ptr[blk];
+        if (std::count(seen.begin(), seen.end(), (uint8_t)1) != new_ptr[blk + 1] - t) {
+          bad = true;
+          return;
+        }
+        for (int32_t kb = 0; kb < m.n_blocks; ++kb) {
+          if (!seen[kb]) continue;
+          new_col[t] = kb;
+          std::memcpy(new_bits + t * kTileWords, &dense[kb * kTileWords], kTileWords * sizeof(uint32_t));
+          ++t;
+        }
+      }
+    });
+  } catch (const std::exception& e) {
+    return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_permute_fill: %s", e.what());
+  }
+  if (bad) return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_permute_fill: new_ptr does not match the mask");
+  return FWN_OK;
+}
+
+}  // extern "C"

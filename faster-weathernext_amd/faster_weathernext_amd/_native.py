@@ -52,7 +52,10 @@ class Tiles(ctypes.Structure):
               ("n_items", ctypes.c_int32), ("n_parts", ctypes.c_int32), ("n_split", ctypes.c_int32),
               ("n_work", ctypes.c_int32), ("items", ctypes.c_void_p), ("split", ctypes.c_void_p),
               ("halves", ctypes.c_void_p), ("work", ctypes.c_void_p), ("work_pairs", ctypes.c_int32),
-              ("reserved", ctypes.c_int32)]
+              ("flags", ctypes.c_int32), ("node", ctypes.c_void_p)]
+
+
+TILES_NODES = 1  # FWN_TILES_NODES: the list is laid out in an order of its own (Tiles.node)
 
 
 class DsMap(ctypes.Structure):
@@ -89,6 +92,9 @@ SIGNATURES = {
     "fwn_tiles_count": [_I32, _I32, _P, _P, _P, _P],
     "fwn_tiles_fill": [_I32, _I32, _P, _P, _P, _P, _P, _P],
     "fwn_tiles_prepare": [_I32, _I32, _I32, _P, _P, _P, _P, _P, _P],
+    "fwn_tiles_node_order": [_I32, _P, _P, _P, _P],
+    "fwn_tiles_permute_count": [_I32, _P, _P, _P, _P, _P],
+    "fwn_tiles_permute_fill": [_I32, _P, _P, _P, _P, _P, _P, _P],
     "fwn_tiles_schedule_count": [_I32, _P, _I32, _P, _P, _P],
     "fwn_tiles_schedule_fill": [_I32, _P, _I32, _P, _P],
     "fwn_tiles_order_count": [_I32, _P, _P, _I32, _I32, _I32, _I32, _I32, _P],

@@ -119,7 +119,7 @@ class _Schedule:
     return nat.Tiles(tl.n_blocks, tl.n_tiles, addr(tl.ptr), addr(tl.col), addr(tl.lanes), addr(tl.groups),
                      self.n_items, self.n_parts, self.n_split, 0 if work is None else work.shape[0],
                      addr(self.items), addr(self.split) if self.n_split else None, addr(tl.halves), addr(work),
-                     pairs, 0)
+                     pairs, 0 if tl.node is None else nat.TILES_NODES, addr(tl.node))
 
   def order_table(self, pairs, order=nat.ORDER_BALANCED, window=0, slots=64):
     """Host order table [n_work, 2] of this schedule for calls of `pairs` (batch, head) pairs."""
@@ -143,6 +143,13 @@ class _Schedule:
     return self._orders[key][1]
 
 
+# A list's own node order (TileList.launch_list): taken when the estimated cost of its tiles
+# (ORDER_TILE_UNITS per tile + ORDER_HALF_UNITS per live 32 x 16 half) is at most ORDERED_GAIN of
+# the given order's. On the refinement-6 mesh the estimates are 0.30 (8 hops) and 0.46 (16 hops) of
+# mesh order, 0.89 of Hilbert order (32 hops).
+ORDERED_GAIN = 0.95
+
+
 class TileList:
   """A tile list prepared for the kernels and resident on one device.
 
@@ -151,9 +158,13 @@ class TileList:
   call, as the reference shares one device copy of the mask across layers (``patch.py:263-266``).
   ``max_item_tiles`` fixes the split-K cap; None lets each launch pick it (``struct_for``).
   ``struct`` is the schedule with the fixed cap, or nat.ITEM_TILES.
+
+  The op's calls run ``launch_list()``: the same mask laid out in a node order of the list's own
+  (``fwn_tiles_node_order``) when that leaves the kernels less to compute, else this list. Nothing
+  outside the kernels sees that order: they address the rows of q, k, v, ... through ``node``.
   """
 
-  def __init__(self, tile_ptr, tile_kb, tile_bits, n_cols, device="cuda", max_item_tiles=None):
+  def __init__(self, tile_ptr, tile_kb, tile_bits, n_cols, device="cuda", max_item_tiles=None, _node=None):
     tile_ptr = nat.as_c(tile_ptr, np.int32)
     tile_kb = nat.as_c(tile_kb, np.int32)
     tile_bits = nat.as_c(tile_bits, np.uint32)
@@ -177,6 +188,8 @@ class TileList:
                                   nat.ptr(tile_bits), nat.ptr(lanes), nat.ptr(groups), nat.ptr(halves)))
     self.device = torch.device(device)
     put = lambda a: torch.from_numpy(a).to(self.device)
+    # The node at each position (n_cols past the last), or None: positions are nodes.
+    self.node = _node
     self.ptr = put(tile_ptr)
     self.col = put(tile_kb)
     self.lanes = put(lanes.view(np.int64))
@@ -197,6 +210,56 @@ class TileList:
     self.items_host, self.split_host = base.items_host, base.split_host
     self.items, self.split = base.items, base.split
     self.struct = base.struct
+    self._perm = None
+    self._transposes = weakref.WeakKeyDictionary()
+    self._ordered = self._lay_out() if _node is None and self.device.type == "cuda" else None
+
+  def _cost(self, n_tiles, halves):
+    return ORDER_TILE_UNITS * n_tiles + ORDER_HALF_UNITS * int(np.unpackbits(halves.view(np.uint8)).sum())
+
+  def _lay_out(self):
+    """This mask's list in a locality order of its own, or None where that would not pay (or the
+    list is not square, or a single block)."""
+    n = self.n_cols
+    if self.n_blocks != -(-n // nat.BLOCK) or self.n_blocks < 2 or n >= 1 << 24 or not self.n_tiles:
+      return None
+    perm = np.empty(n, np.int64)
+    nat.check(nat.lib().fwn_tiles_node_order(n, nat.ptr(self._tile_ptr), nat.ptr(self._tile_col),
+                                             nat.ptr(self._tile_bits), nat.ptr(perm)))
+    node = np.full(self.n_blocks * nat.BLOCK, n, np.int32)
+    node[:n] = perm
+    ordered = self._permuted(perm, torch.from_numpy(node).to(self.device))
+    if (self._cost(ordered.n_tiles, ordered.halves_host) >
+        ORDERED_GAIN * self._cost(self.n_tiles, self.halves_host)):
+      return None
+    self._perm = perm
+    return ordered
+
+  def _permuted(self, perm, node):
+    """The list of mask[perm][:, perm], with the device table `node` of that order."""
+    L = nat.lib()
+    args = (self.n_cols, nat.ptr(self._tile_ptr), nat.ptr(self._tile_col), nat.ptr(self._tile_bits), nat.ptr(perm))
+    tile_ptr = np.zeros(self.n_blocks + 1, np.int32)
+    nat.check(L.fwn_tiles_permute_count(*args, nat.ptr(tile_ptr)))
+    tile_kb = np.empty(int(tile_ptr[-1]), np.int32)
+    tile_bits = np.empty((int(tile_ptr[-1]), nat.BLOCK, nat.BLOCK // 32), np.uint32)
+    nat.check(L.fwn_tiles_permute_fill(*args, nat.ptr(tile_ptr), nat.ptr(tile_kb), nat.ptr(tile_bits)))
+    return TileList(tile_ptr, tile_kb, tile_bits, self.n_cols, self.device, self._fixed_cap, _node=node)
+
+  def launch_list(self, desc):
+    """The list the kernels of a call with descriptor `desc` walk for this mask: the one laid out in
+    its own order where there is one (bf16 kernels), else this one."""
+    return self if self._ordered is None or desc.dtype != nat.BF16 else self._ordered
+
+  def launch_lists(self, tiles_t, desc):
+    """(launch list of this mask, list of the transposed mask `tiles_t` in the same order): the
+    pair whose dS units the backward exchanges."""
+    tl = self.launch_list(desc)
+    if tiles_t is self or tl is self or tiles_t.n_blocks != self.n_blocks or tiles_t.n_cols != self.n_cols:
+      return tl, tl if tiles_t is self else tiles_t
+    if tiles_t not in self._transposes:
+      self._transposes[tiles_t] = tiles_t._permuted(self._perm, tl.node)
+    return tl, self._transposes[tiles_t]
 
   def _schedule(self, cap):
     cap = int(cap) if cap > 0 else nat.ITEM_TILES
@@ -448,7 +511,7 @@ def attention_forward(q, k, v, tiles, scale, with_lse=True, precision="native"):
   v = _same_layout(v, q, "v")
   out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
   desc = _desc(q, scale, out, prec)
-  tl = _as_tiles(tiles, q.shape[1], q.device)
+  tl = _as_tiles(tiles, q.shape[1], q.device).launch_list(desc)
   lse = torch.empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32, device=q.device) if with_lse else None
   ws = workspace(desc, q.device, tl)
   ts = tl.struct_for_desc(desc, "fwd")
@@ -487,12 +550,15 @@ def _backward_into(q, k, v, out, lse, dout, tiles, tiles_t, scale, dq, dk, dv, p
   exchange only."""
   desc = _desc(q, scale, out)
   n = q.shape[1]
-  tl = _as_tiles(tiles, n, q.device)
-  tlt = tl if tiles_t is None else _as_tiles(tiles_t, n, q.device)
+  base = _as_tiles(tiles, n, q.device)
+  base_t = base if tiles_t is None else _as_tiles(tiles_t, n, q.device)
   delta = torch.empty_like(lse)
   L = nat.lib()
   main = torch.cuda.current_stream(q.device)
-  dmap = tl.ds_map(tlt, unit_keys_for(q.dtype)) if DS_EXCHANGE else None
+  dmap = None
+  if DS_EXCHANGE:
+    tl, tlt = base.launch_lists(base_t, desc)
+    dmap = tl.ds_map(tlt, unit_keys_for(q.dtype))
   if dmap is not None:
     # delta, dK/dV writing dS, then dQ from dS, in stream order (fwn_attn_bwd_ds_launch).
     desc = _desc(q, scale, out, _precision(precision, q.dtype))
@@ -504,6 +570,7 @@ def _backward_into(q, k, v, out, lse, dout, tiles, tiles_t, scale, dq, dk, dv, p
                                        dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ds.data_ptr(), ds.numel(),
                                        *_ws_args(ws), main.cuda_stream))
     return
+  tl, tlt = base.launch_list(desc), base_t.launch_list(desc)
   ws_q, ws_kv = workspace(desc, q.device, tl), workspace(desc, q.device, tlt)
   nat.check(L.fwn_attn_bwd_delta_launch(desc, out.data_ptr(), dout.data_ptr(), delta.data_ptr(), main.cuda_stream))
   side = _side_stream(q.device)

@@ -130,8 +130,19 @@ typedef struct fwn_tiles {
   int32_t work_pairs;       /* batch * heads the order table was built for (launches of another
                                shape are refused); the table must come from this `items` array
                                (the launchers check its size, not its entries) */
-  int32_t reserved;         /* 0 */
+  int32_t flags;            /* 0, or FWN_TILES_NODES: the list has the member below */
+  const int32_t* node;      /* read with FWN_TILES_NODES only: [n_blocks * 128], the node (row of q,
+                               k, v, o, lse, ...) at each position of the list's own order, n for
+                               positions past the last (fwn_tiles_node_order, fwn_tiles_permute_*).
+                               The list describes mask[node][:, node]; the tensors stay in node
+                               order and the kernels address their rows through this table. Every
+                               entry below n must appear once (the launchers check n < 2^24, not
+                               the entries; an entry out of range reads zeros and stores nothing) */
 } fwn_tiles;
+
+/* fwn_tiles.flags: the list is laid out in an order of its own (member `node`). Without it the
+ * structure may end before that member. */
+#define FWN_TILES_NODES 1
 
 /* Thread-local message of the last failure on this thread ("" if none). */
 const char* fwn_last_error(void);
@@ -177,6 +188,24 @@ int fwn_tiles_fill(int32_t n_rows, int32_t n_cols, const int64_t* row_ptr, const
 int fwn_tiles_prepare(int32_t n_blocks, int32_t n_tiles, int32_t n_cols, const int32_t* tile_ptr,
                       const int32_t* tile_col, const uint32_t* tile_bits, uint64_t* lanes,
                       uint32_t* groups, uint32_t* halves);
+
+/* A locality order of the nodes of a canonical tile list (n rows = n columns): perm[p] is the node
+ * at position p. Built from the mask alone: breadth-first distances to a few far-apart nodes,
+ * averaged over each node's neighbourhood, then recursive bisection along the principal axis in
+ * runs of whole 128-row blocks. The kernels compute whole 32 x 32 groups, so a list laid out in a
+ * compact order has fewer of them to compute; the reference gets the same effect from the nodes'
+ * latitudes and longitudes (pallas_attn.py:71-82), which the op does not see. A heuristic: for a
+ * mask without locality the order may be no better than the given one. */
+int fwn_tiles_node_order(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
+                         int64_t* perm);
+
+/* Canonical tile list of mask[perm][:, perm] from the mask's own canonical list. Two passes:
+ * fwn_tiles_permute_count writes new_ptr[n_blocks + 1], fwn_tiles_permute_fill
+ * new_col[new_ptr[last]] and new_bits[new_ptr[last] * 128 * 4]. */
+int fwn_tiles_permute_count(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
+                            const int64_t* perm, int32_t* new_ptr);
+int fwn_tiles_permute_fill(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
+                           const int64_t* perm, const int32_t* new_ptr, int32_t* new_col, uint32_t* new_bits);
 
 /* Work items of a tile list: the tiles of each block are cut into ceil(count / max_item_tiles)
  * runs of near-equal length (max_item_tiles <= 0 selects FWN_ITEM_TILES). The reference runs one
