@@ -560,7 +560,7 @@ def attention(args):
   sp = stream.cuda_stream
   # The list the kernels walk, as the package picks it: the mask in a node order of the list's own
   # where that has less to compute, else the given order's.
-  walked = tiles.launch_list(fdesc)
+  walked = tiles.launch_list()
   # The schedule of each kernel (with --order auto, its order table): the forward's, dQ's and
   # dK/dV's (the list is its own transpose); the recomputing kernels take the native descriptor.
   sched = lambda d, kernel: (walked.struct_for_desc(d, kernel) if args.order == "auto" else

@@ -184,7 +184,8 @@ uint64_t workspace_bytes_for(const fwn_attn_desc* d, const fwn_tiles* t) {
 int split_to_slot(const fwn_attn_desc* d, const fwn_tiles* t, void* ws, int slot, const void* x, int64_t sb,
                   int64_t sn, int64_t sh, hipStream_t stream, const uint16_t** out) {
   uint16_t* dst = (uint16_t*)((char*)ws + round256(partial_bytes(d, t)) + (uint64_t)slot * round256(split_bytes(d)));
-  if (hipError_t e = launch_split_x3((const float*)x, sb, sn, sh, d->batch, d->n, d->heads, d->head_dim, dst, stream);
+  if (hipError_t e = launch_split_x3((const float*)x, sb, sn, sh, d->batch, d->n, d->heads, d->head_dim,
+                                     t->flags & FWN_TILES_NODES ? t->node : nullptr, dst, stream);
       e != hipSuccess)
     return fail(FWN_ERR_HIP, "bf16x3 split launch: %s", hipGetErrorString(e));
   *out = dst;
@@ -513,6 +514,13 @@ int fwn_attn_bwd_ds_launch(const fwn_attn_desc* desc, const void* q, const void*
                            const void* dout, const float* lse, float* delta, const fwn_tiles* tiles,
                            const fwn_tiles* tiles_t, const fwn_ds_map* map, void* dq, void* dk, void* dv, void* ds,
                            uint64_t ds_bytes, void* workspace, uint64_t workspace_bytes, void* stream) {
+  // The dS units are numbered by the positions of both lists: one order.
+  if (tiles && tiles_t && tiles != tiles_t) {
+    clear_error();
+    const int32_t* n0 = tiles->flags & FWN_TILES_NODES ? tiles->node : nullptr;
+    const int32_t* n1 = tiles_t->flags & FWN_TILES_NODES ? tiles_t->node : nullptr;
+    if (n0 != n1) return fail(FWN_ERR_TILES, "tiles and tiles_t have different node tables");
+  }
   if (int rc = fwn_attn_bwd_delta_launch(desc, o, dout, delta, stream)) return rc;
   if (int rc = fwn_attn_bwd_dkv_ds_launch(desc, q, k, v, dout, lse, delta, tiles_t ? tiles_t : tiles, map, dk, dv,
                                           ds, ds_bytes, workspace, workspace_bytes, stream))

@@ -85,7 +85,7 @@ __global__ void __launch_bounds__(NT, 2) fwd_kernel(KArgs a) {
     gnext = tile_groups(a, t0);
     if constexpr (G) {
       uint32_t nd[TileDma<D>::OPS];
-      dma.nodes(nd, a.node, kb);
+      dma.nodes(nd, node_block(a, kb));
       dma.gather(rK, K, w, nd, snb);
       if (w == 0 && t0 + 1 < t1) tab.load((t0 + 1) & 1, ((ci32_ptr)a.col)[t0 + 1], lane);
       wait_vmem();  // K(t0), its mask and group bits, the Q fragment and the nodes of tile t0 + 1
@@ -260,7 +260,7 @@ __global__ void __launch_bounds__(NT, 2) dq_kernel(KArgs a) {
     hcur = tile_halves(a, t0);
     if constexpr (G) {
       uint32_t nd[TileDma<D>::OPS];
-      dma.nodes(nd, a.node, kb);
+      dma.nodes(nd, node_block(a, kb));
       dma.gather(rK, K, w, nd, snb, 3u);
       dma.gather(rV, V, w, nd, snb, 3u);
       if (w == 0) tab.load(t0 & 1, kb, lane);
@@ -495,7 +495,7 @@ __global__ void __launch_bounds__(NT, 2) dq_ds_kernel(KArgs a) {
     uint32_t nd[TileDma<D>::OPS];
     if constexpr (G) {
       if (slot < 0)
-        dma.nodes(nd, a.node, kb);
+        dma.nodes(nd, node_block(a, kb));
       else
         dma.nodes(nd, tab.block(slot));
     }
@@ -871,7 +871,7 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
       uint32_t nd[TileDma<D, true>::OPS];
       if (mode != 2) {
         if (slot < 0)
-          dmaQ.nodes(nd, a.node, qb);
+          dmaQ.nodes(nd, node_block(a, qb));
         else
           dmaQ.nodes(nd, tab.block(slot));
       }
@@ -891,7 +891,7 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const uint32_t at = 64u * h + lane;
-          const uint32_t vo = 4u * (slot < 0 ? (uint32_t)a.node[(int64_t)qb * BLK + at] : tab.block(slot)[at]);
+          const uint32_t vo = 4u * (slot < 0 ? (uint32_t)node_block(a, qb)[at] : tab.block(slot)[at]);
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rL, (__attribute__((address_space(3))) void*)(stats + 256 * h), 4,
                                                    (int)vo, 0, 0, 0);
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rD, (__attribute__((address_space(3))) void*)(stats + 1024 + 256 * h),

@@ -77,15 +77,12 @@ struct TileDma {
     voff = (uint32_t)row * snb + chunk;
   }
 
-  // With a node table: the nodes of this lane's rows of tile column block kb, from the table in
-  // global memory or from its 128 entries for the block in LDS.
-  __device__ __forceinline__ void nodes(uint32_t (&nd)[OPS], const int32_t* node, int kb) const {
+  // With a node table: the nodes of this lane's rows of a tile, from its column block's 128 entries
+  // (in global memory or in LDS).
+  template <typename Table>
+  __device__ __forceinline__ void nodes(uint32_t (&nd)[OPS], Table node) const {
 #pragma unroll
-    for (int op = 0; op < OPS; ++op) nd[op] = (uint32_t)node[(int64_t)kb * BLK + first + op * 4 * RPO];
-  }
-  __device__ __forceinline__ void nodes(uint32_t (&nd)[OPS], const __attribute__((address_space(3))) uint32_t* tab) const {
-#pragma unroll
-    for (int op = 0; op < OPS; ++op) nd[op] = tab[first + op * 4 * RPO];
+    for (int op = 0; op < OPS; ++op) nd[op] = (uint32_t)node[first + op * 4 * RPO];
   }
 
   // issue() of a tile whose rows are the given nodes.
@@ -119,25 +116,6 @@ struct TileDma {
                                                16, (int)vo, 0, 0, 0);
     }
   }
-};
-
-// The node table of the tiles being copied, two blocks of 128 entries in LDS: block `slot` is
-// loaded by one wave (lanes 0-31, 16 bytes each) a tile before the copies that read it.
-struct NodeTab {
-  typedef const __attribute__((address_space(3))) uint32_t* ptr;
-  lds_char* base;
-  rsrc_t r;
-
-  __device__ __forceinline__ void init(const KArgs& a, lds_char* lds) {
-    base = lds;
-    r = make_rsrc(a.node, (uint32_t)a.n_blocks * (BLK * 4));
-  }
-  __device__ __forceinline__ void load(int slot, int kb, int lane) const {
-    if (lane < 32)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(base + slot * (BLK * 4)), 16,
-                                               (kb * BLK + 4 * lane) * 4, 0, 0, 0);
-  }
-  __device__ __forceinline__ ptr block(int slot) const { return (ptr)(base + slot * (BLK * 4)); }
 };
 
 // Per-lane LDS byte offsets of the MFMA A operands.

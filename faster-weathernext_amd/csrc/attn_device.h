@@ -127,9 +127,35 @@ __device__ __forceinline__ int node_at(const KArgs& a, int pos) {
   return pos;
 }
 
+// The 128 node table entries of column block kb (a malformed list's blocks past the last read the
+// last one's).
+__device__ __forceinline__ const int32_t* node_block(const KArgs& a, int kb) {
+  const uint32_t last = (uint32_t)a.n_blocks - 1u;
+  return a.node + (int64_t)((uint32_t)kb < last ? (uint32_t)kb : last) * BLK;
+}
+
 // Byte offset of a row from a node table: node * stride, both below 2^24 (one v_mul_u32_u24 or
 // v_mad_u32_u24; a 32-bit product takes four times as long).
 __device__ __forceinline__ uint32_t row_bytes(uint32_t node, uint32_t stride) { return __umul24(node, stride); }
+
+// The node table of the tiles being copied, two blocks of 128 entries in LDS: block `slot` is
+// loaded by one wave (lanes 0-31, 16 bytes each) a tile before the copies that read it.
+struct NodeTab {
+  typedef const __attribute__((address_space(3))) uint32_t* ptr;
+  lds_char* base;
+  rsrc_t r;
+
+  __device__ __forceinline__ void init(const KArgs& a, lds_char* lds) {
+    base = lds;
+    r = make_rsrc(a.node, (uint32_t)a.n_blocks * (BLK * 4));
+  }
+  __device__ __forceinline__ void load(int slot, int kb, int lane) const {
+    if (lane < 32)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(base + slot * (BLK * 4)), 16,
+                                               (kb * BLK + 4 * lane) * 4, 0, 0, 0);
+  }
+  __device__ __forceinline__ ptr block(int slot) const { return (ptr)(base + slot * (BLK * 4)); }
+};
 
 // Without an order table, workgroups are dealt round-robin over the 8 XCDs, each with its own
 // L2. Jobs are ordered (batch, head) major, then work items in block order, and XCD x gets a

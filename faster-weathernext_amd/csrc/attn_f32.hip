@@ -7,6 +7,12 @@
 // needed. Tiles stream into LDS by LDS DMA, double-buffered: in 64-row halves for the backward
 // kernels (HalfDma), in 32-row key groups for the forward (GroupDma).
 //
+// Node tables (G): the rows of a list laid out in an order of its own are gathered by the same LDS
+// DMA instructions. The step-streamed kernels (forward, 16-key dK/dV) load the next step's nodes into
+// registers a step ahead, the tile-streamed ones the next tile's into LDS. Refinement-6 mesh, before
+// -> after: 8-hop 4x128 forward in mesh order 1.915 -> 0.675 ms (0.637 with the tensors themselves in
+// such an order); 32-hop Hilbert 6x128 forward + backward 18.39 -> 16.77 ms.
+//
 // Reference: pallas_attn.py:112-141 (forward), 161-215 (dQ, dK/dV), 274-311 (VJP driver).
 #include "attn_device.h"
 
@@ -84,14 +90,18 @@ struct HalfDma {
   static constexpr int R = 1024 / (D * 4);
   static constexpr int CPR = D / 4;
   static constexpr int NI = 64 / R;
-  uint32_t lo[2];
+  uint32_t lo[2];  // this lane's row and chunk of the source
+  uint32_t ch[2];  // the chunk alone (node tables)
+  uint32_t rl;     // the row alone: row kR + rl of the half
 
   __device__ __forceinline__ void init(int w, int lane, uint32_t snb, bool swizzle) {
-    const int rl = lane / CPR, pc = lane % CPR;
+    const int pc = lane % CPR;
+    rl = (uint32_t)(lane / CPR);
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
-      const int row = (w + 4 * m) * R + rl;  // same low bits for every h and every m of this parity
-      lo[m] = (uint32_t)rl * snb + (uint32_t)((swizzle ? pc ^ swz_row3(row) : pc) << 4);
+      const int row = (w + 4 * m) * R + (int)rl;  // same low bits for every h and every m of this parity
+      ch[m] = (uint32_t)((swizzle ? pc ^ swz_row3(row) : pc) << 4);
+      lo[m] = rl * snb + ch[m];
     }
   }
 
@@ -110,6 +120,25 @@ struct HalfDma {
                                                16, (int)src, 0, 0, 0);
     }
   }
+
+  // issue() through a node table: `node` holds the tile's 128 entries (in global memory or LDS).
+  template <typename Table>
+  __device__ __forceinline__ void gather(rsrc_t r, char* half, Table node, uint32_t snb, int w, int h,
+                                         uint32_t live) const {
+    uint32_t base = (uint32_t)(uintptr_t)half;
+    asm volatile("" : "+s"(base));
+    uint32_t nd[NI / 4];
+#pragma unroll
+    for (int m = 0; m < NI / 4; ++m) nd[m] = (uint32_t)node[64 * h + (w + 4 * m) * R + rl];
+#pragma unroll
+    for (int m = 0; m < NI / 4; ++m) {
+      const int k = w + 4 * m;
+      if (!(live >> (2 * h + ((k * R) >> 5)) & 1u)) continue;
+      const uint32_t src = row_bytes(nd[m], snb) + ch[m & 1];
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(uintptr_t)(base + 1024u * k),
+                                               16, (int)src, 0, 0, 0);
+    }
+  }
 };
 
 // ------------------------------------------------------------------------------------------
@@ -122,14 +151,17 @@ struct GroupDma {
   static constexpr int R = 1024 / (D * 4);
   static constexpr int CPR = D / 4;
   static constexpr int NI = 32 / R;
-  uint32_t lo[2];
+  static constexpr int OPS = NI / 4;
+  uint32_t lo[2], ch[2], rl;  // as HalfDma
 
   __device__ __forceinline__ void init(int w, int lane, uint32_t snb, bool swizzle) {
-    const int rl = lane / CPR, pc = lane % CPR;
+    const int pc = lane % CPR;
+    rl = (uint32_t)(lane / CPR);
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
-      const int row = (w + 4 * m) * R + rl;
-      lo[m] = (uint32_t)rl * snb + (uint32_t)((swizzle ? pc ^ swz_row3(row) : pc) << 4);
+      const int row = (w + 4 * m) * R + (int)rl;
+      ch[m] = (uint32_t)((swizzle ? pc ^ swz_row3(row) : pc) << 4);
+      lo[m] = rl * snb + ch[m];
     }
   }
 
@@ -146,13 +178,29 @@ struct GroupDma {
                                                16, (int)src, 0, 0, 0);
     }
   }
+
+  // The nodes of this lane's rows of a group, from its 32 node table entries, and issue() of those
+  // rows.
+  __device__ __forceinline__ void nodes(uint32_t (&nd)[OPS], const int32_t* node, int w) const {
+#pragma unroll
+    for (int m = 0; m < OPS; ++m) nd[m] = (uint32_t)node[(w + 4 * m) * R + rl];
+  }
+  __device__ __forceinline__ void gather(rsrc_t r, char* buf, const uint32_t (&nd)[OPS], uint32_t snb, int w) const {
+    uint32_t base = (uint32_t)(uintptr_t)buf;
+    asm volatile("" : "+s"(base));
+#pragma unroll
+    for (int m = 0; m < OPS; ++m)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          r, (__attribute__((address_space(3))) void*)(uintptr_t)(base + 1024u * (w + 4 * m)), 16,
+          (int)(row_bytes(nd[m], snb) + ch[m & 1]), 0, 0, 0);
+  }
 };
 
 // Forward, fp32, two workgroups per CU, streamed by 32-key group: the work item's steps are its
 // (tile, key group) pairs in which some wave has a valid element; each step's K and V rows (32 KB
 // at D = 128) go into one of two group buffers, the copy of step s + 1 running while step s is
 // computed, one barrier per step. Groups no wave needs cost neither a copy nor a barrier.
-template <int D>
+template <int D, bool G>
 __global__ void __launch_bounds__(NT, 2) fwd_f32g_kernel(KArgs a) {
   constexpr int GB = 32 * D * 4;  // bytes of 32 rows of K or V
   __shared__ __attribute__((aligned(1024))) char gb0[2 * GB];  // K group (swizzled) | V group (plain)
@@ -165,7 +213,7 @@ __global__ void __launch_bounds__(NT, 2) fwd_f32g_kernel(KArgs a) {
   const uint32_t snb = (uint32_t)a.sn * 4;
   const rsrc_t rK = make_rsrc((const float*)a.k + j.base, a.slice_bytes);
   const rsrc_t rV = make_rsrc((const float*)a.v + j.base, a.slice_bytes);
-  const int qrow = j.blk * BLK + 32 * w + i;
+  const int qrow = node_at<G>(a, j.blk * BLK + 32 * w + i);
   f32x4 qf[D / 8];
   load_frag_f32<D>(qf, make_rsrc((const float*)a.q + j.base, a.slice_bytes), qrow, snb, g);
   F32Offsets<D> off;
@@ -226,26 +274,44 @@ __global__ void __launch_bounds__(NT, 2) fwd_f32g_kernel(KArgs a) {
     rem &= rem - 1u;
     return true;
   };
-  auto copy = [&](char* gb, int t, int c) {
-    const int row0 = ((ci32_ptr)a.col)[t] * BLK + 32 * c;
-    dmaK.issue(rK, gb, row0, snb, w);
-    dmaV.issue(rV, gb + GB, row0, snb, w);
+  auto pos0 = [&](int t, int c) { return ((ci32_ptr)a.col)[t] * BLK + 32 * c; };
+  auto nodes_of = [&](int t, int c) { return node_block(a, ((ci32_ptr)a.col)[t]) + 32 * c; };
+  // The K and V rows of step (t, c); with a node table, the rows of nodes nd.
+  auto copy = [&](char* gb, int t, int c, const uint32_t (&nd)[GroupDma<D>::OPS]) {
+    if constexpr (G) {
+      dmaK.gather(rK, gb, nd, snb, w);
+      dmaV.gather(rV, gb + GB, nd, snb, w);
+    } else {
+      dmaK.issue(rK, gb, pos0(t, c), snb, w);
+      dmaV.issue(rV, gb + GB, pos0(t, c), snb, w);
+    }
   };
-  int tc = 0, cc = 0, tn = 0, cn = 0;
-  bool vc = take(tc, cc), vn = false;
+  int tc = 0, cc = 0, tn = 0, cn = 0, tm = 0, cm = 0;
+  bool vc = take(tc, cc), vn = false, vm = false;
   u32x2 mbc = {0u, 0u}, mbn = {0u, 0u};
+  uint32_t ndA[GroupDma<D>::OPS], ndB[GroupDma<D>::OPS];
   if (vc) {
-    copy(gb0, tc, cc);
+    if constexpr (G) dmaK.nodes(ndA, nodes_of(tc, cc), w);
+    copy(gb0, tc, cc, ndA);
     mbc = tile_bits(a, tc, w, lane);
     vn = take(tn, cn);
+    if constexpr (G) {
+      if (vn) dmaK.nodes(ndA, nodes_of(tn, cn), w);
+      vm = vn && take(tm, cm);
+    }
   }
-  // One step: step (tc, cc) is in `cur`; the copy of step (tn, cn) goes into `nxt`.
-  auto step = [&](char* cur, char* nxt) {
-    wait_vmem();      // this wave's part of the current step (and its mask bits)
+  // One step: step (tc, cc) is in `cur`; the copy of step (tn, cn) goes into `nxt`. With a node table
+  // the rows of step (tn, cn) are in nd, loaded a step ago, and those of step (tm, cm) go into
+  // ndnext.
+  auto step = [&](char* cur, char* nxt, const uint32_t (&nd)[GroupDma<D>::OPS], uint32_t (&ndnext)[GroupDma<D>::OPS]) {
+    wait_vmem();      // this wave's part of the current step (its mask bits, the next step's nodes)
     __syncthreads();  // the step landed; every wave is done with the previous step's buffer
     if (vn) {
-      copy(nxt, tn, cn);
+      copy(nxt, tn, cn, nd);
       mbn = tn != tc ? tile_bits(a, tn, w, lane) : mbc;
+      if constexpr (G) {
+        if (vm) dmaK.nodes(ndnext, nodes_of(tm, cm), w);
+      }
     }
     const uint32_t live = tile_groups(a, tc) >> (4 * w) & 15u;
     if (live >> cc & 1u) group(cc, cur, mbc, tile_halves(a, tc) >> (8 * w + 2 * cc) & 3u);
@@ -253,12 +319,19 @@ __global__ void __launch_bounds__(NT, 2) fwd_f32g_kernel(KArgs a) {
     cc = cn;
     mbc = mbn;
     vc = vn;
-    vn = vc && take(tn, cn);
+    if constexpr (G) {
+      tn = tm;
+      cn = cm;
+      vn = vm;
+      vm = vn && take(tm, cm);
+    } else {
+      vn = vc && take(tn, cn);
+    }
   };
   while (vc) {
-    step(gb0, gb1);
+    step(gb0, gb1, ndA, ndB);
     if (!vc) break;
-    step(gb1, gb0);
+    step(gb1, gb0, ndB, ndA);
   }
   const float ltot = st.l + __shfl_xor(st.l, 32);
   if (j.part >= 0) {
@@ -273,11 +346,12 @@ __global__ void __launch_bounds__(NT, 2) fwd_f32g_kernel(KArgs a) {
 // dQ, fp32. The tile's K and V rows stream in halves (rows 0-63, 64-127) through two half
 // buffers: the copy of one half runs while the other is computed. Two barriers per tile.
 
-template <int D>
+template <int D, bool G>
 __global__ void __launch_bounds__(NT, 1) dq_f32_kernel(KArgs a) {
   constexpr int HB = 64 * D * 4;  // bytes of 64 rows of K or V
   __shared__ __attribute__((aligned(1024))) char h0[2 * HB];  // rows 0-63: K | V
   __shared__ __attribute__((aligned(1024))) char h1[2 * HB];  // rows 64-127: K | V
+  __shared__ __attribute__((aligned(16))) char lnode[G ? 2 * 4 * BLK : 16];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 31, g = lane >> 5;
@@ -287,12 +361,12 @@ __global__ void __launch_bounds__(NT, 1) dq_f32_kernel(KArgs a) {
   const rsrc_t rK = make_rsrc((const float*)a.k + j.base, a.slice_bytes);
   const rsrc_t rV = make_rsrc((const float*)a.v + j.base, a.slice_bytes);
 
-  const int qrow = j.blk * BLK + 32 * w + i;
+  const int qrow = node_at<G>(a, j.blk * BLK + 32 * w + i);
   f32x4 qf[D / 8], df[D / 8];
   load_frag_f32<D>(qf, make_rsrc((const float*)a.q + j.base, a.slice_bytes), qrow, snb, g);
   load_frag_f32<D>(df, make_rsrc((const float*)a.dout + j.obase, a.oslice_bytes), qrow, (uint32_t)a.osn * 4, g);
   float lse_t = 0.f, delta = 0.f;
-  if (qrow < a.n) {
+  if ((unsigned)qrow < (unsigned)a.n) {
     lse_t = a.lse[stat_index(a, j, qrow)] * LOG2E;
     delta = a.delta[stat_index(a, j, qrow)];
   }
@@ -300,6 +374,18 @@ __global__ void __launch_bounds__(NT, 1) dq_f32_kernel(KArgs a) {
   off.init(i, g);
   HalfDma<D> dma;
   dma.init(w, lane, snb, true);
+  NodeTab tab;
+  if constexpr (G) tab.init(a, (lds_char*)lnode);
+  // Half h of key block kb's K and V rows (its nodes: LDS block `slot`).
+  auto copy_half = [&](char* hb, int kb, int slot, int h, uint32_t live) {
+    if constexpr (G) {
+      dma.gather(rK, hb, tab.block(slot), snb, w, h, live);
+      dma.gather(rV, hb + HB, tab.block(slot), snb, w, h, live);
+    } else {
+      dma.issue(rK, hb, kb * BLK, snb, w, h, live);
+      dma.issue(rV, hb + HB, kb * BLK, snb, w, h, live);
+    }
+  };
   f32x16 acc[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) acc[db] = zero16();
@@ -346,8 +432,13 @@ __global__ void __launch_bounds__(NT, 1) dq_f32_kernel(KArgs a) {
   if (t0 < t1) {
     gcur = tile_groups(a, t0);
     const int kb = ((ci32_ptr)a.col)[t0];
-    dma.issue(rK, h0, kb * BLK, snb, w, 0, any_rows(gcur));
-    dma.issue(rV, h0 + HB, kb * BLK, snb, w, 0, any_rows(gcur));
+    if constexpr (G) {
+      dma.gather(rK, h0, node_block(a, kb), snb, w, 0, any_rows(gcur));
+      dma.gather(rV, h0 + HB, node_block(a, kb), snb, w, 0, any_rows(gcur));
+      if (w == 0) tab.load(t0 & 1, kb, lane);
+    } else {
+      copy_half(h0, kb, 0, 0, any_rows(gcur));
+    }
   }
   for (int tt = t0; tt < t1; ++tt) {
     const int t = __builtin_amdgcn_readfirstlane(tt);
@@ -357,8 +448,11 @@ __global__ void __launch_bounds__(NT, 1) dq_f32_kernel(KArgs a) {
     const uint32_t live = gt >> (4 * w) & 15u;  // key groups with p = 0 throughout are skipped
     wait_vmem();      // this wave's part of half 0 of tile t, and the mask bits
     __syncthreads();  // half 0 landed; every wave is done with half 1 of tile t - 1
-    dma.issue(rK, h1, kb * BLK, snb, w, 1, any_rows(gt));
-    dma.issue(rV, h1 + HB, kb * BLK, snb, w, 1, any_rows(gt));
+    copy_half(h1, kb, t & 1, 1, any_rows(gt));
+    // The nodes of tile t + 1 go where tile t - 1's were (last read before this barrier).
+    if constexpr (G) {
+      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, ((ci32_ptr)a.col)[t + 1], lane);
+    }
     if (t + 1 < t1) gcur = tile_groups(a, t + 1);
     // Fenced, so that one group's reads and MFMAs do not overlap the next group's registers.
     __builtin_amdgcn_sched_barrier(0);
@@ -369,9 +463,7 @@ __global__ void __launch_bounds__(NT, 1) dq_f32_kernel(KArgs a) {
     wait_vmem();      // this wave's part of half 1
     __syncthreads();  // half 1 landed; every wave is done with half 0
     if (t + 1 < t1) {
-      const int kbn = ((ci32_ptr)a.col)[t + 1];
-      dma.issue(rK, h0, kbn * BLK, snb, w, 0, any_rows(gcur));
-      dma.issue(rV, h0 + HB, kbn * BLK, snb, w, 0, any_rows(gcur));
+      copy_half(h0, ((ci32_ptr)a.col)[t + 1], (t + 1) & 1, 0, any_rows(gcur));
     }
     __builtin_amdgcn_sched_barrier(0);
     if (live & 4u) group(2, 0, h1, h1 + HB, mb);
@@ -398,11 +490,12 @@ __global__ void __launch_bounds__(NT, 1) dq_f32_kernel(KArgs a) {
 // K rows stream in halves through two half buffers (32 KB each at D = 128), two workgroups per
 // CU. A half's units are loaded together with its K rows, so the barrier that publishes the rows
 // also covers the units.
-template <int D>
+template <int D, bool G>
 __global__ void __launch_bounds__(NT, 2) dq_f32_ds_kernel(KArgs a) {
   constexpr int HB = 64 * D * 4;  // bytes of 64 rows of K
   __shared__ __attribute__((aligned(1024))) char h0[HB];  // rows 0-63
   __shared__ __attribute__((aligned(1024))) char h1[HB];  // rows 64-127
+  __shared__ __attribute__((aligned(16))) char lnode[G ? 2 * 4 * BLK : 16];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 31, g = lane >> 5;
@@ -411,11 +504,21 @@ __global__ void __launch_bounds__(NT, 2) dq_f32_ds_kernel(KArgs a) {
   const uint32_t snb = (uint32_t)a.sn * 4;
   const rsrc_t rK = make_rsrc((const float*)a.k + j.base, a.slice_bytes);
   const rsrc_t rS = make_rsrc((const float*)a.ds + (int64_t)j.bh * (a.ds_slice_bytes >> 2), a.ds_slice_bytes);
-  const int qrow = j.blk * BLK + 32 * w + i;
+  const int qrow = node_at<G>(a, j.blk * BLK + 32 * w + i);
   F32Offsets<D> off;
   off.init(i, g);
   HalfDma<D> dma;
   dma.init(w, lane, snb, true);
+  NodeTab tab;
+  if constexpr (G) tab.init(a, (lds_char*)lnode);
+  // Half h of key block kb's rows (its nodes: LDS block `slot`).
+  auto copy_half = [&](char* hb, int kb, int slot, int h, uint32_t live) {
+    if constexpr (G) {
+      dma.gather(rK, hb, tab.block(slot), snb, w, h, live);
+    } else {
+      dma.issue(rK, hb, kb * BLK, snb, w, h, live);
+    }
+  };
   f32x16 acc[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) acc[db] = zero16();
@@ -470,7 +573,13 @@ __global__ void __launch_bounds__(NT, 2) dq_f32_ds_kernel(KArgs a) {
   if (t0 < t1) {
     gcur = tile_groups(a, t0);
     ucur = (uint32_t)((cmap_ptr)a.ubase)[t0];
-    dma.issue(rK, h0, ((ci32_ptr)a.col)[t0] * BLK, snb, w, 0, any_rows(gcur));
+    const int kb = ((ci32_ptr)a.col)[t0];
+    if constexpr (G) {
+      dma.gather(rK, h0, node_block(a, kb), snb, w, 0, any_rows(gcur));
+      if (w == 0) tab.load(t0 & 1, kb, lane);
+    } else {
+      copy_half(h0, kb, 0, 0, any_rows(gcur));
+    }
     load_units(dsA, gcur, ucur, 0);
   }
   for (int tt = t0; tt < t1; ++tt) {
@@ -481,7 +590,11 @@ __global__ void __launch_bounds__(NT, 2) dq_f32_ds_kernel(KArgs a) {
     const uint32_t hw = tile_halves(a, t) >> (8 * w) & 0xffu;  // bit 2 sb + h: live 16-key halves
     wait_vmem();      // this wave's part of half 0 of tile t and its units
     __syncthreads();  // half 0 landed; every wave is done with half 1 of tile t - 1
-    dma.issue(rK, h1, kb * BLK, snb, w, 1, any_rows(gt));
+    copy_half(h1, kb, t & 1, 1, any_rows(gt));
+    // The nodes of tile t + 1 go where tile t - 1's were (last read before this barrier).
+    if constexpr (G) {
+      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, ((ci32_ptr)a.col)[t + 1], lane);
+    }
     load_units(dsB, gt, ut, 1);
     if (t + 1 < t1) {
       gcur = tile_groups(a, t + 1);
@@ -495,7 +608,7 @@ __global__ void __launch_bounds__(NT, 2) dq_f32_ds_kernel(KArgs a) {
     wait_vmem();      // this wave's part of half 1 and its units
     __syncthreads();  // half 1 landed; every wave is done with half 0
     if (t + 1 < t1) {
-      dma.issue(rK, h0, ((ci32_ptr)a.col)[t + 1] * BLK, snb, w, 0, any_rows(gcur));
+      copy_half(h0, ((ci32_ptr)a.col)[t + 1], (t + 1) & 1, 0, any_rows(gcur));
       load_units(dsA, gcur, ucur, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -521,12 +634,13 @@ __global__ void __launch_bounds__(NT, 2) dq_f32_ds_kernel(KArgs a) {
 // has a per-lane offset fixed at the start plus an immediate per register. Units are numbered
 // over the forward list by the rank of group bit 4 sb + w (query group sb, key group w) in the
 // forward tile's group word; tmap gives that word and the tile's first unit.
-template <int D, bool DS = false>
+template <int D, bool DS, bool G>
 __global__ void __launch_bounds__(NT, 1) dkv_f32_kernel(KArgs a) {
   constexpr int HB = 64 * D * 4;  // bytes of 64 rows of Q or dO
   // rows 0-63 (h0) and 64-127 (h1): Q | dO | lse * log2(e) [64] | delta [64]
   __shared__ __attribute__((aligned(1024))) char h0[2 * HB + 512];
   __shared__ __attribute__((aligned(1024))) char h1[2 * HB + 512];
+  __shared__ __attribute__((aligned(16))) char lnode[G ? 2 * 4 * BLK : 16];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 31, g = lane >> 5;
@@ -539,7 +653,7 @@ __global__ void __launch_bounds__(NT, 1) dkv_f32_kernel(KArgs a) {
   const rsrc_t rL = make_rsrc(a.lse + stat_index(a, j, 0), (uint32_t)a.n * 4);
   const rsrc_t rD = make_rsrc(a.delta + stat_index(a, j, 0), (uint32_t)a.n * 4);
 
-  const int krow = j.blk * BLK + 32 * w + i;
+  const int krow = node_at<G>(a, j.blk * BLK + 32 * w + i);
   f32x4 kf[D / 8], vf[D / 8];
   load_frag_f32<D>(kf, make_rsrc((const float*)a.k + j.base, a.slice_bytes), krow, snb, g);
   load_frag_f32<D>(vf, make_rsrc((const float*)a.v + j.base, a.slice_bytes), krow, snb, g);
@@ -568,13 +682,29 @@ __global__ void __launch_bounds__(NT, 1) dkv_f32_kernel(KArgs a) {
 
   // Half h of query block qb: the Q and dO rows (live groups only) and, by wave 0, the 64 rows'
   // lse and delta (4 bytes per lane; rows past n read zeros).
-  auto copy_half = [&](char* hb, int qb, int h, uint32_t live) {
-    dmaQ.issue(rQ, hb, qb * BLK, snb, w, h, live);
-    dmaO.issue(rO, hb + HB, qb * BLK, osnb, w, h, live);
+  // With a node table: the rows of the nodes in `node` (the block's 128 entries, in LDS or global
+  // memory).
+  NodeTab tab;
+  if constexpr (G) tab.init(a, (lds_char*)lnode);
+  auto copy_stats = [&](char* hb, int row) {
     if (w == 0) {
-      const int so = (qb * BLK + 64 * h + lane) * 4;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rL, (__attribute__((address_space(3))) void*)(hb + 2 * HB), 4, so, 0, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rD, (__attribute__((address_space(3))) void*)(hb + 2 * HB + 256), 4, so, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rL, (__attribute__((address_space(3))) void*)(hb + 2 * HB), 4, row * 4, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rD, (__attribute__((address_space(3))) void*)(hb + 2 * HB + 256), 4, row * 4, 0, 0, 0);
+    }
+  };
+  auto gather_half = [&](char* hb, auto node, int h, uint32_t live) {
+    const int row = w == 0 ? (int)node[64 * h + lane] : 0;
+    dmaQ.gather(rQ, hb, node, snb, w, h, live);
+    dmaO.gather(rO, hb + HB, node, osnb, w, h, live);
+    copy_stats(hb, row);
+  };
+  auto copy_half = [&](char* hb, int qb, int slot, int h, uint32_t live) {
+    if constexpr (G) {
+      gather_half(hb, tab.block(slot), h, live);
+    } else {
+      dmaQ.issue(rQ, hb, qb * BLK, snb, w, h, live);
+      dmaO.issue(rO, hb + HB, qb * BLK, osnb, w, h, live);
+      copy_stats(hb, qb * BLK + 64 * h + lane);
     }
   };
   // After the copy of a half landed: lse -> lse * log2(e), the form the exponent takes.
@@ -649,7 +779,13 @@ __global__ void __launch_bounds__(NT, 1) dkv_f32_kernel(KArgs a) {
   uint32_t gcur = 0u;
   if (t0 < t1) {
     gcur = tile_groups(a, t0);
-    copy_half(h0, ((ci32_ptr)a.col)[t0], 0, any_rows(gcur));
+    const int qb = ((ci32_ptr)a.col)[t0];
+    if constexpr (G) {
+      gather_half(h0, node_block(a, qb), 0, any_rows(gcur));
+      if (w == 0) tab.load(t0 & 1, qb, lane);
+    } else {
+      copy_half(h0, qb, 0, 0, any_rows(gcur));
+    }
   }
   for (int tt = t0; tt < t1; ++tt) {
     const int t = __builtin_amdgcn_readfirstlane(tt);
@@ -664,7 +800,11 @@ __global__ void __launch_bounds__(NT, 1) dkv_f32_kernel(KArgs a) {
     wait_vmem();  // this wave's part of half 0 of tile t, and the mask bits
     scale_lse(h0);
     __syncthreads();  // half 0 landed; every wave is done with half 1 of tile t - 1
-    copy_half(h1, qb, 1, any_rows(gt));
+    copy_half(h1, qb, t & 1, 1, any_rows(gt));
+    // The nodes of tile t + 1 go where tile t - 1's were (last read before this barrier).
+    if constexpr (G) {
+      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, ((ci32_ptr)a.col)[t + 1], lane);
+    }
     if (t + 1 < t1) gcur = tile_groups(a, t + 1);
     // Fenced, so that one group's reads and MFMAs do not overlap the next group's registers.
     __builtin_amdgcn_sched_barrier(0);
@@ -675,7 +815,7 @@ __global__ void __launch_bounds__(NT, 1) dkv_f32_kernel(KArgs a) {
     wait_vmem();  // this wave's part of half 1
     scale_lse(h1);
     __syncthreads();  // half 1 landed; every wave is done with half 0
-    if (t + 1 < t1) copy_half(h0, ((ci32_ptr)a.col)[t + 1], 0, any_rows(gcur));
+    if (t + 1 < t1) copy_half(h0, ((ci32_ptr)a.col)[t + 1], (t + 1) & 1, 0, any_rows(gcur));
     __builtin_amdgcn_sched_barrier(0);
     if (live & 4u) group(2, 0, h1, mb);
     __builtin_amdgcn_sched_barrier(0);
@@ -725,7 +865,7 @@ __device__ __forceinline__ f32x4 mfma16f(float a, float b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-template <bool DS>
+template <bool DS, bool G>
 __global__ void __launch_bounds__(256, 2) dkv16_f32_kernel(KArgs a) {
   constexpr int D = 128;
   constexpr int RB = kRowPad;
@@ -759,7 +899,7 @@ __global__ void __launch_bounds__(256, 2) dkv16_f32_kernel(KArgs a) {
   const rsrc_t rD = make_rsrc(a.delta + stat_index(a, j, 0), (uint32_t)a.n * 4);
   const rsrc_t rS = make_rsrc(DS ? (const void*)(a.ds + (int64_t)j.bh * (a.ds_slice_bytes >> 1)) : (const void*)a.q,
                               DS ? a.ds_slice_bytes : 0u);
-  const int krow = j.blk * BLK + 16 * kg + t16;
+  const int krow = node_at<G>(a, j.blk * BLK + 16 * kg + t16);
   // K and V of this lane's key: kf[u][e] = column 32 g + 4 u + e (k-step 4 u + e).
   f32x4 kf[8], vf[8];
   {
@@ -906,25 +1046,34 @@ __global__ void __launch_bounds__(256, 2) dkv16_f32_kernel(KArgs a) {
     rem &= rem - 1u;
     return true;
   };
-  // Rows row0 .. row0 + 31 of Q (plane 0) and dO (plane 1), one padded row per instruction: wave w
-  // copies rows w + 4 m' of both planes with lanes 0-31 (16 bytes each); then, by wave 0, the
-  // group's lse and delta (rows past n read zeros).
-  auto copy = [&](lds_char* buf, int t, int c) {
-    const int row0 = ((ci32_ptr)a.col)[t] * BLK + 32 * c;
+  auto pos0 = [&](int t, int c) { return ((ci32_ptr)a.col)[t] * BLK + 32 * c; };
+  // The tensors' row at position lane % 32 of step (t, c): a node, loaded a step before its copy.
+  auto lane_row = [&](int t, int c) {
+    if constexpr (G) return node_block(a, ((ci32_ptr)a.col)[t])[32 * c + (lane & 31)];
+    return pos0(t, c) + (lane & 31);
+  };
+  // Step (t, c)'s rows of Q (plane 0) and dO (plane 1), one padded row per instruction: wave w copies
+  // rows w + 4 m' of both planes with lanes 0-31 (16 bytes each); then, by wave 0, the group's lse and
+  // delta (rows past n read zeros). `lrow` is the step's lane_row.
+  auto copy = [&](lds_char* buf, int t, int c, int lrow) {
     uint32_t base = (uint32_t)(uintptr_t)buf;
     asm volatile("" : "+s"(base));
+    const int row0 = G ? 0 : pos0(t, c);
+    int rows[8];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) rows[m] = G ? __builtin_amdgcn_readlane(lrow, wid + 4 * m) : row0 + wid + 4 * m;
     if (lane < 32) {
 #pragma unroll
       for (int m = 0; m < 16; ++m) {
         const int plane = m >> 3, row = wid + 4 * (m & 7);
-        const uint32_t src = (uint32_t)(row0 + row) * (plane ? osnb : snb) + (uint32_t)(16 * lane);
+        const uint32_t src = (uint32_t)rows[m & 7] * (plane ? osnb : snb) + (uint32_t)(16 * lane);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             plane ? rO : rQ, (__attribute__((address_space(3))) void*)(uintptr_t)(base + (uint32_t)(plane * PB + row * RB)),
             16, (int)src, 0, 0, 0);
       }
     }
     if (wid == 0) {
-      const int so = lane < 32 ? (row0 + lane) * 4 : (int)kPastEndF;
+      const int so = lane < 32 ? (G ? lrow : row0 + lane) * 4 : (int)kPastEndF;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rL, (__attribute__((address_space(3))) void*)(buf + SB), 4, so, 0, 0, 0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rD, (__attribute__((address_space(3))) void*)(buf + SB + 256), 4, so, 0,
                                                0, 0);
@@ -932,13 +1081,18 @@ __global__ void __launch_bounds__(256, 2) dkv16_f32_kernel(KArgs a) {
   };
   lds_char* b0 = (lds_char*)gb0;
   lds_char* b1 = (lds_char*)gb1;
-  int tc = 0, cc = 0, tn = 0, cn = 0;
-  bool vc = take(tc, cc), vn = false;
+  int tc = 0, cc = 0, tn = 0, cn = 0, tm = 0, cm = 0;
+  bool vc = take(tc, cc), vn = false, vm = false;
   uint64_t mwc = 0, mwn = 0;
+  int rown = 0, rowm = 0;  // lane rows of steps (tn, cn) and (tm, cm)
   if (vc) {
-    copy(b0, tc, cc);
+    copy(b0, tc, cc, lane_row(tc, cc));
     mwc = mword[(int64_t)tc * 256];
     vn = take(tn, cn);
+    if constexpr (G) {
+      if (vn) rown = lane_row(tn, cn);
+      vm = vn && take(tm, cm);
+    }
   }
   auto step = [&](lds_char* cur, lds_char* nxt) {
     wait_vmem();  // this wave's part of the current step (wave 0: the statistics) and its mask word
@@ -952,8 +1106,11 @@ __global__ void __launch_bounds__(256, 2) dkv16_f32_kernel(KArgs a) {
     }
     __syncthreads();  // the step landed; every wave is done with the previous step's buffer
     if (vn) {
-      copy(nxt, tn, cn);
+      copy(nxt, tn, cn, rown);
       mwn = tn != tc ? mword[(int64_t)tn * 256] : mwc;
+      if constexpr (G) {
+        if (vm) rowm = lane_row(tm, cm);
+      }
     }
     // The 16-query halves of group cc in which the wave's 16 keys have a valid element: some
     // lane's bits 16 cc + 8 m + r (shifted by 4 (g % 2)) are set.
@@ -983,7 +1140,15 @@ __global__ void __launch_bounds__(256, 2) dkv16_f32_kernel(KArgs a) {
     cc = cn;
     mwc = mwn;
     vc = vn;
-    vn = vc && take(tn, cn);
+    if constexpr (G) {
+      tn = tm;
+      cn = cm;
+      vn = vm;
+      rown = rowm;
+      vm = vn && take(tm, cm);
+    } else {
+      vn = vc && take(tn, cn);
+    }
   };
   while (vc) {
     step(b0, b1);
@@ -1072,31 +1237,36 @@ dim3 delta_grid(const KArgs& a) {
   return dim3((unsigned)(((int64_t)a.n + rows - 1) / rows * a.batch));
 }
 
-template <int D>
-hipError_t launch_d(Kind kind, const KArgs& a, hipStream_t stream) {
+template <int D, bool G>
+hipError_t launch_dg(Kind kind, const KArgs& a, hipStream_t stream) {
   const dim3 block(NT);
-  if (kind == Kind::kDelta) {
-    hipLaunchKernelGGL((delta_kernel<float, D>), (delta_grid<float, D>(a)), block, 0, stream, a);
-    return hipGetLastError();
-  }
   const dim3 grid((unsigned)job_count(a));
   // dkv16_f32_kernel: two workgroups per item, laid out in blocks of 16 ids (8 items x 2 halves).
   const dim3 grid2(16u * (((unsigned)job_count(a) + 7u) / 8u));
   switch (kind) {
-    case Kind::kFwd: hipLaunchKernelGGL(fwd_f32g_kernel<D>, grid, block, 0, stream, a); break;
-    case Kind::kDq: hipLaunchKernelGGL(dq_f32_kernel<D>, grid, block, 0, stream, a); break;
+    case Kind::kFwd: hipLaunchKernelGGL((fwd_f32g_kernel<D, G>), grid, block, 0, stream, a); break;
+    case Kind::kDq: hipLaunchKernelGGL((dq_f32_kernel<D, G>), grid, block, 0, stream, a); break;
     case Kind::kDkv:
-      if constexpr (D == 128) hipLaunchKernelGGL((dkv16_f32_kernel<false>), grid2, dim3(256), 0, stream, a);
-      else hipLaunchKernelGGL((dkv_f32_kernel<D, false>), grid, block, 0, stream, a);
+      if constexpr (D == 128) hipLaunchKernelGGL((dkv16_f32_kernel<false, G>), grid2, dim3(256), 0, stream, a);
+      else hipLaunchKernelGGL((dkv_f32_kernel<D, false, G>), grid, block, 0, stream, a);
       break;
     case Kind::kDkvDs:
-      if constexpr (D == 128) hipLaunchKernelGGL((dkv16_f32_kernel<true>), grid2, dim3(256), 0, stream, a);
-      else hipLaunchKernelGGL((dkv_f32_kernel<D, true>), grid, block, 0, stream, a);
+      if constexpr (D == 128) hipLaunchKernelGGL((dkv16_f32_kernel<true, G>), grid2, dim3(256), 0, stream, a);
+      else hipLaunchKernelGGL((dkv_f32_kernel<D, true, G>), grid, block, 0, stream, a);
       break;
-    case Kind::kDqDs: hipLaunchKernelGGL(dq_f32_ds_kernel<D>, grid, block, 0, stream, a); break;
+    case Kind::kDqDs: hipLaunchKernelGGL((dq_f32_ds_kernel<D, G>), grid, block, 0, stream, a); break;
     default: break;
   }
   return hipGetLastError();
+}
+
+template <int D>
+hipError_t launch_d(Kind kind, const KArgs& a, hipStream_t stream) {
+  if (kind == Kind::kDelta) {
+    hipLaunchKernelGGL((delta_kernel<float, D>), (delta_grid<float, D>(a)), dim3(NT), 0, stream, a);
+    return hipGetLastError();
+  }
+  return a.node ? launch_dg<D, true>(kind, a, stream) : launch_dg<D, false>(kind, a, stream);
 }
 
 template <int D>

@@ -33,7 +33,7 @@ struct KArgs {
   const int32_t* tmap;    // dK/dV writing dS: per transposed tile, (ubase, halves) of the forward tile
   uint32_t ds_slice_bytes;  // bytes of one (batch, head) slice of ds: n_units * 1024
   const uint16_t* xa;     // bf16x3 kernels: split operands, [batch * heads][n][2][head_dim] bf16 (hi row,
-  const uint16_t* xb;     //   lo row; written by the split pass): forward k, v; dK/dV q, dout; dQ k
+  const uint16_t* xb;     //   lo row; rows in the list's order; written by the split pass): forward k, v; dK/dV q, dout; dQ k
   uint32_t xslice_bytes;  // bytes of one (batch, head) slice of xa / xb: n * 4 * head_dim
   int32_t n, heads, batch, n_blocks, n_tiles, n_items, n_parts, n_split, n_order;
   int64_t sb, sn, sh;     // strides of q, k, v, dq, dk, dv
@@ -55,9 +55,10 @@ hipError_t launch_f32(Kind kind, int head_dim, const KArgs& a, hipStream_t strea
 hipError_t launch_delta_bf16(int head_dim, const KArgs& a, hipStream_t stream);      // attn_f32.hip
 hipError_t launch_x3(Kind kind, int head_dim, const KArgs& a, hipStream_t stream);    // attn_x3.hip: kFwd, kDkvDs, kDqDs
 // Splits a float32 [batch, n, heads, head_dim] tensor (element strides sb, sn, sh) into dst,
-// [batch * heads][n][2][head_dim] bf16: hi = bf16(x), lo = bf16(x - hi) (attn_x3.hip).
+// [batch * heads][n][2][head_dim] bf16: hi = bf16(x), lo = bf16(x - hi), rows in the order of the
+// node table `node` (NULL: node order) (attn_x3.hip).
 hipError_t launch_split_x3(const float* src, int64_t sb, int64_t sn, int64_t sh, int batch, int n, int heads,
-                           int head_dim, uint16_t* dst, hipStream_t stream);
+                           int head_dim, const int32_t* node, uint16_t* dst, hipStream_t stream);
 hipError_t launch_combine(Kind kind, int dtype, int head_dim, const KArgs& a,
                           hipStream_t stream);                                     // attn_combine.hip
 

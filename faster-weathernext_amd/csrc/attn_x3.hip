@@ -10,7 +10,10 @@
 // The operands that stream through LDS (forward: K, V; dK/dV: Q, dO; dQ: K) are split once per
 // call by split_x3_kernel into [batch * heads][n][2][D] bf16 (hi row, then lo row) and copied by
 // 32-row group; the operands a wave keeps in registers (forward: Q; dK/dV: its K and V rows) are
-// split when loaded; P and dS are split in registers.
+// split when loaded; P and dS are split in registers. A list laid out in a node order of its own gets
+// its streamed operands in that order from the split pass, so only the register rows, the statistics
+// and the outputs go through the node table (32-hop Hilbert 6x128 forward + backward at refinement
+// 6: 6.92 -> 6.35 ms against the given order).
 //
 // The backward is the dS exchange (5 contractions per tile): dK/dV computes S, dP, dV, dK and
 // writes each 32 x 32 dS group as hi and lo bf16 (4 KB, the float32 exchange's unit size and
@@ -30,17 +33,22 @@ struct SplitArgs {
   uint16_t* dst;
   int64_t sb, sn, sh;  // element strides of src
   int32_t batch, n, heads, d;
+  const int32_t* node;  // the row of src at each position of the list's own order, or NULL
 };
 
 // One thread per 8 consecutive elements of a row: 32 bytes read, 16 bytes of hi and 16 of lo
-// written. dst is [batch * heads][n][2][d]: (batch, head) slices of n split rows.
+// written. dst is [batch * heads][n][2][d]: (batch, head) slices of n split rows, in the order of the
+// list that streams them (with its node table the split pass is where the rows are gathered: its
+// reads are whole rows either way).
 __global__ void __launch_bounds__(256) split_x3_kernel(SplitArgs s) {
   const uint32_t per_row = (uint32_t)s.d / 8u;
   const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
   const uint32_t rows = (uint32_t)s.batch * (uint32_t)s.heads * (uint32_t)s.n;
   if (idx >= rows * per_row) return;
   const uint32_t r = idx / per_row, c = idx - r * per_row;
-  const uint32_t bh = r / (uint32_t)s.n, node = r - bh * (uint32_t)s.n;
+  const uint32_t bh = r / (uint32_t)s.n, pos = r - bh * (uint32_t)s.n;
+  const uint32_t node = s.node ? (uint32_t)s.node[pos] : pos;
+  if (node >= (uint32_t)s.n) return;
   const uint32_t b = bh / (uint32_t)s.heads, h = bh - b * (uint32_t)s.heads;
   const float* p = s.src + (int64_t)b * s.sb + (int64_t)node * s.sn + (int64_t)h * s.sh + 8 * c;
   const f32x4 x0 = *(const f32x4*)p, x1 = *(const f32x4*)(p + 4);
@@ -58,7 +66,7 @@ __global__ void __launch_bounds__(256) split_x3_kernel(SplitArgs s) {
 // s + 1 runs while step s is computed, one barrier per step. Per live group a wave issues 3 D/16
 // MFMAs for S^T = K Q^T and 3 D/16 for O^T += V^T P^T, with the online softmax of the bf16
 // forward between them (lazy rescale, masks skipped for fully valid groups).
-template <int D>
+template <int D, bool G>
 __global__ void __launch_bounds__(NT, 2) fwd_x3_kernel(KArgs a) {
   constexpr int GB = X3Dma<D>::GB;
   __shared__ __attribute__((aligned(1024))) char gb0[4 * GB];
@@ -71,7 +79,7 @@ __global__ void __launch_bounds__(NT, 2) fwd_x3_kernel(KArgs a) {
   const int64_t xbase = (int64_t)j.bh * a.n * (2 * D);
   const rsrc_t rK = make_rsrc(a.xa + xbase, a.xslice_bytes);
   const rsrc_t rV = make_rsrc(a.xb + xbase, a.xslice_bytes);
-  const int qrow = j.blk * BLK + 32 * w + i;
+  const int qrow = node_at<G>(a, j.blk * BLK + 32 * w + i);
   u32x4 qh[D / 16], ql[D / 16];
   load_frag_x3<D>(qh, ql, make_rsrc((const float*)a.q + j.base, a.slice_bytes), qrow, (uint32_t)a.sn * 4, g);
   Off<D> off;
@@ -186,7 +194,7 @@ __global__ void __launch_bounds__(NT, 2) fwd_x3_kernel(KArgs a) {
 // into one of two half buffers (planes K hi, K lo of each group: 32 KB at D = 128), two workgroups
 // per CU; a half's units (four 16-byte non-temporal loads per lane: the B operands' hi and lo
 // parts) are loaded with its rows, so the barrier that publishes the rows covers them.
-template <int D>
+template <int D, bool G>
 __global__ void __launch_bounds__(NT, 2) dq_x3_ds_kernel(KArgs a) {
   constexpr int GB = X3Dma<D>::GB;
   __shared__ __attribute__((aligned(1024))) char hb0[4 * GB];
@@ -202,7 +210,7 @@ __global__ void __launch_bounds__(NT, 2) dq_x3_ds_kernel(KArgs a) {
   const uint32_t skip = 32u * 4u * D;
   const rsrc_t rK2 = make_rsrc(a.xa + xbase + 32 * 2 * D, a.xslice_bytes > skip ? a.xslice_bytes - skip : 0u);
   const rsrc_t rS = make_rsrc(a.ds + (int64_t)j.bh * (a.ds_slice_bytes >> 1), a.ds_slice_bytes);
-  const int qrow = j.blk * BLK + 32 * w + i;
+  const int qrow = node_at<G>(a, j.blk * BLK + 32 * w + i);
   Off<D> off;
   off.init(lane);
   X3Dma<D> dma;
@@ -296,15 +304,20 @@ __global__ void __launch_bounds__(NT, 2) dq_x3_ds_kernel(KArgs a) {
   store_acc_f32<D>(make_rsrc((float*)a.out0 + j.base, a.slice_bytes), qrow, (uint32_t)a.sn * 4, acc, a.scale, g);
 }
 
-template <int D>
-hipError_t launch_d(Kind kind, const KArgs& a, hipStream_t stream) {
+template <int D, bool G>
+hipError_t launch_dg(Kind kind, const KArgs& a, hipStream_t stream) {
   const dim3 grid((unsigned)job_count(a)), block(NT);
   switch (kind) {
-    case Kind::kFwd: hipLaunchKernelGGL(fwd_x3_kernel<D>, grid, block, 0, stream, a); break;
-    case Kind::kDqDs: hipLaunchKernelGGL(dq_x3_ds_kernel<D>, grid, block, 0, stream, a); break;
+    case Kind::kFwd: hipLaunchKernelGGL((fwd_x3_kernel<D, G>), grid, block, 0, stream, a); break;
+    case Kind::kDqDs: hipLaunchKernelGGL((dq_x3_ds_kernel<D, G>), grid, block, 0, stream, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
+}
+
+template <int D>
+hipError_t launch_d(Kind kind, const KArgs& a, hipStream_t stream) {
+  return a.node ? launch_dg<D, true>(kind, a, stream) : launch_dg<D, false>(kind, a, stream);
 }
 
 }  // namespace
@@ -320,8 +333,8 @@ hipError_t launch_x3(Kind kind, int head_dim, const KArgs& a, hipStream_t stream
 }
 
 hipError_t launch_split_x3(const float* src, int64_t sb, int64_t sn, int64_t sh, int batch, int n, int heads,
-                           int head_dim, uint16_t* dst, hipStream_t stream) {
-  SplitArgs s{src, dst, sb, sn, sh, batch, n, heads, head_dim};
+                           int head_dim, const int32_t* node, uint16_t* dst, hipStream_t stream) {
+  SplitArgs s{src, dst, sb, sn, sh, batch, n, heads, head_dim, node};
   const uint64_t threads = (uint64_t)batch * heads * n * (head_dim / 8);
   hipLaunchKernelGGL(split_x3_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, s);
   return hipGetLastError();

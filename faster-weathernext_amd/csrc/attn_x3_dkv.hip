@@ -75,7 +75,7 @@ struct X3DmaW {
 // L), through a per-wave LDS stage ([plane][query][16 keys] bf16, 32-byte rows: conflict-free
 // 16-byte reads). A wave whose 16 keys have no valid element in a unit the map has writes zeros
 // for its chunk.
-template <int D>
+template <int D, bool G>
 __global__ void __launch_bounds__(NT4, 2) dkv16_x3_kernel(KArgs a) {
   using Dma = X3DmaW<D, 4>;
   constexpr int GB = Dma::GB;
@@ -105,7 +105,7 @@ __global__ void __launch_bounds__(NT4, 2) dkv16_x3_kernel(KArgs a) {
   const rsrc_t rD = make_rsrc(a.delta + stat_index(a, j, 0), (uint32_t)a.n * 4);
   const rsrc_t rS = make_rsrc(a.ds + (int64_t)j.bh * (a.ds_slice_bytes >> 1), a.ds_slice_bytes);
   const uint32_t snb = (uint32_t)a.sn * 4;
-  const int krow = j.blk * BLK + 16 * kg + t16;
+  const int krow = node_at<G>(a, j.blk * BLK + 16 * kg + t16);
   // K and V rows of this lane's key, columns 32 s + 8 g .. + 7, split.
   u32x4 kh[KS], kl[KS], vh[KS], vl[KS];
   {
@@ -261,11 +261,17 @@ __global__ void __launch_bounds__(NT4, 2) dkv16_x3_kernel(KArgs a) {
     rem &= rem - 1u;
     return true;
   };
-  auto copy = [&](lds_char* buf, int t, int c) {
+  // The tensors' row at position lane % 32 of step (t, c), whose lse and delta wave 0 copies: with a
+  // node table it is loaded a step before. (The split Q and dO rows are in the list's order.)
+  auto lane_row = [&](int t, int c) {
+    if constexpr (G) return node_block(a, ((ci32_ptr)a.col)[t])[32 * c + (lane & 31)];
+    return 0;
+  };
+  auto copy = [&](lds_char* buf, int t, int c, int lrow) {
     const int row0 = ((ci32_ptr)a.col)[t] * BLK + 32 * c;
     dma.issue(rQ, rO, buf, row0, wid);
     if (wid == 0) {
-      const int so = lane < 32 ? (row0 + lane) * 4 : (int)kPastEnd;
+      const int so = lane < 32 ? (G ? lrow : row0 + lane) * 4 : (int)kPastEnd;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rL, (__attribute__((address_space(3))) void*)(buf + SB), 4, so, 0, 0, 0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rD, (__attribute__((address_space(3))) void*)(buf + SB + 256), 4, so, 0,
                                                0, 0);
@@ -273,13 +279,18 @@ __global__ void __launch_bounds__(NT4, 2) dkv16_x3_kernel(KArgs a) {
   };
   lds_char* b0 = (lds_char*)gb0;
   lds_char* b1 = (lds_char*)gb1;
-  int tc = 0, cc = 0, tn = 0, cn = 0;
-  bool vc = take(tc, cc), vn = false;
+  int tc = 0, cc = 0, tn = 0, cn = 0, tm = 0, cm = 0;
+  bool vc = take(tc, cc), vn = false, vm = false;
   uint64_t mwc = 0, mwn = 0;
+  int rown = 0, rowm = 0;  // lane rows of steps (tn, cn) and (tm, cm)
   if (vc) {
-    copy(b0, tc, cc);
+    copy(b0, tc, cc, lane_row(tc, cc));
     mwc = mword[(int64_t)tc * 256];
     vn = take(tn, cn);
+    if constexpr (G) {
+      if (vn) rown = lane_row(tn, cn);
+      vm = vn && take(tm, cm);
+    }
   }
   auto step = [&](lds_char* cur, lds_char* nxt) {
     wait_vmem();  // this wave's part of the current step (wave 0: the statistics) and its mask word
@@ -294,8 +305,11 @@ __global__ void __launch_bounds__(NT4, 2) dkv16_x3_kernel(KArgs a) {
     }
     __syncthreads();  // the step landed; every wave is done with the previous step's buffer
     if (vn) {
-      copy(nxt, tn, cn);
+      copy(nxt, tn, cn, rown);
       mwn = tn != tc ? mword[(int64_t)tn * 256] : mwc;
+      if constexpr (G) {
+        if (vm) rowm = lane_row(tm, cm);
+      }
     }
     // The wave's 16 keys have a valid element in query group cc: some lane's bits of the group
     // (16 c + 8 m + r, shifted by 4 (g % 2)) are set.
@@ -315,7 +329,15 @@ __global__ void __launch_bounds__(NT4, 2) dkv16_x3_kernel(KArgs a) {
     cc = cn;
     mwc = mwn;
     vc = vn;
-    vn = vc && take(tn, cn);
+    if constexpr (G) {
+      tn = tm;
+      cn = cm;
+      vn = vm;
+      rown = rowm;
+      vm = vn && take(tm, cm);
+    } else {
+      vn = vc && take(tn, cn);
+    }
   };
   while (vc) {
     step(b0, b1);
@@ -348,7 +370,10 @@ template <int D>
 hipError_t launch_d(const KArgs& a, hipStream_t stream) {
   // Two workgroups per item, laid out in blocks of 16 ids (8 items x 2 halves).
   const dim3 grid(16u * (((unsigned)job_count(a) + 7u) / 8u));
-  hipLaunchKernelGGL((dkv16_x3_kernel<D>), grid, dim3(NT4), 0, stream, a);
+  if (a.node)
+    hipLaunchKernelGGL((dkv16_x3_kernel<D, true>), grid, dim3(NT4), 0, stream, a);
+  else
+    hipLaunchKernelGGL((dkv16_x3_kernel<D, false>), grid, dim3(NT4), 0, stream, a);
   return hipGetLastError();
 }
 

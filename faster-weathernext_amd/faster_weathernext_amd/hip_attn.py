@@ -246,15 +246,15 @@ class TileList:
     nat.check(L.fwn_tiles_permute_fill(*args, nat.ptr(tile_ptr), nat.ptr(tile_kb), nat.ptr(tile_bits)))
     return TileList(tile_ptr, tile_kb, tile_bits, self.n_cols, self.device, self._fixed_cap, _node=node)
 
-  def launch_list(self, desc):
-    """The list the kernels of a call with descriptor `desc` walk for this mask: the one laid out in
-    its own order where there is one (bf16 kernels), else this one."""
-    return self if self._ordered is None or desc.dtype != nat.BF16 else self._ordered
+  def launch_list(self):
+    """The list the kernels walk for this mask: the one laid out in its own order where there is
+    one, else this one."""
+    return self if self._ordered is None else self._ordered
 
-  def launch_lists(self, tiles_t, desc):
+  def launch_lists(self, tiles_t):
     """(launch list of this mask, list of the transposed mask `tiles_t` in the same order): the
     pair whose dS units the backward exchanges."""
-    tl = self.launch_list(desc)
+    tl = self.launch_list()
     if tiles_t is self or tl is self or tiles_t.n_blocks != self.n_blocks or tiles_t.n_cols != self.n_cols:
       return tl, tl if tiles_t is self else tiles_t
     if tiles_t not in self._transposes:
@@ -511,7 +511,7 @@ def attention_forward(q, k, v, tiles, scale, with_lse=True, precision="native"):
   v = _same_layout(v, q, "v")
   out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
   desc = _desc(q, scale, out, prec)
-  tl = _as_tiles(tiles, q.shape[1], q.device).launch_list(desc)
+  tl = _as_tiles(tiles, q.shape[1], q.device).launch_list()
   lse = torch.empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32, device=q.device) if with_lse else None
   ws = workspace(desc, q.device, tl)
   ts = tl.struct_for_desc(desc, "fwd")
@@ -557,7 +557,7 @@ def _backward_into(q, k, v, out, lse, dout, tiles, tiles_t, scale, dq, dk, dv, p
   main = torch.cuda.current_stream(q.device)
   dmap = None
   if DS_EXCHANGE:
-    tl, tlt = base.launch_lists(base_t, desc)
+    tl, tlt = base.launch_lists(base_t)
     dmap = tl.ds_map(tlt, unit_keys_for(q.dtype))
   if dmap is not None:
     # delta, dK/dV writing dS, then dQ from dS, in stream order (fwn_attn_bwd_ds_launch).
@@ -570,7 +570,7 @@ def _backward_into(q, k, v, out, lse, dout, tiles, tiles_t, scale, dq, dk, dv, p
                                        dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ds.data_ptr(), ds.numel(),
                                        *_ws_args(ws), main.cuda_stream))
     return
-  tl, tlt = base.launch_list(desc), base_t.launch_list(desc)
+  tl, tlt = base.launch_list(), base_t.launch_list()
   ws_q, ws_kv = workspace(desc, q.device, tl), workspace(desc, q.device, tlt)
   nat.check(L.fwn_attn_bwd_delta_launch(desc, out.data_ptr(), dout.data_ptr(), delta.data_ptr(), main.cuda_stream))
   side = _side_stream(q.device)
