@@ -226,11 +226,195 @@ hipError_t launch_t(RowPass pass, const RowArgs& a, hipStream_t stream) {
   return hipErrorInvalidValue;
 }
 
+// ------------------------------------------------------------------------------------------
+// Backward of both passes (autograd of patch.py:240-253, 274-276, 288-292; JAX differentiates the
+// reference's own). One wave per row: x and the gradients are read once, the statistics are
+// recomputed in registers, and the input gradient is written once, so the pass is bound by HBM as
+// the forward is (3 or 4 tensors of traffic). The per-channel sums of the affine's gradients stay in
+// each lane's registers over all rows of its wave (a strided share of one batch member's rows), are
+// added over the workgroup's waves in LDS and go out as one partial row per workgroup, which
+// sums_kernel adds; both orders are fixed. At [1, 40962, 768] float32: with the sums 68 + 6 us (378 MB,
+// 5.6 TB/s), gather_norm's 104 us (504 MB, its scattered rows written whole; 4.8 TB/s); bf16 with sums
+// and the residual's gradient 58 + 6 us. The same gradients as torch operations took 15 to 25
+// launches: a gather, scatter and their gradients 1.64 -> 0.36 ms, a block's training pass 7.38 ->
+// 5.69 ms.
+constexpr int kSumGroups = 16;  // partial rows added in parallel by sums_kernel's workgroup
+
+__device__ __forceinline__ void wave_sum2(float& x, float& y) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    x += __shfl_xor(x, o);
+    y += __shfl_xor(y, o);
+  }
+}
+
+template <typename T, int VPL, bool SUMS>
+__global__ void __launch_bounds__(64 * kWaves) norm_bwd_kernel(RowBwdArgs a) {
+  constexpr int E = Vec<T>::E;
+  extern __shared__ float sums[];  // SUMS: [2][channels]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int b = (int)blockIdx.x / a.blocks, blk = (int)blockIdx.x - b * a.blocks;
+  const size_t c = (size_t)a.channels, base = (size_t)b * a.n;
+  const int nv = a.channels / E;
+  const float inv_c = 1.f / (float)a.channels;
+  const float* mul = a.mul ? a.mul + (size_t)b * c : nullptr;
+  float sm[SUMS ? VPL : 1][E], sa[SUMS ? VPL : 1][E];
+  if constexpr (SUMS) {
+#pragma unroll
+    for (int k = 0; k < VPL; ++k)
+#pragma unroll
+      for (int e = 0; e < E; ++e) sm[k][e] = sa[k][e] = 0.f;
+  }
+  for (int64_t i = (int64_t)blk * kWaves + wave; i < a.n; i += (int64_t)a.blocks * kWaves) {
+    const int64_t src = a.perm_grad ? a.perm_grad[i] : i, dst = a.perm_out ? a.perm_out[i] : i;
+    const bool has = a.g_norm && (uint64_t)src < (uint64_t)a.n;
+    const T* gn = (const T*)a.g_norm + (base + (size_t)(has ? src : 0)) * c;
+    const T* gr = a.g_res ? (const T*)a.g_res + (base + (size_t)i) * c : nullptr;
+    u32x4 gv[VPL], rv[VPL];
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+      const int idx = lane + 64 * k;
+      gv[k] = rv[k] = u32x4{0u, 0u, 0u, 0u};
+      if (has && idx < nv) gv[k] = *(const u32x4*)(gn + (size_t)idx * E);
+      if (gr && idx < nv) rv[k] = *(const u32x4*)(gr + (size_t)idx * E);
+    }
+    u32x4 v[VPL];
+    float f[VPL][E];
+    float mean, rstd;
+    load_row<T, VPL>((const T*)a.x + (base + (size_t)i) * c, true, nv, a.channels, a.eps, lane, v, f, mean, rstd);
+    float g[VPL][E], s1 = 0.f, s2 = 0.f;
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+      const int idx = lane + 64 * k;
+      Vec<T>::unpack(gv[k], g[k]);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        f[k][e] = (f[k][e] - mean) * rstd;
+        if constexpr (SUMS) {
+          sm[k][e] = fmaf(g[k][e], f[k][e], sm[k][e]);
+          sa[k][e] += g[k][e];
+        }
+      }
+      if (mul && idx < nv) {
+#pragma unroll
+        for (int q = 0; q < E / 4; ++q) {
+          const u32x4 m = *(const u32x4*)(mul + (size_t)idx * E + 4 * q);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) g[k][4 * q + e] *= as_float(m[e]);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        s1 += g[k][e];
+        s2 = fmaf(g[k][e], f[k][e], s2);
+      }
+    }
+    wave_sum2(s1, s2);
+    const float m1 = s1 * inv_c, m2 = s2 * inv_c;
+    if ((uint64_t)dst >= (uint64_t)a.n) continue;
+    T* out = (T*)a.gx + (base + (size_t)dst) * c;
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+      const int idx = lane + 64 * k;
+      if (idx >= nv) continue;
+      float r[E], y[E];
+      Vec<T>::unpack(rv[k], r);
+#pragma unroll
+      for (int e = 0; e < E; ++e) y[e] = fmaf(rstd, g[k][e] - m1 - f[k][e] * m2, r[e]);
+      store16(out + (size_t)idx * E, Vec<T>::pack(y));
+    }
+  }
+  if constexpr (SUMS) {
+    for (int w = 0; w < kWaves; ++w) {
+      if (wave == w) {
+#pragma unroll
+        for (int k = 0; k < VPL; ++k) {
+          const int idx = lane + 64 * k;
+          if (idx >= nv) continue;
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            float* p = sums + (size_t)idx * E + e;
+            p[0] = w == 0 ? sm[k][e] : p[0] + sm[k][e];
+            p[c] = w == 0 ? sa[k][e] : p[c] + sa[k][e];
+          }
+        }
+      }
+      __syncthreads();
+    }
+    float* part = a.part + (size_t)blockIdx.x * 2 * c;
+    for (int j = threadIdx.x; j < 2 * a.channels; j += 64 * kWaves) part[j] = sums[j];
+  }
+}
+
+// g_mul and g_add from the partial rows: 64 columns per workgroup, kSumGroups strided shares of a
+// batch member's partial rows, added in LDS.
+__global__ void __launch_bounds__(64 * kSumGroups) sums_kernel(RowBwdArgs a) {
+  __shared__ float red[kSumGroups][64];
+  const int lane = threadIdx.x & 63, grp = (int)threadIdx.x >> 6;
+  const int cols = 2 * a.channels, per = (cols + 63) / 64;
+  const int b = (int)blockIdx.x / per, j = ((int)blockIdx.x - b * per) * 64 + lane;
+  float s = 0.f;
+  if (j < cols) {
+    const float* p = a.part + (size_t)b * a.blocks * cols + j;
+#pragma unroll 8
+    for (int r = grp; r < a.blocks; r += kSumGroups) s += p[(size_t)r * cols];
+  }
+  red[grp][lane] = s;
+  __syncthreads();
+  if (grp != 0 || j >= cols) return;
+#pragma unroll
+  for (int r = 1; r < kSumGroups; ++r) s += red[r][lane];
+  if (j < a.channels)
+    a.g_mul[(size_t)b * a.channels + j] = s;
+  else
+    a.g_add[(size_t)b * a.channels + j - a.channels] = s;
+}
+
+template <typename T, int VPL>
+hipError_t launch_bwd_tv(const RowBwdArgs& a, hipStream_t stream) {
+  const dim3 grid((unsigned)a.blocks * (unsigned)a.batch), block(64 * kWaves);
+  if (!a.part) {
+    hipLaunchKernelGGL((norm_bwd_kernel<T, VPL, false>), grid, block, 0, stream, a);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL((norm_bwd_kernel<T, VPL, true>), grid, block, 2 * (unsigned)a.channels * sizeof(float), stream, a);
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  const unsigned per = (2u * (unsigned)a.channels + 63u) / 64u;
+  hipLaunchKernelGGL(sums_kernel, dim3(per * (unsigned)a.batch), dim3(64 * kSumGroups), 0, stream, a);
+  return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_bwd_t(const RowBwdArgs& a, hipStream_t stream) {
+  const int per_lane = (a.channels / Vec<T>::E + 63) / 64;
+  if (per_lane <= 1) return launch_bwd_tv<T, 1>(a, stream);
+  if (per_lane <= 2) return launch_bwd_tv<T, 2>(a, stream);
+  if (per_lane <= 3) return launch_bwd_tv<T, 3>(a, stream);
+  if (per_lane <= 4) return launch_bwd_tv<T, 4>(a, stream);
+  if (per_lane <= 8) return launch_bwd_tv<T, 8>(a, stream);
+  if constexpr (Vec<T>::E == 4) return launch_bwd_tv<T, 16>(a, stream);  // float32, up to 4,096 channels
+  return hipErrorInvalidValue;
+}
+
 }  // namespace
 
 hipError_t launch_rows(RowPass pass, int dtype, const RowArgs& a, hipStream_t stream) {
   if ((int64_t)a.batch * a.n == 0) return hipSuccess;
   return dtype == FWN_F32 ? launch_t<float>(pass, a, stream) : launch_t<uint16_t>(pass, a, stream);
+}
+
+// Four rows per wave at least (with sums: each workgroup writes a partial row), and about four
+// workgroups per CU over the whole call; without sums twice as many, one row per wave for small calls.
+int32_t rows_bwd_blocks(int32_t batch, int32_t n, bool sums) {
+  const int64_t rows = sums ? 4 * kWaves : kWaves, most = sums ? 1024 : 2048;
+  const int64_t want = ((int64_t)n + rows - 1) / rows, cap = most / (batch > 0 ? batch : 1);
+  const int64_t blocks = want < cap ? want : cap;
+  return (int32_t)(blocks > 1 ? blocks : 1);
+}
+
+hipError_t launch_rows_bwd(int dtype, const RowBwdArgs& a, hipStream_t stream) {
+  return dtype == FWN_F32 ? launch_bwd_t<float>(a, stream) : launch_bwd_t<uint16_t>(a, stream);
 }
 
 }  // namespace fwn

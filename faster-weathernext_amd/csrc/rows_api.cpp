@@ -132,4 +132,58 @@ int fwn_rows_add_norm_affine_launch(const fwn_rows_desc* d, const void* x, const
   return status(launch_rows(RowPass::kNormScatter, d->dtype, a, (hipStream_t)stream), what);
 }
 
+int fwn_rows_norm_bwd_workspace_size(const fwn_rows_desc* d, uint64_t* bytes) {
+  using namespace fwn;
+  clear_error();
+  const char* what = "fwn_rows_norm_bwd_workspace_size";
+  if (!d || !bytes) return fail(FWN_ERR_INVALID_ARG, "%s: null argument", what);
+  if (d->batch < 0 || d->n < 0 || d->channels <= 0) return fail(FWN_ERR_INVALID_ARG, "%s: negative shape", what);
+  *bytes = (uint64_t)rows_bwd_blocks(d->batch, d->n, true) * (uint64_t)d->batch * 2u * (uint64_t)d->channels * 4u;
+  return FWN_OK;
+}
+
+int fwn_rows_norm_bwd_launch(const fwn_rows_desc* d, const void* x, const int64_t* perm, int32_t perm_rows,
+                             const void* g_norm, const void* g_res, const float* mul, void* gx, float* g_mul,
+                             float* g_add, void* workspace, uint64_t workspace_bytes, void* stream) {
+  using namespace fwn;
+  clear_error();
+  const char* what = "fwn_rows_norm_bwd_launch";
+  if (int rc = check_rows(d, x, perm, what, false)) return rc;
+  if (perm ? perm_rows != FWN_ROWS_PERM_GRAD && perm_rows != FWN_ROWS_PERM_OUT : perm_rows != 0)
+    return fail(FWN_ERR_INVALID_ARG, "%s: perm_rows %d", what, perm_rows);
+  if (!gx || !aligned16(gx) || (g_norm && !aligned16(g_norm)) || (g_res && !aligned16(g_res)) || (mul && !aligned16(mul)))
+    return fail(FWN_ERR_INVALID_ARG, "%s: gx must be non-null, and every tensor 16-byte aligned", what);
+  const uint64_t nb = fwn::bytes(d);
+  if (overlap(gx, x, nb) || (g_norm && overlap(gx, g_norm, nb)) || (g_res && overlap(gx, g_res, nb)))
+    return fail(FWN_ERR_INVALID_ARG, "%s: gx must not overlap x, g_norm or g_res", what);
+  if (!g_mul != !g_add) return fail(FWN_ERR_INVALID_ARG, "%s: g_mul and g_add go together", what);
+  RowBwdArgs a{};
+  a.x = x;
+  a.perm_grad = perm_rows == FWN_ROWS_PERM_GRAD ? perm : nullptr;
+  a.perm_out = perm_rows == FWN_ROWS_PERM_OUT ? perm : nullptr;
+  a.g_norm = g_norm;
+  a.g_res = g_res;
+  a.mul = mul;
+  a.gx = gx;
+  a.batch = d->batch;
+  a.n = d->n;
+  a.channels = d->channels;
+  a.eps = d->eps;
+  a.blocks = rows_bwd_blocks(d->batch, d->n, g_mul != nullptr);
+  if ((int64_t)a.blocks * d->batch > INT32_MAX / 128)
+    return fail(FWN_ERR_INVALID_ARG, "%s: batch too large for one launch (%d)", what, d->batch);
+  if (g_mul) {
+    uint64_t need = 0;
+    if (int rc = fwn_rows_norm_bwd_workspace_size(d, &need)) return rc;
+    if (need > 0 && (!workspace || !aligned16(workspace) || workspace_bytes < need))
+      return fail(FWN_ERR_INVALID_ARG, "%s: a 16-byte aligned workspace of %llu bytes is needed", what,
+                  (unsigned long long)need);
+    a.part = (float*)workspace;
+    a.g_mul = g_mul;
+    a.g_add = g_add;
+  }
+  if (d->batch == 0) return FWN_OK;  // no rows, no sums to write
+  return status(launch_rows_bwd(d->dtype, a, (hipStream_t)stream), what);
+}
+
 }  // extern "C"

@@ -18,10 +18,13 @@ residual in front of it in the same pass. The affine's scale and offset come
 from the conditioning vector through LinearNormConditioning's own projections, which the caller
 evaluates: pass ``mul`` (its multiplier of the normalised features) and ``add``.
 
-The forward passes run on the GPU only. Their gradients are computed with torch operations on
-the same device (the gather's transpose is the scatter and vice versa, plus the layer norm's
-analytic backward).
+The forward passes and their gradients run on the GPU only. Each gradient is one HIP pass as well
+(``fwn_rows_norm_bwd_launch``: the layer norm's analytic backward, with the permutation and the
+gradient that bypassed the norm in the same pass), plus a small reduction for mul and add. A
+backward that has to be differentiated again (create_graph) runs as torch operations instead.
 """
+import ctypes
+
 import torch
 
 from . import _native as nat
@@ -127,6 +130,36 @@ def add_layer_norm_affine(x, y, *, mul=None, add=None, eps=1e-5, inplace=False):
   return s, out
 
 
+def _dense(t):
+  """t as the kernels read it: contiguous and 16-byte aligned (None stays None)."""
+  if t is None:
+    return None
+  t = t.contiguous()
+  return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _norm_backward_pass(x, eps, g_norm, g_res=None, mul=None, perm=None, perm_rows=0, sums=False):
+  """(gradient of the rows, g_mul or None, g_add or None): one HIP pass (fwn_rows_norm_bwd_launch)."""
+  x, g_norm, g_res, mul, perm = (_dense(t) for t in (x, g_norm, g_res, mul, perm))
+  d = _desc(x, eps)
+  L = nat.lib()
+  gx = torch.empty_like(x)
+  g_mul = g_add = ws = None
+  if sums:
+    g_mul, g_add = (torch.empty((x.shape[0], x.shape[2]), dtype=torch.float32, device=x.device) for _ in range(2))
+    size = ctypes.c_uint64(0)
+    nat.check(L.fwn_rows_norm_bwd_workspace_size(d, ctypes.byref(size)))
+    ws = torch.empty(int(size.value), dtype=torch.uint8, device=x.device)
+  with torch.cuda.device(x.device):
+    nat.check(L.fwn_rows_norm_bwd_launch(d, _addr(x), _addr(perm), perm_rows, _addr(g_norm), _addr(g_res), _addr(mul),
+                                         _addr(gx), _addr(g_mul), _addr(g_add), _addr(ws),
+                                         0 if ws is None else ws.numel(), _stream(x)))
+  return gx, g_mul, g_add
+
+
+# The same gradients as torch operations, for backwards under create_graph.
+
+
 def _norm_stats(x, eps):
   xf = x.float()
   mean = xf.mean(-1, keepdim=True)
@@ -147,23 +180,35 @@ def _inverse(perm):
   return inv
 
 
+def _affine_norm_backward(x, eps, g_y, mul, need_mul, need_add):
+  """(gradient of x in float32, g_mul, g_add) of layer_norm(x) * mul + add for the gradient g_y."""
+  g_y = g_y.float()
+  xhat, rstd = _norm_stats(x, eps)
+  g_mul = (g_y * xhat).sum(1) if need_mul else None
+  g_add = g_y.sum(1) if need_add else None
+  return _norm_backward(xhat, rstd, g_y * mul[:, None, :] if mul is not None else g_y), g_mul, g_add
+
+
 class _GatherNorm(torch.autograd.Function):
   @staticmethod
   def forward(ctx, x, perm, eps):
     x_out, n_out = gather_layer_norm_forward(x, perm, eps)
     ctx.save_for_backward(x_out, perm)
+    ctx.set_materialize_grads(False)
     ctx.eps = eps
     return x_out, n_out
 
   @staticmethod
   def backward(ctx, g_x, g_n):
     x_out, perm = ctx.saved_tensors
+    if not torch.is_grad_enabled():
+      return _norm_backward_pass(x_out, ctx.eps, g_n, g_x, perm=perm, perm_rows=nat.ROWS_PERM_OUT)[0], None, None
     g = torch.zeros(x_out.shape, device=x_out.device, dtype=torch.float32)
     if g_x is not None:
-      g += g_x.float()
+      g = g + g_x.float()
     if g_n is not None:
       xhat, rstd = _norm_stats(x_out, ctx.eps)
-      g += _norm_backward(xhat, rstd, g_n)
+      g = g + _norm_backward(xhat, rstd, g_n)
     return g[:, _inverse(perm)].to(x_out.dtype), None, None
 
 
@@ -182,13 +227,52 @@ class _NormScatter(torch.autograd.Function):
   @staticmethod
   def backward(ctx, g_out):
     x, perm, mul = ctx.saved_tensors
-    g_y = (g_out if perm is None else g_out[:, perm]).float()  # gradient of the un-scattered rows
-    xhat, rstd = _norm_stats(x, ctx.eps)
-    g_mul = (g_y * xhat).sum(1) if mul is not None and ctx.needs_input_grad[2] else None
-    g_add = g_y.sum(1) if ctx.has_add and ctx.needs_input_grad[3] else None
-    g_xhat = g_y * mul[:, None, :] if mul is not None else g_y
-    g_x = _norm_backward(xhat, rstd, g_xhat).to(x.dtype)
-    return g_x, None, g_mul, g_add, None
+    need_mul, need_add = mul is not None and ctx.needs_input_grad[2], ctx.has_add and ctx.needs_input_grad[3]
+    if torch.is_grad_enabled():
+      g_y = g_out if perm is None else g_out[:, perm]  # gradient of the un-scattered rows
+      g_x, g_mul, g_add = _affine_norm_backward(x, ctx.eps, g_y, mul, need_mul, need_add)
+      return g_x.to(x.dtype), None, g_mul, g_add, None
+    g_x, g_mul, g_add = _norm_backward_pass(x, ctx.eps, g_out, mul=mul, perm=perm,
+                                            perm_rows=0 if perm is None else nat.ROWS_PERM_GRAD,
+                                            sums=need_mul or need_add)
+    return g_x, None, g_mul if need_mul else None, g_add if need_add else None, None
+
+
+class _AddNorm(torch.autograd.Function):
+  """(x + y, layer_norm(x + y) * mul + add): the gradient of the sum adds to the norm's in the
+  norm's backward pass."""
+
+  @staticmethod
+  def forward(ctx, x, y, mul, add, eps):
+    s, out = add_layer_norm_affine(x, y, mul=mul, add=add, eps=eps)
+    ctx.save_for_backward(s, mul)
+    ctx.set_materialize_grads(False)
+    ctx.eps = eps
+    return s, out
+
+  @staticmethod
+  def backward(ctx, g_s, g_out):
+    s, mul = ctx.saved_tensors
+    if g_out is None:
+      return g_s, g_s, None, None, None
+    need_mul, need_add = ctx.needs_input_grad[2], ctx.needs_input_grad[3]
+    if torch.is_grad_enabled():
+      g, g_mul, g_add = _affine_norm_backward(s, ctx.eps, g_out, mul, need_mul, need_add)
+      g = (g if g_s is None else g + g_s.float()).to(s.dtype)
+    else:
+      g, g_mul, g_add = _norm_backward_pass(s, ctx.eps, g_out, g_s, mul, sums=need_mul or need_add)
+    return g, g, g_mul if need_mul else None, g_add if need_add else None, None
+
+
+def residual_norm(x, y, *, mul, add, eps=1e-5):
+  """(x + y, layer_norm_affine(x + y)) with gradients: one pass forward and one backward where x and
+  y share dtype and layout, else torch's add and the norm's own pass."""
+  same = (x.dtype == y.dtype and x.shape == y.shape and x.is_contiguous() and y.is_contiguous() and
+          x.data_ptr() % 16 == 0 and y.data_ptr() % 16 == 0)
+  if same and x.is_cuda and x.dim() == 3 and x.dtype in _DTYPES:
+    return _AddNorm.apply(x, y, mul, add, float(eps))
+  s = x + y
+  return s, layer_norm_affine(s, mul=mul, add=add, eps=eps)
 
 
 def gather_layer_norm(x, perm, *, eps=1e-5):

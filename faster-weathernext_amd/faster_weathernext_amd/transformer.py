@@ -23,7 +23,8 @@ and GELU run in the epilogue of its GEMM (``torch._addmm_activation``, which has
 so the [n, ffw_hidden] activations make one trip to HBM instead of three, every block GEMM
 splits its rows at a multiple of 512 (``mha.linear_rows``), and each residual add runs in one
 pass with the conditioned layer norm after it (``rows.add_layer_norm_affine``); with autograd the
-same functions run as plain Linear, GELU, Linear and separate adds.
+same functions run as plain Linear, GELU, Linear and adds, the attention's add fused with the
+feed-forward's conditioned norm (``rows.residual_norm``).
 Parameters are random-initialised torch parameters; official checkpoints are Haiku parameters of
 the JAX model, which this package does not load.
 """
@@ -36,7 +37,7 @@ from . import patch
 from .hip_attn import TileList
 from .mesh import hilbert_order, khop_mask, mesh_mask
 from .mha import TiledMHA, linear_rows, needs_grad
-from .rows import add_layer_norm_affine, gather_layer_norm, layer_norm_affine, layer_norm_scatter
+from .rows import add_layer_norm_affine, gather_layer_norm, layer_norm_affine, layer_norm_scatter, residual_norm
 
 
 class NormConditioning(torch.nn.Module):
@@ -61,6 +62,11 @@ class NormConditioning(torch.nn.Module):
     """forward(layer_norm(x), cond) as one HIP pass (statistics and affine in float32)."""
     mul, add = self.affine(cond)
     return layer_norm_affine(x, mul=mul.float().contiguous(), add=add.float().contiguous(), eps=eps)
+
+  def residual_norm(self, x, y, cond, eps):
+    """(x + y, norm(x + y)) with gradients, in one HIP pass where x and y allow it."""
+    mul, add = self.affine(cond)
+    return residual_norm(x, y, mul=mul.float().contiguous(), add=add.float().contiguous(), eps=eps)
 
   def add_norm(self, x, y, cond, eps):
     """(x + y, forward(layer_norm(x + y), cond)) as one HIP pass, without autograd."""
@@ -96,8 +102,8 @@ class MeshBlock(torch.nn.Module):
     """`normed` is layernorm(x) when the caller has it already (block 0 gets it from the fused
     gather). Otherwise each conditioned layer norm is one fused pass (``layer_norm_affine``)."""
     h = self.norm_mha(normed, cond) if normed is not None else self.norm_mha.norm(x, cond, self.eps)
-    x = x + self.mha(h)
-    return x + self.feed_forward(self.norm_ffw.norm(x, cond, self.eps))
+    x, h = self.norm_ffw.residual_norm(x, self.mha(h), cond, self.eps)
+    return x + self.feed_forward(h)
 
   def forward_fused(self, x, h, cond, next_norm=None):
     """The block without autograd, from h = norm_mha(layernorm(x)) already computed: each residual

@@ -73,6 +73,28 @@ int fwn_rows_add_norm_affine_launch(const fwn_rows_desc* d, const void* x, const
                                     const float* mul, const float* add, void* sum, void* out,
                                     void* stream);
 
+/* Backward of the passes above: for every row i of x (the rows a pass normalised, with xhat their
+ * layer norm and rstd its 1 / sqrt(var + eps), recomputed from x),
+ *
+ *   g[b, i, :]  = rstd (gm - mean(gm) - xhat mean(gm xhat)) + g_res[b, i, :],  gm = g_norm mul
+ *   g_mul[b, :] = sum over i of g_norm xhat,   g_add[b, :] = sum over i of g_norm
+ *
+ * computed in float32; g is written to gx in the dtype. g_norm (NULL: zeros) is the gradient of
+ * the norm's output, g_res (NULL: zeros) that of the sum or copy x itself also went to, mul as in
+ * the forward (NULL: 1). g_mul and g_add (float32 [batch, channels]) are written when both are
+ * non-NULL; that needs fwn_rows_norm_bwd_workspace_size bytes of workspace (16-byte aligned), used
+ * until the launch's stream work is done, and none otherwise. The sums run in a fixed order.
+ * With perm, `perm_rows` says what it permutes:
+ *   FWN_ROWS_PERM_GRAD: row i's g_norm is row perm[i] of the tensor (backward of norm_scatter);
+ *   FWN_ROWS_PERM_OUT: g is written to row perm[i] of gx (backward of gather_norm).
+ * Entries of perm outside [0, n) read a zero row or drop the row. gx must not overlap the inputs. */
+#define FWN_ROWS_PERM_GRAD 1
+#define FWN_ROWS_PERM_OUT 2
+int fwn_rows_norm_bwd_workspace_size(const fwn_rows_desc* d, uint64_t* bytes);
+int fwn_rows_norm_bwd_launch(const fwn_rows_desc* d, const void* x, const int64_t* perm, int32_t perm_rows,
+                             const void* g_norm, const void* g_res, const float* mul, void* gx, float* g_mul,
+                             float* g_add, void* workspace, uint64_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }  /* extern "C" */
 #endif
