@@ -12,7 +12,7 @@ from dS, on one stream. With --no-ds the dQ kernel recomputes S and dP and runs 
 beside dK/dV on a second stream. Inputs are resident in HBM before the timed region. The metric is effective
 TFLOP/s over live 128x128 tiles (14 * D * 128^2 per live tile, batch and head for fwd + bwd;
 4 * D * 128^2 for forward-only workloads). The live tiles are those of the workload's node order; the
-kernels may walk a list of fewer tiles, laid out in an order of its own (TileList.launch_list), so
+kernels may walk lists of fewer tiles, laid out for them (TileList.launch_list, exchange_lists), so
 the rate can exceed the matrix peak. The mask build is timed separately.
 
 Prints one JSON line (rank 0). `value` comes from K steps with nothing recorded between their
@@ -558,21 +558,27 @@ def attention(args):
   L = nat.lib()
   stream = torch.cuda.current_stream(dev)
   sp = stream.cuda_stream
-  # The list the kernels walk, as the package picks it: the mask in a node order of the list's own
-  # where that has less to compute, else the given order's.
+  # The lists the kernels walk, as the package picks them: the mask laid out for each kernel where
+  # that has less to compute, else the given order's. With the dS exchange (symmetric k-hop mask: the
+  # forward list is its own transpose) dQ and dK/dV have lists of their own.
   walked = tiles.launch_list()
-  # The schedule of each kernel (with --order auto, its order table): the forward's, dQ's and
-  # dK/dV's (the list is its own transpose); the recomputing kernels take the native descriptor.
-  sched = lambda d, kernel: (walked.struct_for_desc(d, kernel) if args.order == "auto" else
-                             walked.struct_for(B, H, kernel=kernel))
+  exchange = None
+  if cfg["backward"] and not args.no_ds and fwn.hip_attn.DS_EXCHANGE:
+    exchange = tiles.exchange_lists(tiles, fwn.hip_attn.unit_keys_for(dtype))
+  walked_dq, walked_kv, dmap = exchange or (walked, walked, None)
+  # The schedule of each kernel (with --order auto, its order table); the recomputing kernels take
+  # the native descriptor.
+  def sched(d, kernel):
+    lst = {"fwd": walked, "dq": walked_dq, "kv": walked_kv}[kernel]
+    return lst.struct_for_desc(d, kernel) if args.order == "auto" else lst.struct_for(B, H, kernel=kernel)
   ts, tsq, tst = sched(fdesc, "fwd"), sched(fdesc, "dq"), sched(fdesc, "kv")
   tsq_n, tst_n = sched(desc, "dq"), sched(desc, "kv")
-  ws = fwn.hip_attn.workspace(fdesc, dev, walked)
+  ws = fwn.hip_attn.workspace(fdesc, dev, walked, walked_dq, walked_kv)
   wsp, wsn = (ws.data_ptr(), ws.numel()) if ws is not None else (None, 0)
   # dK/dV runs on a second stream beside dQ (as the package's backward does), with its own
   # workspace; the step joins the two streams at its end.
   side = torch.cuda.Stream(dev)
-  ws2 = fwn.hip_attn.workspace(desc, dev, walked)
+  ws2 = fwn.hip_attn.workspace(desc, dev, walked, walked_dq, walked_kv)
   ws2p, ws2n = (ws2.data_ptr(), ws2.numel()) if ws2 is not None else (None, 0)
 
   def fwd(st):
@@ -592,11 +598,6 @@ def attention(args):
                                         lse.data_ptr(), delta.data_ptr(), tst_n, dk.data_ptr(), dv.data_ptr(),
                                         ws2p if own else wsp, ws2n if own else wsn, st.cuda_stream))
 
-  # The bf16 backward's dS exchange, as the package runs it (symmetric k-hop mask: the forward
-  # list is its own transpose, so one list serves both kernels).
-  dmap = None
-  if cfg["backward"] and not args.no_ds and fwn.hip_attn.DS_EXCHANGE:
-    dmap = walked.ds_map(walked, fwn.hip_attn.unit_keys_for(dtype))
   if dmap is not None:
     dsbuf = torch.empty(max(dmap.ds_bytes(desc), 256), dtype=torch.uint8, device=dev)
 
@@ -675,14 +676,15 @@ def attention(args):
   value = total_flops / (ms_step * 1e-3) / 1e12
   # `value` counts the workload's live tiles, those of its own node order, so that it measures the
   # same work whatever the kernels walk; the per-kernel rates and the roofline count the tiles of
-  # the list the kernels walk.
-  unit_flops = D * 128 * 128 * walked.n_tiles * B * H
+  # the list each kernel walks.
+  per_tile = D * 128 * 128 * B * H
   # Algorithmic FLOPs per launch: forward 4*D per live entry; the backward's 10*D (FA2 count: S,
   # dP, dV, dK, dQ at 2*D each). The recomputing kernels split it as dQ 4*D (dQ + half of the S/dP
   # recompute) and dK/dV 6*D; with the dS exchange dK/dV computes S, dP, dV, dK (8*D) and dQ only
   # dQ (2*D).
-  algo = {"fwd": 4 * unit_flops, "dq": 4 * unit_flops, "dkv": 6 * unit_flops, "delta": 0,
-          "dkv_ds": 8 * unit_flops, "dq_ds": 2 * unit_flops}
+  algo = {"fwd": 4 * per_tile * walked.n_tiles, "dq": 4 * per_tile * walked_dq.n_tiles,
+          "dkv": 6 * per_tile * walked_kv.n_tiles, "delta": 0,
+          "dkv_ds": 8 * per_tile * walked_kv.n_tiles, "dq_ds": 2 * per_tile * walked_dq.n_tiles}
   dominant = max((k_ for k_ in per_solo if algo.get(k_)), key=lambda k_: per_solo[k_])
   achieved = algo[dominant] / (per_solo[dominant] * 1e-3) / 1e12
   peak = PEAK[cfg["dtype"]]
@@ -703,8 +705,11 @@ def attention(args):
                  "heads": H, "head_dim": D, "order": "hilbert" if cfg["reorder"] else "subdivision",
                  "sigma": cfg["sigma"], "live_tiles": T, "tile_density": round(tiles.density, 4),
                  "live_group_fraction": round(tiles.group_fraction, 4),
-                 "walked_tiles": walked.n_tiles, "walked_order": "given" if walked is tiles else "list",
-                 "walked_group_fraction": round(walked.group_fraction, 4),
+                 "walked_tiles": {"fwd": walked.n_tiles, "dq": walked_dq.n_tiles, "kv": walked_kv.n_tiles},
+                 "walked_layout": "given" if walked is tiles else "packed",
+                 "walked_group_fraction": {"fwd": round(walked.group_fraction, 4),
+                                           "dq": round(walked_dq.group_fraction, 4),
+                                           "kv": round(walked_kv.group_fraction, 4)},
                  "valid_entries": int(mask.nnz),
                  "item_tiles": {kn: walked.item_cap_for(B, H, kn) for kn in ("fwd", "dq", "kv")},
                  "order_tables": {"fwd": ts.n_work > 0, "dq": tsq.n_work > 0, "kv": tst.n_work > 0},
@@ -712,7 +717,7 @@ def attention(args):
       "roofline": {"bound": "mfma", "kernel": dominant, "achieved": round(achieved, 3), "peak": peak,
                    "unit": "TFLOP/s", "frac": round(achieved / peak, 4), "traffic": traffic,
                    "traffic_source": traffic_src, "ms": round(per_solo[dominant], 4),
-                   "work": "algorithmic FLOPs over whole live 128x128 tiles of the list the kernels walk "
+                   "work": "algorithmic FLOPs over whole 128x128 tiles of the list the kernel walks "
                            "(config.walked_tiles); they skip 32x32 groups without a valid element "
                            "(config.walked_group_fraction of them execute), so frac can exceed 1" + ("; bf16x3: fp32-equivalent products against the bf16 MFMA "
                                              "peak / 3" if x3 and peak != PEAK["f32"] else ""),

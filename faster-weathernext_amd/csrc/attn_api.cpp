@@ -136,7 +136,10 @@ int check_tiles(const fwn_attn_desc* d, const fwn_tiles* t, const char* name) {
                 t->n_split);
   if (t->flags & ~FWN_TILES_NODES) return fail(FWN_ERR_INVALID_ARG, "%s: unknown flags 0x%x", name, t->flags);
   if (t->flags & FWN_TILES_NODES) {
-    if (!t->node) return fail(FWN_ERR_TILES, "%s: null node table", name);
+    if (!t->row_node || (t->n_tiles > 0 && !t->col_node)) return fail(FWN_ERR_TILES, "%s: null node table", name);
+    if (!aligned16(t->col_node)) return fail(FWN_ERR_INVALID_ARG, "%s: col_node is not 16-byte aligned", name);
+    if ((int64_t)t->n_tiles * FWN_BLOCK * 4 >= (int64_t)1 << 31)
+      return fail(FWN_ERR_INVALID_ARG, "%s: too many tiles for a node table (%d)", name, t->n_tiles);
     // The kernels form row offsets as 24-bit products of the node and the row stride. The stride
     // is below 2^24 bytes for lists of two or more blocks (a slice spans less than 2 GiB).
     const int64_t elem = d->dtype == FWN_BF16 ? 2 : 4;
@@ -184,8 +187,7 @@ uint64_t workspace_bytes_for(const fwn_attn_desc* d, const fwn_tiles* t) {
 int split_to_slot(const fwn_attn_desc* d, const fwn_tiles* t, void* ws, int slot, const void* x, int64_t sb,
                   int64_t sn, int64_t sh, hipStream_t stream, const uint16_t** out) {
   uint16_t* dst = (uint16_t*)((char*)ws + round256(partial_bytes(d, t)) + (uint64_t)slot * round256(split_bytes(d)));
-  if (hipError_t e = launch_split_x3((const float*)x, sb, sn, sh, d->batch, d->n, d->heads, d->head_dim,
-                                     t->flags & FWN_TILES_NODES ? t->node : nullptr, dst, stream);
+  if (hipError_t e = launch_split_x3((const float*)x, sb, sn, sh, d->batch, d->n, d->heads, d->head_dim, dst, stream);
       e != hipSuccess)
     return fail(FWN_ERR_HIP, "bf16x3 split launch: %s", hipGetErrorString(e));
   *out = dst;
@@ -238,7 +240,8 @@ void set_tiles(KArgs& a, const fwn_tiles* t, void* ws) {
   a.lanes = t->lanes;
   a.groups = t->groups;
   a.halves = t->halves;
-  a.node = t->flags & FWN_TILES_NODES ? t->node : nullptr;
+  a.row_node = t->flags & FWN_TILES_NODES ? t->row_node : nullptr;
+  a.col_node = t->flags & FWN_TILES_NODES ? t->col_node : nullptr;
   a.items = (const int32_t*)t->items;
   a.split = t->split;
   a.n_tiles = t->n_tiles;
@@ -270,13 +273,15 @@ int64_t ds_unit_bytes(const fwn_ds_map* m) { return m->unit_keys == 16 ? 1024 : 
 // The dS exchange needs a map and buffer that match the call: the unit size of the dtype (16
 // keys for bf16, 32 for float32), n_units from fwn_tiles_ds_map, one (batch, head) slice of
 // units addressable with 32-bit offsets, and ds_bytes >= batch * heads * n_units * unit bytes.
-int check_ds(const fwn_attn_desc* d, const fwn_ds_map* m, const void* ds, uint64_t ds_bytes, bool need_ubase,
-             bool need_tmap) {
+int check_ds(const fwn_attn_desc* d, const fwn_ds_map* m, const void* ds, uint64_t ds_bytes, const fwn_tiles* tiles,
+             bool need_ubase, bool need_tmap) {
   if (!m) return fail(FWN_ERR_INVALID_ARG, "ds map is null");
   const int32_t want = d->dtype == FWN_BF16 ? 16 : 32;
   if (m->unit_keys != want)
     return fail(FWN_ERR_INVALID_ARG, "ds map: unit_keys %d, the %s exchange uses %d", m->unit_keys,
                 d->dtype == FWN_BF16 ? "bf16" : "float32", want);
+  if (tiles && m->table != (tiles->flags & FWN_TILES_NODES ? 1 : 0))
+    return fail(FWN_ERR_INVALID_ARG, "ds map: table %d does not fit the list's flags", m->table);
   if (m->n_units < 0 || m->n_units * ds_unit_bytes(m) >= ((int64_t)1 << 31))
     return fail(FWN_ERR_INVALID_ARG, "ds map: %lld units of %lld bytes (a (batch, head) slice must stay below 2 GiB)",
                 (long long)m->n_units, (long long)ds_unit_bytes(m));
@@ -454,7 +459,7 @@ int fwn_attn_bwd_dkv_ds_launch(const fwn_attn_desc* desc, const void* q, const v
                                void* workspace, uint64_t workspace_bytes, void* stream) {
   clear_error();
   if (int rc = check_desc(desc)) return rc;
-  if (int rc = check_ds(desc, map, ds, ds_bytes, false, true)) return rc;
+  if (int rc = check_ds(desc, map, ds, ds_bytes, tiles_t, false, true)) return rc;
   if (int rc = check_tensor(q, "q")) return rc;
   if (int rc = check_tensor(k, "k")) return rc;
   if (int rc = check_tensor(v, "v")) return rc;
@@ -490,7 +495,7 @@ int fwn_attn_bwd_dq_ds_launch(const fwn_attn_desc* desc, const void* k, const vo
                               uint64_t workspace_bytes, void* stream) {
   clear_error();
   if (int rc = check_desc(desc)) return rc;
-  if (int rc = check_ds(desc, map, ds, ds_bytes, true, false)) return rc;
+  if (int rc = check_ds(desc, map, ds, ds_bytes, tiles, true, false)) return rc;
   if (int rc = check_tensor(k, "k")) return rc;
   if (int rc = check_tensor(dq, "dq")) return rc;
   if (int rc = check_disjoint(desc, false, "dq")) return rc;
@@ -517,8 +522,8 @@ int fwn_attn_bwd_ds_launch(const fwn_attn_desc* desc, const void* q, const void*
   // The dS units are numbered by the positions of both lists: one order.
   if (tiles && tiles_t && tiles != tiles_t) {
     clear_error();
-    const int32_t* n0 = tiles->flags & FWN_TILES_NODES ? tiles->node : nullptr;
-    const int32_t* n1 = tiles_t->flags & FWN_TILES_NODES ? tiles_t->node : nullptr;
+    const int32_t* n0 = tiles->flags & FWN_TILES_NODES ? tiles->row_node : nullptr;
+    const int32_t* n1 = tiles_t->flags & FWN_TILES_NODES ? tiles_t->row_node : nullptr;
     if (n0 != n1) return fail(FWN_ERR_TILES, "tiles and tiles_t have different node tables");
   }
   if (int rc = fwn_attn_bwd_delta_launch(desc, o, dout, delta, stream)) return rc;

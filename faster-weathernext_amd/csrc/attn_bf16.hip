@@ -18,16 +18,17 @@
 // logical chunk, and the 32 lanes of a transpose read hit 4 consecutive rows x 4 consecutive
 // chunks.
 //
-// Node tables (G): a list laid out in a node order of its own walks fewer tiles and live groups than
-// one in the caller's order, and the kernels then address rows through the list's node table: the
-// LDS DMA takes any per-lane source address, so a gathered tile copy costs one LDS read and one
-// multiply-add per 1 KB instruction, the nodes of the next tile having been copied into LDS (512
-// bytes, one instruction of one wave) a tile ahead. Forward + backward, refinement-6 mesh, order
-// given by the caller -> the list's own: 16 hops, 4 heads, mesh order 1.269 -> 0.682 ms (17,183 ->
-// 7,047 tiles; 0.742 with the tensors themselves in such an order, events between the kernels); 8
-// hops, 8 members 6.64 -> 2.93 ms; 32 hops, 6 heads, Hilbert order 2.745 -> 2.54 ms. The variants
-// without G stay for lists whose order is good already (hip_attn.ORDERED_GAIN) and for callers of
-// the C ABI that pass no table.
+// Node tables (G): a list laid out for the kernels (a compact node order of its own, each block's
+// live columns packed into tiles) walks fewer tiles and live groups than one in the caller's order,
+// and the kernels then address rows through its node tables: the LDS DMA takes any per-lane source
+// address, so a gathered tile copy costs one LDS read and one multiply-add per 1 KB instruction, the
+// nodes of the next tile having been copied into LDS (512 bytes, one instruction of one wave) a tile
+// ahead. The forward's list packs single columns: a refinement-6 block with the 16-hop mask has 13
+// tiles of 88% live groups where the unpacked list has 22 of 56%. Forward + backward, us, list in the
+// caller's order -> laid out (in a compact order alone): 16 hops, 4 heads, mesh order 1261 -> 656
+// (682); 8 hops, 8 members 6645 -> 2681 (2928); 32 hops, 6 heads, Hilbert order 2740 -> 2469 (2539). The
+// forward alone, order alone -> packed: 190 -> 158, 793 -> 604 and 715 -> 632. The variants without G stay for lists
+// that no layout improves (hip_attn.LAID_OUT_GAIN) and for callers of the C ABI that pass no tables.
 //
 // Reference: pallas_attn.py:112-141 (forward), 161-215 (dQ, dK/dV), 274-311 (VJP driver).
 #include "attn_bf16_tiles.h"
@@ -85,9 +86,9 @@ __global__ void __launch_bounds__(NT, 2) fwd_kernel(KArgs a) {
     gnext = tile_groups(a, t0);
     if constexpr (G) {
       uint32_t nd[TileDma<D>::OPS];
-      dma.nodes(nd, node_block(a, kb));
+      dma.nodes(nd, tile_nodes(a, t0));
       dma.gather(rK, K, w, nd, snb);
-      if (w == 0 && t0 + 1 < t1) tab.load((t0 + 1) & 1, ((ci32_ptr)a.col)[t0 + 1], lane);
+      if (w == 0 && t0 + 1 < t1) tab.load((t0 + 1) & 1, t0 + 1, lane);
       wait_vmem();  // K(t0), its mask and group bits, the Q fragment and the nodes of tile t0 + 1
       dma.gather(rV, V, w, nd, snb);
     } else {
@@ -142,7 +143,7 @@ __global__ void __launch_bounds__(NT, 2) fwd_kernel(KArgs a) {
         uint32_t nd[TileDma<D>::OPS];
         dma.nodes(nd, tab.block((t + 1) & 1));
         dma.gather(rK, K, w, nd, snb, copy_next);
-        if (w == 0 && t + 2 < t1) tab.load(t & 1, ((ci32_ptr)a.col)[t + 2], lane);
+        if (w == 0 && t + 2 < t1) tab.load(t & 1, t + 2, lane);
       } else {
         dma.issue(rK, K, w, ((ci32_ptr)a.col)[t + 1] * BLK, snb, copy_next);
       }
@@ -260,10 +261,10 @@ __global__ void __launch_bounds__(NT, 2) dq_kernel(KArgs a) {
     hcur = tile_halves(a, t0);
     if constexpr (G) {
       uint32_t nd[TileDma<D>::OPS];
-      dma.nodes(nd, node_block(a, kb));
+      dma.nodes(nd, tile_nodes(a, t0));
       dma.gather(rK, K, w, nd, snb, 3u);
       dma.gather(rV, V, w, nd, snb, 3u);
-      if (w == 0) tab.load(t0 & 1, kb, lane);
+      if (w == 0) tab.load(t0 & 1, t0, lane);
     } else {
       dma.issue(rK, K, w, kb * BLK, snb, 3u);
       dma.issue(rV, V, w, kb * BLK, snb, 3u);
@@ -327,7 +328,7 @@ __global__ void __launch_bounds__(NT, 2) dq_kernel(KArgs a) {
       dma.nodes(nd, tab.block(t & 1));
       dma.gather(rK, K, w, nd, snb, copy & 12u);
       dma.gather(rV, V, w, nd, snb, copy & 12u);
-      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, ((ci32_ptr)a.col)[t + 1], lane);
+      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, t + 1, lane);
     } else {
       dma.issue(rK, K, w, kb * BLK, snb, copy & 12u);
       dma.issue(rV, V, w, kb * BLK, snb, copy & 12u);
@@ -488,16 +489,17 @@ __global__ void __launch_bounds__(NT, 2) dq_ds_kernel(KArgs a) {
   // read (live16 bit x: rows 16x .. 16x + 15), so the others are not copied (12% of the rows of
   // live 32-row groups at C3, 6% at the C5 shape; dQ -2% and -1.3%). Op `op` of this wave fills
   // rows 4 RPO op + RPO w .. + RPO - 1, inside one 16-row chunk.
-  // With a node table the rows are the nodes in LDS block `slot`, or (slot < 0, the first tile)
-  // in global memory.
-  auto copy16 = [&](lds_char* tile, int kb, int slot, uint32_t live16) {
+  // Rows of column block kb or, with node tables, of the nodes of tile t (read from LDS or, for the
+  // item's first tile, from global memory: `first` is a constant at every call, as a choice at run
+  // time puts global loads, and waits for the copies in flight, into the loop).
+  auto copy16 = [&](bool first, lds_char* tile, int t, int kb, uint32_t live16) {
     constexpr int RPO = Tile<D>::ROWS_PER_OP;
     uint32_t nd[TileDma<D>::OPS];
     if constexpr (G) {
-      if (slot < 0)
-        dma.nodes(nd, node_block(a, kb));
+      if (first)
+        dma.nodes(nd, tile_nodes(a, t));
       else
-        dma.nodes(nd, tab.block(slot));
+        dma.nodes(nd, tab.block(t & 1));
     }
     uint32_t base = (uint32_t)(uintptr_t)tile + (uint32_t)w * 1024u;
     asm volatile("" : "+s"(base));
@@ -528,10 +530,10 @@ __global__ void __launch_bounds__(NT, 2) dq_ds_kernel(KArgs a) {
     const uint32_t ht = hcur;
     const bool more = t + 1 < t1;
     const uint32_t hl = h1, ul = u1;
-    if (more) copy16(nxt, c1, (t + 1) & 1, live16(h1));
+    if (more) copy16(false, nxt, t + 1, c1, live16(h1));
     // The nodes of tile t + 2 go where tile t's were (read before this barrier).
     if constexpr (G) {
-      if (w == 0 && t + 2 < t1) tab.load(t & 1, c2, lane);
+      if (w == 0 && t + 2 < t1) tab.load(t & 1, t + 2, lane);
     }
     hcur = h1;
     c1 = c2;
@@ -579,7 +581,7 @@ __global__ void __launch_bounds__(NT, 2) dq_ds_kernel(KArgs a) {
   lds_char* K1 = (lds_char*)lk1;
   if (t0 < t1) {
     const uint32_t hf0 = tile_halves(a, t0);
-    copy16(K0, ((ci32_ptr)a.col)[t0], -1, live16(hf0));
+    copy16(true, K0, t0, ((ci32_ptr)a.col)[t0], live16(hf0));
     load_units(dsA, hf0, (uint32_t)((cmap_ptr)a.ubase)[t0]);
     hcur = hf0;
     if (t0 + 1 < t1) {
@@ -587,7 +589,7 @@ __global__ void __launch_bounds__(NT, 2) dq_ds_kernel(KArgs a) {
       h1 = tile_halves(a, t0 + 1);
       u1 = (uint32_t)((cmap_ptr)a.ubase)[t0 + 1];
       if constexpr (G) {
-        if (w == 0) tab.load((t0 + 1) & 1, c1, lane);
+        if (w == 0) tab.load((t0 + 1) & 1, t0 + 1, lane);
       }
     }
     if (t0 + 2 < t1) {
@@ -834,6 +836,7 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
   __shared__ __attribute__((aligned(1024))) char lds0[2 * TB + 1536];  // Q | dO | lse[128] | gap | delta[128]
   __shared__ __attribute__((aligned(1024))) char lds1[2 * TB + 1536];
   __shared__ __attribute__((aligned(16))) char lnode[G ? 2 * 4 * BLK : 16];
+  __shared__ __attribute__((aligned(16))) char lunit[G && DS ? 2 * 4 * UnitTab::WORDS : 16];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);  // keys 16 wid .. 16 wid + 15 of the block
   const int g = lane >> 4, t16 = lane & 15;
@@ -864,16 +867,16 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
   if constexpr (G) tab.init(a, (lds_char*)lnode);
   auto stats_wave = [&](int mode) { return mode == 0 ? wid == 0 : (mode == 1 && (wid & 3) == 0); };
   bool stats_cur = false;  // this wave copied the current tile's lse and delta (it rescales them)
-  // With a node table, slot is the LDS block of query block qb's nodes (< 0: read from global
-  // memory, the first tile).
-  auto issue = [&](int qb, lds_char* buf, uint32_t copy, int mode, int slot) {
+  // Tile t, of query block qb or, with node tables, of the tile's own nodes (read from LDS or, for the
+  // item's first tile, from global memory; `first` is a constant at every call).
+  auto issue = [&](bool first, int t, int qb, lds_char* buf, uint32_t copy, int mode) {
     if constexpr (G) {
       uint32_t nd[TileDma<D, true>::OPS];
       if (mode != 2) {
-        if (slot < 0)
-          dmaQ.nodes(nd, node_block(a, qb));
+        if (first)
+          dmaQ.nodes(nd, tile_nodes(a, t));
         else
-          dmaQ.nodes(nd, tab.block(slot));
+          dmaQ.nodes(nd, tab.block(t & 1));
       }
       if (mode == 0) {
         if (wid < 4) {
@@ -891,7 +894,7 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const uint32_t at = 64u * h + lane;
-          const uint32_t vo = 4u * (slot < 0 ? (uint32_t)node_block(a, qb)[at] : tab.block(slot)[at]);
+          const uint32_t vo = 4u * (first ? (uint32_t)tile_nodes(a, t)[at] : tab.block(t & 1)[at]);
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rL, (__attribute__((address_space(3))) void*)(stats + 256 * h), 4,
                                                    (int)vo, 0, 0, 0);
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rD, (__attribute__((address_space(3))) void*)(stats + 1024 + 256 * h),
@@ -930,7 +933,13 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
   rsrc_t rS;
   u32x4 dsv = {0u, 0u, 0u, 0u};
   uint32_t pend = 0u, ubc = 0u, hfc = 0u;
-  typedef const __attribute__((address_space(4))) uint32_t* cmap_ptr;
+  // With node tables: the numbers of this wave's units in the current tile, by query group, read from
+  // LDS during the step before (the choice of the copying wave right after the barrier, which needs
+  // hfc, then waits for nothing).
+  u32x4 uc = {0u, 0u, 0u, 0u}, ucn = uc;
+  uint32_t hfn = 0u;
+  UnitTab utab;
+  if constexpr (DS && G) utab.init(a, (lds_char*)lunit);
   if constexpr (DS) {
     rS = make_rsrc(a.ds + (int64_t)j.bh * (a.ds_slice_bytes >> 1), a.ds_slice_bytes);
     pend = a.ds_slice_bytes;
@@ -975,7 +984,7 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
         const uint32_t ns4 = (uint32_t)__builtin_popcount(hfc >> (s + 4) & 0x01010101u);
         mode = ((wid < 4) == (ns <= ns4)) ? 1 : 2;
       }
-      issue(cnext, nxt, any_rows(gnext), mode, (t + 1) & 1);
+      issue(false, t + 1, cnext, nxt, any_rows(gnext), mode);
       stats_nxt = stats_wave(mode);
     }
     if (t + 2 < t1) {
@@ -983,8 +992,16 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
       cnext = ((ci32_ptr)a.col)[t + 2];
       // The nodes of tile t + 2 go where tile t's were (read before this barrier).
       if constexpr (G) {
-        if (wid == 0) tab.load(t & 1, cnext, lane);
+        if (wid == 0) tab.load(t & 1, t + 2, lane);
       }
+    }
+    if constexpr (DS && G) {
+      if (t + 1 < t1) {  // landed by this barrier
+        ucn = utab.units((t + 1) & 1, wid);
+        hfn = utab.live((t + 1) & 1);
+      }
+      // The units of tile t + 2 go where tile t's were (read during the last step).
+      if (wid == 1 && t + 2 < t1) utab.load(t & 1, t + 2, lane);
     }
     uint32_t live, full;
     KeyWave<D>::live_units(mw, live, full);
@@ -995,16 +1012,24 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
         if constexpr (DS) {
           store_ds();
           kw.unit(cur, cur + TB, stats + 128 * c, stats + 1024 + 128 * c, c, mw, full >> c & 1u, g, a.c2, &dsv);
-          const uint32_t bit = 8u * c + (uint32_t)wid;
-          pend = (ubc + (uint32_t)__builtin_popcount(hfc & ((1u << bit) - 1u))) * 1024u;
+          if constexpr (G) {
+            // A unit the map does not have (-1: a map of other lists) lies past the slice.
+            pend = (int)uc[c] >= 0 ? uc[c] * 1024u : a.ds_slice_bytes;
+          } else {
+            const uint32_t bit = 8u * c + (uint32_t)wid;
+            pend = (ubc + (uint32_t)__builtin_popcount(hfc & ((1u << bit) - 1u))) * 1024u;
+          }
         } else {
           kw.unit(cur, cur + TB, stats + 128 * c, stats + 1024 + 128 * c, c, mw, full >> c & 1u, g, a.c2);
         }
       }
     if constexpr (DS) {
-      if (t + 1 < t1) {
-        ubc = ((cmap_ptr)a.tmap)[2 * (t + 1)];
-        hfc = ((cmap_ptr)a.tmap)[2 * (t + 1) + 1];
+      if constexpr (G) {
+        uc = ucn;
+        hfc = __builtin_amdgcn_readfirstlane(hfn);
+      } else if (t + 1 < t1) {
+        ubc = ((cu32_ptr)a.tmap)[2 * (t + 1)];
+        hfc = ((cu32_ptr)a.tmap)[2 * (t + 1) + 1];
       }
     }
     stats_cur = stats_nxt;
@@ -1024,12 +1049,20 @@ __global__ void __launch_bounds__(NT8, 1) dkv16_kernel(KArgs a) {
       cnext = ((ci32_ptr)a.col)[t0 + 1];
     }
     if constexpr (DS) {
-      ubc = ((cmap_ptr)a.tmap)[2 * t0];
-      hfc = ((cmap_ptr)a.tmap)[2 * t0 + 1];
+      if constexpr (G) {
+        const ci32_ptr m = (ci32_ptr)a.tmap + (int64_t)t0 * UnitTab::WORDS;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) uc[c] = (uint32_t)m[4 * wid + c];
+        hfc = (uint32_t)m[32];
+        if (wid == 1 && t0 + 1 < t1) utab.load((t0 + 1) & 1, t0 + 1, lane);
+      } else {
+        ubc = ((cu32_ptr)a.tmap)[2 * t0];
+        hfc = ((cu32_ptr)a.tmap)[2 * t0 + 1];
+      }
     }
-    issue(((ci32_ptr)a.col)[t0], b0, any_rows(tile_groups(a, t0)), 0, -1);
+    issue(true, t0, ((ci32_ptr)a.col)[t0], b0, any_rows(tile_groups(a, t0)), 0);
     if constexpr (G) {
-      if (wid == 0 && t0 + 1 < t1) tab.load((t0 + 1) & 1, cnext, lane);
+      if (wid == 0 && t0 + 1 < t1) tab.load((t0 + 1) & 1, t0 + 1, lane);
     }
     stats_cur = wid == 0;
   }
@@ -1057,7 +1090,7 @@ hipError_t launch_dg(Kind kind, const KArgs& a, hipStream_t stream) {
 
 template <int D>
 hipError_t launch_d(Kind kind, const KArgs& a, hipStream_t stream) {
-  return a.node ? launch_dg<D, true>(kind, a, stream) : launch_dg<D, false>(kind, a, stream);
+  return a.row_node ? launch_dg<D, true>(kind, a, stream) : launch_dg<D, false>(kind, a, stream);
 }
 
 }  // namespace

@@ -77,8 +77,8 @@ struct TileDma {
     voff = (uint32_t)row * snb + chunk;
   }
 
-  // With a node table: the nodes of this lane's rows of a tile, from its column block's 128 entries
-  // (in global memory or in LDS).
+  // With a node table: the nodes of this lane's rows of a tile, from the tile's 128 entries (in
+  // global memory or in LDS).
   template <typename Table>
   __device__ __forceinline__ void nodes(uint32_t (&nd)[OPS], Table node) const {
 #pragma unroll

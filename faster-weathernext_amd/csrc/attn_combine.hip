@@ -80,7 +80,7 @@ __global__ void __launch_bounds__(kThreads) fwd_combine_kernel(KArgs a) {
   const int r = cell.r, d = cell.d;
   const int pos = s.blk * BLK + r;
   if (!s.ok) return;
-  const int row = a.node ? a.node[pos] : pos;  // the node table covers every block
+  const int row = a.row_node ? a.row_node[pos] : pos;  // the table covers every block
   if ((unsigned)row >= (unsigned)a.n) return;
   float M = -__builtin_inff();
   for (int c = 0; c < s.np; ++c) M = fmaxf(M, slot_ptr<D>(a, s, c)[128 * D + r]);
@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(kThreads) bwd_combine_kernel(KArgs a) {
   const int r = cell.r, d = cell.d;
   const int pos = s.blk * BLK + r;
   if (!s.ok) return;
-  const int row = a.node ? a.node[pos] : pos;  // the node table covers every block
+  const int row = a.row_node ? a.row_node[pos] : pos;  // the table covers every block
   if ((unsigned)row >= (unsigned)a.n) return;
   const int64_t out_off = (int64_t)s.b * a.sb + (int64_t)s.h * a.sh + (int64_t)row * a.sn + d;
 #pragma unroll

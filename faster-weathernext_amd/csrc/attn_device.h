@@ -118,28 +118,24 @@ struct Job {
   bool skip;     // an empty entry of the order table: the workgroup does nothing
 };
 
-// The node (row of the tensors) at position `pos` of the list's order: the position itself, or
-// with a node table (G) its entry. Positions past the last block (a malformed item) are past the
-// tensors' rows, whose loads read zeros and whose stores drop.
+// The node (row of the tensors) of row `pos` of the list's blocks: the row itself, or with node
+// tables (G) its entry. Rows past the last block (a malformed item) are past the tensors' rows,
+// whose loads read zeros and whose stores drop.
 template <bool G>
 __device__ __forceinline__ int node_at(const KArgs& a, int pos) {
-  if constexpr (G) return pos < a.n_blocks * BLK ? a.node[pos] : a.n;
+  if constexpr (G) return pos < a.n_blocks * BLK ? a.row_node[pos] : a.n;
   return pos;
 }
 
-// The 128 node table entries of column block kb (a malformed list's blocks past the last read the
-// last one's).
-__device__ __forceinline__ const int32_t* node_block(const KArgs& a, int kb) {
-  const uint32_t last = (uint32_t)a.n_blocks - 1u;
-  return a.node + (int64_t)((uint32_t)kb < last ? (uint32_t)kb : last) * BLK;
-}
+// The nodes of the 128 columns of tile t (tiles of an item lie in [0, n_tiles)).
+__device__ __forceinline__ const int32_t* tile_nodes(const KArgs& a, int t) { return a.col_node + (int64_t)t * BLK; }
 
 // Byte offset of a row from a node table: node * stride, both below 2^24 (one v_mul_u32_u24 or
 // v_mad_u32_u24; a 32-bit product takes four times as long).
 __device__ __forceinline__ uint32_t row_bytes(uint32_t node, uint32_t stride) { return __umul24(node, stride); }
 
-// The node table of the tiles being copied, two blocks of 128 entries in LDS: block `slot` is
-// loaded by one wave (lanes 0-31, 16 bytes each) a tile before the copies that read it.
+// The nodes of the tiles being copied, 128 entries each, in two LDS blocks: block `slot` is loaded by
+// one wave (lanes 0-31, 16 bytes each) a tile before the copies that read it.
 struct NodeTab {
   typedef const __attribute__((address_space(3))) uint32_t* ptr;
   lds_char* base;
@@ -147,14 +143,40 @@ struct NodeTab {
 
   __device__ __forceinline__ void init(const KArgs& a, lds_char* lds) {
     base = lds;
-    r = make_rsrc(a.node, (uint32_t)a.n_blocks * (BLK * 4));
+    r = make_rsrc(a.col_node, (uint32_t)a.n_tiles * (BLK * 4));
   }
-  __device__ __forceinline__ void load(int slot, int kb, int lane) const {
+  __device__ __forceinline__ void load(int slot, int t, int lane) const {
     if (lane < 32)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(base + slot * (BLK * 4)), 16,
-                                               (kb * BLK + 4 * lane) * 4, 0, 0, 0);
+                                               (t * BLK + 4 * lane) * 4, 0, 0, 0);
   }
   __device__ __forceinline__ ptr block(int slot) const { return (ptr)(base + slot * (BLK * 4)); }
+};
+
+// The dS unit numbers of the tiles (fwn_tiles_unit_map: 36 words each) in two LDS blocks, loaded like
+// the nodes (lanes 0-8). They go through LDS because each tile's are read once: a scalar load of
+// them misses the scalar cache every time, and a wave's LDS waits would wait for it as well.
+struct UnitTab {
+  static constexpr int WORDS = 36;
+  lds_char* base;
+  rsrc_t r;
+
+  __device__ __forceinline__ void init(const KArgs& a, lds_char* lds) {
+    base = lds;
+    r = make_rsrc(a.tmap, (uint32_t)a.n_tiles * (WORDS * 4));
+  }
+  __device__ __forceinline__ void load(int slot, int t, int lane) const {
+    if (lane < WORDS / 4)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(base + slot * (WORDS * 4)), 16,
+                                               t * (WORDS * 4) + 16 * lane, 0, 0, 0);
+  }
+  // Units of 16-key group kg by query group, and the tile's live word.
+  __device__ __forceinline__ u32x4 units(int slot, int kg) const {
+    return *(const __attribute__((address_space(3))) u32x4*)(base + slot * (WORDS * 4) + 16 * kg);
+  }
+  __device__ __forceinline__ uint32_t live(int slot) const {
+    return *(const __attribute__((address_space(3))) uint32_t*)(base + slot * (WORDS * 4) + 128);
+  }
 };
 
 // Without an order table, workgroups are dealt round-robin over the 8 XCDs, each with its own

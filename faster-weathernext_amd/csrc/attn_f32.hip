@@ -7,11 +7,12 @@
 // needed. Tiles stream into LDS by LDS DMA, double-buffered: in 64-row halves for the backward
 // kernels (HalfDma), in 32-row key groups for the forward (GroupDma).
 //
-// Node tables (G): the rows of a list laid out in an order of its own are gathered by the same LDS
-// DMA instructions. The step-streamed kernels (forward, 16-key dK/dV) load the next step's nodes into
-// registers a step ahead, the tile-streamed ones the next tile's into LDS. Refinement-6 mesh, before
-// -> after: 8-hop 4x128 forward in mesh order 1.915 -> 0.675 ms (0.637 with the tensors themselves in
-// such an order); 32-hop Hilbert 6x128 forward + backward 18.39 -> 16.77 ms.
+// Node tables (G): the rows of a list laid out for the kernels are gathered by the same LDS DMA
+// instructions. The step-streamed kernels (forward, 16-key dK/dV) load the next step's nodes into
+// registers a step ahead, the tile-streamed ones the next tile's into LDS. Refinement-6 mesh, list in
+// the caller's order -> in a compact order -> packed as well: 8-hop 4x128 forward in mesh order 1917 ->
+// 675 -> 485 us; 32-hop Hilbert 6x128 forward + backward 18.45 -> 16.8 -> 16.3 ms (the forward 5.77 ->
+// 5.20 -> 4.65).
 //
 // Reference: pallas_attn.py:112-141 (forward), 161-215 (dQ, dK/dV), 274-311 (VJP driver).
 #include "attn_device.h"
@@ -275,7 +276,7 @@ __global__ void __launch_bounds__(NT, 2) fwd_f32g_kernel(KArgs a) {
     return true;
   };
   auto pos0 = [&](int t, int c) { return ((ci32_ptr)a.col)[t] * BLK + 32 * c; };
-  auto nodes_of = [&](int t, int c) { return node_block(a, ((ci32_ptr)a.col)[t]) + 32 * c; };
+  auto nodes_of = [&](int t, int c) { return tile_nodes(a, t) + 32 * c; };
   // The K and V rows of step (t, c); with a node table, the rows of nodes nd.
   auto copy = [&](char* gb, int t, int c, const uint32_t (&nd)[GroupDma<D>::OPS]) {
     if constexpr (G) {
@@ -433,9 +434,9 @@ __global__ void __launch_bounds__(NT, 1) dq_f32_kernel(KArgs a) {
     gcur = tile_groups(a, t0);
     const int kb = ((ci32_ptr)a.col)[t0];
     if constexpr (G) {
-      dma.gather(rK, h0, node_block(a, kb), snb, w, 0, any_rows(gcur));
-      dma.gather(rV, h0 + HB, node_block(a, kb), snb, w, 0, any_rows(gcur));
-      if (w == 0) tab.load(t0 & 1, kb, lane);
+      dma.gather(rK, h0, tile_nodes(a, t0), snb, w, 0, any_rows(gcur));
+      dma.gather(rV, h0 + HB, tile_nodes(a, t0), snb, w, 0, any_rows(gcur));
+      if (w == 0) tab.load(t0 & 1, t0, lane);
     } else {
       copy_half(h0, kb, 0, 0, any_rows(gcur));
     }
@@ -451,7 +452,7 @@ __global__ void __launch_bounds__(NT, 1) dq_f32_kernel(KArgs a) {
     copy_half(h1, kb, t & 1, 1, any_rows(gt));
     // The nodes of tile t + 1 go where tile t - 1's were (last read before this barrier).
     if constexpr (G) {
-      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, ((ci32_ptr)a.col)[t + 1], lane);
+      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, t + 1, lane);
     }
     if (t + 1 < t1) gcur = tile_groups(a, t + 1);
     // Fenced, so that one group's reads and MFMAs do not overlap the next group's registers.
@@ -575,8 +576,8 @@ __global__ void __launch_bounds__(NT, 2) dq_f32_ds_kernel(KArgs a) {
     ucur = (uint32_t)((cmap_ptr)a.ubase)[t0];
     const int kb = ((ci32_ptr)a.col)[t0];
     if constexpr (G) {
-      dma.gather(rK, h0, node_block(a, kb), snb, w, 0, any_rows(gcur));
-      if (w == 0) tab.load(t0 & 1, kb, lane);
+      dma.gather(rK, h0, tile_nodes(a, t0), snb, w, 0, any_rows(gcur));
+      if (w == 0) tab.load(t0 & 1, t0, lane);
     } else {
       copy_half(h0, kb, 0, 0, any_rows(gcur));
     }
@@ -593,7 +594,7 @@ __global__ void __launch_bounds__(NT, 2) dq_f32_ds_kernel(KArgs a) {
     copy_half(h1, kb, t & 1, 1, any_rows(gt));
     // The nodes of tile t + 1 go where tile t - 1's were (last read before this barrier).
     if constexpr (G) {
-      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, ((ci32_ptr)a.col)[t + 1], lane);
+      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, t + 1, lane);
     }
     load_units(dsB, gt, ut, 1);
     if (t + 1 < t1) {
@@ -641,6 +642,7 @@ __global__ void __launch_bounds__(NT, 1) dkv_f32_kernel(KArgs a) {
   __shared__ __attribute__((aligned(1024))) char h0[2 * HB + 512];
   __shared__ __attribute__((aligned(1024))) char h1[2 * HB + 512];
   __shared__ __attribute__((aligned(16))) char lnode[G ? 2 * 4 * BLK : 16];
+  __shared__ __attribute__((aligned(16))) char lunit[G && DS ? 2 * 4 * UnitTab::WORDS : 16];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 31, g = lane >> 5;
@@ -673,6 +675,9 @@ __global__ void __launch_bounds__(NT, 1) dkv_f32_kernel(KArgs a) {
   // the current tile's first unit and group word.
   char* dsb = nullptr;
   uint32_t dsl = 0u, ubc = 0u, gfc = 0u;
+  int tcur = 0;
+  UnitTab utab;
+  if constexpr (DS && G) utab.init(a, (lds_char*)lunit);
   typedef const __attribute__((address_space(4))) uint32_t* cmap_ptr;
   if constexpr (DS) {
     dsb = (char*)a.ds + (int64_t)j.bh * a.ds_slice_bytes;
@@ -745,11 +750,20 @@ __global__ void __launch_bounds__(NT, 1) dkv_f32_kernel(KArgs a) {
       dp[r] = p * dp[r];
     }
     if constexpr (DS) {
-      const uint32_t bit = 4u * (uint32_t)sb + (uint32_t)w;
-      const uint32_t so = (ubc + (uint32_t)__builtin_popcount(gfc & 0xffffu & ((1u << bit) - 1u))) * 4096u;
+      uint32_t so;
+      bool have;
+      if constexpr (G) {
+        const int u = (int)utab.units(tcur & 1, 2 * w)[sb];
+        so = (uint32_t)u * 4096u;
+        have = u >= 0;
+      } else {
+        const uint32_t bit = 4u * (uint32_t)sb + (uint32_t)w;
+        so = (ubc + (uint32_t)__builtin_popcount(gfc & 0xffffu & ((1u << bit) - 1u))) * 4096u;
+        have = gfc >> bit & 1u;
+      }
       // A plain pointer has no range check: store only a unit the map has, inside the slice (a
       // map of other lists cannot write outside the buffer).
-      if ((gfc >> bit & 1u) && so + 4096u <= a.ds_slice_bytes) {
+      if (have && (uint64_t)so + 4096u <= a.ds_slice_bytes) {
         float* u = (float*)(dsb + (so + dsl));
 #pragma unroll
         for (int r = 0; r < 16; ++r) u[4 * (16 * (r >> 3) + (r & 7))] = dp[r];
@@ -781,8 +795,11 @@ __global__ void __launch_bounds__(NT, 1) dkv_f32_kernel(KArgs a) {
     gcur = tile_groups(a, t0);
     const int qb = ((ci32_ptr)a.col)[t0];
     if constexpr (G) {
-      gather_half(h0, node_block(a, qb), 0, any_rows(gcur));
-      if (w == 0) tab.load(t0 & 1, qb, lane);
+      gather_half(h0, tile_nodes(a, t0), 0, any_rows(gcur));
+      if (w == 0) tab.load(t0 & 1, t0, lane);
+      if constexpr (DS) {
+        if (w == 1) utab.load(t0 & 1, t0, lane);
+      }
     } else {
       copy_half(h0, qb, 0, 0, any_rows(gcur));
     }
@@ -794,16 +811,22 @@ __global__ void __launch_bounds__(NT, 1) dkv_f32_kernel(KArgs a) {
     const uint32_t gt = gcur;
     const uint32_t live = gt >> (4 * w) & 15u;  // query groups with p = 0 throughout are skipped
     if constexpr (DS) {
-      ubc = ((cmap_ptr)a.tmap)[2 * t];
-      gfc = ((cmap_ptr)a.tmap)[2 * t + 1];
+      tcur = t;
+      if constexpr (!G) {
+        ubc = ((cmap_ptr)a.tmap)[2 * t];
+        gfc = ((cmap_ptr)a.tmap)[2 * t + 1];
+      }
     }
     wait_vmem();  // this wave's part of half 0 of tile t, and the mask bits
     scale_lse(h0);
     __syncthreads();  // half 0 landed; every wave is done with half 1 of tile t - 1
     copy_half(h1, qb, t & 1, 1, any_rows(gt));
-    // The nodes of tile t + 1 go where tile t - 1's were (last read before this barrier).
+    // The nodes and units of tile t + 1 go where tile t - 1's were (last read before this barrier).
     if constexpr (G) {
-      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, ((ci32_ptr)a.col)[t + 1], lane);
+      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, t + 1, lane);
+      if constexpr (DS) {
+        if (w == 1 && t + 1 < t1) utab.load((t + 1) & 1, t + 1, lane);
+      }
     }
     if (t + 1 < t1) gcur = tile_groups(a, t + 1);
     // Fenced, so that one group's reads and MFMAs do not overlap the next group's registers.
@@ -1047,9 +1070,15 @@ __global__ void __launch_bounds__(256, 2) dkv16_f32_kernel(KArgs a) {
     return true;
   };
   auto pos0 = [&](int t, int c) { return ((ci32_ptr)a.col)[t] * BLK + 32 * c; };
-  // The tensors' row at position lane % 32 of step (t, c): a node, loaded a step before its copy.
+  // The tensors' row of column lane % 32 of step (t, c): with node tables, lanes 0-31 hold its node and
+  // lane 32 the step's dS unit, loaded a step before they are used (a scalar load of the unit would
+  // miss the scalar cache, and the wave's LDS waits would wait for it).
   auto lane_row = [&](int t, int c) {
-    if constexpr (G) return node_block(a, ((ci32_ptr)a.col)[t])[32 * c + (lane & 31)];
+    if constexpr (G) {
+      const int32_t* p = tile_nodes(a, t) + 32 * c + (lane & 31);
+      if constexpr (DS) p = lane < 32 ? p : a.tmap + (int64_t)t * UnitTab::WORDS + 4 * kg + c;
+      return *p;
+    }
     return pos0(t, c) + (lane & 31);
   };
   // Step (t, c)'s rows of Q (plane 0) and dO (plane 1), one padded row per instruction: wave w copies
@@ -1085,8 +1114,11 @@ __global__ void __launch_bounds__(256, 2) dkv16_f32_kernel(KArgs a) {
   bool vc = take(tc, cc), vn = false, vm = false;
   uint64_t mwc = 0, mwn = 0;
   int rown = 0, rowm = 0;  // lane rows of steps (tn, cn) and (tm, cm)
+  int unitc = -1;          // unit of step (tc, cc), with node tables
   if (vc) {
-    copy(b0, tc, cc, lane_row(tc, cc));
+    const int rowc = lane_row(tc, cc);
+    copy(b0, tc, cc, rowc);
+    unitc = __builtin_amdgcn_readlane(rowc, 32);
     mwc = mword[(int64_t)tc * 256];
     vn = take(tn, cn);
     if constexpr (G) {
@@ -1122,11 +1154,16 @@ __global__ void __launch_bounds__(256, 2) dkv16_f32_kernel(KArgs a) {
     bool have_unit = false;
     uint32_t u_idx = 0u;
     if constexpr (DS) {
-      const uint32_t ub = ((cmap_ptr)a.tmap)[2 * tc];
-      const uint32_t gw = ((cmap_ptr)a.tmap)[2 * tc + 1];
-      const uint32_t bit = 4u * (uint32_t)cc + (uint32_t)(kg >> 1);
-      have_unit = (gw >> bit & 1u) != 0u;
-      u_idx = ub + (uint32_t)__builtin_popcount(gw & 0xffffu & ((1u << bit) - 1u));
+      if constexpr (G) {
+        have_unit = unitc >= 0;
+        u_idx = (uint32_t)unitc;
+      } else {
+        const uint32_t ub = ((cmap_ptr)a.tmap)[2 * tc];
+        const uint32_t gw = ((cmap_ptr)a.tmap)[2 * tc + 1];
+        const uint32_t bit = 4u * (uint32_t)cc + (uint32_t)(kg >> 1);
+        have_unit = (gw >> bit & 1u) != 0u;
+        u_idx = ub + (uint32_t)__builtin_popcount(gw & 0xffffu & ((1u << bit) - 1u));
+      }
     }
     // One store path after the unit (dS of a unit the map has, zeros where these 16 keys have no
     // valid element): a store inside the unit's branch, and another beside it, made the register
@@ -1144,6 +1181,7 @@ __global__ void __launch_bounds__(256, 2) dkv16_f32_kernel(KArgs a) {
       tn = tm;
       cn = cm;
       vn = vm;
+      unitc = __builtin_amdgcn_readlane(rown, 32);
       rown = rowm;
       vm = vn && take(tm, cm);
     } else {
@@ -1266,7 +1304,7 @@ hipError_t launch_d(Kind kind, const KArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL((delta_kernel<float, D>), (delta_grid<float, D>(a)), dim3(NT), 0, stream, a);
     return hipGetLastError();
   }
-  return a.node ? launch_dg<D, true>(kind, a, stream) : launch_dg<D, false>(kind, a, stream);
+  return a.row_node ? launch_dg<D, true>(kind, a, stream) : launch_dg<D, false>(kind, a, stream);
 }
 
 template <int D>

@@ -24,16 +24,18 @@ struct KArgs {
   const uint32_t* halves;  // per tile: bit 8r + 2c + h = ... in columns 32c + 16h..; NULL = all live
   const int32_t* items;   // fwn_item[n_items] as int32 quadruples (block, t0, t1, part)
   const int32_t* split;   // [n_split * 3] block, first partial slot, slot count (combine pass)
-  const int32_t* node;    // [n_blocks * 128] node at each position of the list's own order (n past the last),
-                          //   or NULL: positions are nodes
+  const int32_t* row_node;  // [n_blocks * 128] node of each row of the list's blocks (n past the last), or
+                            //   NULL: the list is in node order
+  const int32_t* col_node;  // [n_tiles * 128] node of each tile column (n: padding), with row_node
   const int32_t* order;   // order table: [n_order][2] (pair b * heads + h, item) per workgroup, or NULL
   float* work;            // partial slots: [n_parts][batch * heads][128][2 * head_dim + 2] float32
   uint16_t* ds;           // dS units (bf16 backward with the dS exchange): [batch * heads][n_units][512]
   const int32_t* ubase;   // dq from dS: first unit of each tile of the forward list
-  const int32_t* tmap;    // dK/dV writing dS: per transposed tile, (ubase, halves) of the forward tile
+  const int32_t* tmap;    // dK/dV writing dS: per transposed tile, (ubase, halves) of the forward tile; with
+                          //   row_node 36 words per tile (fwn_tiles_unit_map)
   uint32_t ds_slice_bytes;  // bytes of one (batch, head) slice of ds: n_units * 1024
   const uint16_t* xa;     // bf16x3 kernels: split operands, [batch * heads][n][2][head_dim] bf16 (hi row,
-  const uint16_t* xb;     //   lo row; rows in the list's order; written by the split pass): forward k, v; dK/dV q, dout; dQ k
+  const uint16_t* xb;     //   lo row; written by the split pass): forward k, v; dK/dV q, dout; dQ k
   uint32_t xslice_bytes;  // bytes of one (batch, head) slice of xa / xb: n * 4 * head_dim
   int32_t n, heads, batch, n_blocks, n_tiles, n_items, n_parts, n_split, n_order;
   int64_t sb, sn, sh;     // strides of q, k, v, dq, dk, dv
@@ -55,10 +57,9 @@ hipError_t launch_f32(Kind kind, int head_dim, const KArgs& a, hipStream_t strea
 hipError_t launch_delta_bf16(int head_dim, const KArgs& a, hipStream_t stream);      // attn_f32.hip
 hipError_t launch_x3(Kind kind, int head_dim, const KArgs& a, hipStream_t stream);    // attn_x3.hip: kFwd, kDkvDs, kDqDs
 // Splits a float32 [batch, n, heads, head_dim] tensor (element strides sb, sn, sh) into dst,
-// [batch * heads][n][2][head_dim] bf16: hi = bf16(x), lo = bf16(x - hi), rows in the order of the
-// node table `node` (NULL: node order) (attn_x3.hip).
+// [batch * heads][n][2][head_dim] bf16: hi = bf16(x), lo = bf16(x - hi) (attn_x3.hip).
 hipError_t launch_split_x3(const float* src, int64_t sb, int64_t sn, int64_t sh, int batch, int n, int heads,
-                           int head_dim, const int32_t* node, uint16_t* dst, hipStream_t stream);
+                           int head_dim, uint16_t* dst, hipStream_t stream);
 hipError_t launch_combine(Kind kind, int dtype, int head_dim, const KArgs& a,
                           hipStream_t stream);                                     // attn_combine.hip
 

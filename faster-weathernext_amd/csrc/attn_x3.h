@@ -67,10 +67,15 @@ struct X3Dma {
   static constexpr int NI = 32 / RPO;
   static constexpr int GB = 32 * 2 * D;  // bytes of one plane
   static constexpr int XROW = 4 * D;     // bytes of one split row (hi, lo)
+  static constexpr int ROWS = NI >= 4 ? NI / 4 : 1;  // distinct rows of a lane in one plane's instructions
   uint32_t voff;
+  uint32_t chunk;  // this lane's chunk alone, and its row within an instruction's (node tables)
+  uint32_t rl;
 
   __device__ __forceinline__ void init(int w, int lane) {
     const int row = RPO * (w % NI) + lane / C;
+    rl = (uint32_t)(lane / C);
+    chunk = (uint32_t)(((lane % C) ^ swz<C>(row)) << 4);
     voff = (uint32_t)(lane / C) * XROW + (uint32_t)(((lane % C) ^ swz<C>(row)) << 4);
   }
 
@@ -92,6 +97,44 @@ struct X3Dma {
       }
       if (!(planes >> plane & 1u)) continue;
       const uint32_t src = (uint32_t)(row0 + RPO * sub) * XROW + voff + (uint32_t)(plane & 1) * (2 * D);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          m < D / 32 ? rA : rB,
+          (__attribute__((address_space(3))) void*)(uintptr_t)(base + (uint32_t)(plane * GB + sub * 1024)), 16,
+          (int)src, 0, 0, 0);
+    }
+  }
+
+  // The nodes of this lane's rows of a 32-row group, from the group's 32 entries; and issue() of the
+  // split rows of nodes na (planes 0, 1) and nb (planes 2, 3).
+  template <typename Table>
+  __device__ __forceinline__ void nodes(uint32_t (&nd)[ROWS], Table node, int w) const {
+#pragma unroll
+    for (int k = 0; k < ROWS; ++k) nd[k] = (uint32_t)node[RPO * (NI >= 4 ? w + 4 * k : w & 1) + rl];
+  }
+  // The same from entry i in lane i % 32 of `lanes`.
+  __device__ __forceinline__ void nodes(uint32_t (&nd)[ROWS], int lanes, int w) const {
+#pragma unroll
+    for (int k = 0; k < ROWS; ++k)
+      nd[k] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(4u * ((uint32_t)(RPO * (NI >= 4 ? w + 4 * k : w & 1)) + rl)), lanes);
+  }
+  __device__ __forceinline__ void gather(rsrc_t rA, rsrc_t rB, lds_char* buf, const uint32_t (&na)[ROWS],
+                                         const uint32_t (&nb)[ROWS], int w, uint32_t planes = 15u) const {
+    uint32_t base = (uint32_t)(uintptr_t)buf;
+    asm volatile("" : "+s"(base));
+#pragma unroll
+    for (int m = 0; m < D / 16; ++m) {
+      int plane, sub, k = 0;
+      if constexpr (NI >= 4) {
+        plane = 4 * m / NI;
+        sub = w + (4 * m) % NI;
+        k = m % (NI / 4);
+      } else {
+        plane = 2 * m + (w >> 1);
+        sub = w & 1;
+      }
+      if (!(planes >> plane & 1u)) continue;
+      const uint32_t nd = m < D / 32 ? na[k] : nb[k];
+      const uint32_t src = row_bytes(nd, XROW) + chunk + (uint32_t)(plane & 1) * (2 * D);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           m < D / 32 ? rA : rB,
           (__attribute__((address_space(3))) void*)(uintptr_t)(base + (uint32_t)(plane * GB + sub * 1024)), 16,

@@ -10,10 +10,9 @@
 // The operands that stream through LDS (forward: K, V; dK/dV: Q, dO; dQ: K) are split once per
 // call by split_x3_kernel into [batch * heads][n][2][D] bf16 (hi row, then lo row) and copied by
 // 32-row group; the operands a wave keeps in registers (forward: Q; dK/dV: its K and V rows) are
-// split when loaded; P and dS are split in registers. A list laid out in a node order of its own gets
-// its streamed operands in that order from the split pass, so only the register rows, the statistics
-// and the outputs go through the node table (32-hop Hilbert 6x128 forward + backward at refinement
-// 6: 6.92 -> 6.35 ms against the given order).
+// split when loaded; P and dS are split in registers. Lists
+// with node tables gather the split rows as the float32 kernels gather theirs (32-hop Hilbert 6x128
+// forward + backward at refinement 6: 6.96 -> 6.17 ms against the list in the caller's order).
 //
 // The backward is the dS exchange (5 contractions per tile): dK/dV computes S, dP, dV, dK and
 // writes each 32 x 32 dS group as hi and lo bf16 (4 KB, the float32 exchange's unit size and
@@ -33,22 +32,17 @@ struct SplitArgs {
   uint16_t* dst;
   int64_t sb, sn, sh;  // element strides of src
   int32_t batch, n, heads, d;
-  const int32_t* node;  // the row of src at each position of the list's own order, or NULL
 };
 
 // One thread per 8 consecutive elements of a row: 32 bytes read, 16 bytes of hi and 16 of lo
-// written. dst is [batch * heads][n][2][d]: (batch, head) slices of n split rows, in the order of the
-// list that streams them (with its node table the split pass is where the rows are gathered: its
-// reads are whole rows either way).
+// written. dst is [batch * heads][n][2][d]: (batch, head) slices of n split rows.
 __global__ void __launch_bounds__(256) split_x3_kernel(SplitArgs s) {
   const uint32_t per_row = (uint32_t)s.d / 8u;
   const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
   const uint32_t rows = (uint32_t)s.batch * (uint32_t)s.heads * (uint32_t)s.n;
   if (idx >= rows * per_row) return;
   const uint32_t r = idx / per_row, c = idx - r * per_row;
-  const uint32_t bh = r / (uint32_t)s.n, pos = r - bh * (uint32_t)s.n;
-  const uint32_t node = s.node ? (uint32_t)s.node[pos] : pos;
-  if (node >= (uint32_t)s.n) return;
+  const uint32_t bh = r / (uint32_t)s.n, node = r - bh * (uint32_t)s.n;
   const uint32_t b = bh / (uint32_t)s.heads, h = bh - b * (uint32_t)s.heads;
   const float* p = s.src + (int64_t)b * s.sb + (int64_t)node * s.sn + (int64_t)h * s.sh + 8 * c;
   const f32x4 x0 = *(const f32x4*)p, x1 = *(const f32x4*)(p + 4);
@@ -146,24 +140,45 @@ __global__ void __launch_bounds__(NT, 2) fwd_x3_kernel(KArgs a) {
     rem &= rem - 1u;
     return true;
   };
-  auto copy = [&](lds_char* buf, int t, int c) { dma.issue(rK, rV, buf, ((ci32_ptr)a.col)[t] * BLK + 32 * c, w); };
+  // With node tables, the node of column lane % 32 of step (t, c), loaded a step before its copy.
+  auto lane_node = [&](int t, int c) {
+    if constexpr (G) return tile_nodes(a, t)[32 * c + (lane & 31)];
+    return 0;
+  };
+  auto copy = [&](lds_char* buf, int t, int c, int lnode) {
+    if constexpr (G) {
+      uint32_t nd[X3Dma<D>::ROWS];
+      dma.nodes(nd, lnode, w);
+      dma.gather(rK, rV, buf, nd, nd, w);
+    } else {
+      dma.issue(rK, rV, buf, ((ci32_ptr)a.col)[t] * BLK + 32 * c, w);
+    }
+  };
   lds_char* b0 = (lds_char*)gb0;
   lds_char* b1 = (lds_char*)gb1;
-  int tc = 0, cc = 0, tn = 0, cn = 0;
-  bool vc = take(tc, cc), vn = false;
+  int tc = 0, cc = 0, tn = 0, cn = 0, tm = 0, cm = 0;
+  bool vc = take(tc, cc), vn = false, vm = false;
   u32x2 mbc = {0u, 0u}, mbn = {0u, 0u};
+  int noden = 0, nodem = 0;  // lane nodes of steps (tn, cn) and (tm, cm)
   if (vc) {
-    copy(b0, tc, cc);
+    copy(b0, tc, cc, lane_node(tc, cc));
     mbc = tile_bits(a, tc, w, lane);
     vn = take(tn, cn);
+    if constexpr (G) {
+      if (vn) noden = lane_node(tn, cn);
+      vm = vn && take(tm, cm);
+    }
   }
   // One step: step (tc, cc) is in `cur`; the copy of step (tn, cn) goes into `nxt`.
   auto step = [&](lds_char* cur, lds_char* nxt) {
-    wait_vmem();      // this wave's part of the current step (and its mask bits)
+    wait_vmem();      // this wave's part of the current step (its mask bits, the next step's nodes)
     __syncthreads();  // the step landed; every wave is done with the previous step's buffer
     if (vn) {
-      copy(nxt, tn, cn);
+      copy(nxt, tn, cn, noden);
       mbn = tn != tc ? tile_bits(a, tn, w, lane) : mbc;
+      if constexpr (G) {
+        if (vm) nodem = lane_node(tm, cm);
+      }
     }
     const uint32_t gt = tile_groups(a, tc);
     if (gt >> (4 * w + cc) & 1u) group(cc, cur, mbc, gt >> (16 + 4 * w + cc) & 1u);
@@ -171,7 +186,15 @@ __global__ void __launch_bounds__(NT, 2) fwd_x3_kernel(KArgs a) {
     cc = cn;
     mbc = mbn;
     vc = vn;
-    vn = vc && take(tn, cn);
+    if constexpr (G) {
+      tn = tm;
+      cn = cm;
+      vn = vm;
+      noden = nodem;
+      vm = vn && take(tm, cm);
+    } else {
+      vn = vc && take(tn, cn);
+    }
   };
   while (vc) {
     step(b0, b1);
@@ -184,8 +207,11 @@ __global__ void __launch_bounds__(NT, 2) fwd_x3_kernel(KArgs a) {
     return;
   }
   const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
-  store_acc_f32<D>(make_rsrc((float*)a.out0 + j.obase, a.oslice_bytes), qrow, (uint32_t)a.osn * 4, o, inv, g);
-  if (g == 0) write_lse(a, j, qrow, st, ltot);
+  // The row again (a register held through the loop would spill).
+  asm volatile("" ::: "memory");
+  const int orow = node_at<G>(a, j.blk * BLK + 32 * w + i);
+  store_acc_f32<D>(make_rsrc((float*)a.out0 + j.obase, a.oslice_bytes), orow, (uint32_t)a.osn * 4, o, inv, g);
+  if (g == 0) write_lse(a, j, orow, st, ltot);
 }
 
 // dQ, float32 tensors, bf16x3 products, from the dS units of dkv16_x3_kernel: per work item
@@ -199,6 +225,7 @@ __global__ void __launch_bounds__(NT, 2) dq_x3_ds_kernel(KArgs a) {
   constexpr int GB = X3Dma<D>::GB;
   __shared__ __attribute__((aligned(1024))) char hb0[4 * GB];
   __shared__ __attribute__((aligned(1024))) char hb1[4 * GB];
+  __shared__ __attribute__((aligned(16))) char lnode[G ? 2 * 4 * BLK : 16];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 31, g = lane >> 5;
@@ -250,9 +277,25 @@ __global__ void __launch_bounds__(NT, 2) dq_x3_ds_kernel(KArgs a) {
 #pragma unroll
       for (int c = 0; c < 2; ++c) acc[db] = mfma_x3(th[db][c], tl[db][c], d[c], d[2 + c], acc[db]);
   };
-  auto copy = [&](lds_char* hb, int kb, int h, uint32_t live) {
+  NodeTab tab;
+  if constexpr (G) tab.init(a, (lds_char*)lnode);
+  // Half h of tile t: of key block kb or, with node tables, of the tile's own nodes (read from LDS or, for
+  // the first half of the item's first tile, from global memory; `first` is a constant at every call).
+  auto copy = [&](bool first, lds_char* hb, int t, int kb, int h, uint32_t live) {
     const uint32_t planes = (live >> (2 * h) & 1u ? 3u : 0u) | (live >> (2 * h + 1) & 1u ? 12u : 0u);
-    dma.issue(rK, rK2, hb, kb * BLK + 64 * h, w, planes);
+    if constexpr (G) {
+      uint32_t na[X3Dma<D>::ROWS], nb[X3Dma<D>::ROWS];
+      if (first) {
+        dma.nodes(na, tile_nodes(a, t), w);
+        dma.nodes(nb, tile_nodes(a, t) + 32, w);
+      } else {
+        dma.nodes(na, tab.block(t & 1) + 64 * h, w);
+        dma.nodes(nb, tab.block(t & 1) + 64 * h + 32, w);
+      }
+      dma.gather(rK, rK, hb, na, nb, w, planes);
+    } else {
+      dma.issue(rK, rK2, hb, kb * BLK + 64 * h, w, planes);
+    }
   };
 
   int t0, t1;
@@ -264,7 +307,10 @@ __global__ void __launch_bounds__(NT, 2) dq_x3_ds_kernel(KArgs a) {
   if (t0 < t1) {
     gcur = tile_groups(a, t0);
     ucur = ((cmap_ptr)a.ubase)[t0];
-    copy(h0, ((ci32_ptr)a.col)[t0], 0, any_rows(gcur));
+    copy(true, h0, t0, ((ci32_ptr)a.col)[t0], 0, any_rows(gcur));
+    if constexpr (G) {
+      if (w == 0) tab.load(t0 & 1, t0, lane);
+    }
     load_units(dsA, gcur, ucur, 0);
   }
   for (int tt = t0; tt < t1; ++tt) {
@@ -274,7 +320,11 @@ __global__ void __launch_bounds__(NT, 2) dq_x3_ds_kernel(KArgs a) {
     const uint32_t live = gt >> (4 * w) & 15u;
     wait_vmem();      // this wave's part of half 0 of tile t and its units
     __syncthreads();  // half 0 landed; every wave is done with half 1 of tile t - 1
-    copy(h1, kb, 1, any_rows(gt));
+    copy(false, h1, t, kb, 1, any_rows(gt));
+    // The nodes of tile t + 1 go where tile t - 1's were (last read before this barrier).
+    if constexpr (G) {
+      if (w == 0 && t + 1 < t1) tab.load((t + 1) & 1, t + 1, lane);
+    }
     load_units(dsB, gt, ut, 1);
     if (t + 1 < t1) {
       gcur = tile_groups(a, t + 1);
@@ -288,7 +338,7 @@ __global__ void __launch_bounds__(NT, 2) dq_x3_ds_kernel(KArgs a) {
     wait_vmem();      // this wave's part of half 1 and its units
     __syncthreads();  // half 1 landed; every wave is done with half 0
     if (t + 1 < t1) {
-      copy(h0, ((ci32_ptr)a.col)[t + 1], 0, any_rows(gcur));
+      copy(false, h0, t + 1, ((ci32_ptr)a.col)[t + 1], 0, any_rows(gcur));
       load_units(dsA, gcur, ucur, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -317,7 +367,7 @@ hipError_t launch_dg(Kind kind, const KArgs& a, hipStream_t stream) {
 
 template <int D>
 hipError_t launch_d(Kind kind, const KArgs& a, hipStream_t stream) {
-  return a.node ? launch_dg<D, true>(kind, a, stream) : launch_dg<D, false>(kind, a, stream);
+  return a.row_node ? launch_dg<D, true>(kind, a, stream) : launch_dg<D, false>(kind, a, stream);
 }
 
 }  // namespace
@@ -333,8 +383,8 @@ hipError_t launch_x3(Kind kind, int head_dim, const KArgs& a, hipStream_t stream
 }
 
 hipError_t launch_split_x3(const float* src, int64_t sb, int64_t sn, int64_t sh, int batch, int n, int heads,
-                           int head_dim, const int32_t* node, uint16_t* dst, hipStream_t stream) {
-  SplitArgs s{src, dst, sb, sn, sh, batch, n, heads, head_dim, node};
+                           int head_dim, uint16_t* dst, hipStream_t stream) {
+  SplitArgs s{src, dst, sb, sn, sh, batch, n, heads, head_dim};
   const uint64_t threads = (uint64_t)batch * heads * n * (head_dim / 8);
   hipLaunchKernelGGL(split_x3_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, s);
   return hipGetLastError();

@@ -35,10 +35,15 @@ struct X3DmaW {
   static constexpr int NI = 32 / RPO;
   static constexpr int GB = 32 * 2 * D;
   static constexpr int XROW = 4 * D;
+  static constexpr int ROWS = NI >= NW ? NI / NW : 1;  // distinct rows of a lane in one plane's instructions
   uint32_t voff;
+  uint32_t chunk;  // this lane's chunk alone, and its row within an instruction's (node tables)
+  uint32_t rl;
 
   __device__ __forceinline__ void init(int w, int lane) {
     const int row = RPO * (w % NI) + lane / C;
+    rl = (uint32_t)(lane / C);
+    chunk = (uint32_t)(((lane % C) ^ swz16<C>(row)) << 4);
     voff = (uint32_t)(lane / C) * XROW + (uint32_t)(((lane % C) ^ swz16<C>(row)) << 4);
   }
 
@@ -49,6 +54,25 @@ struct X3DmaW {
     for (int m = 0; m < 4 * NI / NW; ++m) {
       const int k = w + NW * m, plane = k / NI, sub = k % NI;
       const uint32_t src = (uint32_t)(row0 + RPO * sub) * XROW + voff + (uint32_t)(plane & 1) * (2 * D);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          plane < 2 ? rA : rB,
+          (__attribute__((address_space(3))) void*)(uintptr_t)(base + (uint32_t)(plane * GB + sub * 1024)), 16,
+          (int)src, 0, 0, 0);
+    }
+  }
+
+  // issue() of the split rows of a group's 32 nodes, entry i in lane i % 32 of `nodes`.
+  __device__ __forceinline__ void gather(rsrc_t rA, rsrc_t rB, lds_char* buf, int nodes, int w) const {
+    uint32_t base = (uint32_t)(uintptr_t)buf;
+    asm volatile("" : "+s"(base));
+    uint32_t nd[ROWS];
+#pragma unroll
+    for (int k = 0; k < ROWS; ++k)
+      nd[k] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(4u * ((uint32_t)(RPO * ((w + NW * k) % NI)) + rl)), nodes);
+#pragma unroll
+    for (int m = 0; m < 4 * NI / NW; ++m) {
+      const int k = w + NW * m, plane = k / NI, sub = k % NI;
+      const uint32_t src = row_bytes(nd[m % ROWS], XROW) + chunk + (uint32_t)(plane & 1) * (2 * D);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           plane < 2 ? rA : rB,
           (__attribute__((address_space(3))) void*)(uintptr_t)(base + (uint32_t)(plane * GB + sub * 1024)), 16,
@@ -261,15 +285,21 @@ __global__ void __launch_bounds__(NT4, 2) dkv16_x3_kernel(KArgs a) {
     rem &= rem - 1u;
     return true;
   };
-  // The tensors' row at position lane % 32 of step (t, c), whose lse and delta wave 0 copies: with a
-  // node table it is loaded a step before. (The split Q and dO rows are in the list's order.)
+  // With node tables: lanes 0-31 hold the node of column lane of step (t, c) and lane 32 the step's dS
+  // unit, loaded a step before they are used (a scalar load of the unit would miss the scalar
+  // cache, and the wave's LDS waits would wait for it).
   auto lane_row = [&](int t, int c) {
-    if constexpr (G) return node_block(a, ((ci32_ptr)a.col)[t])[32 * c + (lane & 31)];
+    if constexpr (G)
+      return *(lane < 32 ? tile_nodes(a, t) + 32 * c + lane : a.tmap + (int64_t)t * UnitTab::WORDS + 4 * kg + c);
     return 0;
   };
   auto copy = [&](lds_char* buf, int t, int c, int lrow) {
-    const int row0 = ((ci32_ptr)a.col)[t] * BLK + 32 * c;
-    dma.issue(rQ, rO, buf, row0, wid);
+    const int row0 = G ? 0 : ((ci32_ptr)a.col)[t] * BLK + 32 * c;
+    if constexpr (G) {
+      dma.gather(rQ, rO, buf, lrow, wid);
+    } else {
+      dma.issue(rQ, rO, buf, row0, wid);
+    }
     if (wid == 0) {
       const int so = lane < 32 ? (G ? lrow : row0 + lane) * 4 : (int)kPastEnd;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rL, (__attribute__((address_space(3))) void*)(buf + SB), 4, so, 0, 0, 0);
@@ -283,8 +313,11 @@ __global__ void __launch_bounds__(NT4, 2) dkv16_x3_kernel(KArgs a) {
   bool vc = take(tc, cc), vn = false, vm = false;
   uint64_t mwc = 0, mwn = 0;
   int rown = 0, rowm = 0;  // lane rows of steps (tn, cn) and (tm, cm)
+  int unitc = -1;          // unit of step (tc, cc), with node tables
   if (vc) {
-    copy(b0, tc, cc, lane_row(tc, cc));
+    const int rowc = lane_row(tc, cc);
+    copy(b0, tc, cc, rowc);
+    unitc = __builtin_amdgcn_readlane(rowc, 32);
     mwc = mword[(int64_t)tc * 256];
     vn = take(tn, cn);
     if constexpr (G) {
@@ -315,11 +348,18 @@ __global__ void __launch_bounds__(NT4, 2) dkv16_x3_kernel(KArgs a) {
     // (16 c + 8 m + r, shifted by 4 (g % 2)) are set.
     const uint64_t mw = mwc >> mshift;
     const bool live = __builtin_amdgcn_ballot_w64((((uint32_t)(mw >> (16 * cc))) & 0x0F0Fu) != 0u) != 0u;
-    const uint32_t ub = ((cmap_ptr)a.tmap)[2 * tc];
-    const uint32_t gw = ((cmap_ptr)a.tmap)[2 * tc + 1];
-    const uint32_t bit = 4u * (uint32_t)cc + (uint32_t)(kg >> 1);
-    const bool have_unit = (gw >> bit & 1u) != 0u;
-    const uint32_t u = ub + (uint32_t)__builtin_popcount(gw & 0xffffu & ((1u << bit) - 1u));
+    bool have_unit;
+    uint32_t u;
+    if constexpr (G) {
+      have_unit = unitc >= 0;
+      u = (uint32_t)unitc;
+    } else {
+      const uint32_t ub = ((cmap_ptr)a.tmap)[2 * tc];
+      const uint32_t gw = ((cmap_ptr)a.tmap)[2 * tc + 1];
+      const uint32_t bit = 4u * (uint32_t)cc + (uint32_t)(kg >> 1);
+      have_unit = (gw >> bit & 1u) != 0u;
+      u = ub + (uint32_t)__builtin_popcount(gw & 0xffffu & ((1u << bit) - 1u));
+    }
     // One store path after the unit (a store inside the unit's branch and another beside it made
     // the register allocator place dK^T / dV^T differently on each path and copy them every step).
     u32x4 dh = {0u, 0u, 0u, 0u}, dl = {0u, 0u, 0u, 0u};
@@ -333,6 +373,7 @@ __global__ void __launch_bounds__(NT4, 2) dkv16_x3_kernel(KArgs a) {
       tn = tm;
       cn = cm;
       vn = vm;
+      unitc = __builtin_amdgcn_readlane(rown, 32);
       rown = rowm;
       vm = vn && take(tm, cm);
     } else {
@@ -370,7 +411,7 @@ template <int D>
 hipError_t launch_d(const KArgs& a, hipStream_t stream) {
   // Two workgroups per item, laid out in blocks of 16 ids (8 items x 2 halves).
   const dim3 grid(16u * (((unsigned)job_count(a) + 7u) / 8u));
-  if (a.node)
+  if (a.row_node)
     hipLaunchKernelGGL((dkv16_x3_kernel<D, true>), grid, dim3(NT4), 0, stream, a);
   else
     hipLaunchKernelGGL((dkv16_x3_kernel<D, false>), grid, dim3(NT4), 0, stream, a);

@@ -1,5 +1,6 @@
-// A locality order of a tile list's nodes, computed from its mask alone, and the list of the
-// permuted mask.
+// A locality order of a tile list's nodes, computed from its mask alone, the list of the permuted
+// mask, the same with each block's live columns packed together, and the dS unit numbering of such
+// lists.
 //
 // The kernels compute whole 32 x 32 groups of a live tile, so their work depends on how compactly
 // each node's neighbourhood lies in the node numbering. The mask is the only description of the
@@ -206,6 +207,30 @@ void for_entries(const List& m, const int64_t* perm, const std::vector<int32_t>&
   }
 }
 
+// The live column groups of block blk in ascending order (any row with an element in them).
+void live_groups(const List& m, int64_t blk, int32_t group, std::vector<int32_t>& out) {
+  out.clear();
+  const int32_t rows = std::min(FWN_BLOCK, m.n - (int32_t)blk * FWN_BLOCK);
+  for (int32_t t = m.ptr[blk]; t < m.ptr[blk + 1]; ++t) {
+    uint32_t any[kWords] = {};
+    const uint32_t* w = m.bits + t * kTileWords;
+    for (int32_t r = 0; r < rows; ++r)
+      for (int32_t q = 0; q < kWords; ++q) any[q] |= w[r * kWords + q];
+    for (int32_t c = 0; c < FWN_BLOCK; c += group) {
+      const uint32_t mask = group == 32 ? 0xffffffffu : ((1u << group) - 1u) << (c % 32);
+      if ((any[c / 32] & mask) && m.col[t] * FWN_BLOCK + c < m.n) out.push_back((m.col[t] * FWN_BLOCK + c) / group);
+    }
+  }
+}
+
+bool good_group(int32_t group) { return group == 1 || group == 16 || group == 32; }
+
+// One unit of a dS numbering: the 16- or 32-column group it covers and its number.
+struct Unit {
+  int32_t col, unit;
+  bool operator<(const Unit& o) const { return col < o.col; }
+};
+
 int inverse(const char* what, int32_t n, const int64_t* perm, std::vector<int32_t>& inv) {
   if (!perm) return fwn::fail(FWN_ERR_INVALID_ARG, "%s: null perm", what);
   inv.assign(n, -1);
@@ -328,6 +353,155 @@ int fwn_tiles_permute_fill(int32_t n, const int32_t* tile_ptr, const int32_t* ti
     return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_permute_fill: %s", e.what());
   }
   if (bad) return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_permute_fill: new_ptr does not match the mask");
+  return FWN_OK;
+}
+
+int fwn_tiles_compact_count(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
+                            int32_t group, int32_t* new_ptr) {
+  fwn::clear_error();
+  List m;
+  if (int rc = make_list(m, "fwn_tiles_compact_count", n, tile_ptr, tile_col, tile_bits)) return rc;
+  if (!new_ptr || !good_group(group))
+    return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_compact_count: null output or group %d (1, 16 or 32)", group);
+  try {
+    std::vector<int32_t> count(m.n_blocks);
+    parallel_for(m.n_blocks, 4, [&](int64_t b, int64_t e) {
+      std::vector<int32_t> live;
+      for (int64_t blk = b; blk < e; ++blk) {
+        live_groups(m, blk, group, live);
+        count[blk] = (int32_t)(((int64_t)live.size() * group + FWN_BLOCK - 1) / FWN_BLOCK);
+      }
+    });
+    new_ptr[0] = 0;
+    for (int32_t blk = 0; blk < m.n_blocks; ++blk) new_ptr[blk + 1] = new_ptr[blk] + count[blk];  // at most n_tiles
+  } catch (const std::exception& e) {
+    return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_compact_count: %s", e.what());
+  }
+  return FWN_OK;
+}
+
+int fwn_tiles_compact_fill(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
+                           int32_t group, const int32_t* new_ptr, int32_t* cols, uint32_t* new_bits) {
+  fwn::clear_error();
+  List m;
+  if (int rc = make_list(m, "fwn_tiles_compact_fill", n, tile_ptr, tile_col, tile_bits)) return rc;
+  if (!new_ptr || !good_group(group) || (new_ptr[m.n_blocks] > 0 && (!cols || !new_bits)))
+    return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_compact_fill: null output or group %d (1, 16 or 32)", group);
+  std::atomic<bool> bad(false);
+  try {
+    parallel_for(m.n_blocks, 4, [&](int64_t b, int64_t e) {
+      std::vector<int32_t> live, at((size_t)m.n_blocks * FWN_BLOCK / group, -1);
+      for (int64_t blk = b; blk < e; ++blk) {
+        live_groups(m, blk, group, live);
+        const int64_t t0 = new_ptr[blk], tiles = new_ptr[blk + 1] - t0;
+        if (tiles != ((int64_t)live.size() * group + FWN_BLOCK - 1) / FWN_BLOCK) {
+          bad = true;
+          return;
+        }
+        std::memset(new_bits + t0 * kTileWords, 0, tiles * kTileWords * sizeof(uint32_t));
+        std::fill(cols + t0 * FWN_BLOCK, cols + (t0 + tiles) * FWN_BLOCK, n);
+        for (size_t k = 0; k < live.size(); ++k) {
+          at[live[k]] = (int32_t)(k * group);
+          for (int32_t c = 0; c < group; ++c)
+            cols[t0 * FWN_BLOCK + k * group + c] = std::min(live[k] * group + c, n);
+        }
+        const int32_t rows = std::min(FWN_BLOCK, n - (int32_t)blk * FWN_BLOCK);
+        for (int32_t t = m.ptr[blk]; t < m.ptr[blk + 1]; ++t)
+          for (int32_t r = 0; r < rows; ++r)
+            for (int32_t q = 0; q < kWords; ++q)
+              for (uint32_t v = m.bits[t * kTileWords + r * kWords + q]; v; v &= v - 1) {
+                const int32_t c = m.col[t] * FWN_BLOCK + 32 * q + __builtin_ctz(v);
+                if (c >= n) continue;
+                const int32_t to = at[c / group] + c % group;
+                new_bits[(t0 + to / FWN_BLOCK) * kTileWords + r * kWords + to % FWN_BLOCK / 32] |= 1u << (to % 32);
+              }
+      }
+    });
+  } catch (const std::exception& e) {
+    return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_compact_fill: %s", e.what());
+  }
+  if (bad) return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_compact_fill: new_ptr does not match the mask");
+  return FWN_OK;
+}
+
+int fwn_tiles_unit_map(int32_t n, const int32_t* tile_ptr, const uint32_t* bits, const int32_t* cols,
+                       const int32_t* tile_ptr_t, const uint32_t* bits_t, const int32_t* cols_t, int32_t unit_keys,
+                       int32_t* ubase, int32_t* tmap, int64_t* n_units) {
+  fwn::clear_error();
+  if (n <= 0 || !tile_ptr || !tile_ptr_t || !n_units || (unit_keys != 16 && unit_keys != 32))
+    return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_unit_map: null argument or unit_keys %d (16 or 32)", unit_keys);
+  const int32_t n_blocks = (n + FWN_BLOCK - 1) / FWN_BLOCK;
+  const int32_t n_tiles = tile_ptr[n_blocks], n_tiles_t = tile_ptr_t[n_blocks];
+  if ((n_tiles > 0 && (!bits || !cols || !ubase)) || (n_tiles_t > 0 && (!bits_t || !cols_t || !tmap)))
+    return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_unit_map: null tile arrays");
+  try {
+    // The units of each 32-row group, in the order of their columns.
+    std::vector<std::vector<Unit>> units((size_t)n_blocks * 4);
+    int64_t total = 0;
+    const int32_t per = FWN_BLOCK / unit_keys;  // units of a 32-row group in one tile
+    for (int32_t blk = 0; blk < n_blocks; ++blk)
+      for (int32_t t = tile_ptr[blk]; t < tile_ptr[blk + 1]; ++t) {
+        ubase[t] = (int32_t)total;
+        const uint32_t* w = bits + t * kTileWords;
+        for (int32_t g = 0; g < 4; ++g)
+          for (int32_t x = 0; x < per; ++x) {
+            const int32_t c0 = x * unit_keys;
+            const uint32_t mask = unit_keys == 32 ? 0xffffffffu : 0xffffu << (c0 % 32);
+            uint32_t any = 0;
+            for (int32_t r = 32 * g; r < 32 * g + 32; ++r) any |= w[r * kWords + c0 / 32] & mask;
+            if (!any) continue;
+            const int32_t c = cols[(int64_t)t * FWN_BLOCK + c0];
+            if (c < 0 || c >= n || c % unit_keys)
+              return fwn::fail(FWN_ERR_TILES, "fwn_tiles_unit_map: tile %d is not compacted in groups of %d", t, unit_keys);
+            units[4 * blk + g].push_back(Unit{c / unit_keys, (int32_t)total++});
+            if (total > INT32_MAX) return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_unit_map: more than 2^31 units");
+          }
+      }
+    for (auto& u : units) std::sort(u.begin(), u.end());
+    std::atomic<int64_t> found(0);
+    std::atomic<bool> bad(false);
+    parallel_for(n_blocks, 4, [&](int64_t b, int64_t e) {
+      int64_t mine = 0;
+      for (int64_t blk = b; blk < e; ++blk)
+        for (int32_t t = tile_ptr_t[blk]; t < tile_ptr_t[blk + 1]; ++t) {
+          int32_t* m = tmap + (int64_t)t * 36;
+          const uint32_t* w = bits_t + t * kTileWords;
+          uint32_t live = 0;
+          for (int32_t kg = 0; kg < 8; ++kg)
+            for (int32_t c = 0; c < 4; ++c) {
+              m[4 * kg + c] = -1;
+              uint32_t own = 0, any = 0;
+              const int32_t r0 = unit_keys == 32 ? 32 * (kg / 2) : 16 * kg;
+              for (int32_t r = r0; r < r0 + unit_keys; ++r) any |= w[r * kWords + c];
+              for (int32_t r = 16 * kg; r < 16 * kg + 16; ++r) own |= w[r * kWords + c];
+              if (own) live |= 1u << (8 * c + kg);
+              if (!any) continue;
+              const int32_t q = cols_t[(int64_t)t * FWN_BLOCK + 32 * c], key = ((int32_t)blk * FWN_BLOCK + r0) / unit_keys;
+              if (q < 0 || q >= n || q % 32) {
+                bad = true;
+                return;
+              }
+              const auto& u = units[q / 32];
+              const auto it = std::lower_bound(u.begin(), u.end(), Unit{key, 0});
+              if (it == u.end() || it->col != key) {
+                bad = true;
+                return;
+              }
+              m[4 * kg + c] = it->unit;
+              if (unit_keys == 16 || kg % 2 == 0) ++mine;
+            }
+          m[32] = (int32_t)live;
+          m[33] = m[34] = m[35] = 0;
+        }
+      found += mine;
+    });
+    // Each unit of one list is one of the other's, and as many: none is written twice or never.
+    if (bad || found != total)
+      return fwn::fail(FWN_ERR_TILES, "fwn_tiles_unit_map: the lists have different units (not transposes)");
+    *n_units = total;
+  } catch (const std::exception& e) {
+    return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_unit_map: %s", e.what());
+  }
   return FWN_OK;
 }
 

@@ -52,15 +52,15 @@ class Tiles(ctypes.Structure):
               ("n_items", ctypes.c_int32), ("n_parts", ctypes.c_int32), ("n_split", ctypes.c_int32),
               ("n_work", ctypes.c_int32), ("items", ctypes.c_void_p), ("split", ctypes.c_void_p),
               ("halves", ctypes.c_void_p), ("work", ctypes.c_void_p), ("work_pairs", ctypes.c_int32),
-              ("flags", ctypes.c_int32), ("node", ctypes.c_void_p)]
+              ("flags", ctypes.c_int32), ("row_node", ctypes.c_void_p), ("col_node", ctypes.c_void_p)]
 
 
-TILES_NODES = 1  # FWN_TILES_NODES: the list is laid out in an order of its own (Tiles.node)
+TILES_NODES = 1  # FWN_TILES_NODES: the list is laid out in an order of its own (Tiles.row_node, col_node)
 
 
 class DsMap(ctypes.Structure):
   _fields_ = [("n_units", ctypes.c_int64), ("ubase", ctypes.c_void_p), ("tmap", ctypes.c_void_p),
-              ("unit_keys", ctypes.c_int32), ("reserved", ctypes.c_int32)]
+              ("unit_keys", ctypes.c_int32), ("table", ctypes.c_int32)]
 
 
 ITEM_TILES = 64  # FWN_ITEM_TILES: default longest run of tiles per work item
@@ -96,6 +96,9 @@ SIGNATURES = {
     "fwn_tiles_node_order": [_I32, _P, _P, _P, _P],
     "fwn_tiles_permute_count": [_I32, _P, _P, _P, _P, _P],
     "fwn_tiles_permute_fill": [_I32, _P, _P, _P, _P, _P, _P, _P],
+    "fwn_tiles_compact_count": [_I32, _P, _P, _P, _I32, _P],
+    "fwn_tiles_compact_fill": [_I32, _P, _P, _P, _I32, _P, _P, _P],
+    "fwn_tiles_unit_map": [_I32, _P, _P, _P, _P, _P, _P, _I32, _P, _P, _P],
     "fwn_tiles_schedule_count": [_I32, _P, _I32, _P, _P, _P],
     "fwn_tiles_schedule_fill": [_I32, _P, _I32, _P, _P],
     "fwn_tiles_order_count": [_I32, _P, _P, _I32, _I32, _I32, _I32, _I32, _P],

@@ -119,7 +119,7 @@ class _Schedule:
     return nat.Tiles(tl.n_blocks, tl.n_tiles, addr(tl.ptr), addr(tl.col), addr(tl.lanes), addr(tl.groups),
                      self.n_items, self.n_parts, self.n_split, 0 if work is None else work.shape[0],
                      addr(self.items), addr(self.split) if self.n_split else None, addr(tl.halves), addr(work),
-                     pairs, 0 if tl.node is None else nat.TILES_NODES, addr(tl.node))
+                     pairs, *tl._nodes())
 
   def order_table(self, pairs, order=nat.ORDER_BALANCED, window=0, slots=64):
     """Host order table [n_work, 2] of this schedule for calls of `pairs` (batch, head) pairs."""
@@ -143,11 +143,11 @@ class _Schedule:
     return self._orders[key][1]
 
 
-# A list's own node order (TileList.launch_list): taken when the estimated cost of its tiles
-# (ORDER_TILE_UNITS per tile + ORDER_HALF_UNITS per live 32 x 16 half) is at most ORDERED_GAIN of
-# the given order's. On the refinement-6 mesh the estimates are 0.30 (8 hops) and 0.46 (16 hops) of
-# mesh order, 0.89 of Hilbert order (32 hops).
-ORDERED_GAIN = 0.95
+# Lists laid out for the kernels (TileList.launch_list): taken when the estimated cost of their tiles
+# (ORDER_TILE_UNITS per tile + ORDER_HALF_UNITS per live 32 x 16 half) is at most LAID_OUT_GAIN of the
+# given list's. On the refinement-6 mesh the forward's estimates are 0.24 (8 hops) and 0.37 (16
+# hops) of mesh order's list, 0.77 of Hilbert order's (32 hops).
+LAID_OUT_GAIN = 0.95
 
 
 class TileList:
@@ -159,12 +159,22 @@ class TileList:
   ``max_item_tiles`` fixes the split-K cap; None lets each launch pick it (``struct_for``).
   ``struct`` is the schedule with the fixed cap, or nat.ITEM_TILES.
 
-  The op's calls run ``launch_list()``: the same mask laid out in a node order of the list's own
-  (``fwn_tiles_node_order``) when that leaves the kernels less to compute, else this list. Nothing
-  outside the kernels sees that order: they address the rows of q, k, v, ... through ``node``.
+  The op's calls run lists laid out for its kernels (``launch_list``, ``exchange_lists``) when those
+  leave less to compute, else this list: the mask in a node order of its own
+  (``fwn_tiles_node_order``), each block's live columns packed into as few tiles as hold them
+  (``fwn_tiles_compact_*``). Nothing outside the kernels sees that layout: they address the rows of
+  q, k, v, ... through node tables.
   """
 
-  def __init__(self, tile_ptr, tile_kb, tile_bits, n_cols, device="cuda", max_item_tiles=None, _node=None):
+  def __init__(self, tile_ptr, tile_kb, tile_bits, n_cols, device="cuda", max_item_tiles=None):
+    self._build(tile_ptr, tile_kb, tile_bits, n_cols, device, max_item_tiles)
+    self._layout = _Layout.choose(self) if self.device.type == "cuda" else None
+
+  def _nodes(self):
+    """The node members of the C struct: flags, row_node, col_node."""
+    return 0, None, None
+
+  def _build(self, tile_ptr, tile_kb, tile_bits, n_cols, device, max_item_tiles):
     tile_ptr = nat.as_c(tile_ptr, np.int32)
     tile_kb = nat.as_c(tile_kb, np.int32)
     tile_bits = nat.as_c(tile_bits, np.uint32)
@@ -188,8 +198,6 @@ class TileList:
                                   nat.ptr(tile_bits), nat.ptr(lanes), nat.ptr(groups), nat.ptr(halves)))
     self.device = torch.device(device)
     put = lambda a: torch.from_numpy(a).to(self.device)
-    # The node at each position (n_cols past the last), or None: positions are nodes.
-    self.node = _node
     self.ptr = put(tile_ptr)
     self.col = put(tile_kb)
     self.lanes = put(lanes.view(np.int64))
@@ -210,56 +218,27 @@ class TileList:
     self.items_host, self.split_host = base.items_host, base.split_host
     self.items, self.split = base.items, base.split
     self.struct = base.struct
-    self._perm = None
-    self._transposes = weakref.WeakKeyDictionary()
-    self._ordered = self._lay_out() if _node is None and self.device.type == "cuda" else None
 
-  def _cost(self, n_tiles, halves):
-    return ORDER_TILE_UNITS * n_tiles + ORDER_HALF_UNITS * int(np.unpackbits(halves.view(np.uint8)).sum())
-
-  def _lay_out(self):
-    """This mask's list in a locality order of its own, or None where that would not pay (or the
-    list is not square, or a single block)."""
-    n = self.n_cols
-    if self.n_blocks != -(-n // nat.BLOCK) or self.n_blocks < 2 or n >= 1 << 24 or not self.n_tiles:
-      return None
-    perm = np.empty(n, np.int64)
-    nat.check(nat.lib().fwn_tiles_node_order(n, nat.ptr(self._tile_ptr), nat.ptr(self._tile_col),
-                                             nat.ptr(self._tile_bits), nat.ptr(perm)))
-    node = np.full(self.n_blocks * nat.BLOCK, n, np.int32)
-    node[:n] = perm
-    ordered = self._permuted(perm, torch.from_numpy(node).to(self.device))
-    if (self._cost(ordered.n_tiles, ordered.halves_host) >
-        ORDERED_GAIN * self._cost(self.n_tiles, self.halves_host)):
-      return None
-    self._perm = perm
-    return ordered
-
-  def _permuted(self, perm, node):
-    """The list of mask[perm][:, perm], with the device table `node` of that order."""
-    L = nat.lib()
-    args = (self.n_cols, nat.ptr(self._tile_ptr), nat.ptr(self._tile_col), nat.ptr(self._tile_bits), nat.ptr(perm))
-    tile_ptr = np.zeros(self.n_blocks + 1, np.int32)
-    nat.check(L.fwn_tiles_permute_count(*args, nat.ptr(tile_ptr)))
-    tile_kb = np.empty(int(tile_ptr[-1]), np.int32)
-    tile_bits = np.empty((int(tile_ptr[-1]), nat.BLOCK, nat.BLOCK // 32), np.uint32)
-    nat.check(L.fwn_tiles_permute_fill(*args, nat.ptr(tile_ptr), nat.ptr(tile_kb), nat.ptr(tile_bits)))
-    return TileList(tile_ptr, tile_kb, tile_bits, self.n_cols, self.device, self._fixed_cap, _node=node)
+  @property
+  def cost(self):
+    """Estimated cost of the list's tiles for one (batch, head) pair (ORDER_* units)."""
+    halves = int(np.unpackbits(self.halves_host.view(np.uint8)).sum())
+    return ORDER_TILE_UNITS * self.n_tiles + ORDER_HALF_UNITS * halves
 
   def launch_list(self):
-    """The list the kernels walk for this mask: the one laid out in its own order where there is
-    one, else this one."""
-    return self if self._ordered is None else self._ordered
+    """The list the forward (and each recomputing backward kernel) walks for this mask: the one laid
+    out for it where there is one, else this one."""
+    return self if self._layout is None else self._layout.forward
 
-  def launch_lists(self, tiles_t):
-    """(launch list of this mask, list of the transposed mask `tiles_t` in the same order): the
-    pair whose dS units the backward exchanges."""
-    tl = self.launch_list()
-    if tiles_t is self or tl is self or tiles_t.n_blocks != self.n_blocks or tiles_t.n_cols != self.n_cols:
-      return tl, tl if tiles_t is self else tiles_t
-    if tiles_t not in self._transposes:
-      self._transposes[tiles_t] = tiles_t._permuted(self._perm, tl.node)
-    return tl, self._transposes[tiles_t]
+  def exchange_lists(self, tiles_t, unit_keys):
+    """(list for dQ, list for dK/dV, dS map) of the dS exchange with `tiles_t`, the transposed
+    mask's list (this list itself for a symmetric mask), or None when it is not the exact
+    transpose (the recomputing backward applies then). Built on first use and kept."""
+    dmap = self.ds_map(tiles_t, unit_keys)
+    if dmap is None:
+      return None
+    laid_out = self._layout and self._layout.exchange(tiles_t, unit_keys)
+    return laid_out or (self, tiles_t, dmap)
 
   def _schedule(self, cap):
     cap = int(cap) if cap > 0 else nat.ITEM_TILES
@@ -346,6 +325,100 @@ class TileList:
     return float(bits) / (16 * self.n_tiles)
 
 
+class _Arrays:
+  """Canonical tile arrays on the host (tile_ptr, column blocks, bits) of an n x n mask."""
+
+  def __init__(self, n, ptr, col, bits):
+    self.n, self.ptr, self.col, self.bits = n, ptr, col, bits
+    self.args = (n, nat.ptr(ptr), nat.ptr(col), nat.ptr(bits))
+
+  def permuted(self, perm):
+    """The arrays of mask[perm][:, perm]."""
+    L = nat.lib()
+    ptr = np.zeros_like(self.ptr)
+    nat.check(L.fwn_tiles_permute_count(*self.args, nat.ptr(perm), nat.ptr(ptr)))
+    col, bits = np.empty(int(ptr[-1]), np.int32), np.empty((int(ptr[-1]), nat.BLOCK, nat.BLOCK // 32), np.uint32)
+    nat.check(L.fwn_tiles_permute_fill(*self.args, nat.ptr(perm), nat.ptr(ptr), nat.ptr(col), nat.ptr(bits)))
+    return _Arrays(self.n, ptr, col, bits)
+
+
+class _PackedList(TileList):
+  """The list of `arrays` with each block's live column groups of `group` columns packed
+  (``fwn_tiles_compact_*``). ``cols`` holds the column of each tile column; ``node[c]`` is the node of
+  row or column c (n past the last)."""
+
+  def __init__(self, arrays, group, node, row_node, device, max_item_tiles):
+    L = nat.lib()
+    self.n = arrays.n
+    ptr = np.zeros_like(arrays.ptr)
+    nat.check(L.fwn_tiles_compact_count(*arrays.args, group, nat.ptr(ptr)))
+    tiles = int(ptr[-1])
+    self.cols = np.empty((tiles, nat.BLOCK), np.int32)
+    bits = np.empty((tiles, nat.BLOCK, nat.BLOCK // 32), np.uint32)
+    nat.check(L.fwn_tiles_compact_fill(*arrays.args, group, nat.ptr(ptr), nat.ptr(self.cols), nat.ptr(bits)))
+    self._row_node = row_node
+    self._col_node = torch.from_numpy(node[self.cols]).to(device)
+    self._layout = None
+    # A tile's column block is its index within the block: the kernels read col_node instead.
+    index = (np.arange(tiles) - np.repeat(ptr[:-1], np.diff(ptr))).astype(np.int32)
+    self._build(ptr, index, bits, (len(ptr) - 1) * nat.BLOCK, device, max_item_tiles)
+
+  def _nodes(self):
+    return nat.TILES_NODES, self._row_node.data_ptr(), self._col_node.data_ptr()
+
+
+class _Layout:
+  """A mask laid out for the kernels: its node order and the packed lists built from it.
+
+  The forward's list packs single columns: per block the union of its rows' keys, so nearly every
+  column of a tile is used. The dS exchange hands 32-query x 16-key (bf16) or x 32-key units from
+  dK/dV to dQ, so its lists pack whole groups: dQ's by `unit_keys` keys, dK/dV's by 32 queries."""
+
+  def __init__(self, arrays, perm, device, cap):
+    self.arrays, self.perm, self._device, self._cap = arrays, perm, device, cap
+    n = arrays.n
+    self._node = np.concatenate([perm.astype(np.int32), np.full(nat.BLOCK, n, np.int32)])
+    rows = (len(arrays.ptr) - 1) * nat.BLOCK
+    self._row_node = torch.from_numpy(self._node[np.minimum(np.arange(rows), n)]).to(device)
+    self._pairs = weakref.WeakKeyDictionary()
+    self.forward = self.packed(arrays, 1)
+
+  def packed(self, arrays, group):
+    return _PackedList(arrays, group, self._node, self._row_node, self._device, self._cap)
+
+  @classmethod
+  def choose(cls, tl):
+    """The layout of TileList `tl`'s mask, or None where it would not pay (LAID_OUT_GAIN) or the list
+    is not square or a single block."""
+    n = tl.n_cols
+    if tl.n_blocks != -(-n // nat.BLOCK) or tl.n_blocks < 2 or n >= 1 << 24 or not tl.n_tiles:
+      return None
+    given = _Arrays(n, tl._tile_ptr, tl._tile_col, tl._tile_bits)
+    perm = np.empty(n, np.int64)
+    nat.check(nat.lib().fwn_tiles_node_order(*given.args, nat.ptr(perm)))
+    # The packed list of the mask in its own order or, if that is no better, in the given one.
+    best = None
+    for p in (perm, np.arange(n, dtype=np.int64)):
+      arrays = given if best else given.permuted(p)
+      layout = cls(arrays, p, tl.device, tl._fixed_cap)
+      if best is None or layout.forward.cost < best.forward.cost:
+        best = layout
+      if best.forward.cost <= LAID_OUT_GAIN * tl.cost:
+        break
+    return best if best.forward.cost <= LAID_OUT_GAIN * tl.cost else None
+
+  def exchange(self, tiles_t, unit_keys):
+    """(list for dQ, list for dK/dV, map) in this layout; `tiles_t` is the exact transpose."""
+    pairs = self._pairs.setdefault(tiles_t, {})
+    if unit_keys not in pairs:
+      own = tiles_t._layout is self
+      arrays_t = self.arrays if own else _Arrays(self.arrays.n, tiles_t._tile_ptr, tiles_t._tile_col,
+                                                 tiles_t._tile_bits).permuted(self.perm)
+      dq, kv = self.packed(self.arrays, unit_keys), self.packed(arrays_t, 32)
+      pairs[unit_keys] = (dq, kv, DsMap.of_packed(dq, kv, unit_keys))
+    return pairs[unit_keys]
+
+
 class DsMap:
   """Unit numbering of the backward's dS exchange (``fwn_tiles_ds_map``): the dK/dV kernel writes
   each unit of dS = P (dP - delta) once, and the dQ kernel reads it instead of recomputing S and
@@ -353,13 +426,13 @@ class DsMap:
   (bf16, the set bits of the forward list's half words) or 32 (float32, its group bits),
   numbered tile by tile; ``struct`` is the C view."""
 
-  def __init__(self, n_units, ubase, tmap, unit_keys, device):
+  def __init__(self, n_units, ubase, tmap, unit_keys, device, table=0):
     self.n_units = int(n_units)
     self.unit_keys = int(unit_keys)
     self.ubase = torch.from_numpy(ubase).to(device)
     self.tmap = torch.from_numpy(tmap).to(device)
     addr = lambda t: t.data_ptr() if t.numel() else None
-    self.struct = nat.DsMap(self.n_units, addr(self.ubase), addr(self.tmap), self.unit_keys, 0)
+    self.struct = nat.DsMap(self.n_units, addr(self.ubase), addr(self.tmap), self.unit_keys, table)
 
   @classmethod
   def build(cls, tl, tlt, unit_keys=16):
@@ -378,6 +451,18 @@ class DsMap:
       return None
     nat.check(status)
     return cls(n_units[0], ubase[:tl.n_tiles], tmap[:tlt.n_tiles], unit_keys, tl.device)
+
+  @classmethod
+  def of_packed(cls, tl, tlt, unit_keys):
+    """The map of a packed pair (``fwn_tiles_unit_map``): a unit of `tlt` finds its number in a
+    table, as its tile's queries come from several tiles of `tl`."""
+    ubase = np.zeros(max(tl.n_tiles, 1), np.int32)
+    tmap = np.zeros((max(tlt.n_tiles, 1), 9, 4), np.int32)
+    n_units = np.zeros(1, np.int64)
+    nat.check(nat.lib().fwn_tiles_unit_map(tl.n, nat.ptr(tl._tile_ptr), nat.ptr(tl._tile_bits), nat.ptr(tl.cols),
+                                           nat.ptr(tlt._tile_ptr), nat.ptr(tlt._tile_bits), nat.ptr(tlt.cols),
+                                           int(unit_keys), nat.ptr(ubase), nat.ptr(tmap), nat.ptr(n_units)))
+    return cls(n_units[0], ubase[:tl.n_tiles], tmap[:tlt.n_tiles], unit_keys, tl.device, table=1)
 
   def ds_bytes(self, desc):
     n = ctypes.c_uint64(0)
@@ -555,11 +640,10 @@ def _backward_into(q, k, v, out, lse, dout, tiles, tiles_t, scale, dq, dk, dv, p
   delta = torch.empty_like(lse)
   L = nat.lib()
   main = torch.cuda.current_stream(q.device)
-  dmap = None
-  if DS_EXCHANGE:
-    tl, tlt = base.launch_lists(base_t)
-    dmap = tl.ds_map(tlt, unit_keys_for(q.dtype))
-  if dmap is not None:
+  exchange = base.exchange_lists(base_t, unit_keys_for(q.dtype))
+  # Without the exchange the kernels walk the same lists (dK and dV are then the same bit for bit).
+  tl, tlt, dmap = exchange or (base.launch_list(), base_t.launch_list(), None)
+  if DS_EXCHANGE and dmap is not None:
     # delta, dK/dV writing dS, then dQ from dS, in stream order (fwn_attn_bwd_ds_launch).
     desc = _desc(q, scale, out, _precision(precision, q.dtype))
     ws = workspace(desc, q.device, tl, tlt)
@@ -570,7 +654,6 @@ def _backward_into(q, k, v, out, lse, dout, tiles, tiles_t, scale, dq, dk, dv, p
                                        dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ds.data_ptr(), ds.numel(),
                                        *_ws_args(ws), main.cuda_stream))
     return
-  tl, tlt = base.launch_list(), base_t.launch_list()
   ws_q, ws_kv = workspace(desc, q.device, tl), workspace(desc, q.device, tlt)
   nat.check(L.fwn_attn_bwd_delta_launch(desc, out.data_ptr(), dout.data_ptr(), delta.data_ptr(), main.cuda_stream))
   side = _side_stream(q.device)

@@ -130,18 +130,19 @@ typedef struct fwn_tiles {
   int32_t work_pairs;       /* batch * heads the order table was built for (launches of another
                                shape are refused); the table must come from this `items` array
                                (the launchers check its size, not its entries) */
-  int32_t flags;            /* 0, or FWN_TILES_NODES: the list has the member below */
-  const int32_t* node;      /* read with FWN_TILES_NODES only: [n_blocks * 128], the node (row of q,
-                               k, v, o, lse, ...) at each position of the list's own order, n for
-                               positions past the last (fwn_tiles_node_order, fwn_tiles_permute_*).
-                               The list describes mask[node][:, node]; the tensors stay in node
-                               order and the kernels address their rows through this table. Every
-                               entry below n must appear once (the launchers check n < 2^24, not
-                               the entries; an entry out of range reads zeros and stores nothing) */
+  int32_t flags;            /* 0, or FWN_TILES_NODES: the list has the two members below */
+  const int32_t* row_node;  /* [n_blocks * 128]: the node (row of q, k, v, o, lse, ...) of each row of
+                               the list's blocks, n for rows past the last */
+  const int32_t* col_node;  /* [n_tiles * 128], 16-byte aligned: the node of each column of each tile,
+                               n for columns of padding (whose mask bits must be clear); `col` is
+                               not read then */
 } fwn_tiles;
 
-/* fwn_tiles.flags: the list is laid out in an order of its own (member `node`). Without it the
- * structure may end before that member. */
+/* fwn_tiles.flags: the list is laid out in an order of its own (fwn_tiles_node_order,
+ * fwn_tiles_permute_*), its tiles' columns gathered per block (fwn_tiles_compact_*). The tensors stay
+ * in node order and the kernels address their rows through the two tables. Every node below n must
+ * be the row of one position; the launchers check n < 2^24, not the entries (an entry of n or
+ * more reads zeros and stores nothing). Without the flag the structure may end before them. */
 #define FWN_TILES_NODES 1
 
 /* Thread-local message of the last failure on this thread ("" if none). */
@@ -206,6 +207,17 @@ int fwn_tiles_permute_count(int32_t n, const int32_t* tile_ptr, const int32_t* t
                             const int64_t* perm, int32_t* new_ptr);
 int fwn_tiles_permute_fill(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
                            const int64_t* perm, const int32_t* new_ptr, int32_t* new_col, uint32_t* new_bits);
+
+/* The tile list with each block's columns compacted: of the groups of `group` (1, 16 or 32)
+ * consecutive columns, those in which some row of the block has a valid element, in ascending
+ * order, packed into tiles of 128 columns. fwn_tiles_compact_count writes new_ptr[n_blocks + 1];
+ * fwn_tiles_compact_fill writes cols[new_ptr[last] * 128], the column of each tile column (n for
+ * padding), and new_bits[new_ptr[last] * 128 * 4]. A column of a compacted list is not a column
+ * block's, so its launches need FWN_TILES_NODES. No reference counterpart. */
+int fwn_tiles_compact_count(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
+                            int32_t group, int32_t* new_ptr);
+int fwn_tiles_compact_fill(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
+                           int32_t group, const int32_t* new_ptr, int32_t* cols, uint32_t* new_bits);
 
 /* Work items of a tile list: the tiles of each block are cut into ceil(count / max_item_tiles)
  * runs of near-equal length (max_item_tiles <= 0 selects FWN_ITEM_TILES). The reference runs one
@@ -335,7 +347,8 @@ typedef struct fwn_ds_map {
                             bits word (as int32: halves for 16, groups for 32) of the same tile of
                             the forward list */
   int32_t unit_keys;     /* 16 (bf16 calls) or 32 (float32 calls) */
-  int32_t reserved;      /* 0 */
+  int32_t table;         /* 0, or 1: tmap is [tiles_t->n_tiles][9][4] (fwn_tiles_unit_map), as lists with
+                            FWN_TILES_NODES need */
 } fwn_ds_map;
 
 /* Builds the unit numbering (host arrays) from the canonical arrays of both lists (tile_ptr,
@@ -348,6 +361,18 @@ int fwn_tiles_ds_map(int32_t n_blocks, const int32_t* tile_ptr, const int32_t* t
                      const uint32_t* tile_bits, const int32_t* tile_ptr_t, const int32_t* tile_col_t,
                      const uint32_t* tile_bits_t, int32_t unit_keys, int32_t* ubase, int32_t* tmap,
                      int64_t* n_units);
+
+/* The unit numbering of a compacted pair of lists (host arrays): the forward list (tile_ptr, bits,
+ * cols) with columns compacted in groups of unit_keys, whose units are numbered tile by tile by the
+ * rank of their bit as above, and the transposed list (.._t) compacted in groups of 32. Both lists'
+ * rows and columns are positions in one order of the n nodes. ubase[n_tiles];
+ * tmap[n_tiles_t * 36]: entry [kg][c] (kg < 8, c < 4) of a transposed tile is the unit of its rows 16 kg
+ * .. + 15 and columns 32 c .. + 31 (for unit_keys 32, that of the 32 rows they lie in), -1 when there is
+ * none, and entry [8][0] the word with bit 8 c + kg set where the rows have a valid element there.
+ * FWN_ERR_TILES when the lists do not have the same units (they are not transposes). */
+int fwn_tiles_unit_map(int32_t n, const int32_t* tile_ptr, const uint32_t* bits, const int32_t* cols,
+                       const int32_t* tile_ptr_t, const uint32_t* bits_t, const int32_t* cols_t, int32_t unit_keys,
+                       int32_t* ubase, int32_t* tmap, int64_t* n_units);
 
 /* Bytes of the dS buffer: batch * heads * n_units * (1024 for unit_keys 16, 4096 for 32);
  * 256-byte aligned device memory. */

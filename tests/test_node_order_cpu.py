@@ -1,6 +1,7 @@
-"""The locality order of a tile list's nodes and the permuted list (``fwn_tiles_node_order``,
-``fwn_tiles_permute_count``, ``fwn_tiles_permute_fill``): the order is a permutation for any mask, the
-permuted list is the one built from the permuted mask, and the order shrinks a mesh's list."""
+"""The locality order of a tile list's nodes, the permuted and the packed lists and the dS unit
+numbering of packed pairs (``fwn_tiles_node_order``, ``fwn_tiles_permute_*``, ``fwn_tiles_compact_*``,
+``fwn_tiles_unit_map``): the order is a permutation for any mask, the permuted list is the one built
+from the permuted mask, a packed list holds the mask's entries, and every dS unit has one number."""
 import numpy as np
 import pytest
 from scipy import sparse
@@ -68,6 +69,103 @@ def test_order_is_deterministic_and_compact_on_a_shuffled_mesh():
   assert tiles <= _arrays(mask, hilbert)[0][-1] < tp[-1]
 
 
+def _compact(n, tp, kb, bits, group):
+  new_ptr = np.zeros_like(tp)
+  args = (n, nat.ptr(tp), nat.ptr(kb), nat.ptr(bits), group)
+  nat.check(nat.lib().fwn_tiles_compact_count(*args, nat.ptr(new_ptr)))
+  cols = np.full((new_ptr[-1], 128), -7, np.int32)
+  new_bits = np.full((new_ptr[-1], 128, 4), 0xFFFFFFFF, np.uint32)
+  nat.check(nat.lib().fwn_tiles_compact_fill(*args, nat.ptr(new_ptr), nat.ptr(cols), nat.ptr(new_bits)))
+  return new_ptr, cols, new_bits
+
+
+def _bools(bits):
+  return np.unpackbits(bits.view(np.uint8), axis=-1, bitorder="little").reshape(len(bits), 128, 128).astype(bool)
+
+
+@pytest.mark.parametrize("group", [1, 16, 32])
+@pytest.mark.parametrize("name", [n for n, _ in _masks()])
+def test_packed_list_holds_the_mask(name, group):
+  """Unpacked through its columns, a packed list is the mask; every column group it holds is live
+  in the block, whole, once and in order; only a block's last tile is padded."""
+  mask = dict(_masks())[name].tocsr()
+  n = mask.shape[0]
+  ptr, cols, bits = _compact(n, *_arrays(mask), group)
+  dense, got = mask.toarray(), np.zeros((n, n + 1), bool)
+  b = _bools(bits)
+  for blk in range(len(ptr) - 1):
+    r0, r1 = 128 * blk, min(n, 128 * blk + 128)
+    c = cols[ptr[blk]:ptr[blk + 1]].ravel()
+    live = c[c < n]
+    assert np.all(np.diff(live) > 0) and np.all(c[len(live):] == n)
+    want = np.unique(np.nonzero(dense[r0:r1].any(0))[0] // group)
+    assert np.array_equal(np.unique(live // group), want)
+    assert len(live) == sum(min(group, n - g * group) for g in want)
+    assert ptr[blk + 1] - ptr[blk] == -(-len(want) * group // 128)
+    for t in range(ptr[blk], ptr[blk + 1]):
+      assert not b[t][:, cols[t] == n].any() and not b[t][r1 - r0:].any()
+      got[r0:r1, cols[t]] |= b[t][:r1 - r0]
+  assert np.array_equal(got[:, :n], dense)
+
+
+def _unit_map(n, f, t, unit_keys):
+  (ptr, cols, bits), (ptr_t, cols_t, bits_t) = f, t
+  ubase, tmap, units = np.zeros(max(len(cols), 1), np.int32), np.full((max(len(cols_t), 1), 9, 4), -9, np.int32), np.zeros(1, np.int64)
+  status = nat.lib().fwn_tiles_unit_map(n, nat.ptr(ptr), nat.ptr(bits), nat.ptr(cols), nat.ptr(ptr_t), nat.ptr(bits_t),
+                                        nat.ptr(cols_t), unit_keys, nat.ptr(ubase), nat.ptr(tmap), nat.ptr(units))
+  return status, ubase, tmap, int(units[0])
+
+
+@pytest.mark.parametrize("unit_keys", [16, 32])
+@pytest.mark.parametrize("name", [n for n, _ in _masks()])
+def test_unit_map_numbers_every_unit_once(name, unit_keys):
+  """The number dQ gives a unit (its tile's first plus the rank of its bit) is the one dK/dV's table
+  holds for the same 32 queries and keys; the numbers are 0 .. n_units - 1."""
+  mask = dict(_masks())[name].tocsr()
+  n = mask.shape[0]
+  f, t = _compact(n, *_arrays(mask), unit_keys), _compact(n, *_arrays(mask.T.tocsr()), 32)
+  status, ubase, tmap, units = _unit_map(n, f, t, unit_keys)
+  assert status == nat.OK
+  want = {}
+  (ptr, cols, bits), (ptr_t, cols_t, bits_t) = f, t
+  b = _bools(bits)
+  for blk in range(len(ptr) - 1):
+    for tile in range(ptr[blk], ptr[blk + 1]):
+      u = ubase[tile]
+      for g in range(4):
+        for c0 in range(0, 128, unit_keys):
+          if b[tile, 32 * g:32 * g + 32, c0:c0 + unit_keys].any():
+            want[4 * blk + g, cols[tile, c0] // unit_keys] = u
+            u += 1
+  assert sorted(want.values()) == list(range(units))
+  b, seen = _bools(bits_t), set()
+  for blk in range(len(ptr_t) - 1):
+    for tile in range(ptr_t[blk], ptr_t[blk + 1]):
+      for kg in range(8):
+        for c in range(4):
+          r0 = 16 * kg // unit_keys * unit_keys
+          live = b[tile, r0:r0 + unit_keys, 32 * c:32 * c + 32].any()
+          own = b[tile, 16 * kg:16 * kg + 16, 32 * c:32 * c + 32].any()
+          assert bool(tmap[tile, 8, 0] >> (8 * c + kg) & 1) == own
+          unit = tmap[tile, kg, c]
+          assert (unit >= 0) == live
+          if live:
+            assert unit == want[cols_t[tile, 32 * c] // 32, (128 * blk + r0) // unit_keys]
+            seen.add(int(unit))
+  assert seen == set(range(units))
+
+
+def test_unit_map_refuses_lists_that_are_not_transposes():
+  m = sparse.identity(300, dtype=bool, format="lil")
+  m[3, 290] = True
+  m = m.tocsr()
+  n = m.shape[0]
+  f, wrong = _compact(n, *_arrays(m), 16), _compact(n, *_arrays(m), 32)
+  assert _unit_map(n, f, wrong, 16)[0] == nat.ERR_TILES
+  assert _unit_map(n, f, _compact(n, *_arrays(m.T.tocsr()), 32), 16)[0] == nat.OK
+  assert _unit_map(n, _compact(n, *_arrays(m), 1), _compact(n, *_arrays(m.T.tocsr()), 32), 16)[0] == nat.ERR_TILES
+
+
 def test_bad_arguments_are_refused():
   tp, kb, bits = _arrays(fwn.mesh_mask(2, 1)[0])
   n, L = 162, nat.lib()
@@ -83,6 +181,10 @@ def test_bad_arguments_are_refused():
   col = kb.copy()
   col[0] = 99
   assert L.fwn_tiles_node_order(n, nat.ptr(tp), nat.ptr(col), nat.ptr(bits), nat.ptr(perm)) == nat.ERR_TILES
+  for group in (0, 2, 64):
+    assert L.fwn_tiles_compact_count(*good, group, nat.ptr(ptr)) == nat.ERR_INVALID_ARG
+  assert L.fwn_tiles_compact_fill(*good, 1, nat.ptr(np.array([0, 1, 1], np.int32)), nat.ptr(np.zeros(128, np.int32)),
+                                  nat.ptr(np.zeros((1, 128, 4), np.uint32))) == nat.ERR_INVALID_ARG
   # a pointer array of another order's list
   assert L.fwn_tiles_permute_fill(*good, nat.ptr(perm), nat.ptr(np.array([0, 1, 2], np.int32)), nat.ptr(np.zeros(2, np.int32)),
                                   nat.ptr(np.zeros((2, 128, 4), np.uint32))) == nat.ERR_INVALID_ARG
@@ -94,7 +196,7 @@ def test_launchers_check_the_node_table():
   size = np.zeros(1, np.uint64)
   desc = nat.AttnDesc(1, 256, 1, 32, nat.F32, 1.0, 32 * 256, 32, 32)
   def status(flags, node, d=desc, blocks=2):
-    t = nat.Tiles(blocks, 1, F, F, F, F, blocks, 0, 0, 0, F, None, None, None, 0, flags, node)
+    t = nat.Tiles(blocks, 1, F, F, F, F, blocks, 0, 0, 0, F, None, None, None, 0, flags, node, node)
     return nat.lib().fwn_attn_workspace_size(d, t, nat.ptr(size))
   assert status(0, None) == nat.OK and status(nat.TILES_NODES, F) == nat.OK
   assert status(2, F) == nat.ERR_INVALID_ARG

@@ -1,5 +1,5 @@
-"""Tile lists laid out in a node order of their own (``TileList.launch_list``): the kernels gather
-and scatter the rows through the node table, so the op's results are those of the mask in the
+"""Tile lists laid out for the kernels (``TileList.launch_list``, ``exchange_lists``: a node order of
+their own, packed columns): the kernels gather and scatter the rows through the node tables, so the op's results are those of the mask in the
 caller's order. Against the float64 dense oracle at block edges, every head size, split work items,
 non-symmetric masks, packed tensors and both backwards."""
 import numpy as np
@@ -61,11 +61,11 @@ def _run(case, q, k, v, do, tiles, tiles_t, scale, packed=False):
 def test_matches_dense_reference(case, d, n, directed, cap, exchange, packed, monkeypatch):
   print(f"node order {case} d={d} n={n} directed={directed} cap={cap} exchange={exchange} packed={packed}", flush=True)
   monkeypatch.setattr(hip_attn, "DS_EXCHANGE", exchange)
-  monkeypatch.setattr(hip_attn, "ORDERED_GAIN", 10.0)  # the order applies whatever it saves
+  monkeypatch.setattr(hip_attn, "LAID_OUT_GAIN", 10.0)  # the layout applies whatever it saves
   mask = _shuffled_mesh(n, 3, n + d, directed)
   tiles = fwn.TileList.from_mask(mask, device=DEV, max_item_tiles=cap)
   tiles_t = fwn.TileList.from_mask(mask.T.tocsr(), device=DEV, max_item_tiles=cap) if directed else None
-  assert tiles._ordered is not None
+  assert tiles._layout is not None
   rng = np.random.default_rng(n)
   b, h = 2, 2
   q, k, v, do = (rounded(rng.standard_normal((b, n, h, d)), CASES[case][0]) for _ in range(4))
@@ -90,14 +90,14 @@ def test_lse_and_empty_rows(case):
     mask[:, r] = False
   mask = mask.tocsr()
   tiles = fwn.TileList.from_mask(mask, device=DEV)
-  assert tiles._ordered is not None
+  assert tiles._layout is not None
   rng = np.random.default_rng(3)
   q, k, v = (dev(rounded(rng.standard_normal((1, n, h, d)), dtype), dtype) for _ in range(3))
   out, lse = fwn.attention_forward(q, k, v, tiles, d ** -0.5, precision=precision)
-  plain = tiles._ordered
-  tiles._ordered = None
+  plain = tiles._layout
+  tiles._layout = None
   out0, lse0 = fwn.attention_forward(q, k, v, tiles, d ** -0.5, precision=precision)
-  tiles._ordered = plain
+  tiles._layout = plain
   assert not host(out)[0, empty].any()
   _check(host(out), host(out0), case, "out")
   keep = np.setdiff1d(np.arange(n), empty)
@@ -109,11 +109,11 @@ def test_lse_and_empty_rows(case):
 def test_order_is_kept_only_where_it_pays():
   """A mesh in mesh order takes an order of its own; a mask without locality, a single block and a
   list whose order saves nothing keep the given one."""
-  assert fwn.TileList.from_mask(fwn.mesh_mask(4, 4)[0], device=DEV)._ordered is not None
+  assert fwn.TileList.from_mask(fwn.mesh_mask(4, 4)[0], device=DEV)._layout is not None
   rng = np.random.default_rng(0)
   m = fwn.mesh_mask(2, 2)[0]
-  assert fwn.TileList.from_mask(m[:128][:, :128].tocsr(), device=DEV)._ordered is None
+  assert fwn.TileList.from_mask(m[:128][:, :128].tocsr(), device=DEV)._layout is None
   dense = sparse.csr_matrix(np.ones((300, 300), bool))
-  assert fwn.TileList.from_mask(dense, device=DEV)._ordered is None
+  assert fwn.TileList.from_mask(dense, device=DEV)._layout is None
   noise = (sparse.random(600, 600, 0.2, random_state=1) + sparse.identity(600)).astype(bool).tocsr()
-  assert fwn.TileList.from_mask(noise, device=DEV)._ordered is None
+  assert fwn.TileList.from_mask(noise, device=DEV)._layout is None
