@@ -564,7 +564,7 @@ def attention(args):
   walked = tiles.launch_list()
   exchange = None
   if cfg["backward"] and not args.no_ds and fwn.hip_attn.DS_EXCHANGE:
-    exchange = tiles.exchange_lists(tiles, fwn.hip_attn.unit_keys_for(dtype))
+    exchange = tiles.exchange_lists(tiles, fwn.hip_attn.products_of(fdesc))
   walked_dq, walked_kv, dmap = exchange or (walked, walked, None)
   # The schedule of each kernel (with --order auto, its order table); the recomputing kernels take
   # the native descriptor.

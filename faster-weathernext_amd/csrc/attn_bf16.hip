@@ -23,11 +23,14 @@
 // and the kernels then address rows through its node tables: the LDS DMA takes any per-lane source
 // address, so a gathered tile copy costs one LDS read and one multiply-add per 1 KB instruction, the
 // nodes of the next tile having been copied into LDS (512 bytes, one instruction of one wave) a tile
-// ahead. The forward's list packs single columns: a refinement-6 block with the 16-hop mask has 13
-// tiles of 88% live groups where the unpacked list has 22 of 56%. Forward + backward, us, list in the
-// caller's order -> laid out (in a compact order alone): 16 hops, 4 heads, mesh order 1261 -> 656
-// (682); 8 hops, 8 members 6645 -> 2681 (2928); 32 hops, 6 heads, Hilbert order 2740 -> 2469 (2539). The
-// forward alone, order alone -> packed: 190 -> 158, 793 -> 604 and 715 -> 632. The variants without G stay for lists
+// ahead. The forward's list packs single columns, those live for the same waves together: a
+// refinement-6 block with the 16-hop mask has 13 tiles with 9.8 live groups (31% of them without a
+// mask) where the unpacked list has 22 with 9.0, and the tile's runs are chosen so that the four
+// waves have the same number of live groups (the largest 4% over the mean; 28% in ascending order).
+// Forward + backward, us, list in the caller's order -> compact order -> packed -> balanced: 16 hops, 4
+// heads, mesh order 1266 -> 682 -> 656 -> 638; 8 hops, 8 members 6642 -> 2928 -> 2681 -> 2591; 32 hops, 6
+// heads, Hilbert order 2735 -> 2539 -> 2469 -> 2414. The forward alone, from the compact order: 190 ->
+// 157 -> 146, 793 -> 601 -> 575 and 715 -> 623 -> 570. The variants without G stay for lists
 // that no layout improves (hip_attn.LAID_OUT_GAIN) and for callers of the C ABI that pass no tables.
 //
 // Reference: pallas_attn.py:112-141 (forward), 161-215 (dQ, dK/dV), 274-311 (VJP driver).

@@ -10,9 +10,9 @@
 // Node tables (G): the rows of a list laid out for the kernels are gathered by the same LDS DMA
 // instructions. The step-streamed kernels (forward, 16-key dK/dV) load the next step's nodes into
 // registers a step ahead, the tile-streamed ones the next tile's into LDS. Refinement-6 mesh, list in
-// the caller's order -> in a compact order -> packed as well: 8-hop 4x128 forward in mesh order 1917 ->
-// 675 -> 485 us; 32-hop Hilbert 6x128 forward + backward 18.45 -> 16.8 -> 16.3 ms (the forward 5.77 ->
-// 5.20 -> 4.65).
+// the caller's order -> in a compact order -> packed -> balanced: 8-hop 4x128 forward in mesh order 1915
+// -> 675 -> 485 -> 448 us; 32-hop Hilbert 6x128 forward + backward 18.44 -> 16.8 -> 16.3 -> 15.7 ms (the
+// forward 5.77 -> 5.20 -> 4.65 -> 4.43, dQ 2.66 -> 2.45 -> 2.41 -> 2.25).
 //
 // Reference: pallas_attn.py:112-141 (forward), 161-215 (dQ, dK/dV), 274-311 (VJP driver).
 #include "attn_device.h"

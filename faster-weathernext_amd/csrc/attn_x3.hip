@@ -12,7 +12,7 @@
 // 32-row group; the operands a wave keeps in registers (forward: Q; dK/dV: its K and V rows) are
 // split when loaded; P and dS are split in registers. Lists
 // with node tables gather the split rows as the float32 kernels gather theirs (32-hop Hilbert 6x128
-// forward + backward at refinement 6: 6.96 -> 6.17 ms against the list in the caller's order).
+// forward + backward at refinement 6: 6.96 -> 6.13 ms against the list in the caller's order).
 //
 // The backward is the dS exchange (5 contractions per tile): dK/dV computes S, dP, dV, dK and
 // writes each 32 x 32 dS group as hi and lo bf16 (4 KB, the float32 exchange's unit size and

@@ -207,20 +207,146 @@ void for_entries(const List& m, const int64_t* perm, const std::vector<int32_t>&
   }
 }
 
-// The live column groups of block blk in ascending order (any row with an element in them).
-void live_groups(const List& m, int64_t blk, int32_t group, std::vector<int32_t>& out) {
-  out.clear();
+// One run of columns that a packed list keeps together, with the load it gives each of the four
+// parts of a workgroup that meet at the tile barriers.
+struct Run {
+  int32_t first;    // index of its first column in the block's column order
+  uint8_t load[4];
+};
+
+// The columns of block blk in the order they are packed, and their runs of `width` columns.
+// group 1: the columns some row has an element in, sorted by the 32-row groups they are live in, then by
+// those all of whose rows have the element, so that a 32-column run is live (or needs no mask) for
+// all of a wave's rows or none; runs of 32. group 16 or 32: the live aligned groups, one run each.
+// Loads: the 32-row groups a run is live in (`pairs` false), or the count of live 16-row groups s and
+// s + 4 (`pairs`: dK/dV's waves by SIMD).
+void block_runs(const List& m, int64_t blk, int32_t group, bool pairs, std::vector<int32_t>& cols,
+                std::vector<Run>& runs) {
+  cols.clear();
+  runs.clear();
   const int32_t rows = std::min(FWN_BLOCK, m.n - (int32_t)blk * FWN_BLOCK);
+  struct Column {
+    int32_t col;
+    uint8_t live16, full32;
+  };
+  std::vector<Column> all;
   for (int32_t t = m.ptr[blk]; t < m.ptr[blk + 1]; ++t) {
-    uint32_t any[kWords] = {};
+    // any[g]: columns with an element in rows 16 g ..; every[g]: in all of rows 32 g .. + 31.
+    uint32_t any[8][kWords] = {}, every[4][kWords];
+    std::memset(every, 0xff, sizeof(every));
     const uint32_t* w = m.bits + t * kTileWords;
-    for (int32_t r = 0; r < rows; ++r)
-      for (int32_t q = 0; q < kWords; ++q) any[q] |= w[r * kWords + q];
-    for (int32_t c = 0; c < FWN_BLOCK; c += group) {
-      const uint32_t mask = group == 32 ? 0xffffffffu : ((1u << group) - 1u) << (c % 32);
-      if ((any[c / 32] & mask) && m.col[t] * FWN_BLOCK + c < m.n) out.push_back((m.col[t] * FWN_BLOCK + c) / group);
+    for (int32_t r = 0; r < FWN_BLOCK; ++r)
+      for (int32_t q = 0; q < kWords; ++q) {
+        const uint32_t v = r < rows ? w[r * kWords + q] : 0u;
+        any[r / 16][q] |= v;
+        every[r / 32][q] &= v;
+      }
+    for (int32_t c = 0; c < FWN_BLOCK; ++c) {
+      const int32_t col = m.col[t] * FWN_BLOCK + c;
+      Column x{col, 0, 0};
+      for (int32_t g = 0; g < 8; ++g) x.live16 |= (any[g][c / 32] >> (c % 32) & 1u) << g;
+      for (int32_t g = 0; g < 4; ++g) x.full32 |= (every[g][c / 32] >> (c % 32) & 1u) << g;
+      if (x.live16 && col < m.n) all.push_back(x);
     }
   }
+  auto live32 = [](uint8_t l) {
+    return (uint8_t)((l & 3 ? 1 : 0) | (l & 12 ? 2 : 0) | (l & 48 ? 4 : 0) | (l & 192 ? 8 : 0));
+  };
+  std::vector<uint8_t> live;  // of each packed column
+  if (group == 1) {
+    std::stable_sort(all.begin(), all.end(), [&](const Column& a, const Column& b) {
+      const uint8_t la = live32(a.live16), lb = live32(b.live16);
+      const int pa = __builtin_popcount(la), pb = __builtin_popcount(lb);
+      if (pa != pb) return pa > pb;
+      if (la != lb) return la < lb;
+      return a.full32 < b.full32;
+    });
+    for (const Column& x : all) {
+      cols.push_back(x.col);
+      live.push_back(x.live16);
+    }
+  } else {
+    for (size_t k = 0; k < all.size();) {
+      const int32_t g = all[k].col / group;
+      const size_t at = cols.size();
+      for (int32_t c = 0; c < group; ++c) cols.push_back(std::min(g * group + c, m.n));
+      live.resize(at + group, 0);
+      for (; k < all.size() && all[k].col / group == g; ++k) live[at + all[k].col % group] = all[k].live16;
+    }
+  }
+  const int32_t width = group == 1 ? 32 : group;
+  for (int32_t i = 0; i < (int32_t)cols.size(); i += width) {
+    uint8_t l = 0;
+    for (int32_t c = i; c < std::min((int32_t)cols.size(), i + width); ++c) l |= live[c];
+    Run r{i, {}};
+    for (int32_t p = 0; p < 4; ++p)
+      r.load[p] = (uint8_t)(pairs ? (l >> p & 1) + (l >> (p + 4) & 1) : live32(l) >> p & 1);
+    runs.push_back(r);
+  }
+}
+
+// Distributes the runs over tiles of `cap` runs so that the four parts of the workgroup have about
+// the same load in each tile, which is what the tile barriers cost: minimises the sum over the tiles
+// of the largest part's load (weighted 64, against the sum of squares that leads there), by dealing
+// the runs out heaviest first and then exchanging pairs while that helps, within a fixed number of
+// trials. slot[k] is the place (tile * cap + position) of run k; runs of a tile keep their order.
+void balance(const std::vector<Run>& runs, int32_t cap, std::vector<int32_t>& slot) {
+  const int32_t n = (int32_t)runs.size(), tiles = (n + cap - 1) / cap, places = tiles * cap;
+  std::vector<Run> item(runs);
+  item.resize(places, Run{-1, {0, 0, 0, 0}});  // empty places have no load
+  std::vector<int32_t> order(places);
+  for (int32_t i = 0; i < places; ++i) order[i] = i;
+  auto total = [&](int32_t i) { return item[i].load[0] + item[i].load[1] + item[i].load[2] + item[i].load[3]; };
+  std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return total(a) > total(b); });
+  struct Tile {
+    int32_t load[4] = {}, count = 0;
+  };
+  std::vector<Tile> tile(tiles);
+  auto value = [](const int32_t (&l)[4]) {
+    const int32_t top = std::max(std::max(l[0], l[1]), std::max(l[2], l[3]));
+    return 64 * top + l[0] * l[0] + l[1] * l[1] + l[2] * l[2] + l[3] * l[3];
+  };
+  std::vector<int32_t> at(places);  // tile of each item
+  int32_t start = 0;
+  for (int32_t i : order) {
+    int32_t best = -1, best_cost = 0;
+    for (int32_t k = 0; k < tiles; ++k) {
+      const int32_t t = (start + k) % tiles;
+      if (tile[t].count == cap) continue;
+      int32_t l[4];
+      for (int p = 0; p < 4; ++p) l[p] = tile[t].load[p] + item[i].load[p];
+      const int32_t cost = value(l) - value(tile[t].load);
+      if (best < 0 || cost < best_cost) best = t, best_cost = cost;
+    }
+    for (int p = 0; p < 4; ++p) tile[best].load[p] += item[i].load[p];
+    ++tile[best].count;
+    at[i] = best;
+    start = (best + 1) % tiles;
+  }
+  int64_t trials = 400000;
+  for (bool more = true; more && trials > 0;) {
+    more = false;
+    for (int32_t a = 0; a < places && trials > 0; ++a)
+      for (int32_t b = a + 1; b < places; ++b) {
+        if (at[a] == at[b] || !std::memcmp(item[a].load, item[b].load, 4)) continue;
+        --trials;
+        Tile &x = tile[at[a]], &y = tile[at[b]];
+        int32_t lx[4], ly[4];
+        for (int p = 0; p < 4; ++p) {
+          const int32_t d = item[b].load[p] - item[a].load[p];
+          lx[p] = x.load[p] + d;
+          ly[p] = y.load[p] - d;
+        }
+        if (value(lx) + value(ly) >= value(x.load) + value(y.load)) continue;
+        std::memcpy(x.load, lx, sizeof(lx));
+        std::memcpy(y.load, ly, sizeof(ly));
+        std::swap(at[a], at[b]);
+        more = true;
+      }
+  }
+  slot.assign(n, 0);
+  std::vector<int32_t> used(tiles, 0);
+  for (int32_t k = 0; k < n; ++k) slot[k] = at[k] * cap + used[at[k]]++;
 }
 
 bool good_group(int32_t group) { return group == 1 || group == 16 || group == 32; }
@@ -366,10 +492,11 @@ int fwn_tiles_compact_count(int32_t n, const int32_t* tile_ptr, const int32_t* t
   try {
     std::vector<int32_t> count(m.n_blocks);
     parallel_for(m.n_blocks, 4, [&](int64_t b, int64_t e) {
-      std::vector<int32_t> live;
+      std::vector<int32_t> cols;
+      std::vector<Run> runs;
       for (int64_t blk = b; blk < e; ++blk) {
-        live_groups(m, blk, group, live);
-        count[blk] = (int32_t)(((int64_t)live.size() * group + FWN_BLOCK - 1) / FWN_BLOCK);
+        block_runs(m, blk, group, false, cols, runs);
+        count[blk] = (int32_t)((cols.size() + FWN_BLOCK - 1) / FWN_BLOCK);
       }
     });
     new_ptr[0] = 0;
@@ -381,30 +508,45 @@ int fwn_tiles_compact_count(int32_t n, const int32_t* tile_ptr, const int32_t* t
 }
 
 int fwn_tiles_compact_fill(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
-                           int32_t group, const int32_t* new_ptr, int32_t* cols, uint32_t* new_bits) {
+                           int32_t group, int32_t parts, int32_t window, const int32_t* new_ptr, int32_t* cols,
+                           uint32_t* new_bits) {
   fwn::clear_error();
   List m;
   if (int rc = make_list(m, "fwn_tiles_compact_fill", n, tile_ptr, tile_col, tile_bits)) return rc;
-  if (!new_ptr || !good_group(group) || (new_ptr[m.n_blocks] > 0 && (!cols || !new_bits)))
-    return fwn::fail(FWN_ERR_INVALID_ARG, "fwn_tiles_compact_fill: null output or group %d (1, 16 or 32)", group);
+  if (!new_ptr || !good_group(group) || (new_ptr[m.n_blocks] > 0 && (!cols || !new_bits)) || parts < 0 ||
+      parts > FWN_PARTS_PAIRS16 || window < 0)
+    return fwn::fail(FWN_ERR_INVALID_ARG,
+                     "fwn_tiles_compact_fill: null output, group %d (1, 16 or 32), parts %d or window %d", group, parts,
+                     window);
   std::atomic<bool> bad(false);
   try {
     parallel_for(m.n_blocks, 4, [&](int64_t b, int64_t e) {
-      std::vector<int32_t> live, at((size_t)m.n_blocks * FWN_BLOCK / group, -1);
+      const int32_t width = group == 1 ? 32 : group;
+      std::vector<int32_t> packed, slot, place, at((size_t)m.n_blocks * FWN_BLOCK, -1);
+      std::vector<Run> runs, part;
       for (int64_t blk = b; blk < e; ++blk) {
-        live_groups(m, blk, group, live);
+        block_runs(m, blk, group, parts == FWN_PARTS_PAIRS16, packed, runs);
         const int64_t t0 = new_ptr[blk], tiles = new_ptr[blk + 1] - t0;
-        if (tiles != ((int64_t)live.size() * group + FWN_BLOCK - 1) / FWN_BLOCK) {
+        if (tiles != (int64_t)(packed.size() + FWN_BLOCK - 1) / FWN_BLOCK) {
           bad = true;
           return;
         }
+        if (tiles == 0) continue;
+        slot.clear();
+        const size_t cap = FWN_BLOCK / width, step = window ? window * cap : runs.size();
+        for (size_t k = 0; k < runs.size(); k += step) {
+          part.assign(runs.begin() + k, runs.begin() + std::min(runs.size(), k + step));
+          balance(part, (int32_t)cap, place);
+          for (int32_t x : place) slot.push_back((int32_t)k + x);
+        }
         std::memset(new_bits + t0 * kTileWords, 0, tiles * kTileWords * sizeof(uint32_t));
         std::fill(cols + t0 * FWN_BLOCK, cols + (t0 + tiles) * FWN_BLOCK, n);
-        for (size_t k = 0; k < live.size(); ++k) {
-          at[live[k]] = (int32_t)(k * group);
-          for (int32_t c = 0; c < group; ++c)
-            cols[t0 * FWN_BLOCK + k * group + c] = std::min(live[k] * group + c, n);
-        }
+        for (size_t k = 0; k < runs.size(); ++k)
+          for (int32_t c = 0; c < width && runs[k].first + c < (int32_t)packed.size(); ++c) {
+            const int32_t col = packed[runs[k].first + c], to = slot[k] * width + c;
+            cols[t0 * FWN_BLOCK + to] = col;
+            if (col < n) at[col] = to;
+          }
         const int32_t rows = std::min(FWN_BLOCK, n - (int32_t)blk * FWN_BLOCK);
         for (int32_t t = m.ptr[blk]; t < m.ptr[blk + 1]; ++t)
           for (int32_t r = 0; r < rows; ++r)
@@ -412,7 +554,7 @@ int fwn_tiles_compact_fill(int32_t n, const int32_t* tile_ptr, const int32_t* ti
               for (uint32_t v = m.bits[t * kTileWords + r * kWords + q]; v; v &= v - 1) {
                 const int32_t c = m.col[t] * FWN_BLOCK + 32 * q + __builtin_ctz(v);
                 if (c >= n) continue;
-                const int32_t to = at[c / group] + c % group;
+                const int32_t to = at[c];
                 new_bits[(t0 + to / FWN_BLOCK) * kTileWords + r * kWords + to % FWN_BLOCK / 32] |= 1u << (to % 32);
               }
       }

@@ -63,6 +63,7 @@ class DsMap(ctypes.Structure):
               ("unit_keys", ctypes.c_int32), ("table", ctypes.c_int32)]
 
 
+PARTS_ROWS32, PARTS_PAIRS16 = 0, 1  # FWN_PARTS_*: whose work a packed list balances per tile
 ITEM_TILES = 64  # FWN_ITEM_TILES: default longest run of tiles per work item
 ORDER_ITEMS, ORDER_BALANCED, ORDER_MAKESPAN = 0, 1, 2  # FWN_ORDER_*
 SCRATCH_BYTES = 64 << 20  # FWN_SCRATCH_BYTES: static scratch of fwn_attn_fwd_launch_noalloc
@@ -97,7 +98,7 @@ SIGNATURES = {
     "fwn_tiles_permute_count": [_I32, _P, _P, _P, _P, _P],
     "fwn_tiles_permute_fill": [_I32, _P, _P, _P, _P, _P, _P, _P],
     "fwn_tiles_compact_count": [_I32, _P, _P, _P, _I32, _P],
-    "fwn_tiles_compact_fill": [_I32, _P, _P, _P, _I32, _P, _P, _P],
+    "fwn_tiles_compact_fill": [_I32, _P, _P, _P, _I32, _I32, _I32, _P, _P, _P],
     "fwn_tiles_unit_map": [_I32, _P, _P, _P, _P, _P, _P, _I32, _P, _P, _P],
     "fwn_tiles_schedule_count": [_I32, _P, _I32, _P, _P, _P],
     "fwn_tiles_schedule_fill": [_I32, _P, _I32, _P, _P],

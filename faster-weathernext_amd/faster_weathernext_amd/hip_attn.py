@@ -82,14 +82,27 @@ ORDER_TILE_UNITS = 20
 ORDER_HALF_UNITS = 1
 
 
+# Keys per dS unit of the exchange, by products.
+DS_UNIT_KEYS = {"bf16": 16, "f32": 32, "bf16x3": 32}
+# Windows (tiles) within which dQ's packed list balances its waves' work per tile; 0: whole blocks.
+# Balancing mixes distant keys into a tile, which costs the memory-bound dQ kernels locality in L2.
+# Measured on MI355X, ms, windows of 1 (ascending order), 8 and whole blocks: bf16 C3 0.154 / 0.154 /
+# 0.151, C4 0.598 / 0.572 / 0.572, C5 shape 0.509 / 0.510 / 0.529; C5 shape with split products 1.019
+# / 1.031 / 1.097, with IEEE float32 products (bound by its matrix cores) 2.40 / 2.35 / 2.25.
+DQ_WINDOW = {"bf16": 8, "f32": 0, "bf16x3": 1}
+
+
+def products_of(desc):
+  """The kernels' products for a call with descriptor `desc`: "bf16", "f32" (IEEE) or "bf16x3"."""
+  if desc.precision == nat.PREC_BF16X3:
+    return "bf16x3"
+  return "bf16" if desc.dtype == nat.BF16 else "f32"
+
+
 def order_plan(desc, kernel):
   """(cut, window, slots) of the order table for `kernel` ("fwd", "dq" or "kv") of a call with
   descriptor `desc`."""
-  if desc.precision == nat.PREC_BF16X3:
-    products = "bf16x3"
-  else:
-    products = "bf16" if desc.dtype == nat.BF16 else "f32"
-  return ORDER_CUTS[kernel], ORDER_WINDOWS[products][kernel], ORDER_SLOTS[kernel]
+  return ORDER_CUTS[kernel], ORDER_WINDOWS[products_of(desc)][kernel], ORDER_SLOTS[kernel]
 
 
 class _Schedule:
@@ -143,10 +156,12 @@ class _Schedule:
     return self._orders[key][1]
 
 
-# Lists laid out for the kernels (TileList.launch_list): taken when the estimated cost of their tiles
-# (ORDER_TILE_UNITS per tile + ORDER_HALF_UNITS per live 32 x 16 half) is at most LAID_OUT_GAIN of the
-# given list's. On the refinement-6 mesh the forward's estimates are 0.24 (8 hops) and 0.37 (16
-# hops) of mesh order's list, 0.77 of Hilbert order's (32 hops).
+# Lists laid out for the kernels (TileList.launch_list): taken when both the number of tiles and
+# their estimated cost (ORDER_TILE_UNITS per tile + ORDER_HALF_UNITS per live 32 x 16 half) are at
+# most LAID_OUT_GAIN of the given list's. On the refinement-6 mesh the forward's cost is 0.20 (8
+# hops) and 0.33 (16 hops) of mesh order's list, 0.73 of Hilbert order's (32 hops), its tiles 0.14,
+# 0.25 and 0.64. A mask without locality (random entries) has as many tiles in any order; it keeps
+# the given list, and with it that list's results bit for bit.
 LAID_OUT_GAIN = 0.95
 
 
@@ -230,14 +245,15 @@ class TileList:
     out for it where there is one, else this one."""
     return self if self._layout is None else self._layout.forward
 
-  def exchange_lists(self, tiles_t, unit_keys):
+  def exchange_lists(self, tiles_t, products):
     """(list for dQ, list for dK/dV, dS map) of the dS exchange with `tiles_t`, the transposed
-    mask's list (this list itself for a symmetric mask), or None when it is not the exact
-    transpose (the recomputing backward applies then). Built on first use and kept."""
-    dmap = self.ds_map(tiles_t, unit_keys)
+    mask's list (this list itself for a symmetric mask), for kernels with these products (see
+    ``products_of``), or None when it is not the exact transpose (the recomputing backward
+    applies then). Built on first use and kept."""
+    dmap = self.ds_map(tiles_t, DS_UNIT_KEYS[products])
     if dmap is None:
       return None
-    laid_out = self._layout and self._layout.exchange(tiles_t, unit_keys)
+    laid_out = self._layout and self._layout.exchange(tiles_t, products)
     return laid_out or (self, tiles_t, dmap)
 
   def _schedule(self, cap):
@@ -347,7 +363,7 @@ class _PackedList(TileList):
   (``fwn_tiles_compact_*``). ``cols`` holds the column of each tile column; ``node[c]`` is the node of
   row or column c (n past the last)."""
 
-  def __init__(self, arrays, group, node, row_node, device, max_item_tiles):
+  def __init__(self, arrays, group, parts, window, node, row_node, device, max_item_tiles):
     L = nat.lib()
     self.n = arrays.n
     ptr = np.zeros_like(arrays.ptr)
@@ -355,7 +371,7 @@ class _PackedList(TileList):
     tiles = int(ptr[-1])
     self.cols = np.empty((tiles, nat.BLOCK), np.int32)
     bits = np.empty((tiles, nat.BLOCK, nat.BLOCK // 32), np.uint32)
-    nat.check(L.fwn_tiles_compact_fill(*arrays.args, group, nat.ptr(ptr), nat.ptr(self.cols), nat.ptr(bits)))
+    nat.check(L.fwn_tiles_compact_fill(*arrays.args, group, parts, window, nat.ptr(ptr), nat.ptr(self.cols), nat.ptr(bits)))
     self._row_node = row_node
     self._col_node = torch.from_numpy(node[self.cols]).to(device)
     self._layout = None
@@ -383,8 +399,8 @@ class _Layout:
     self._pairs = weakref.WeakKeyDictionary()
     self.forward = self.packed(arrays, 1)
 
-  def packed(self, arrays, group):
-    return _PackedList(arrays, group, self._node, self._row_node, self._device, self._cap)
+  def packed(self, arrays, group, parts=nat.PARTS_ROWS32, window=0):
+    return _PackedList(arrays, group, parts, window, self._node, self._row_node, self._device, self._cap)
 
   @classmethod
   def choose(cls, tl):
@@ -403,20 +419,27 @@ class _Layout:
       layout = cls(arrays, p, tl.device, tl._fixed_cap)
       if best is None or layout.forward.cost < best.forward.cost:
         best = layout
-      if best.forward.cost <= LAID_OUT_GAIN * tl.cost:
-        break
-    return best if best.forward.cost <= LAID_OUT_GAIN * tl.cost else None
+      if best._pays(tl):
+        return best
+    return None
 
-  def exchange(self, tiles_t, unit_keys):
-    """(list for dQ, list for dK/dV, map) in this layout; `tiles_t` is the exact transpose."""
+  def _pays(self, tl):
+    return (self.forward.n_tiles <= LAID_OUT_GAIN * tl.n_tiles and
+            self.forward.cost <= LAID_OUT_GAIN * tl.cost)
+
+  def exchange(self, tiles_t, products):
+    """(list for dQ, list for dK/dV, map) in this layout for kernels with these products; `tiles_t`
+    is the exact transpose."""
     pairs = self._pairs.setdefault(tiles_t, {})
-    if unit_keys not in pairs:
+    unit_keys, window = DS_UNIT_KEYS[products], DQ_WINDOW[products]
+    if products not in pairs:
       own = tiles_t._layout is self
       arrays_t = self.arrays if own else _Arrays(self.arrays.n, tiles_t._tile_ptr, tiles_t._tile_col,
                                                  tiles_t._tile_bits).permuted(self.perm)
-      dq, kv = self.packed(self.arrays, unit_keys), self.packed(arrays_t, 32)
-      pairs[unit_keys] = (dq, kv, DsMap.of_packed(dq, kv, unit_keys))
-    return pairs[unit_keys]
+      dq = self.packed(self.arrays, unit_keys, window=window)
+      kv = self.packed(arrays_t, 32, nat.PARTS_PAIRS16)
+      pairs[products] = (dq, kv, DsMap.of_packed(dq, kv, unit_keys))
+    return pairs[products]
 
 
 class DsMap:
@@ -640,12 +663,13 @@ def _backward_into(q, k, v, out, lse, dout, tiles, tiles_t, scale, dq, dk, dv, p
   delta = torch.empty_like(lse)
   L = nat.lib()
   main = torch.cuda.current_stream(q.device)
-  exchange = base.exchange_lists(base_t, unit_keys_for(q.dtype))
+  exact = _desc(q, scale, out, _precision(precision, q.dtype))  # the exchange's descriptor
+  exchange = base.exchange_lists(base_t, products_of(exact))
   # Without the exchange the kernels walk the same lists (dK and dV are then the same bit for bit).
   tl, tlt, dmap = exchange or (base.launch_list(), base_t.launch_list(), None)
   if DS_EXCHANGE and dmap is not None:
     # delta, dK/dV writing dS, then dQ from dS, in stream order (fwn_attn_bwd_ds_launch).
-    desc = _desc(q, scale, out, _precision(precision, q.dtype))
+    desc = exact
     ws = workspace(desc, q.device, tl, tlt)
     ds = torch.empty(max(dmap.ds_bytes(desc), 256), dtype=torch.uint8, device=q.device)
     ts, tst = tl.struct_for_desc(desc, "dq"), tlt.struct_for_desc(desc, "kv")

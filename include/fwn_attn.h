@@ -209,15 +209,24 @@ int fwn_tiles_permute_fill(int32_t n, const int32_t* tile_ptr, const int32_t* ti
                            const int64_t* perm, const int32_t* new_ptr, int32_t* new_col, uint32_t* new_bits);
 
 /* The tile list with each block's columns compacted: of the groups of `group` (1, 16 or 32)
- * consecutive columns, those in which some row of the block has a valid element, in ascending
- * order, packed into tiles of 128 columns. fwn_tiles_compact_count writes new_ptr[n_blocks + 1];
- * fwn_tiles_compact_fill writes cols[new_ptr[last] * 128], the column of each tile column (n for
- * padding), and new_bits[new_ptr[last] * 128 * 4]. A column of a compacted list is not a column
- * block's, so its launches need FWN_TILES_NODES. No reference counterpart. */
+ * consecutive columns, those in which some row of the block has a valid element, packed into tiles of
+ * 128 columns. fwn_tiles_compact_count writes new_ptr[n_blocks + 1]; fwn_tiles_compact_fill writes
+ * cols[new_ptr[last] * 128], the column of each tile column (n for padding), and
+ * new_bits[new_ptr[last] * 128 * 4]. Which groups share a tile is chosen so that the parts of a
+ * workgroup that meet at the tile's barrier have about the same work in it: its four waves of 32
+ * rows (FWN_PARTS_ROWS32), or the wave pairs of 16-row groups s and s + 4 that share a SIMD in the
+ * bf16 dK/dV kernel (FWN_PARTS_PAIRS16). The choice is made within windows of `window` tiles' worth of
+ * consecutive groups (0: the whole block; 1: ascending order). With group 1 the columns are first sorted by the 32-row
+ * groups they are live in and full in, so that 32-column groups are so for all of their columns.
+ * A column of a compacted list is not a column block's, so its launches need FWN_TILES_NODES. No
+ * reference counterpart. */
+#define FWN_PARTS_ROWS32 0
+#define FWN_PARTS_PAIRS16 1
 int fwn_tiles_compact_count(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
                             int32_t group, int32_t* new_ptr);
 int fwn_tiles_compact_fill(int32_t n, const int32_t* tile_ptr, const int32_t* tile_col, const uint32_t* tile_bits,
-                           int32_t group, const int32_t* new_ptr, int32_t* cols, uint32_t* new_bits);
+                           int32_t group, int32_t parts, int32_t window, const int32_t* new_ptr, int32_t* cols,
+                           uint32_t* new_bits);
 
 /* Work items of a tile list: the tiles of each block are cut into ceil(count / max_item_tiles)
  * runs of near-equal length (max_item_tiles <= 0 selects FWN_ITEM_TILES). The reference runs one

@@ -69,10 +69,11 @@ def test_order_is_deterministic_and_compact_on_a_shuffled_mesh():
   assert tiles <= _arrays(mask, hilbert)[0][-1] < tp[-1]
 
 
-def _compact(n, tp, kb, bits, group):
+def _compact(n, tp, kb, bits, group, parts=0, window=0):
   new_ptr = np.zeros_like(tp)
   args = (n, nat.ptr(tp), nat.ptr(kb), nat.ptr(bits), group)
   nat.check(nat.lib().fwn_tiles_compact_count(*args, nat.ptr(new_ptr)))
+  args = (*args, parts, window)
   cols = np.full((new_ptr[-1], 128), -7, np.int32)
   new_bits = np.full((new_ptr[-1], 128, 4), 0xFFFFFFFF, np.uint32)
   nat.check(nat.lib().fwn_tiles_compact_fill(*args, nat.ptr(new_ptr), nat.ptr(cols), nat.ptr(new_bits)))
@@ -83,29 +84,43 @@ def _bools(bits):
   return np.unpackbits(bits.view(np.uint8), axis=-1, bitorder="little").reshape(len(bits), 128, 128).astype(bool)
 
 
-@pytest.mark.parametrize("group", [1, 16, 32])
+@pytest.mark.parametrize("group,parts,window", [(1, 0, 0), (16, 0, 0), (16, 0, 2), (32, 0, 1), (32, 1, 0)])
 @pytest.mark.parametrize("name", [n for n, _ in _masks()])
-def test_packed_list_holds_the_mask(name, group):
+def test_packed_list_holds_the_mask(name, group, parts, window):
   """Unpacked through its columns, a packed list is the mask; every column group it holds is live
-  in the block, whole, once and in order; only a block's last tile is padded."""
+  in the block, whole and once, in as few tiles as hold them."""
   mask = dict(_masks())[name].tocsr()
   n = mask.shape[0]
-  ptr, cols, bits = _compact(n, *_arrays(mask), group)
+  ptr, cols, bits = _compact(n, *_arrays(mask), group, parts, window)
   dense, got = mask.toarray(), np.zeros((n, n + 1), bool)
   b = _bools(bits)
   for blk in range(len(ptr) - 1):
     r0, r1 = 128 * blk, min(n, 128 * blk + 128)
-    c = cols[ptr[blk]:ptr[blk + 1]].ravel()
-    live = c[c < n]
-    assert np.all(np.diff(live) > 0) and np.all(c[len(live):] == n)
+    c = cols[ptr[blk]:ptr[blk + 1]].reshape(-1, group)
+    c = c[c[:, 0] < n]
+    assert np.all(c[:, 0] % group == 0) and np.array_equal(c, np.minimum(c[:, :1] + np.arange(group), n))
     want = np.unique(np.nonzero(dense[r0:r1].any(0))[0] // group)
-    assert np.array_equal(np.unique(live // group), want)
-    assert len(live) == sum(min(group, n - g * group) for g in want)
+    assert np.array_equal(np.sort(c[:, 0] // group), want)
     assert ptr[blk + 1] - ptr[blk] == -(-len(want) * group // 128)
     for t in range(ptr[blk], ptr[blk + 1]):
       assert not b[t][:, cols[t] == n].any() and not b[t][r1 - r0:].any()
       got[r0:r1, cols[t]] |= b[t][:r1 - r0]
   assert np.array_equal(got[:, :n], dense)
+
+
+def test_packed_list_balances_the_waves():
+  """Per tile, the part of a workgroup with the most live runs has at most 15% more than the mean of
+  its four parts, over a mesh's blocks (36 to 70% more when the runs are packed in ascending order)."""
+  mask, _, _, _ = fwn.mesh_mask(5, 8)
+  n = mask.shape[0]
+  tp, kb, bits = _arrays(mask)
+  arrays = _permuted(n, tp, kb, bits, _order(n, tp, kb, bits))
+  for group, parts in ((16, 0), (32, 1)):
+    b = _bools(_compact(n, *arrays, group, parts)[2])
+    rows = 32 if parts == 0 else 16
+    live = b.reshape(len(b), 128 // rows, rows, 128 // group, group).any((2, 4)).sum(2)
+    load = live if parts == 0 else live[:, :4] + live[:, 4:]
+    assert load.max(1).sum() <= 1.15 * load.mean(1).sum(), (group, load.max(1).sum() / load.mean(1).sum())
 
 
 def _unit_map(n, f, t, unit_keys):
@@ -183,7 +198,7 @@ def test_bad_arguments_are_refused():
   assert L.fwn_tiles_node_order(n, nat.ptr(tp), nat.ptr(col), nat.ptr(bits), nat.ptr(perm)) == nat.ERR_TILES
   for group in (0, 2, 64):
     assert L.fwn_tiles_compact_count(*good, group, nat.ptr(ptr)) == nat.ERR_INVALID_ARG
-  assert L.fwn_tiles_compact_fill(*good, 1, nat.ptr(np.array([0, 1, 1], np.int32)), nat.ptr(np.zeros(128, np.int32)),
+  assert L.fwn_tiles_compact_fill(*good, 1, 0, 0, nat.ptr(np.array([0, 1, 1], np.int32)), nat.ptr(np.zeros(128, np.int32)),
                                   nat.ptr(np.zeros((1, 128, 4), np.uint32))) == nat.ERR_INVALID_ARG
   # a pointer array of another order's list
   assert L.fwn_tiles_permute_fill(*good, nat.ptr(perm), nat.ptr(np.array([0, 1, 2], np.int32)), nat.ptr(np.zeros(2, np.int32)),
