@@ -92,11 +92,15 @@ DS_UNIT_KEYS = {"bf16": 16, "f32": 32, "bf16x3": 32}
 DQ_WINDOW = {"bf16": 8, "f32": 0, "bf16x3": 1}
 
 
+def _products(dtype, precision):
+  if precision == nat.PREC_BF16X3:
+    return "bf16x3"
+  return "bf16" if dtype == torch.bfloat16 else "f32"
+
+
 def products_of(desc):
   """The kernels' products for a call with descriptor `desc`: "bf16", "f32" (IEEE) or "bf16x3"."""
-  if desc.precision == nat.PREC_BF16X3:
-    return "bf16x3"
-  return "bf16" if desc.dtype == nat.BF16 else "f32"
+  return _products(torch.bfloat16 if desc.dtype == nat.BF16 else torch.float32, desc.precision)
 
 
 def order_plan(desc, kernel):
@@ -226,6 +230,8 @@ class TileList:
     self._tile_col = tile_kb
     self._tile_bits = tile_bits
     self._ds_maps = {}
+    self._exchanges = weakref.WeakKeyDictionary()
+    self._plans = {}
     self._fixed_cap = None if max_item_tiles is None else int(max_item_tiles)
     self._schedules = {}
     base = self._schedule(nat.ITEM_TILES if self._fixed_cap is None else self._fixed_cap)
@@ -250,11 +256,27 @@ class TileList:
     mask's list (this list itself for a symmetric mask), for kernels with these products (see
     ``products_of``), or None when it is not the exact transpose (the recomputing backward
     applies then). Built on first use and kept."""
-    dmap = self.ds_map(tiles_t, DS_UNIT_KEYS[products])
-    if dmap is None:
-      return None
-    laid_out = self._layout and self._layout.exchange(tiles_t, products)
-    return laid_out or (self, tiles_t, dmap)
+    exchange = self._exchange(tiles_t, products)
+    return None if exchange is None else (exchange.dq, exchange.kv, exchange.dmap)
+
+  def _exchange(self, tiles_t, products):
+    """The _Exchange with `tiles_t` for these products, or None (``exchange_lists``)."""
+    made = self._exchanges.get(tiles_t)
+    if made is None:
+      made = self._exchanges[tiles_t] = {}
+    if products not in made:
+      dmap = self.ds_map(tiles_t, DS_UNIT_KEYS[products])
+      laid_out = dmap and self._layout and self._layout.exchange(tiles_t, products)
+      made[products] = _Exchange(*(laid_out or (self, tiles_t, dmap))) if dmap else None
+    return made[products]
+
+  def forward_plan(self, q, o, scale, precision):
+    """(descriptor, C struct, workspace bytes) of a forward call over this list, kept by the call's
+    shape and strides (``_plan``)."""
+    def make(desc):
+      ts = self.struct_for_desc(desc, "fwd")
+      return ts, _workspace_size(desc, ts)
+    return _plan(self._plans, q, o, scale, precision, make)
 
   def _schedule(self, cap):
     cap = int(cap) if cap > 0 else nat.ITEM_TILES
@@ -493,6 +515,47 @@ class DsMap:
     return int(n.value)
 
 
+class _Exchange:
+  """The lists and map of one dS exchange (``TileList.exchange_lists``) and its calls' plans."""
+
+  def __init__(self, dq, kv, dmap):
+    self.dq, self.kv, self.dmap = dq, kv, dmap
+    self._plans = {}
+
+  def plan(self, q, o, scale, precision):
+    """(descriptor, dQ's C struct, dK/dV's, workspace bytes, dS bytes) of a backward call."""
+    def make(desc):
+      ts, tst = self.dq.struct_for_desc(desc, "dq"), self.kv.struct_for_desc(desc, "kv")
+      return ts, tst, max(_workspace_size(desc, ts), _workspace_size(desc, tst)), max(self.dmap.ds_bytes(desc), 256)
+    return _plan(self._plans, q, o, scale, precision, make)
+
+
+def _workspace_size(desc, struct):
+  n = ctypes.c_uint64(0)
+  nat.check(nat.lib().fwn_attn_workspace_size(desc, struct, ctypes.byref(n)))
+  return int(n.value)
+
+
+# Plans kept per list: a program's calls repeat a few shapes, and forming a call's descriptor, its
+# schedules and workspace sizes takes longer than a small call's kernels (forward + backward of a
+# refinement-3 layer: 100 us of host time, 55 with the plans kept).
+PLANS = 32
+
+
+def _plan(plans, q, o, scale, precision, make):
+  """(descriptor, *make(descriptor)) of a call with q's shape, strides and dtype and o's strides:
+  values that depend on nothing else, kept in `plans` (at most PLANS, then started over)."""
+  key = (q.shape, q.stride(), o.stride(), q.dtype, scale, precision)
+  plan = plans.get(key)
+  if plan is None:
+    desc = _desc(q, scale, o, precision)
+    plan = (desc, *make(desc))
+    if len(plans) >= PLANS:
+      plans.clear()
+    plans[key] = plan
+  return plan
+
+
 # The backward uses the dS exchange (DsMap) when the lists allow it; False keeps the
 # recomputing dQ kernel beside dK/dV for every call.
 DS_EXCHANGE = True
@@ -618,11 +681,10 @@ def attention_forward(q, k, v, tiles, scale, with_lse=True, precision="native"):
   k = _same_layout(k, q, "k")
   v = _same_layout(v, q, "v")
   out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-  desc = _desc(q, scale, out, prec)
   tl = _as_tiles(tiles, q.shape[1], q.device).launch_list()
+  desc, ts, ws_bytes = tl.forward_plan(q, out, float(scale), prec)
   lse = torch.empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32, device=q.device) if with_lse else None
-  ws = workspace(desc, q.device, tl)
-  ts = tl.struct_for_desc(desc, "fwd")
+  ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
   nat.check(nat.lib().fwn_attn_fwd_launch(desc, q.data_ptr(), k.data_ptr(), v.data_ptr(), ts, out.data_ptr(),
                                           lse.data_ptr() if with_lse else None, *_ws_args(ws), _stream(q.device)))
   return out, lse
@@ -656,28 +718,27 @@ def _backward_into(q, k, v, out, lse, dout, tiles, tiles_t, scale, dq, dk, dv, p
   other's last workgroups leave idle. The sequence is what fwn_attn_bwd_launch enqueues on one
   stream, with the dQ and dK/dV launches overlapped. ``precision`` "bf16x3" applies to the dS
   exchange only."""
-  desc = _desc(q, scale, out)
   n = q.shape[1]
   base = _as_tiles(tiles, n, q.device)
   base_t = base if tiles_t is None else _as_tiles(tiles_t, n, q.device)
   delta = torch.empty_like(lse)
   L = nat.lib()
   main = torch.cuda.current_stream(q.device)
-  exact = _desc(q, scale, out, _precision(precision, q.dtype))  # the exchange's descriptor
-  exchange = base.exchange_lists(base_t, products_of(exact))
-  # Without the exchange the kernels walk the same lists (dK and dV are then the same bit for bit).
-  tl, tlt, dmap = exchange or (base.launch_list(), base_t.launch_list(), None)
-  if DS_EXCHANGE and dmap is not None:
+  prec = _precision(precision, q.dtype)
+  exchange = base._exchange(base_t, _products(q.dtype, prec))
+  if DS_EXCHANGE and exchange is not None:
     # delta, dK/dV writing dS, then dQ from dS, in stream order (fwn_attn_bwd_ds_launch).
-    desc = exact
-    ws = workspace(desc, q.device, tl, tlt)
-    ds = torch.empty(max(dmap.ds_bytes(desc), 256), dtype=torch.uint8, device=q.device)
-    ts, tst = tl.struct_for_desc(desc, "dq"), tlt.struct_for_desc(desc, "kv")
+    desc, ts, tst, ws_bytes, ds_bytes = exchange.plan(q, out, float(scale), prec)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
+    ds = torch.empty(ds_bytes, dtype=torch.uint8, device=q.device)
     nat.check(L.fwn_attn_bwd_ds_launch(desc, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                                       dout.data_ptr(), lse.data_ptr(), delta.data_ptr(), ts, tst, dmap.struct,
-                                       dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ds.data_ptr(), ds.numel(),
+                                       dout.data_ptr(), lse.data_ptr(), delta.data_ptr(), ts, tst, exchange.dmap.struct,
+                                       dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ds.data_ptr(), ds_bytes,
                                        *_ws_args(ws), main.cuda_stream))
     return
+  # Without the exchange the kernels walk the same lists (dK and dV are then the same bit for bit).
+  tl, tlt = (exchange.dq, exchange.kv) if exchange else (base.launch_list(), base_t.launch_list())
+  desc = _desc(q, scale, out)
   ws_q, ws_kv = workspace(desc, q.device, tl), workspace(desc, q.device, tlt)
   nat.check(L.fwn_attn_bwd_delta_launch(desc, out.data_ptr(), dout.data_ptr(), delta.data_ptr(), main.cuda_stream))
   side = _side_stream(q.device)
