@@ -371,6 +371,46 @@ __global__ void __launch_bounds__(64 * kSumGroups) sums_kernel(RowBwdArgs a) {
     a.g_add[(size_t)b * a.channels + j - a.channels] = s;
 }
 
+// ------------------------------------------------------------------------------------------
+// The conditioning of several norms in one launch: one thread per output column, its weight row read
+// straight from memory (64 bytes at 32 bf16 conditioning features; read once for 4 batch members).
+// Bound by launches, not by bytes: each norm's own GEMM, add and two casts are four or five launches.
+// The 49 norms of a 24-layer transformer of 768 channels, issued back to back: 1.7 to 2.0 ms norm by
+// norm, 58 us here (most of it the host's); its whole refinement-6 forward 30.04 -> 29.84 ms.
+template <typename T>
+__device__ __forceinline__ float load_one(const void* p, size_t i) {
+  if constexpr (sizeof(T) == 4) {
+    return ((const float*)p)[i];
+  } else {
+    return as_float((uint32_t)((const uint16_t*)p)[i] << 16);
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) cond_kernel(CondArgs a) {
+  const int cols = 2 * a.channels, per = (cols + 255) / 256;
+  const int l = (int)blockIdx.x / per, j = ((int)blockIdx.x - l * per) * 256 + (int)threadIdx.x;
+  if (j >= cols) return;
+  const void* w = a.weight[l];
+  const float first = load_one<T>(a.bias[l], (size_t)j) + (j < a.channels ? 1.f : 0.f);
+  float* out = (j < a.channels ? a.mul + j : a.add + (j - a.channels)) + (size_t)l * a.batch * a.channels;
+  constexpr int MEMBERS = 4;  // one pass over the weight row for this many batch members
+  for (int b0 = 0; b0 < a.batch; b0 += MEMBERS) {
+    const int nb = a.batch - b0 < MEMBERS ? a.batch - b0 : MEMBERS;
+    float sum[MEMBERS] = {};
+#pragma unroll 8
+    for (int k = 0; k < a.cond_size; ++k) {
+      const float wk = load_one<T>(w, (size_t)j * a.cond_size + k);
+#pragma unroll
+      for (int m = 0; m < MEMBERS; ++m)
+        sum[m] = fmaf(wk, load_one<T>(a.cond, (size_t)(b0 + (m < nb ? m : 0)) * a.cond_size + k), sum[m]);
+    }
+#pragma unroll
+    for (int m = 0; m < MEMBERS; ++m)
+      if (m < nb) out[(size_t)(b0 + m) * a.channels] = sum[m] + first;
+  }
+}
+
 template <typename T, int VPL>
 hipError_t launch_bwd_tv(const RowBwdArgs& a, hipStream_t stream) {
   const dim3 grid((unsigned)a.blocks * (unsigned)a.batch), block(64 * kWaves);
@@ -411,6 +451,15 @@ int32_t rows_bwd_blocks(int32_t batch, int32_t n, bool sums) {
   const int64_t want = ((int64_t)n + rows - 1) / rows, cap = most / (batch > 0 ? batch : 1);
   const int64_t blocks = want < cap ? want : cap;
   return (int32_t)(blocks > 1 ? blocks : 1);
+}
+
+hipError_t launch_cond(int dtype, const CondArgs& a, hipStream_t stream) {
+  const dim3 grid((unsigned)a.count * ((2u * (unsigned)a.channels + 255u) / 256u)), block(256);
+  if (dtype == FWN_F32)
+    hipLaunchKernelGGL(cond_kernel<float>, grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL(cond_kernel<uint16_t>, grid, block, 0, stream, a);
+  return hipGetLastError();
 }
 
 hipError_t launch_rows_bwd(int dtype, const RowBwdArgs& a, hipStream_t stream) {

@@ -186,4 +186,33 @@ int fwn_rows_norm_bwd_launch(const fwn_rows_desc* d, const void* x, const int64_
   return status(launch_rows_bwd(d->dtype, a, (hipStream_t)stream), what);
 }
 
+int fwn_cond_affine_launch(int32_t count, int32_t batch, int32_t channels, int32_t cond_size, int32_t dtype,
+                           const void* cond, const void* const* weight, const void* const* bias, float* mul,
+                           float* add, void* stream) {
+  using namespace fwn;
+  clear_error();
+  const char* what = "fwn_cond_affine_launch";
+  if (count < 1 || count > FWN_COND_MAX || batch <= 0 || cond_size <= 0)
+    return fail(FWN_ERR_INVALID_ARG, "%s: count %d (1 to %d), batch %d, cond_size %d", what, count, FWN_COND_MAX, batch,
+                cond_size);
+  if (channels <= 0 || channels > FWN_ROWS_MAX_CHANNELS)
+    return fail(FWN_ERR_INVALID_ARG, "%s: %d channels (1 to %d)", what, channels, FWN_ROWS_MAX_CHANNELS);
+  if (dtype != FWN_F32 && dtype != FWN_BF16) return fail(FWN_ERR_UNSUPPORTED, "%s: dtype must be f32 or bf16", what);
+  if (!cond || !weight || !bias || !mul || !add) return fail(FWN_ERR_INVALID_ARG, "%s: null argument", what);
+  CondArgs a{};
+  for (int32_t l = 0; l < count; ++l) {
+    if (!weight[l] || !bias[l]) return fail(FWN_ERR_INVALID_ARG, "%s: null weight or bias of norm %d", what, l);
+    a.weight[l] = weight[l];
+    a.bias[l] = bias[l];
+  }
+  a.cond = cond;
+  a.mul = mul;
+  a.add = add;
+  a.count = count;
+  a.batch = batch;
+  a.channels = channels;
+  a.cond_size = cond_size;
+  return status(launch_cond(dtype, a, (hipStream_t)stream), what);
+}
+
 }  // extern "C"

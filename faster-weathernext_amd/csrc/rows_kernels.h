@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "fwn_rows.h"
+
 namespace fwn {
 
 struct RowArgs {
@@ -23,6 +25,17 @@ enum class RowPass { kGatherNorm, kNormScatter };
 
 // Launches one pass; dtype is FWN_F32 or FWN_BF16 and channels a validated multiple of 8.
 hipError_t launch_rows(RowPass pass, int dtype, const RowArgs& a, hipStream_t stream);
+
+struct CondArgs {
+  const void* weight[FWN_COND_MAX];  // [2 * channels, cond_size] of each norm
+  const void* bias[FWN_COND_MAX];    // [2 * channels]
+  const void* cond;                  // [batch, cond_size]
+  float* mul;                        // [count, batch, channels]
+  float* add;
+  int32_t count, batch, channels, cond_size;
+};
+
+hipError_t launch_cond(int dtype, const CondArgs& a, hipStream_t stream);
 
 struct RowBwdArgs {
   const void* x;

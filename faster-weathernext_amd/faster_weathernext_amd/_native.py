@@ -75,6 +75,7 @@ class RowsDesc(ctypes.Structure):
 
 
 ROWS_MAX_CHANNELS = 4096  # FWN_ROWS_MAX_CHANNELS
+COND_MAX = 64  # FWN_COND_MAX: norms of one fwn_cond_affine_launch
 ROWS_PERM_GRAD, ROWS_PERM_OUT = 1, 2  # FWN_ROWS_PERM_*: what the backward's perm permutes
 
 
@@ -121,6 +122,7 @@ SIGNATURES = {
     "fwn_rows_norm_scatter_launch": [_ROWS, _P, _P, _P, _P, _P, _P],
     "fwn_rows_norm_affine_launch": [_ROWS, _P, _P, _P, _P, _P],
     "fwn_rows_add_norm_affine_launch": [_ROWS, _P, _P, _P, _P, _P, _P, _P],
+    "fwn_cond_affine_launch": [_I32, _I32, _I32, _I32, _I32, _P, _P, _P, _P, _P, _P],
     "fwn_rows_norm_bwd_workspace_size": [_ROWS, _P],
     "fwn_rows_norm_bwd_launch": [_ROWS, _P, _P, _I32, _P, _P, _P, _P, _P, _P, _P, _U64, _P],
 }

@@ -275,6 +275,23 @@ def residual_norm(x, y, *, mul, add, eps=1e-5):
   return s, layer_norm_affine(s, mul=mul, add=add, eps=eps)
 
 
+def cond_affine(cond, weights, biases):
+  """[(mul, add)] of each norm, float32 [batch, channels]: 1 + scale and offset from its weight
+  [2 * channels, cond_size] and bias, as ``LinearNormConditioning`` projects them, in one HIP launch
+  for up to COND_MAX norms (no autograd). cond is [batch, cond_size] in the weights' dtype."""
+  batch, size = cond.shape
+  channels = weights[0].shape[0] // 2
+  out = torch.empty((2, len(weights), batch, channels), dtype=torch.float32, device=cond.device)
+  with torch.cuda.device(cond.device):
+    for lo in range(0, len(weights), nat.COND_MAX):
+      hi = min(lo + nat.COND_MAX, len(weights))
+      table = lambda ts: (ctypes.c_void_p * (hi - lo))(*(t.data_ptr() for t in ts[lo:hi]))
+      nat.check(nat.lib().fwn_cond_affine_launch(hi - lo, batch, channels, size, _DTYPES[cond.dtype], _addr(cond),
+                                                 table(weights), table(biases), _addr(out[0, lo]), _addr(out[1, lo]),
+                                                 _stream(cond)))
+  return list(zip(out[0].unbind(0), out[1].unbind(0)))
+
+
 def gather_layer_norm(x, perm, *, eps=1e-5):
   """x [batch, n, channels] -> (x[:, perm], layer_norm(x[:, perm])): the Hilbert gather before
   the layer loop (``patch.py:274-276``) and block 0's ``st.layernorm(x, create_scale=False,

@@ -37,7 +37,8 @@ from . import patch
 from .hip_attn import TileList
 from .mesh import hilbert_order, khop_mask, mesh_mask
 from .mha import TiledMHA, linear_rows, needs_grad
-from .rows import add_layer_norm_affine, gather_layer_norm, layer_norm_affine, layer_norm_scatter, residual_norm
+from .rows import (add_layer_norm_affine, cond_affine, gather_layer_norm, layer_norm_affine, layer_norm_scatter,
+                   residual_norm)
 
 
 class NormConditioning(torch.nn.Module):
@@ -58,20 +59,54 @@ class NormConditioning(torch.nn.Module):
     mul, add = self.affine(cond)
     return x * mul[:, None, :] + add[:, None, :]
 
+  def affine_f32(self, cond):
+    """affine(cond) as the norm passes take it: contiguous float32."""
+    mul, add = self.affine(cond)
+    return mul.float().contiguous(), add.float().contiguous()
+
   def norm(self, x, cond, eps):
     """forward(layer_norm(x), cond) as one HIP pass (statistics and affine in float32)."""
-    mul, add = self.affine(cond)
-    return layer_norm_affine(x, mul=mul.float().contiguous(), add=add.float().contiguous(), eps=eps)
+    mul, add = self.affine_f32(cond)
+    return layer_norm_affine(x, mul=mul, add=add, eps=eps)
 
   def residual_norm(self, x, y, cond, eps):
     """(x + y, norm(x + y)) with gradients, in one HIP pass where x and y allow it."""
-    mul, add = self.affine(cond)
-    return residual_norm(x, y, mul=mul.float().contiguous(), add=add.float().contiguous(), eps=eps)
+    mul, add = self.affine_f32(cond)
+    return residual_norm(x, y, mul=mul, add=add, eps=eps)
 
-  def add_norm(self, x, y, cond, eps):
-    """(x + y, forward(layer_norm(x + y), cond)) as one HIP pass, without autograd."""
-    mul, add = self.affine(cond)
-    return add_layer_norm_affine(x, y, mul=mul.float().contiguous(), add=add.float().contiguous(), eps=eps)
+  def add_norm(self, x, y, cond, eps, affine=None):
+    """(x + y, forward(layer_norm(x + y), cond)) as one HIP pass, without autograd; `affine` is
+    ``affine_f32(cond)`` where the caller has it."""
+    mul, add = affine or self.affine_f32(cond)
+    return add_layer_norm_affine(x, y, mul=mul, add=add, eps=eps)
+
+  def plain(self, cond):
+    """Whether ``affine`` is the linear map as built, on parameters the conditioning kernel reads: no
+    subclass, hook, parametrization or autocast that would see or change the call."""
+    lin = self.linear
+    return (type(self) is NormConditioning and type(lin) is torch.nn.Linear and not torch.is_autocast_enabled("cuda")
+            and not (lin._forward_hooks or lin._forward_pre_hooks) and cond.dim() == 2 and cond.is_cuda
+            and cond.dtype in (torch.float32, torch.bfloat16) and cond.is_contiguous() and cond.numel() > 0
+            and all(type(t) is torch.nn.Parameter and t.dtype == cond.dtype and t.device == cond.device and
+                    t.is_contiguous() for t in (lin.weight, lin.bias))
+            and lin.weight.shape[1] == cond.shape[1])
+
+
+# Batch members times conditioning features up to which one conditioning launch for all norms beats
+# their projections one by one. Its threads read a weight row each, so its time grows with the
+# product where a GEMM's hardly does; at 4,096 (8 x 512) it is ahead in every shape measured (5 to 49
+# norms of 256 to 2,048 channels: 46 to 329 us against 150 to 1,700), at 32,768 (64 x 512) behind in
+# most (309 to 2,360 against 150 to 1,690).
+COND_WORK = 1 << 12
+
+
+def affines_f32(norms, cond):
+  """``affine_f32(cond)`` of each norm, without autograd, in one launch; None for each where a norm is
+  not ``plain`` or the projections are large enough for a GEMM each."""
+  if (cond.numel() <= COND_WORK and all(norm.plain(cond) for norm in norms) and
+      len({norm.linear.weight.shape for norm in norms}) == 1):
+    return cond_affine(cond, [norm.linear.weight for norm in norms], [norm.linear.bias for norm in norms])
+  return [None] * len(norms)
 
 
 class MeshBlock(torch.nn.Module):
@@ -105,16 +140,16 @@ class MeshBlock(torch.nn.Module):
     x, h = self.norm_ffw.residual_norm(x, self.mha(h), cond, self.eps)
     return x + self.feed_forward(h)
 
-  def forward_fused(self, x, h, cond, next_norm=None):
+  def forward_fused(self, x, h, cond, next_norm=None, affines=(None, None)):
     """The block without autograd, from h = norm_mha(layernorm(x)) already computed: each residual
     add runs in one pass with the conditioned layer norm that reads it (``add_layer_norm_affine``),
-    the feed-forward's own and, when `next_norm` is given, the next block's. Returns (x, the next
-    block's h or None)."""
-    x, h = self.norm_ffw.add_norm(x, self.mha(h), cond, self.eps)
+    the feed-forward's own and, when `next_norm` is given, the next block's. `affines` are the two
+    norms' ``affine_f32(cond)`` where the caller has them. Returns (x, the next block's h or None)."""
+    x, h = self.norm_ffw.add_norm(x, self.mha(h), cond, self.eps, affines[0])
     f = self.feed_forward(h)
     if next_norm is None:
       return x + f, None
-    return next_norm.add_norm(x, f, cond, self.eps)
+    return next_norm.add_norm(x, f, cond, self.eps, affines[1])
 
 
 class MeshTransformer(torch.nn.Module):
@@ -167,20 +202,26 @@ class MeshTransformer(torch.nn.Module):
 
   def forward(self, x, cond):
     d = x.shape[-1]
-    normed = None
+    normed = final = None
     if self.perm is not None:
       x, normed = gather_layer_norm(x, self.perm, eps=self.eps)
     elif len(self.blocks):
       normed = F.layer_norm(x, (d,), eps=self.eps)
     if len(self.blocks) and not needs_grad(x, self):
-      # Without autograd the residual adds are fused into the conditioned layer norms after them.
+      # Without autograd the residual adds are fused into the conditioned layer norms after them, and
+      # every norm's conditioning is evaluated up front in one launch.
+      nexts = [block.norm_mha for block in self.blocks[1:]] + [None]
+      norms = [block.norm_ffw for block in self.blocks] + nexts[:-1] + [self.final_norm]
+      affines = affines_f32(norms, cond)
+      ffw, final = affines[:len(self.blocks)], affines[-1]
       h = self.blocks[0].norm_mha(normed, cond)
       for i, block in enumerate(self.blocks):
-        x, h = block.forward_fused(x, h, cond, self.blocks[i + 1].norm_mha if i + 1 < len(self.blocks) else None)
+        x, h = block.forward_fused(x, h, cond, nexts[i], (ffw[i], affines[len(self.blocks) + i]))
     else:
       for i, block in enumerate(self.blocks):
         x = block(x, cond, normed if i == 0 else None)
-    mul, add = self.final_norm.affine(cond)
     if self.perm is not None:
-      return layer_norm_scatter(x, self.perm, mul=mul.float().contiguous(), add=add.float().contiguous(), eps=self.eps)
+      mul, add = final or self.final_norm.affine_f32(cond)
+      return layer_norm_scatter(x, self.perm, mul=mul, add=add, eps=self.eps)
+    mul, add = self.final_norm.affine(cond)
     return F.layer_norm(x, (d,), eps=self.eps) * mul[:, None, :] + add[:, None, :]

@@ -73,6 +73,19 @@ int fwn_rows_add_norm_affine_launch(const fwn_rows_desc* d, const void* x, const
                                     const float* mul, const float* add, void* sum, void* out,
                                     void* stream);
 
+/* The conditioning of `count` (1 to FWN_COND_MAX) norms from one conditioning vector: for norm l, with
+ * weight[l] a contiguous [2 * channels, cond_size] matrix and bias[l] of 2 * channels entries, both
+ * in `dtype` as cond [batch, cond_size],
+ *   mul[l, b, c] = 1 + weight[l][c, :] . cond[b, :] + bias[l][c]
+ *   add[l, b, c] = weight[l][channels + c, :] . cond[b, :] + bias[l][channels + c]
+ * in float32, the affine the norm passes take (LinearNormConditioning's projections, which the
+ * reference evaluates norm by norm, patch.py:240-253, 288-292). mul and add are float32 [count,
+ * batch, channels]. weight and bias are host arrays of device pointers, read before returning. */
+#define FWN_COND_MAX 64
+int fwn_cond_affine_launch(int32_t count, int32_t batch, int32_t channels, int32_t cond_size, int32_t dtype,
+                           const void* cond, const void* const* weight, const void* const* bias, float* mul,
+                           float* add, void* stream);
+
 /* Backward of the passes above: for every row i of x (the rows a pass normalised, with xhat their
  * layer norm and rstd its 1 / sqrt(var + eps), recomputed from x),
  *
