@@ -23,8 +23,8 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 ARCH = "gfx950"
 
 DEVICE_SOURCES = ["attn_bf16.hip", "attn_x3.hip", "attn_x3_dkv.hip", "attn_f32.hip", "attn_combine.hip",
-                  "attn_noalloc.hip", "rows.hip"]
-HOST_SOURCES = ["attn_api.cpp", "mask_host.cpp", "node_order.cpp", "rows_api.cpp"]
+                  "attn_noalloc.hip", "rows.hip", "linear.hip"]
+HOST_SOURCES = ["attn_api.cpp", "mask_host.cpp", "node_order.cpp", "rows_api.cpp", "linear_api.cpp"]
 
 
 def _run(cmd):

@@ -122,6 +122,8 @@ SIGNATURES = {
     "fwn_rows_norm_scatter_launch": [_ROWS, _P, _P, _P, _P, _P, _P],
     "fwn_rows_norm_affine_launch": [_ROWS, _P, _P, _P, _P, _P],
     "fwn_rows_add_norm_affine_launch": [_ROWS, _P, _P, _P, _P, _P, _P, _P],
+    "fwn_linear_wgrad_workspace_size": [_I64, _I32, _I32, _P],
+    "fwn_linear_wgrad_launch": [_I64, _I32, _I32, _P, _P, _P, _P, _P, _U64, _P],
     "fwn_cond_affine_launch": [_I32, _I32, _I32, _I32, _I32, _P, _P, _P, _P, _P, _P],
     "fwn_rows_norm_bwd_workspace_size": [_ROWS, _P],
     "fwn_rows_norm_bwd_launch": [_ROWS, _P, _P, _I32, _P, _P, _P, _P, _P, _P, _P, _U64, _P],

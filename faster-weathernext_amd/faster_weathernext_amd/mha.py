@@ -14,8 +14,11 @@ input of the final projection. The parameters are plain torch Linear layers init
 torch; official WeatherNext checkpoints are Haiku parameters of the JAX model, which this
 package does not load.
 """
+import ctypes
+
 import torch
 
+from . import _native as nat
 from . import patch
 from .hip_attn import TileList, tiled_flash_attention, tiled_flash_attention_qkv
 
@@ -51,6 +54,87 @@ def needs_grad(x, module):
   return torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in module.parameters()))
 
 
+def linear_wgrad(g, x, bias):
+  """(g^T x, g's column sums or None) of contiguous bfloat16 g [M, N] and x [M, K], N and K multiples
+  of 64: the gradients of a Linear's weight and bias in two HIP launches (``fwn_linear_wgrad_launch``)."""
+  (m, outs), ins = g.shape, x.shape[1]
+  dw = torch.empty((outs, ins), dtype=g.dtype, device=g.device)
+  db = torch.empty(outs, dtype=g.dtype, device=g.device) if bias else None
+  size = ctypes.c_uint64()
+  nat.check(nat.lib().fwn_linear_wgrad_workspace_size(m, outs, ins, ctypes.byref(size)))
+  with torch.cuda.device(g.device):
+    work = torch.empty(size.value, dtype=torch.uint8, device=g.device)
+    nat.check(nat.lib().fwn_linear_wgrad_launch(m, outs, ins, g.data_ptr(), x.data_ptr(), dw.data_ptr(),
+                                                db.data_ptr() if bias else None, work.data_ptr(), size.value,
+                                                torch.cuda.current_stream(g.device).cuda_stream))
+  return dw, db
+
+
+class _Linear(torch.autograd.Function):
+  """F.linear with the faster row split, and with ``linear_wgrad`` for the weight's and bias's gradients."""
+
+  @staticmethod
+  def forward(ctx, x, weight, bias):
+    ctx.save_for_backward(x, weight)
+    ctx.has_bias = bias is not None
+    return linear_rows(x.reshape(-1, x.shape[-1]), weight, bias).view(*x.shape[:-1], weight.shape[0])
+
+  @staticmethod
+  def backward(ctx, grad):
+    x, weight = ctx.saved_tensors
+    need_x, need_w, need_b = ctx.needs_input_grad
+    need_b = need_b and ctx.has_bias
+    g, x2 = grad.reshape(-1, grad.shape[-1]), x.reshape(-1, x.shape[-1])
+    dx = dw = db = None
+    if torch.is_grad_enabled():  # create_graph: differentiable operations
+      return (torch.mm(g, weight).view(x.shape) if need_x else None, torch.mm(g.t(), x2) if need_w else None,
+              g.sum(0) if need_b else None)
+    if need_x:
+      dx = linear_rows(g, weight.t()).view(x.shape)
+    if need_w:
+      g, x2 = g.contiguous(), x2.contiguous()
+      if (g.data_ptr() | x2.data_ptr()) & 15:
+        dw, db = torch.mm(g.t(), x2), g.sum(0) if need_b else None
+      else:
+        dw, db = linear_wgrad(g, x2, need_b)
+    elif need_b:
+      db = g.sum(0)
+    return dx, dw, db
+
+
+# Rows from which a Linear's training pass runs as ``_Linear``. The two gradients at 8,192 rows, GEMM
+# and column sum against ``linear_wgrad``: 57 and 16 us (64 x 64), 67 and 24 (384 x 384), 77 and 39
+# (2,048 x 512); at 2,562 rows of 768 x 768 40 and 25, which the Function's host time takes back.
+WGRAD_ROWS = 8192
+# Largest weight whose gradient is ``linear_wgrad``: half of the 256 CUs' 256 x 256 tiles. Above it a
+# GEMM's own tiles fill the chip (20,484 rows: 4,096 x 1,024 299 and 175 us, 8,192 x 2,048 645 and
+# 594, for 64 MB of partials).
+WGRAD_ENTRIES = 128 * 256 * 256
+
+
+def is_plain(module, kind):
+  """Whether calling `module` is calling kind.forward: no subclass, hook, parametrization or wrapper."""
+  return (type(module) is kind and "forward" not in module.__dict__ and
+          not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or
+               module._backward_pre_hooks) and not torch.nn.modules.module._has_any_global_hook())
+
+
+def linear(lin, x):
+  """lin(x) with gradients: as ``_Linear`` where x and lin's parameters are plain bfloat16 tensors on one
+  GPU, sizes are whole 64s and there are rows enough; else the module as it is."""
+  if (x.dtype == torch.bfloat16 and x.is_cuda and x.numel() >= WGRAD_ROWS * x.shape[-1] > 0 and is_plain(lin, torch.nn.Linear)
+      and type(x) in (torch.Tensor, torch.nn.Parameter) and type(lin.weight) is torch.nn.Parameter and
+      lin.weight.dtype == x.dtype and lin.weight.device == x.device and lin.weight.is_contiguous() and
+      x.shape[-1] == lin.weight.shape[1] and
+      all(s % 64 == 0 and 0 < s <= 16384 for s in lin.weight.shape) and lin.weight.numel() <= WGRAD_ENTRIES and
+      (lin.bias is None or (type(lin.bias) is torch.nn.Parameter and lin.bias.dtype == x.dtype and
+                            lin.bias.device == x.device)) and
+      not torch.is_autocast_enabled("cuda") and not torch.compiler.is_compiling() and
+      not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0):
+    return _Linear.apply(x, lin.weight, lin.bias)
+  return lin(x)
+
+
 class TiledMHA(torch.nn.Module):
   """x [batch, n, d_model] -> x's attention update [batch, n, d_model].
 
@@ -74,10 +158,10 @@ class TiledMHA(torch.nn.Module):
     b, n, d = x.shape
     hd = self.num_heads * self.key_size
     if needs_grad(x, self):
-      qkv = self.qkv(x).view(b, n, 3, self.num_heads, self.key_size)
+      qkv = linear(self.qkv, x).view(b, n, 3, self.num_heads, self.key_size)
       out = tiled_flash_attention_qkv(qkv, self.tiles, scale=self.key_size ** -0.5, tiles_t=self.tiles_t,
                                       precision=self.precision)
-      return self.final(out.view(b, n, hd))
+      return linear(self.final, out.view(b, n, hd))
     # Without autograd the projections run through linear_rows (the faster GEMM row split).
     qkv = linear_rows(x.reshape(b * n, d), self.qkv.weight).view(b, n, 3, self.num_heads, self.key_size)
     out = tiled_flash_attention_qkv(qkv, self.tiles, scale=self.key_size ** -0.5, tiles_t=self.tiles_t,

@@ -23,8 +23,8 @@ and GELU run in the epilogue of its GEMM (``torch._addmm_activation``, which has
 so the [n, ffw_hidden] activations make one trip to HBM instead of three, every block GEMM
 splits its rows at a multiple of 512 (``mha.linear_rows``), and each residual add runs in one
 pass with the conditioned layer norm after it (``rows.add_layer_norm_affine``); with autograd the
-same functions run as plain Linear, GELU, Linear and adds, the attention's add fused with the
-feed-forward's conditioned norm (``rows.residual_norm``).
+same functions run as Linear (``mha.linear``), GELU, Linear and adds, the attention's add fused with
+the feed-forward's conditioned norm (``rows.residual_norm``).
 Parameters are random-initialised torch parameters; official checkpoints are Haiku parameters of
 the JAX model, which this package does not load.
 """
@@ -36,7 +36,7 @@ from scipy import sparse
 from . import patch
 from .hip_attn import TileList
 from .mesh import hilbert_order, khop_mask, mesh_mask
-from .mha import TiledMHA, linear_rows, needs_grad
+from .mha import TiledMHA, is_plain, linear, linear_rows, needs_grad
 from .rows import (add_layer_norm_affine, cond_affine, gather_layer_norm, layer_norm_affine, layer_norm_scatter,
                    residual_norm)
 
@@ -84,8 +84,8 @@ class NormConditioning(torch.nn.Module):
     """Whether ``affine`` is the linear map as built, on parameters the conditioning kernel reads: no
     subclass, hook, parametrization or autocast that would see or change the call."""
     lin = self.linear
-    return (type(self) is NormConditioning and type(lin) is torch.nn.Linear and not torch.is_autocast_enabled("cuda")
-            and not (lin._forward_hooks or lin._forward_pre_hooks) and cond.dim() == 2 and cond.is_cuda
+    return (type(self) is NormConditioning and not torch.is_autocast_enabled("cuda")
+            and is_plain(lin, torch.nn.Linear) and cond.dim() == 2 and cond.is_cuda
             and cond.dtype in (torch.float32, torch.bfloat16) and cond.is_contiguous() and cond.numel() > 0
             and all(type(t) is torch.nn.Parameter and t.dtype == cond.dtype and t.device == cond.device and
                     t.is_contiguous() for t in (lin.weight, lin.bias))
@@ -128,6 +128,8 @@ class MeshBlock(torch.nn.Module):
     both GEMMs use the faster row split (``linear_rows``)."""
     l1, l2 = self.ffw[0], self.ffw[2]
     if needs_grad(h, self.ffw):
+      if is_plain(self.ffw, torch.nn.Sequential) and len(self.ffw) == 3:
+        return linear(l2, self.ffw[1](linear(l1, h)))
       return self.ffw(h)
     lead = h.shape[:-1]
     y = linear_rows(h.reshape(-1, h.shape[-1]), l1.weight, l1.bias, gelu=True)

@@ -108,6 +108,19 @@ int fwn_rows_norm_bwd_launch(const fwn_rows_desc* d, const void* x, const int64_
                              const void* g_norm, const void* g_res, const float* mul, void* gx, float* g_mul,
                              float* g_add, void* workspace, uint64_t workspace_bytes, void* stream);
 
+/* dw[o, i] = sum over r of g[r, o] * x[r, i] and, where db is given, db[o] = sum over r of g[r, o]:
+ * the gradients of y = x w^T + b with respect to w and b, as the transformer block's projections and
+ * feed-forward take them (patch.py:165-177, 233-253). g is [rows, outs], x [rows, ins], dw [outs, ins],
+ * db [outs], all contiguous bfloat16, 16-byte aligned; sums are float32, rounded to bfloat16 once.
+ * outs and ins are positive multiples of FWN_LINEAR_UNIT, each at most FWN_LINEAR_MAX; rows >= 1.
+ * The workspace (fwn_linear_wgrad_workspace_size bytes, 16-byte aligned) holds float32 partial sums;
+ * its contents before the call do not matter. */
+#define FWN_LINEAR_UNIT 64
+#define FWN_LINEAR_MAX 16384
+int fwn_linear_wgrad_workspace_size(int64_t rows, int32_t outs, int32_t ins, uint64_t* bytes);
+int fwn_linear_wgrad_launch(int64_t rows, int32_t outs, int32_t ins, const void* g, const void* x, void* dw, void* db,
+                            void* workspace, uint64_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }  /* extern "C" */
 #endif

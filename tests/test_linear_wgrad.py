@@ -1,0 +1,98 @@
+"""A Linear's weight and bias gradients over many rows (``fwn_linear_wgrad_launch``) against float64 at
+the edges of its split (32-row stages, 256 x 256 tiles with ragged columns, one row range to many),
+and ``mha.linear`` against the module it stands for."""
+import ctypes
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from faster_weathernext_amd import _native as nat
+from faster_weathernext_amd import mha
+
+DEV = "cuda"
+
+
+def _framed(rows, cols, g):
+  """A [rows, cols] tensor inside NaNs: a read outside it shows."""
+  buf = torch.full(((rows + 8) * cols,), float("nan"), device=DEV, dtype=torch.bfloat16)
+  t = buf[4 * cols:(rows + 4) * cols].view(rows, cols)
+  t.copy_(torch.randn(rows, cols, device=DEV, generator=g))
+  return t
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,outs,ins", [(1, 64, 64), (31, 64, 256), (32, 256, 64), (33, 256, 256), (127, 192, 320),
+                                           (128, 320, 192), (129, 512, 256), (257, 768, 2304), (1000, 128, 384),
+                                           (4097, 256, 256), (70001, 64, 128), (9001, 1536, 384)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_wgrad_matches_float64(rows, outs, ins, bias):
+  gen = torch.Generator(device=DEV).manual_seed(rows + outs)
+  g, x = _framed(rows, outs, gen), _framed(rows, ins, gen)
+  dw, db = mha.linear_wgrad(g, x, bias)
+  # float32 sums of `rows` terms in some order, then one rounding to bf16 (8 significant bits: half
+  # an ulp is at most 2^-8 of the value).
+  want, terms = g.double().t() @ x.double(), g.double().abs().t() @ x.double().abs()
+  assert bool(((dw.double() - want).abs() <= 2.0 ** -8 * want.abs() + rows * 2.0 ** -23 * terms).all())
+  if bias:
+    want, terms = g.double().sum(0), g.double().abs().sum(0)
+    assert bool(((db.double() - want).abs() <= 2.0 ** -8 * want.abs() + rows * 2.0 ** -23 * terms).all())
+  else:
+    assert db is None
+
+
+def test_invalid_arguments_are_refused():
+  lib, size = nat.lib(), ctypes.c_uint64()
+  for bad in ((0, 64, 64), (5, 63, 64), (5, 64, 96), (5, 64, 0), (5, 1 << 15, 64)):
+    assert lib.fwn_linear_wgrad_workspace_size(*bad, ctypes.byref(size)) != 0
+    assert lib.fwn_linear_wgrad_launch(*bad, 16, 16, 16, 16, 16, 1 << 40, None) != 0
+  assert lib.fwn_linear_wgrad_workspace_size(40962, 768, 768, None) != 0
+  assert lib.fwn_linear_wgrad_workspace_size(40962, 768, 768, ctypes.byref(size)) == 0 and size.value > 0
+  for bad in ((None, 16, 16, 16, 16), (16, None, 16, 16, 16), (16, 16, None, 16, 16), (16, 16, 16, 16, None),
+              (24, 16, 16, 16, 16), (16, 24, 16, 16, 16), (16, 16, 24, 16, 16), (16, 16, 16, 24, 16), (16, 16, 16, 16, 24)):
+    assert lib.fwn_linear_wgrad_launch(40962, 768, 768, *bad, size.value, None) != 0
+  assert lib.fwn_linear_wgrad_launch(40962, 768, 768, 16, 16, 16, 16, 16, size.value - 1, None) != 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["plain", "no_bias", "3d", "strided", "frozen_weight", "frozen_input", "frozen_bias",
+                                  "odd_size", "hooked", "graph", "saved_hooks"])
+def test_linear_matches_the_module(monkeypatch, form):
+  monkeypatch.setattr(mha, "WGRAD_ROWS", 1)
+  torch.manual_seed(1)
+  lin = torch.nn.Linear(96 if form == "odd_size" else 128, 192, bias=form != "no_bias", device=DEV, dtype=torch.bfloat16)
+  x = torch.randn(2, 350, 96 if form == "odd_size" else 256, device=DEV).to(torch.bfloat16)
+  if form == "strided":
+    x = x[..., ::2]
+  elif form != "odd_size":
+    x = x[..., :128].contiguous()
+  x = x.requires_grad_(form != "frozen_input")
+  lin.weight.requires_grad_(form != "frozen_weight")
+  if lin.bias is not None:
+    lin.bias.requires_grad_(form != "frozen_bias")
+  if form == "hooked":
+    lin.register_forward_hook(lambda mod, args, out: out * 2)
+  g = torch.randn(2, 350, 192, device=DEV).to(torch.bfloat16)
+  leaves = [t for t in (x, *lin.parameters()) if t.requires_grad]
+  calls = []
+  monkeypatch.setattr(mha._Linear, "forward", staticmethod(lambda ctx, *a, f=mha._Linear.forward: calls.append(1) or f(ctx, *a)))
+
+  def run(f, graph):
+    packs = []
+    if form == "saved_hooks":
+      with torch.autograd.graph.saved_tensors_hooks(lambda t: packs.append(1) or t.cpu(), lambda t: t.to(DEV)):
+        out = f(x)
+      assert packs
+    else:
+      out = f(x)
+    return [out, *torch.autograd.grad(out, leaves, g, create_graph=graph)]
+
+  got, want = run(lambda t: mha.linear(lin, t), form == "graph"), run(lin, form == "graph")
+  assert len(calls) == (form not in ("odd_size", "hooked"))
+  if form == "graph":  # second derivatives through the first ones
+    second = lambda grads: torch.autograd.grad(sum((t.float() ** 2).sum() for t in grads[1:]), [x, lin.weight])
+    got, want = got + list(second(got)), want + list(second(want))
+  # Each side rounds float32 sums to bf16 (2^-9) at most twice along the way.
+  for a, b in zip(got, want):
+    assert a.shape == b.shape and a.dtype == b.dtype
+    assert float((a.double() - b.double()).norm() / b.double().norm()) <= 2.0 ** -7
