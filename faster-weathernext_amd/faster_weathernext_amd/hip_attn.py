@@ -267,7 +267,7 @@ class TileList:
     if products not in made:
       dmap = self.ds_map(tiles_t, DS_UNIT_KEYS[products])
       laid_out = dmap and self._layout and self._layout.exchange(tiles_t, products)
-      made[products] = _Exchange(*(laid_out or (self, tiles_t, dmap))) if dmap else None
+      made[products] = _Exchange(*(laid_out or (self, tiles_t, dmap)), kept=bool(laid_out)) if dmap else None
     return made[products]
 
   def forward_plan(self, q, o, scale, precision):
@@ -516,11 +516,25 @@ class DsMap:
 
 
 class _Exchange:
-  """The lists and map of one dS exchange (``TileList.exchange_lists``) and its calls' plans."""
+  """The lists and map of one dS exchange (``TileList.exchange_lists``) and its calls' plans.
 
-  def __init__(self, dq, kv, dmap):
-    self.dq, self.kv, self.dmap = dq, kv, dmap
+  Lists laid out for the exchange are its own (`kept`). The program's two lists are referred to
+  weakly: the exchange is kept by one of them for as long as the other lives, and must not keep
+  either alive."""
+
+  def __init__(self, dq, kv, dmap, kept):
+    self._lists = (dq, kv) if kept else (weakref.ref(dq), weakref.ref(kv))
+    self._kept = kept
+    self.dmap = dmap
     self._plans = {}
+
+  @property
+  def dq(self):
+    return self._lists[0] if self._kept else self._lists[0]()
+
+  @property
+  def kv(self):
+    return self._lists[1] if self._kept else self._lists[1]()
 
   def plan(self, q, o, scale, precision):
     """(descriptor, dQ's C struct, dK/dV's, workspace bytes, dS bytes) of a backward call."""

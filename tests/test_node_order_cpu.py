@@ -2,6 +2,9 @@
 numbering of packed pairs (``fwn_tiles_node_order``, ``fwn_tiles_permute_*``, ``fwn_tiles_compact_*``,
 ``fwn_tiles_unit_map``): the order is a permutation for any mask, the permuted list is the one built
 from the permuted mask, a packed list holds the mask's entries, and every dS unit has one number."""
+import gc
+import weakref
+
 import numpy as np
 import pytest
 from scipy import sparse
@@ -220,3 +223,21 @@ def test_launchers_check_the_node_table():
   big = nat.AttnDesc(1, n, 1, 32, nat.BF16, 1.0, 32 * n, 32, 32)
   assert status(0, None, big, n // 128) == nat.OK
   assert status(nat.TILES_NODES, F, big, n // 128) == nat.ERR_INVALID_ARG
+
+
+def test_an_exchange_keeps_no_list_alive():
+  """The exchange kept by a list refers to the program's lists weakly: a transposed list goes when the
+  program drops it, though the list it was used with lives on."""
+  mask = sparse.random(300, 300, 0.05, format="csr", random_state=np.random.RandomState(1)).astype(bool)
+  tl, tlt = (fwn.TileList.from_mask(m, device="cpu") for m in (mask, mask.T.tocsr()))
+  sym = fwn.TileList.from_mask((mask + mask.T).tocsr(), device="cpu")
+  for products in ("bf16", "f32", "bf16x3"):
+    assert tl.exchange_lists(tlt, products)[:2] == (tl, tlt)
+    assert sym.exchange_lists(sym, products)[:2] == (sym, sym)
+  refs = [weakref.ref(t) for t in (tl, tlt, sym)]
+  del tlt
+  gc.collect()
+  assert refs[1]() is None and not len(tl._exchanges)
+  del tl, sym
+  gc.collect()
+  assert refs[0]() is None and refs[2]() is None
