@@ -21,6 +21,7 @@ import torch
 from . import _native as nat
 from . import patch
 from .hip_attn import TileList, tiled_flash_attention, tiled_flash_attention_qkv
+from .rows import as_torch
 
 # hipBLASLt's bf16 GEMMs on MI355X run much faster when the row count is a multiple of 512: for
 # the block's four GEMMs at n = 40,962 nodes, 680 us per block against 519 us at 40,960 rows.
@@ -86,7 +87,7 @@ class _Linear(torch.autograd.Function):
     need_b = need_b and ctx.has_bias
     g, x2 = grad.reshape(-1, grad.shape[-1]), x.reshape(-1, x.shape[-1])
     dx = dw = db = None
-    if torch.is_grad_enabled():  # create_graph: differentiable operations
+    if as_torch(grad):
       return (torch.mm(g, weight).view(x.shape) if need_x else None, torch.mm(g.t(), x2) if need_w else None,
               g.sum(0) if need_b else None)
     if need_x:

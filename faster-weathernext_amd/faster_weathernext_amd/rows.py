@@ -21,7 +21,8 @@ evaluates: pass ``mul`` (its multiplier of the normalised features) and ``add``.
 The forward passes and their gradients run on the GPU only. Each gradient is one HIP pass as well
 (``fwn_rows_norm_bwd_launch``: the layer norm's analytic backward, with the permutation and the
 gradient that bypassed the norm in the same pass), plus a small reduction for mul and add. A
-backward that has to be differentiated again (create_graph) runs as torch operations instead.
+backward that has to be differentiated again (create_graph) or whose gradients are batched
+(is_grads_batched) runs as torch operations instead.
 """
 import ctypes
 
@@ -157,7 +158,15 @@ def _norm_backward_pass(x, eps, g_norm, g_res=None, mul=None, perm=None, perm_ro
   return gx, g_mul, g_add
 
 
-# The same gradients as torch operations, for backwards under create_graph.
+# The same gradients as torch operations, for backwards under create_graph or of batched gradients.
+
+
+def as_torch(*grads):
+  """Whether a backward with these gradients has to run as torch operations: it is differentiated
+  again (create_graph), or they are vmap's batched tensors (is_grads_batched), which have no memory."""
+  return torch.is_grad_enabled() or any(
+      g is not None and (torch._C._functorch.is_legacy_batchedtensor(g) or
+                         torch._C._functorch.is_functorch_wrapped_tensor(g)) for g in grads)
 
 
 def _norm_stats(x, eps):
@@ -201,7 +210,7 @@ class _GatherNorm(torch.autograd.Function):
   @staticmethod
   def backward(ctx, g_x, g_n):
     x_out, perm = ctx.saved_tensors
-    if not torch.is_grad_enabled():
+    if not as_torch(g_x, g_n):
       return _norm_backward_pass(x_out, ctx.eps, g_n, g_x, perm=perm, perm_rows=nat.ROWS_PERM_OUT)[0], None, None
     g = torch.zeros(x_out.shape, device=x_out.device, dtype=torch.float32)
     if g_x is not None:
@@ -228,7 +237,7 @@ class _NormScatter(torch.autograd.Function):
   def backward(ctx, g_out):
     x, perm, mul = ctx.saved_tensors
     need_mul, need_add = mul is not None and ctx.needs_input_grad[2], ctx.has_add and ctx.needs_input_grad[3]
-    if torch.is_grad_enabled():
+    if as_torch(g_out):
       g_y = g_out if perm is None else g_out[:, perm]  # gradient of the un-scattered rows
       g_x, g_mul, g_add = _affine_norm_backward(x, ctx.eps, g_y, mul, need_mul, need_add)
       return g_x.to(x.dtype), None, g_mul, g_add, None
@@ -256,7 +265,7 @@ class _AddNorm(torch.autograd.Function):
     if g_out is None:
       return g_s, g_s, None, None, None
     need_mul, need_add = ctx.needs_input_grad[2], ctx.needs_input_grad[3]
-    if torch.is_grad_enabled():
+    if as_torch(g_s, g_out):
       g, g_mul, g_add = _affine_norm_backward(s, ctx.eps, g_out, mul, need_mul, need_add)
       g = (g if g_s is None else g + g_s.float()).to(s.dtype)
     else:

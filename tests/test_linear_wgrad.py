@@ -56,7 +56,7 @@ def test_invalid_arguments_are_refused():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("form", ["plain", "no_bias", "3d", "strided", "frozen_weight", "frozen_input", "frozen_bias",
-                                  "odd_size", "hooked", "graph", "saved_hooks"])
+                                  "odd_size", "hooked", "graph", "saved_hooks", "batched"])
 def test_linear_matches_the_module(monkeypatch, form):
   monkeypatch.setattr(mha, "WGRAD_ROWS", 1)
   torch.manual_seed(1)
@@ -85,6 +85,8 @@ def test_linear_matches_the_module(monkeypatch, form):
       assert packs
     else:
       out = f(x)
+    if form == "batched":
+      return [out, *torch.autograd.grad(out, leaves, torch.stack([g, -g.flip(1)]), is_grads_batched=True)]
     return [out, *torch.autograd.grad(out, leaves, g, create_graph=graph)]
 
   got, want = run(lambda t: mha.linear(lin, t), form == "graph"), run(lin, form == "graph")

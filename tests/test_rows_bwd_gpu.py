@@ -1,7 +1,7 @@
 """Gradients of the row passes as one HIP pass (``fwn_rows_norm_bwd_launch``): against float64 torch at
 the sizes where the kernel's split changes (one vector per lane to sixteen, ragged channel counts,
 rows fewer than a workgroup's, several batch members), with each gradient missing or strided, and
-under create_graph, where the torch composite runs."""
+under create_graph or with batched gradients, where the torch composite runs."""
 import numpy as np
 import pytest
 import torch
@@ -122,6 +122,24 @@ def test_second_derivatives():
                  leaf(mul.double()), leaf(add.double()), g1.double())
   for a, r in zip(got, want):
     assert _rel(a, r) <= 1e-5
+
+
+def test_batched_gradients():
+  """is_grads_batched hands the backward vmap's batched tensors: each member's gradients as by itself."""
+  b, n, c = 2, 12, 24
+  x, g1, g2, y, mul, add, perm = _data(b, n, c, torch.float32, 7)
+  leaves = [t.clone().requires_grad_(True) for t in (x, mul, add)]
+  xa, ma, da = leaves
+  grads = torch.stack([g1, g2, y])
+  outs = {"scatter": (rows.layer_norm_scatter(xa, perm, mul=ma, add=da), leaves),
+          "affine": (rows.layer_norm_affine(xa, mul=ma, add=da), leaves),
+          "gather": (rows.gather_layer_norm(xa, perm)[1], [xa]),
+          "residual": (rows.residual_norm(xa, y, mul=ma, add=da)[1], leaves)}
+  for name, (out, wrt) in outs.items():
+    got = torch.autograd.grad(out, wrt, grads, is_grads_batched=True, retain_graph=True)
+    for i, g in enumerate(grads):
+      for a, r in zip(got, torch.autograd.grad(out, wrt, g, retain_graph=True)):
+        assert _rel(a[i], r) <= 1e-5, name
 
 
 def test_bad_arguments_are_refused():
