@@ -62,9 +62,23 @@ struct Vec<uint16_t> {  // bfloat16 bits
   }
 };
 
-// Output rows are written once and not read again by the pass: non-temporal stores stream them
-// past the caches (gather pass at [1, 40962, 768] float32: 74.5 -> 56.3 us, 6.7 TB/s).
-__device__ __forceinline__ void store16(void* p, const u32x4& v) { __builtin_nontemporal_store(v, (u32x4*)p); }
+// A row is read once by a pass: its loads are non-temporal, so that they do not push other rows out of
+// the caches. Outputs are what the program's next kernel reads: they are stored through the caches
+// while a tensor stays in the 256 MB memory-side cache, and non-temporally (`stream`) from
+// kStreamBytes up. Gather + scatter, float32, us, with plain loads and non-temporal stores / non-temporal
+// loads and plain stores / both non-temporal: forward and backward of [1, 40962, 768] (126 MB a tensor)
+// 362 / 337 / 350, [2, 40962, 768] (252 MB) 700 / 719 / 683, [4, 40962, 1280] 2872 / 2929 / 2827; forward of
+// [1, 40962, 768] 124 / 118 / 119. Below 64 MB all three are within 3%. A choice by pass only moves
+// the time to the next one.
+constexpr uint64_t kStreamBytes = 192ull << 20;
+
+__device__ __forceinline__ u32x4 load16(const void* p) { return __builtin_nontemporal_load((const u32x4*)p); }
+__device__ __forceinline__ void store16(void* p, const u32x4& v, bool stream) {
+  if (stream)
+    __builtin_nontemporal_store(v, (u32x4*)p);
+  else
+    *(u32x4*)p = v;
+}
 
 __device__ __forceinline__ float wave_sum(float x) {
 #pragma unroll
@@ -85,11 +99,11 @@ __device__ __forceinline__ void load_row(const T* row, bool ok, int nv, int chan
   for (int k = 0; k < VPL; ++k) {
     const int idx = lane + 64 * k;
     v[k] = u32x4{0u, 0u, 0u, 0u};
-    if (ok && idx < nv) v[k] = *(const u32x4*)(row + (size_t)idx * E);
+    if (ok && idx < nv) v[k] = load16(row + (size_t)idx * E);
     Vec<T>::unpack(v[k], f[k]);
     if (row2) {
       u32x4 w = u32x4{0u, 0u, 0u, 0u};
-      if (ok && idx < nv) w = *(const u32x4*)(row2 + (size_t)idx * E);
+      if (ok && idx < nv) w = load16(row2 + (size_t)idx * E);
       float g[E];
       Vec<T>::unpack(w, g);
 #pragma unroll
@@ -137,12 +151,12 @@ __global__ void __launch_bounds__(64 * kWaves) gather_norm_kernel(RowArgs a) {
   for (int k = 0; k < VPL; ++k) {
     const int idx = lane + 64 * k;
     if (idx >= nv) continue;
-    store16(xo + (size_t)idx * E, v[k]);
+    store16(xo + (size_t)idx * E, v[k], a.stream);
     if (no) {
       float y[E];
 #pragma unroll
       for (int e = 0; e < E; ++e) y[e] = (f[k][e] - mean) * rstd;
-      store16(no + (size_t)idx * E, Vec<T>::pack(y));
+      store16(no + (size_t)idx * E, Vec<T>::pack(y), a.stream);
     }
   }
 }
@@ -169,7 +183,7 @@ __global__ void __launch_bounds__(64 * kWaves) norm_scatter_kernel(RowArgs a) {
     T* so = (T*)a.x_out + (size_t)row * c;
 #pragma unroll
     for (int k = 0; k < VPL; ++k)
-      if (lane + 64 * k < nv) store16(so + (size_t)(lane + 64 * k) * E, v[k]);
+      if (lane + 64 * k < nv) store16(so + (size_t)(lane + 64 * k) * E, v[k], a.stream);
   }
   T* o = (T*)a.out + (size_t)(b * a.n + dst) * c;
   const float* mul = a.mul ? a.mul + (size_t)b * c : nullptr;
@@ -197,7 +211,7 @@ __global__ void __launch_bounds__(64 * kWaves) norm_scatter_kernel(RowArgs a) {
         for (int e = 0; e < 4; ++e) y[4 * q + e] += as_float(m[e]);
       }
     }
-    store16(o + (size_t)idx * E, Vec<T>::pack(y));
+    store16(o + (size_t)idx * E, Vec<T>::pack(y), a.stream);
   }
 }
 
@@ -233,8 +247,8 @@ hipError_t launch_t(RowPass pass, const RowArgs& a, hipStream_t stream) {
 // the forward is (3 or 4 tensors of traffic). The per-channel sums of the affine's gradients stay in
 // each lane's registers over all rows of its wave (a strided share of one batch member's rows), are
 // added over the workgroup's waves in LDS and go out as one partial row per workgroup, which
-// sums_kernel adds; both orders are fixed. At [1, 40962, 768] float32: with the sums 68 + 6 us (378 MB,
-// 5.6 TB/s), gather_norm's 104 us (504 MB, its scattered rows written whole; 4.8 TB/s); bf16 with sums
+// sums_kernel adds; both orders are fixed. At [1, 40962, 768] float32: with the sums 76 + 6 us (378 MB,
+// 5.0 TB/s), gather_norm's 81 us (504 MB, its scattered rows written whole; 6.2 TB/s); bf16 with sums
 // and the residual's gradient 58 + 6 us. The same gradients as torch operations took 15 to 25
 // launches: a gather, scatter and their gradients 1.64 -> 0.36 ms, a block's training pass by
 // 1.5 ms.
@@ -276,8 +290,8 @@ __global__ void __launch_bounds__(64 * kWaves) norm_bwd_kernel(RowBwdArgs a) {
     for (int k = 0; k < VPL; ++k) {
       const int idx = lane + 64 * k;
       gv[k] = rv[k] = u32x4{0u, 0u, 0u, 0u};
-      if (has && idx < nv) gv[k] = *(const u32x4*)(gn + (size_t)idx * E);
-      if (gr && idx < nv) rv[k] = *(const u32x4*)(gr + (size_t)idx * E);
+      if (has && idx < nv) gv[k] = load16(gn + (size_t)idx * E);
+      if (gr && idx < nv) rv[k] = load16(gr + (size_t)idx * E);
     }
     u32x4 v[VPL];
     float f[VPL][E];
@@ -322,7 +336,7 @@ __global__ void __launch_bounds__(64 * kWaves) norm_bwd_kernel(RowBwdArgs a) {
       Vec<T>::unpack(rv[k], r);
 #pragma unroll
       for (int e = 0; e < E; ++e) y[e] = fmaf(rstd, g[k][e] - m1 - f[k][e] * m2, r[e]);
-      store16(out + (size_t)idx * E, Vec<T>::pack(y));
+      store16(out + (size_t)idx * E, Vec<T>::pack(y), a.stream);
     }
   }
   if constexpr (SUMS) {
@@ -437,10 +451,17 @@ hipError_t launch_bwd_t(const RowBwdArgs& a, hipStream_t stream) {
   return hipErrorInvalidValue;
 }
 
+// Whether a pass streams its outputs past the caches (kStreamBytes).
+bool streams(int dtype, int64_t batch, int64_t n, int64_t channels) {
+  return (uint64_t)(batch * n) * (uint64_t)(channels * (dtype == FWN_F32 ? 4 : 2)) >= kStreamBytes;
+}
+
 }  // namespace
 
-hipError_t launch_rows(RowPass pass, int dtype, const RowArgs& a, hipStream_t stream) {
+hipError_t launch_rows(RowPass pass, int dtype, const RowArgs& args, hipStream_t stream) {
+  RowArgs a = args;
   if ((int64_t)a.batch * a.n == 0) return hipSuccess;
+  a.stream = streams(dtype, a.batch, a.n, a.channels);
   return dtype == FWN_F32 ? launch_t<float>(pass, a, stream) : launch_t<uint16_t>(pass, a, stream);
 }
 
@@ -462,7 +483,9 @@ hipError_t launch_cond(int dtype, const CondArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-hipError_t launch_rows_bwd(int dtype, const RowBwdArgs& a, hipStream_t stream) {
+hipError_t launch_rows_bwd(int dtype, const RowBwdArgs& args, hipStream_t stream) {
+  RowBwdArgs a = args;
+  a.stream = streams(dtype, a.batch, a.n, a.channels);
   return dtype == FWN_F32 ? launch_bwd_t<float>(a, stream) : launch_bwd_t<uint16_t>(a, stream);
 }
 

@@ -19,6 +19,7 @@ struct RowArgs {
   const void* addend;  // scatter: added to x before the norm (the sum goes to x_out, required then), or null
   int32_t batch, n, channels;
   float eps;
+  bool stream;  // set by launch_rows: outputs stored non-temporally
 };
 
 enum class RowPass { kGatherNorm, kNormScatter };
@@ -50,6 +51,7 @@ struct RowBwdArgs {
   float* g_add;
   int32_t batch, n, channels, blocks;  // blocks: workgroups per batch member
   float eps;
+  bool stream;  // set by launch_rows_bwd: gx stored non-temporally
 };
 
 // Workgroups per batch member of the backward pass.
