@@ -17,6 +17,8 @@ device memory and the stream. Tensors must be on a ROCm device: there is no CPU 
 """
 import collections
 import ctypes
+import heapq
+import math
 import threading
 import weakref
 
@@ -82,6 +84,22 @@ ORDER_TILE_UNITS = 20
 ORDER_HALF_UNITS = 1
 
 
+# dK/dV runs one workgroup per CU, so a call of few jobs leaves the chip idle in its last round: 1.27
+# rounds take as long as 2 (81 blocks x 4 heads at refinement 5). Below FILL_ROUNDS rounds, some blocks'
+# jobs are cut into up to FILL_PIECES runs of tiles (_PackedList._filled) where the simulated end, with
+# the combine pass (FILL_UNITS: its launch, and each slot's partial sums, in units of a job's cost by
+# products), is below FILL_GAIN of the whole jobs'. Below head_dim 128 more than one workgroup fits a CU,
+# so only calls of less than a round are. Backward on MI355X, us, whole -> filled: IEEE float32
+# refinement 5, 16 hops, 4 x 128 966 -> 868, 1 x 64 385 -> 197, refinement 4, 8 hops 4 x 128 191 -> 155, 2 x
+# 32 95 -> 62 (4 x 32 at refinement 5, over a round, 320 -> 329); split products 357 -> 352, 127 -> 97,
+# 95 -> 84, 55 -> 49. bf16 jobs are too short: 164 -> 164, 89 -> 93, 50.5 -> 51.1, head_dim 64 3 to 15%
+# slower.
+FILL_ROUNDS = 4
+FILL_PIECES = 6
+FILL_UNITS = {"f32": (10, 0.1), "bf16x3": (25, 0.3)}
+FILL_GAIN = 0.95
+
+
 # Keys per dS unit of the exchange, by products.
 DS_UNIT_KEYS = {"bf16": 16, "f32": 32, "bf16x3": 32}
 # Windows (tiles) within which dQ's packed list balances its waves' work per tile; 0: whole blocks.
@@ -109,19 +127,43 @@ def order_plan(desc, kernel):
   return ORDER_CUTS[kernel], ORDER_WINDOWS[products_of(desc)][kernel], ORDER_SLOTS[kernel]
 
 
+def _cut_items(tile_ptr, pieces):
+  """(items [n, 4], split [max(n_split, 1), 3], (n_items, n_parts, n_split)) of blocks cut into
+  `pieces` runs each, as fwn_tiles_schedule_fill lays them out."""
+  items, split, part = [], [], 0
+  for b, p in enumerate(int(p) for p in pieces):
+    t, count = int(tile_ptr[b]), int(tile_ptr[b + 1] - tile_ptr[b])
+    if p > 1:
+      split.append((b, part, p))
+    for c in range(p):
+      length = count // p + (c < count % p)
+      items.append((b, t, t + length, part if p > 1 else -1))
+      part += p > 1
+      t += length
+  return (np.array(items, np.int32), np.array(split or [(0, 0, 0)], np.int32), (len(items), part, len(split)))
+
+
+# What a list builds on first use (schedules, order tables, exchanges) is put in place with
+# setdefault: of two threads that build one, both use the first, since a call holds only addresses.
+
+
 class _Schedule:
   """One split-K schedule of a TileList: its work items, split records and C struct, plus the
   order tables built for it (``ordered_struct``)."""
 
-  def __init__(self, tl, tile_ptr, cap):
+  def __init__(self, tl, tile_ptr, cap, pieces=None):
+    """Items of at most `cap` tiles, or with `pieces` [n_blocks] each block's tiles in that many
+    near-equal runs."""
     L = nat.lib()
     counts = np.zeros(3, np.int32)
     nat.check(L.fwn_tiles_schedule_count(tl.n_blocks, nat.ptr(tile_ptr), int(cap), nat.ptr(counts[0:]),
                                          nat.ptr(counts[1:]), nat.ptr(counts[2:])))
-    self.n_items, self.n_parts, self.n_split = (int(c) for c in counts)
-    items = np.zeros((self.n_items, 4), np.int32)
-    split = np.zeros((max(self.n_split, 1), 3), np.int32)
+    items = np.zeros((int(counts[0]), 4), np.int32)
+    split = np.zeros((max(int(counts[2]), 1), 3), np.int32)
     nat.check(L.fwn_tiles_schedule_fill(tl.n_blocks, nat.ptr(tile_ptr), int(cap), nat.ptr(items), nat.ptr(split)))
+    if pieces is not None:
+      items, split, counts = _cut_items(tile_ptr, pieces)
+    self.n_items, self.n_parts, self.n_split = (int(c) for c in counts)
     self.items_host = items
     self.split_host = split[:self.n_split]
     self.items = torch.from_numpy(items).to(tl.device)
@@ -138,12 +180,30 @@ class _Schedule:
                      addr(self.items), addr(self.split) if self.n_split else None, addr(tl.halves), addr(work),
                      pairs, *tl._nodes())
 
+  def _tile_cost(self):
+    halves = np.unpackbits(self._tl.halves_host.astype("<u4").view(np.uint8).reshape(-1, 4), axis=1).sum(1)
+    return (ORDER_TILE_UNITS + ORDER_HALF_UNITS * halves).astype(np.int32)
+
+  def makespan(self, pairs, order, window, slots):
+    """Estimated end of a launch for `pairs` (batch, head) pairs with that order table: each XCD's jobs
+    in launch order, each to the first free of its `slots` workgroups."""
+    sums = np.concatenate([[0], np.cumsum(self._tile_cost())])
+    cost = (ORDER_ITEM_UNITS + sums[self.items_host[:, 2]] - sums[self.items_host[:, 1]]).tolist()
+    work = self.order_table(pairs, order, window, slots)
+    end = 0
+    for xcd in range(8):
+      free = [0] * slots
+      for pair, item in work[xcd::8].tolist():
+        if pair >= 0:
+          heapq.heapreplace(free, free[0] + cost[item])
+      end = max(end, max(free))
+    return end
+
   def order_table(self, pairs, order=nat.ORDER_BALANCED, window=0, slots=64):
     """Host order table [n_work, 2] of this schedule for calls of `pairs` (batch, head) pairs."""
     L = nat.lib()
     n = np.zeros(1, np.int32)
-    halves = np.unpackbits(self._tl.halves_host.astype("<u4").view(np.uint8).reshape(-1, 4), axis=1).sum(1)
-    cost = (ORDER_TILE_UNITS + ORDER_HALF_UNITS * halves).astype(np.int32)
+    cost = self._tile_cost()
     args = (self.n_items, nat.ptr(self.items_host), nat.ptr(cost) if len(cost) else None, ORDER_ITEM_UNITS,
             int(pairs), int(order), int(window), int(slots))
     nat.check(L.fwn_tiles_order_count(*args, nat.ptr(n)))
@@ -156,7 +216,7 @@ class _Schedule:
     key = (int(pairs), int(order), int(window), int(slots))
     if key not in self._orders:
       work = torch.from_numpy(self.order_table(pairs, order, window, slots)).to(self._tl.device)
-      self._orders[key] = (work, self._struct(work, int(pairs)))
+      self._orders.setdefault(key, (work, self._struct(work, int(pairs))))
     return self._orders[key][1]
 
 
@@ -263,11 +323,11 @@ class TileList:
     """The _Exchange with `tiles_t` for these products, or None (``exchange_lists``)."""
     made = self._exchanges.get(tiles_t)
     if made is None:
-      made = self._exchanges[tiles_t] = {}
+      made = self._exchanges.setdefault(tiles_t, {})
     if products not in made:
       dmap = self.ds_map(tiles_t, DS_UNIT_KEYS[products])
       laid_out = dmap and self._layout and self._layout.exchange(tiles_t, products)
-      made[products] = _Exchange(*(laid_out or (self, tiles_t, dmap)), kept=bool(laid_out)) if dmap else None
+      made.setdefault(products, _Exchange(*(laid_out or (self, tiles_t, dmap)), kept=bool(laid_out)) if dmap else None)
     return made[products]
 
   def forward_plan(self, q, o, scale, precision):
@@ -281,7 +341,7 @@ class TileList:
   def _schedule(self, cap):
     cap = int(cap) if cap > 0 else nat.ITEM_TILES
     if cap not in self._schedules:
-      self._schedules[cap] = _Schedule(self, self._tile_ptr, cap)
+      self._schedules.setdefault(cap, _Schedule(self, self._tile_ptr, cap))
     return self._schedules[cap]
 
   def item_cap_for(self, batch, heads, kernel="fwd"):
@@ -339,7 +399,7 @@ class TileList:
     # this list), so lists evicted from _as_tiles' cache take their maps with them.
     maps = self._ds_maps.setdefault(int(unit_keys), weakref.WeakKeyDictionary())
     if tiles_t not in maps:
-      maps[tiles_t] = DsMap.build(self, tiles_t, unit_keys)
+      maps.setdefault(tiles_t, DsMap.build(self, tiles_t, unit_keys))
     return maps[tiles_t]
 
   @classmethod
@@ -397,12 +457,47 @@ class _PackedList(TileList):
     self._row_node = row_node
     self._col_node = torch.from_numpy(node[self.cols]).to(device)
     self._layout = None
+    self._fills = {}
     # A tile's column block is its index within the block: the kernels read col_node instead.
     index = (np.arange(tiles) - np.repeat(ptr[:-1], np.diff(ptr))).astype(np.int32)
     self._build(ptr, index, bits, (len(ptr) - 1) * nat.BLOCK, device, max_item_tiles)
 
   def _nodes(self):
     return nat.TILES_NODES, self._row_node.data_ptr(), self._col_node.data_ptr()
+
+  def struct_for_desc(self, desc, kernel="fwd"):
+    filled = self._filled(desc) if kernel == "kv" and self._fixed_cap is None else None
+    if filled is None:
+      return super().struct_for_desc(desc, kernel)
+    return filled.ordered_struct(desc.batch * desc.heads, *order_plan(desc, "kv"))
+
+  def _filled(self, desc):
+    """The dK/dV schedule of a call of few rounds (FILL_ROUNDS) whose last round fills the chip: evenly
+    spaced blocks cut into runs of tiles. None where whole blocks are estimated to end as soon."""
+    whole = self.schedule_for(desc.batch, desc.heads, "kv")
+    products, pairs = products_of(desc), desc.batch * desc.heads
+    slots = 8 * ORDER_SLOTS["kv"]
+    rounds = whole.n_items * pairs / slots
+    if (products not in FILL_UNITS or whole.n_split or not 0 < rounds < FILL_ROUNDS or
+        (desc.head_dim < 128 and rounds >= 1)):
+      return None
+    key = products, pairs
+    if key not in self._fills:
+      rest = rounds - int(rounds)
+      # The rest of a round in p pieces a job: ceil(rest * p) pieces per slot, of 1 / p of a round each.
+      _, p = min((math.ceil(rest * p) / p, p) for p in range(1, FILL_PIECES + 1))
+      filled = None
+      if p > 1:
+        cut = np.diff(np.arange(self.n_blocks + 1) * rest / rounds // 1) > 0
+        pieces = np.where(cut, np.clip(np.diff(self._tile_ptr) // 2, 1, p), 1)
+        made = _Schedule(self, self._tile_ptr, 0, pieces)
+        launch, slot = FILL_UNITS[products]
+        plan = order_plan(desc, "kv")
+        if (made.makespan(pairs, *plan) + launch + slot * made.n_parts * pairs <
+            FILL_GAIN * whole.makespan(pairs, *plan)):
+          filled = made
+      self._fills.setdefault(key, filled)
+    return self._fills[key]
 
 
 class _Layout:
@@ -460,7 +555,7 @@ class _Layout:
                                                  tiles_t._tile_bits).permuted(self.perm)
       dq = self.packed(self.arrays, unit_keys, window=window)
       kv = self.packed(arrays_t, 32, nat.PARTS_PAIRS16)
-      pairs[products] = (dq, kv, DsMap.of_packed(dq, kv, unit_keys))
+      pairs.setdefault(products, (dq, kv, DsMap.of_packed(dq, kv, unit_keys)))
     return pairs[products]
 
 
