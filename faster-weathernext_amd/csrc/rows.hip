@@ -250,7 +250,7 @@ hipError_t launch_t(RowPass pass, const RowArgs& a, hipStream_t stream) {
 // sums_kernel adds; both orders are fixed. At [1, 40962, 768] float32: with the sums 76 + 6 us (378 MB,
 // 5.0 TB/s), gather_norm's 81 us (504 MB, its scattered rows written whole; 6.2 TB/s); bf16 with sums
 // and the residual's gradient 58 + 6 us. The same gradients as torch operations took 15 to 25
-// launches: a gather, scatter and their gradients 1.64 -> 0.36 ms, a block's training pass by
+// launches: a gather, scatter and their gradients 1.64 -> 0.33 ms, a block's training pass by
 // 1.5 ms.
 constexpr int kSumGroups = 16;  // partial rows added in parallel by sums_kernel's workgroup
 
