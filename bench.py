@@ -122,23 +122,25 @@ def parse():
 TRAFFIC_DIR = os.path.join(ROOT, "profiles")
 
 
-def measured_traffic(workload, kernel, precision="native"):
+def measured_traffic(workload, kernel, precision="native", walked_tiles=None):
   """HBM bytes per launch of `kernel` on `workload` from the committed PMC summary, if there is one.
 
   The summary (profiles/hbm_traffic_<kernel>_<workload>.txt, with a _bf16x3 suffix for the
   split-precision kernels) holds a line `traffic_bytes_per_launch <N>`: FETCH_SIZE + WRITE_SIZE per
-  dispatch, each scaled by what the same counter reads for a copy of known size.
+  dispatch, each scaled by what the same counter reads for a copy of known size. With `walked_tiles`, the
+  tiles of a list laid out for the kernel, it counts only if it was taken on that list (a line
+  `walked_tiles <N>`).
   """
   suffix = "" if precision == "native" else "_" + precision
   path = os.path.join(TRAFFIC_DIR, f"hbm_traffic_{kernel}_{workload}{suffix}.txt")
   if not os.path.exists(path):
     return None, None
   with open(path) as f:
-    for line in f:
-      parts = line.split()
-      if len(parts) == 2 and parts[0] == "traffic_bytes_per_launch":
-        return int(float(parts[1])), os.path.relpath(path, ROOT)
-  return None, None
+    found = dict(line.split() for line in f if len(line.split()) == 2)
+  if "traffic_bytes_per_launch" not in found or (walked_tiles is not None and
+                                                 found.get("walked_tiles") != str(walked_tiles)):
+    return None, None
+  return int(float(found["traffic_bytes_per_launch"])), os.path.relpath(path, ROOT)
 
 
 def copy_calibration(mib, steps, warmup):
@@ -690,7 +692,9 @@ def attention(args):
   peak = PEAK[cfg["dtype"]]
   if x3 and (dominant == "fwd" or dmap is not None):
     peak = round(PEAK["bf16"] / 3, 1)  # three bf16 MFMA products per counted fp32 product
-  traffic, traffic_src = measured_traffic(args.workload, dominant, args.precision)
+  dominant_list = walked_kv if "dkv" in dominant else walked_dq if "dq" in dominant else walked
+  traffic, traffic_src = measured_traffic(args.workload, dominant, args.precision,
+                                          None if walked is tiles else dominant_list.n_tiles)
   rate = lambda name, ms: round(algo[name] / (ms * 1e-3) / 1e12, 3)
 
   result = {
