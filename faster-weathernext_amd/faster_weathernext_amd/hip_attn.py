@@ -220,13 +220,33 @@ class _Schedule:
     return self._orders[key][1]
 
 
-# Lists laid out for the kernels (TileList.launch_list): taken when both the number of tiles and
-# their estimated cost (ORDER_TILE_UNITS per tile + ORDER_HALF_UNITS per live 32 x 16 half) are at
-# most LAID_OUT_GAIN of the given list's. On the refinement-6 mesh the forward's cost is 0.20 (8
-# hops) and 0.33 (16 hops) of mesh order's list, 0.73 of Hilbert order's (32 hops), its tiles 0.14,
-# 0.25 and 0.64. A mask without locality (random entries) has as many tiles in any order; it keeps
-# the given list, and with it that list's results bit for bit.
+# Lists laid out for the kernels: taken when both the number of tiles and their estimated cost
+# (ORDER_TILE_UNITS per tile + ORDER_HALF_UNITS per live 32 x 16 half) are at most LAID_OUT_GAIN of the
+# given list's. On the refinement-6 mesh the forward's cost is 0.20 (8 hops) and 0.33 (16 hops) of mesh
+# order's list, 0.73 of Hilbert order's (32 hops), its tiles 0.14, 0.25 and 0.64. A mask without
+# locality (random entries) has as many tiles in any order; it keeps the given list, and with it that
+# list's results bit for bit.
 LAID_OUT_GAIN = 0.95
+
+
+def _exchange_gain(products):
+  """The most tiles, cost and dS units the lists laid out for the exchange may have, of the given pair's.
+
+  They pack whole groups and not single columns, so they are judged apart from the forward's: a few
+  rows that reach everywhere leave the forward's list 0.79 of the cost and these 2.1 times of it, with
+  3.8 times the units (8-hop refinement-6 mesh with 20 such rows). Backward of 4 heads x 128 on MI355X, us,
+  given -> packed pair:
+    cost 1.80 to 2.1, units 3.1 to 3.8: that mesh, bf16 1153 -> 2771, float32 8118 -> 16684, split products
+      2883 -> 7395; refinement 5, 4 hops with 12 such rows 252 -> 337, 1980 -> 2261, 716 -> 851
+    cost and units 0.98 to 1.0: random 2% of 2,562 nodes, bf16 116 -> 138, float32 580 -> 438, split 228 ->
+      174; with 64 heads 722 -> 758, 4691 -> 4792, 1687 -> 1737
+    cost 0.91 and units 0.86 to 0.93: random 0.5% of 2,562 nodes, bf16 112 -> 122, float32 574 -> 389, split
+      225 -> 167; with 64 heads 690 -> 649, 4197 -> 3853, 1681 -> 1604
+    cost 0.82, units 0.90: 32-hop refinement-6 mesh, Hilbert order, 1331 -> 1203, 8667 -> 7477, 3396 -> 3044.
+  In bf16 gathering and the table of unit numbers cost a pair of equal work 3 to 18%. In float32 they
+  cost at most 3%, and calls of few rounds, which only the packed lists fill (FILL_ROUNDS), gain up to
+  44%."""
+  return LAID_OUT_GAIN if products == "bf16" else max(LAID_OUT_GAIN, 1.0)
 
 
 class TileList:
@@ -303,8 +323,7 @@ class TileList:
   @property
   def cost(self):
     """Estimated cost of the list's tiles for one (batch, head) pair (ORDER_* units)."""
-    halves = int(np.unpackbits(self.halves_host.view(np.uint8)).sum())
-    return ORDER_TILE_UNITS * self.n_tiles + ORDER_HALF_UNITS * halves
+    return _cost(self.n_tiles, int(np.unpackbits(self.halves_host.view(np.uint8)).sum()))
 
   def launch_list(self):
     """The list the forward (and each recomputing backward kernel) walks for this mask: the one laid
@@ -315,7 +334,8 @@ class TileList:
     """(list for dQ, list for dK/dV, dS map) of the dS exchange with `tiles_t`, the transposed
     mask's list (this list itself for a symmetric mask), for kernels with these products (see
     ``products_of``), or None when it is not the exact transpose (the recomputing backward
-    applies then). Built on first use and kept."""
+    applies then). The lists are those laid out for the exchange where they pay (_exchange_gain), else
+    the given two. Built on first use and kept."""
     exchange = self._exchange(tiles_t, products)
     return None if exchange is None else (exchange.dq, exchange.kv, exchange.dmap)
 
@@ -326,7 +346,7 @@ class TileList:
       made = self._exchanges.setdefault(tiles_t, {})
     if products not in made:
       dmap = self.ds_map(tiles_t, DS_UNIT_KEYS[products])
-      laid_out = dmap and self._layout and self._layout.exchange(tiles_t, products)
+      laid_out = dmap and self._layout and self._layout.exchange(self, tiles_t, products, dmap)
       made.setdefault(products, _Exchange(*(laid_out or (self, tiles_t, dmap)), kept=bool(laid_out)) if dmap else None)
     return made[products]
 
@@ -440,27 +460,45 @@ class _Arrays:
     return _Arrays(self.n, ptr, col, bits)
 
 
-class _PackedList(TileList):
-  """The list of `arrays` with each block's live column groups of `group` columns packed
-  (``fwn_tiles_compact_*``). ``cols`` holds the column of each tile column; ``node[c]`` is the node of
-  row or column c (n past the last)."""
+def _cost(tiles, halves):
+  return ORDER_TILE_UNITS * tiles + ORDER_HALF_UNITS * halves
 
-  def __init__(self, arrays, group, parts, window, node, row_node, device, max_item_tiles):
+
+class _Packed:
+  """`arrays` with each block's live column groups of `group` columns packed (``fwn_tiles_compact_*``),
+  on the host: tile pointers, the column of each tile column, the bits, and the estimated cost."""
+
+  def __init__(self, arrays, group, parts=nat.PARTS_ROWS32, window=0):
     L = nat.lib()
-    self.n = arrays.n
-    ptr = np.zeros_like(arrays.ptr)
-    nat.check(L.fwn_tiles_compact_count(*arrays.args, group, nat.ptr(ptr)))
-    tiles = int(ptr[-1])
-    self.cols = np.empty((tiles, nat.BLOCK), np.int32)
-    bits = np.empty((tiles, nat.BLOCK, nat.BLOCK // 32), np.uint32)
-    nat.check(L.fwn_tiles_compact_fill(*arrays.args, group, parts, window, nat.ptr(ptr), nat.ptr(self.cols), nat.ptr(bits)))
+    self.ptr = np.zeros_like(arrays.ptr)
+    nat.check(L.fwn_tiles_compact_count(*arrays.args, group, nat.ptr(self.ptr)))
+    self.n_tiles = int(self.ptr[-1])
+    self.cols = np.empty((self.n_tiles, nat.BLOCK), np.int32)
+    self.bits = np.empty((self.n_tiles, nat.BLOCK, nat.BLOCK // 32), np.uint32)
+    nat.check(L.fwn_tiles_compact_fill(*arrays.args, group, parts, window, nat.ptr(self.ptr), nat.ptr(self.cols),
+                                       nat.ptr(self.bits)))
+    words = np.bitwise_or.reduce(self.bits.reshape(self.n_tiles, nat.BLOCK // 32, 32, nat.BLOCK // 32), axis=2)
+    self.cost = _cost(self.n_tiles, int(np.count_nonzero(words & 0xffff) + np.count_nonzero(words >> 16)))
+
+  def pays(self, tl, gain):
+    """Whether this list has at most `gain` of TileList `tl`'s tiles and of their cost."""
+    return self.n_tiles <= gain * tl.n_tiles and self.cost <= gain * tl.cost
+
+
+class _PackedList(TileList):
+  """The list of a _Packed of `n` nodes. ``cols`` holds the column of each tile column; ``node[c]`` is the
+  node of row or column c (n past the last)."""
+
+  def __init__(self, packed, n, node, row_node, device, max_item_tiles):
+    self.n, self.cols = n, packed.cols
+    ptr, tiles = packed.ptr, packed.n_tiles
     self._row_node = row_node
     self._col_node = torch.from_numpy(node[self.cols]).to(device)
     self._layout = None
     self._fills = {}
     # A tile's column block is its index within the block: the kernels read col_node instead.
     index = (np.arange(tiles) - np.repeat(ptr[:-1], np.diff(ptr))).astype(np.int32)
-    self._build(ptr, index, bits, (len(ptr) - 1) * nat.BLOCK, device, max_item_tiles)
+    self._build(ptr, index, packed.bits, (len(ptr) - 1) * nat.BLOCK, device, max_item_tiles)
 
   def _nodes(self):
     return nat.TILES_NODES, self._row_node.data_ptr(), self._col_node.data_ptr()
@@ -507,17 +545,20 @@ class _Layout:
   column of a tile is used. The dS exchange hands 32-query x 16-key (bf16) or x 32-key units from
   dK/dV to dQ, so its lists pack whole groups: dQ's by `unit_keys` keys, dK/dV's by 32 queries."""
 
-  def __init__(self, arrays, perm, device, cap):
+  def __init__(self, arrays, perm, device, cap, packed):
     self.arrays, self.perm, self._device, self._cap = arrays, perm, device, cap
     n = arrays.n
     self._node = np.concatenate([perm.astype(np.int32), np.full(nat.BLOCK, n, np.int32)])
     rows = (len(arrays.ptr) - 1) * nat.BLOCK
     self._row_node = torch.from_numpy(self._node[np.minimum(np.arange(rows), n)]).to(device)
     self._pairs = weakref.WeakKeyDictionary()
-    self.forward = self.packed(arrays, 1)
+    self.forward = self._list(packed)
+
+  def _list(self, packed):
+    return _PackedList(packed, self.arrays.n, self._node, self._row_node, self._device, self._cap)
 
   def packed(self, arrays, group, parts=nat.PARTS_ROWS32, window=0):
-    return _PackedList(arrays, group, parts, window, self._node, self._row_node, self._device, self._cap)
+    return self._list(_Packed(arrays, group, parts, window))
 
   @classmethod
   def choose(cls, tl):
@@ -529,33 +570,34 @@ class _Layout:
     given = _Arrays(n, tl._tile_ptr, tl._tile_col, tl._tile_bits)
     perm = np.empty(n, np.int64)
     nat.check(nat.lib().fwn_tiles_node_order(*given.args, nat.ptr(perm)))
-    # The packed list of the mask in its own order or, if that is no better, in the given one.
-    best = None
-    for p in (perm, np.arange(n, dtype=np.int64)):
-      arrays = given if best else given.permuted(p)
-      layout = cls(arrays, p, tl.device, tl._fixed_cap)
-      if best is None or layout.forward.cost < best.forward.cost:
-        best = layout
-      if best._pays(tl):
-        return best
-    return None
+    # The packed list of the mask in its own order or, if that does not pay and costs more, in the given one.
+    arrays = given.permuted(perm)
+    packed = _Packed(arrays, 1)
+    if not packed.pays(tl, LAID_OUT_GAIN):
+      cost, arrays, perm = packed.cost, given, np.arange(n, dtype=np.int64)
+      packed = _Packed(arrays, 1)
+      if packed.cost >= cost or not packed.pays(tl, LAID_OUT_GAIN):
+        return None
+    return cls(arrays, perm, tl.device, tl._fixed_cap, packed)
 
-  def _pays(self, tl):
-    return (self.forward.n_tiles <= LAID_OUT_GAIN * tl.n_tiles and
-            self.forward.cost <= LAID_OUT_GAIN * tl.cost)
-
-  def exchange(self, tiles_t, products):
-    """(list for dQ, list for dK/dV, map) in this layout for kernels with these products; `tiles_t`
-    is the exact transpose."""
+  def exchange(self, tl, tiles_t, products, given):
+    """(list for dQ, list for dK/dV, map) in this layout for kernels with these products, or None where
+    `tl`, whose layout this is, `tiles_t`, its exact transpose, and their map `given` are as good
+    (_exchange_gain)."""
     pairs = self._pairs.setdefault(tiles_t, {})
     unit_keys, window = DS_UNIT_KEYS[products], DQ_WINDOW[products]
     if products not in pairs:
       own = tiles_t._layout is self
       arrays_t = self.arrays if own else _Arrays(self.arrays.n, tiles_t._tile_ptr, tiles_t._tile_col,
                                                  tiles_t._tile_bits).permuted(self.perm)
-      dq = self.packed(self.arrays, unit_keys, window=window)
-      kv = self.packed(arrays_t, 32, nat.PARTS_PAIRS16)
-      pairs.setdefault(products, (dq, kv, DsMap.of_packed(dq, kv, unit_keys)))
+      dq = _Packed(self.arrays, unit_keys, window=window)
+      kv = _Packed(arrays_t, 32, nat.PARTS_PAIRS16)
+      made, gain = None, _exchange_gain(products)
+      if dq.pays(tl, gain) and kv.pays(tiles_t, gain):
+        dq, kv = self._list(dq), self._list(kv)
+        dmap = DsMap.of_packed(dq, kv, unit_keys)
+        made = (dq, kv, dmap) if dmap.n_units <= gain * given.n_units else None
+      pairs.setdefault(products, made)
     return pairs[products]
 
 

@@ -11,6 +11,7 @@ from scipy import sparse
 
 import faster_weathernext_amd as fwn
 from faster_weathernext_amd import _native as nat
+from faster_weathernext_amd import hip_attn
 
 
 def _arrays(mask, perm=None):
@@ -241,3 +242,42 @@ def test_an_exchange_keeps_no_list_alive():
   del tl, sym
   gc.collect()
   assert refs[0]() is None and refs[2]() is None
+
+
+@pytest.mark.parametrize("name", ["mesh", "hilbert", "global rows", "directed global rows", "random", "coarse"])
+def test_exchange_lists_are_no_costlier_than_the_given_ones(name):
+  """The lists of the dS exchange are judged by themselves: where a few rows and columns that reach
+  everywhere spoil the order, or the mask has no locality, the forward's list pays and the given two are
+  walked in the backward; in any case neither their tiles, nor their cost, nor the dS buffer grow."""
+  coarse, wide = name == "coarse", "global" in name
+  mask, _, _, perm = fwn.mesh_mask(2 if coarse else 4, 2 if coarse else 4, reorder=name not in ("mesh", "random"))
+  n = mask.shape[0]
+  if wide:
+    mask = mask.tolil()
+    for r in np.random.default_rng(0).choice(n, 6, replace=False):
+      mask[r, :] = True
+      mask[:, r] = True
+    if name != "global rows":
+      mask[5, 2000] = True
+      mask[2000, 5] = False
+    mask = mask.tocsr()
+  elif name == "random":
+    mask = (sparse.random(n, n, 0.01, random_state=1) + sparse.identity(n)).astype(bool).tocsr()
+    mask = (mask + mask.T).tocsr()
+  tl = fwn.TileList.from_mask(mask, perm, device="cpu")
+  tlt = fwn.TileList.from_mask(mask.T.tocsr(), perm, device="cpu") if "directed" in name else tl
+  tl._layout = hip_attn._Layout.choose(tl)  # as a list on the GPU has it
+  assert tl._layout is not None
+  kept = {}
+  for products, unit_keys in hip_attn.DS_UNIT_KEYS.items():
+    dq, kv, dmap = tl.exchange_lists(tlt, products)
+    given = tl.ds_map(tlt, unit_keys)
+    kept[products] = (dq, kv, dmap) == (tl, tlt, given)
+    assert kept[products] or (dq is not tl and kv is not tlt and dmap is not given)
+    gain = 0.95 if products == "bf16" else 1.0
+    for laid_out, own in ((dq.n_tiles, tl.n_tiles), (dq.cost, tl.cost), (kv.n_tiles, tlt.n_tiles), (kv.cost, tlt.cost),
+                          (dmap.n_units, given.n_units)):
+      assert laid_out == own if kept[products] else laid_out <= gain * own
+    assert dmap.struct.table == dq.struct.flags == kv.struct.flags == (0 if kept[products] else 1)
+  assert kept["bf16"] == (name not in ("mesh", "hilbert"))
+  assert kept["f32"] == kept["bf16x3"] == wide
