@@ -34,6 +34,11 @@ constexpr int kSmooth = 3;      // neighbourhood averages of the distances
 constexpr int kDims = 8;        // coordinates per node (kLandmarks, padded for the vector units)
 constexpr int32_t kLeaf = 16;   // nodes of a bisection leaf: the finest width the kernels skip
 constexpr int kAxisSamples = 512;
+constexpr int64_t kSerialVisits = 1 << 14;
+// Rows looked at over all searches of a list: meshes take 2 to 17 per row of a tile. A list that takes
+// more than these (a path of 10^5 nodes, a shuffled band) is left in its own order: 40,962 nodes in a
+// row take 0.7 s, the searches stop after about 2 s (5 s for lists of 10^5 tiles).
+constexpr int64_t kVisitsPerRow = 24, kVisits = INT64_C(1) << 25;
 
 struct List {
   int32_t n, n_blocks;
@@ -42,46 +47,101 @@ struct List {
   const uint32_t* bits;
 };
 
-// Breadth-first distances from `src`: a node is one step further than the nearest node its row
-// of the mask holds. Nodes not reached get the largest distance plus one. Each level reads the
-// tiles whose column block has a node of the last level, for rows not reached yet.
-void distances(const List& m, int32_t src, std::vector<int32_t>& dist) {
-  std::vector<uint32_t> front((size_t)m.n_blocks * kWords, 0u), next(front.size(), 0u);
-  std::vector<uint8_t> any(m.n_blocks, 0), next_any(m.n_blocks, 0);
-  dist.assign(m.n, -1);
-  dist[src] = 0;
-  front[src / 32] |= 1u << (src % 32);
-  any[src / FWN_BLOCK] = 1;
-  int32_t level = 0;
-  for (bool more = true; more;) {
-    ++level;
-    std::atomic<bool> found(false);
-    parallel_for(m.n_blocks, 16, [&](int64_t b, int64_t e) {
-      for (int64_t blk = b; blk < e; ++blk) {
-        uint32_t* out = &next[blk * kWords];
-        std::memset(out, 0, kWords * sizeof(uint32_t));
-        next_any[blk] = 0;
-        const int32_t r0 = (int32_t)blk * FWN_BLOCK, rows = std::min(FWN_BLOCK, m.n - r0);
-        for (int32_t t = m.ptr[blk]; t < m.ptr[blk + 1]; ++t) {
-          if (!any[m.col[t]]) continue;
-          const uint32_t* f = &front[(int64_t)m.col[t] * kWords];
-          const uint32_t* w = m.bits + t * kTileWords;
-          for (int32_t r = 0; r < rows; ++r, w += kWords) {
-            if (!((w[0] & f[0]) | (w[1] & f[1]) | (w[2] & f[2]) | (w[3] & f[3])) || dist[r0 + r] >= 0) continue;
-            dist[r0 + r] = level;
-            out[r / 32] |= 1u << (r % 32);
-            next_any[blk] = 1;
-          }
-        }
-        if (next_any[blk]) found = true;
+// The list's tiles by column block, and the rows of each tile that hold an entry.
+struct Columns {
+  std::vector<int32_t> ptr, tile;  // tiles of column block kb: tile[ptr[kb]] .. tile[ptr[kb + 1]]
+  std::vector<int32_t> blk;        // row block of each tile
+  std::vector<uint32_t> rows;      // [n_tiles][kWords], rows past the last node clear
+
+  explicit Columns(const List& m) : ptr(m.n_blocks + 1, 0), tile(m.ptr[m.n_blocks]), blk(tile.size()), rows(tile.size() * kWords) {
+    for (size_t t = 0; t < tile.size(); ++t) ++ptr[m.col[t] + 1];
+    for (int32_t k = 0; k < m.n_blocks; ++k) ptr[k + 1] += ptr[k];
+    std::vector<int32_t> at(ptr.begin(), ptr.end() - 1);
+    for (int32_t b = 0; b < m.n_blocks; ++b)
+      for (int32_t t = m.ptr[b]; t < m.ptr[b + 1]; ++t) {
+        tile[at[m.col[t]]++] = t;
+        blk[t] = b;
+      }
+    parallel_for((int64_t)tile.size(), 256, [&](int64_t begin, int64_t end) {
+      for (int64_t t = begin; t < end; ++t) {
+        const uint32_t* w = m.bits + t * kTileWords;
+        const int32_t last = std::min(FWN_BLOCK, m.n - blk[t] * FWN_BLOCK);
+        for (int32_t r = 0; r < last; ++r, w += kWords)
+          if (w[0] | w[1] | w[2] | w[3]) rows[t * kWords + r / 32] |= 1u << (r % 32);
       }
     });
-    front.swap(next);
-    any.swap(next_any);
-    more = found;
+  }
+};
+
+// Breadth-first distances from `src`: a node is one step further than the nearest node its row
+// of the mask holds. Nodes not reached get the largest distance plus one. Each level reads the
+// tiles whose column block has a node of the last level, and of those the rows with an entry that
+// are not reached yet: its cost follows the front, not the list, as a mask of long paths has
+// thousands of levels. `visits` counts the rows and tiles looked at; false when it passes `most`.
+bool distances(const List& m, const Columns& cols, int32_t src, int64_t most, int64_t& visits, std::vector<int32_t>& dist) {
+  struct Rows {
+    uint32_t w[kWords] = {};
+    bool any() const { return w[0] | w[1] | w[2] | w[3]; }
+    void set(int32_t r) { w[r / 32] |= 1u << (r % 32); }
+  };
+  std::vector<Rows> front(m.n_blocks), next(m.n_blocks), left(m.n_blocks);  // left: rows not reached
+  std::vector<std::vector<int32_t>> todo(m.n_blocks);                       // tiles of a level by row block
+  std::vector<int32_t> active{src / FWN_BLOCK}, blocks;
+  for (int32_t i = 0; i < m.n; ++i) left[i / FWN_BLOCK].set(i % FWN_BLOCK);
+  dist.assign(m.n, -1);
+  dist[src] = 0;
+  front[active[0]].set(src % FWN_BLOCK);
+  left[active[0]].w[src % FWN_BLOCK / 32] &= ~(1u << (src % 32));
+  int32_t level = 0;
+  while (!active.empty()) {
+    ++level;
+    int64_t count = 0;
+    blocks.clear();
+    for (int32_t kb : active)
+      for (int32_t k = cols.ptr[kb]; k < cols.ptr[kb + 1]; ++k) {
+        const int32_t t = cols.tile[k], blk = cols.blk[t];
+        int32_t rows = 0;
+        for (int32_t q = 0; q < kWords; ++q) rows += __builtin_popcount(cols.rows[(int64_t)t * kWords + q] & left[blk].w[q]);
+        count += 1 + rows;
+        if (!rows) continue;
+        if (todo[blk].empty()) blocks.push_back(blk);
+        todo[blk].push_back(t);
+      }
+    visits += count;
+    if (visits > most) return false;
+    // Small levels in this thread: starting the others takes longer.
+    const int64_t grain = count < kSerialVisits ? std::max<int64_t>(1, (int64_t)blocks.size()) : 4;
+    parallel_for((int64_t)blocks.size(), grain, [&](int64_t b, int64_t e) {
+      for (int64_t i = b; i < e; ++i) {
+        const int32_t blk = blocks[i];
+        Rows out;
+        for (int32_t t : todo[blk]) {
+          const uint32_t* f = front[m.col[t]].w;
+          for (int32_t q = 0; q < kWords; ++q)
+            for (uint32_t v = cols.rows[(int64_t)t * kWords + q] & left[blk].w[q] & ~out.w[q]; v; v &= v - 1) {
+              const int32_t r = 32 * q + __builtin_ctz(v);
+              const uint32_t* w = m.bits + t * kTileWords + r * kWords;
+              if (!((w[0] & f[0]) | (w[1] & f[1]) | (w[2] & f[2]) | (w[3] & f[3]))) continue;
+              dist[blk * FWN_BLOCK + r] = level;
+              out.set(r);
+            }
+        }
+        next[blk] = out;
+        todo[blk].clear();
+      }
+    });
+    for (int32_t kb : active) front[kb] = Rows();
+    active.clear();
+    for (int32_t blk : blocks) {
+      if (!next[blk].any()) continue;
+      front[blk] = next[blk];
+      for (int32_t q = 0; q < kWords; ++q) left[blk].w[q] &= ~next[blk].w[q];
+      active.push_back(blk);
+    }
   }
   for (int32_t i = 0; i < m.n; ++i)
     if (dist[i] < 0) dist[i] = level;
+  return true;
 }
 
 // One neighbourhood average of the coordinates: each node's are replaced by the mean over the
@@ -382,14 +442,21 @@ int fwn_tiles_node_order(int32_t n, const int32_t* tile_ptr, const int32_t* tile
     // Landmarks: the node furthest from node 0, then each time the node furthest from all so far.
     std::vector<int32_t> dist, nearest;
     std::vector<float> x((size_t)m.n_blocks * FWN_BLOCK * kDims, 0.f), y(x.size(), 0.f);
-    distances(m, 0, dist);
+    const Columns cols(m);
+    const int64_t most = std::max(kVisits, kVisitsPerRow * FWN_BLOCK * tile_ptr[m.n_blocks]);
+    int64_t visits = 0;
+    bool near = distances(m, cols, 0, most, visits, dist);
     int32_t src = (int32_t)(std::max_element(dist.begin(), dist.end()) - dist.begin());
-    for (int l = 0; l < kLandmarks; ++l) {
-      distances(m, src, dist);
+    for (int l = 0; near && l < kLandmarks; ++l) {
+      near = distances(m, cols, src, most, visits, dist);
       for (int32_t i = 0; i < n; ++i) x[(int64_t)i * kDims + l] = (float)dist[i];
       if (l == 0) nearest = dist;
       for (int32_t i = 0; i < n; ++i) nearest[i] = std::min(nearest[i], dist[i]);
       src = (int32_t)(std::max_element(nearest.begin(), nearest.end()) - nearest.begin());
+    }
+    if (!near) {
+      for (int32_t i = 0; i < n; ++i) perm[i] = i;
+      return FWN_OK;
     }
     for (int s = 0; s < kSmooth; ++s) {
       average(m, x, y);

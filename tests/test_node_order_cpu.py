@@ -3,6 +3,7 @@ numbering of packed pairs (``fwn_tiles_node_order``, ``fwn_tiles_permute_*``, ``
 ``fwn_tiles_unit_map``): the order is a permutation for any mask, the permuted list is the one built
 from the permuted mask, a packed list holds the mask's entries, and every dS unit has one number."""
 import gc
+import time
 import weakref
 
 import numpy as np
@@ -71,6 +72,24 @@ def test_order_is_deterministic_and_compact_on_a_shuffled_mesh():
   assert np.array_equal(perm, _order(n, tp, kb, bits))
   tiles = _permuted(n, tp, kb, bits, perm)[0][-1]
   assert tiles <= _arrays(mask, hilbert)[0][-1] < tp[-1]
+
+
+def _band(n, width):
+  off = range(-width, width + 1)
+  return sparse.diags([np.ones(n - abs(k)) for k in off], list(off)).astype(bool).tocsr()
+
+
+@pytest.mark.parametrize("n,width,own", [(40962, 1, True), (40962, 16, True), (100000, 1, False)])
+def test_order_of_a_long_path_takes_seconds(n, width, own):
+  """A mask of long paths has tens of thousands of breadth-first levels: the searches cost what their
+  fronts do (a scan of the list, or a start of threads, per level took 70 s and more for the first
+  of these; 0.7 s now), and one that takes too many steps leaves the nodes in their own order."""
+  lists = _arrays(_band(n, width))
+  start = time.perf_counter()
+  perm = _order(n, *lists)
+  assert time.perf_counter() - start < 15
+  assert np.array_equal(np.sort(perm), np.arange(n))
+  assert np.array_equal(perm, np.arange(n)) == (not own)
 
 
 def _compact(n, tp, kb, bits, group, parts=0, window=0):
