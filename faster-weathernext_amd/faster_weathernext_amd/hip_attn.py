@@ -740,9 +740,14 @@ def _as_tiles(tiles, n, device):
   key = (id(tp), id(kb), id(bits), n, str(device))
   with _cache_lock:
     hit = _cache.get(key)
-    if hit is None or hit[0] is not tp or hit[1] is not kb or hit[2] is not bits:
-      hit = (tp, kb, bits, TileList(np.asarray(tp), np.asarray(kb), np.asarray(bits), n, device))
-      _cache[key] = hit
+    if hit is not None and hit[0] is tp and hit[1] is kb and hit[2] is bits:
+      _cache.move_to_end(key)
+      return hit[3]
+  # Built outside the lock, which every call with arrays takes; of two threads that build the same
+  # list, both use the first one put in place.
+  made = (tp, kb, bits, TileList(np.asarray(tp), np.asarray(kb), np.asarray(bits), n, device))
+  with _cache_lock:
+    hit = _cache.setdefault(key, made)
     _cache.move_to_end(key)
     while len(_cache) > CACHE_LISTS:
       _cache.popitem(last=False)

@@ -2,12 +2,15 @@
 numbering of packed pairs (``fwn_tiles_node_order``, ``fwn_tiles_permute_*``, ``fwn_tiles_compact_*``,
 ``fwn_tiles_unit_map``): the order is a permutation for any mask, the permuted list is the one built
 from the permuted mask, a packed list holds the mask's entries, and every dS unit has one number."""
+import collections
 import gc
+import threading
 import time
 import weakref
 
 import numpy as np
 import pytest
+import torch
 from scipy import sparse
 
 import faster_weathernext_amd as fwn
@@ -300,3 +303,36 @@ def test_exchange_lists_are_no_costlier_than_the_given_ones(name):
     assert dmap.struct.table == dq.struct.flags == kv.struct.flags == (0 if kept[products] else 1)
   assert kept["bf16"] == (name not in ("mesh", "hilbert"))
   assert kept["f32"] == kept["bf16x3"] == wide
+
+
+def test_a_list_in_the_making_holds_up_no_other_call(monkeypatch):
+  """Lists of array triples are built outside the cache's lock: while one is being made, calls with
+  other arrays go on, and two threads that make the same one use the same."""
+  monkeypatch.setattr(hip_attn, "_cache", collections.OrderedDict())
+  first, second = (_arrays(fwn.mesh_mask(2, k)[0]) for k in (1, 2))
+  cpu = torch.device("cpu")
+  ready = hip_attn._as_tiles(second, 162, cpu)
+  started, go = threading.Semaphore(0), threading.Event()
+
+  def make(*args):
+    started.release()
+    assert go.wait(30)
+    return fwn.TileList(*args)
+
+  monkeypatch.setattr(hip_attn, "TileList", type("Slow", (), {"__new__": staticmethod(lambda cls, *a: make(*a))}))
+  made = []
+  threads = [threading.Thread(target=lambda: made.append(hip_attn._as_tiles(first, 162, cpu))) for _ in range(2)]
+  for t in threads:
+    t.start()
+  try:
+    assert started.acquire(timeout=30)
+    other = threading.Thread(target=lambda: made.append(hip_attn._as_tiles(second, 162, cpu)))
+    other.start()
+    other.join(30)
+    assert made == [ready]
+    assert started.acquire(timeout=30)
+  finally:
+    go.set()
+    for t in threads:
+      t.join()
+  assert len(made) == 3 and made[1] is made[2] is hip_attn._as_tiles(first, 162, cpu)
