@@ -72,32 +72,32 @@ def linear_wgrad(g, x, bias):
 
 
 class _Linear(torch.autograd.Function):
-  """F.linear with the faster row split, and with ``linear_wgrad`` for the weight's and bias's gradients."""
+  """F.linear of x [M, K] with the faster row split, and with ``linear_wgrad`` for the weight's and
+  bias's gradients. Its output is a tensor of its own, not a view: a program may write into it."""
 
   @staticmethod
   def forward(ctx, x, weight, bias):
     ctx.save_for_backward(x, weight)
     ctx.has_bias = bias is not None
-    return linear_rows(x.reshape(-1, x.shape[-1]), weight, bias).view(*x.shape[:-1], weight.shape[0])
+    return linear_rows(x, weight, bias)
 
   @staticmethod
-  def backward(ctx, grad):
+  def backward(ctx, g):
     x, weight = ctx.saved_tensors
     need_x, need_w, need_b = ctx.needs_input_grad
     need_b = need_b and ctx.has_bias
-    g, x2 = grad.reshape(-1, grad.shape[-1]), x.reshape(-1, x.shape[-1])
     dx = dw = db = None
-    if as_torch(grad):
-      return (torch.mm(g, weight).view(x.shape) if need_x else None, torch.mm(g.t(), x2) if need_w else None,
+    if as_torch(g):
+      return (torch.mm(g, weight) if need_x else None, torch.mm(g.t(), x) if need_w else None,
               g.sum(0) if need_b else None)
     if need_x:
-      dx = linear_rows(g, weight.t()).view(x.shape)
+      dx = linear_rows(g, weight.t())
     if need_w:
-      g, x2 = g.contiguous(), x2.contiguous()
-      if (g.data_ptr() | x2.data_ptr()) & 15:
-        dw, db = torch.mm(g.t(), x2), g.sum(0) if need_b else None
+      g, x = g.contiguous(), x.contiguous()
+      if (g.data_ptr() | x.data_ptr()) & 15:
+        dw, db = torch.mm(g.t(), x), g.sum(0) if need_b else None
       else:
-        dw, db = linear_wgrad(g, x2, need_b)
+        dw, db = linear_wgrad(g, x, need_b)
     elif need_b:
       db = g.sum(0)
     return dx, dw, db
@@ -132,7 +132,8 @@ def linear(lin, x):
                             lin.bias.device == x.device)) and
       not torch.is_autocast_enabled("cuda") and not torch.compiler.is_compiling() and
       not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0):
-    return _Linear.apply(x, lin.weight, lin.bias)
+    y = _Linear.apply(x.reshape(-1, x.shape[-1]), lin.weight, lin.bias)
+    return y.view(*x.shape[:-1], y.shape[-1])
   return lin(x)
 
 

@@ -98,3 +98,31 @@ def test_linear_matches_the_module(monkeypatch, form):
   for a, b in zip(got, want):
     assert a.shape == b.shape and a.dtype == b.dtype
     assert float((a.double() - b.double()).norm() / b.double().norm()) <= 2.0 ** -7
+
+
+def test_output_may_be_written_in_place():
+  """A Linear's output is its caller's: an in-place activation or residual add after it works as after
+  the module, on the output and on a view of it."""
+  torch.manual_seed(4)
+  lin = torch.nn.Linear(64, 128, dtype=torch.bfloat16)
+  x = torch.randn(6, 64).to(torch.bfloat16).requires_grad_(True)
+  for shape in ((6, 128), (2, 3, 128)):
+    y = mha._Linear.apply(x, lin.weight, lin.bias).view(shape)
+    want = lin(x).view(shape)
+    assert torch.equal(torch.nn.functional.silu(y, inplace=True), torch.nn.functional.silu(want, inplace=True))
+    (y.add_(1.0) * 2).sum()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", [torch.nn.SiLU(inplace=True), torch.nn.ReLU(inplace=True)])
+def test_in_place_activation_after_linear(monkeypatch, act):
+  monkeypatch.setattr(mha, "WGRAD_ROWS", 1)
+  torch.manual_seed(5)
+  lin = torch.nn.Linear(64, 128, device=DEV, dtype=torch.bfloat16)
+  x = torch.randn(3, 100, 64, device=DEV).to(torch.bfloat16).requires_grad_(True)
+  g = torch.randn(3, 100, 128, device=DEV).to(torch.bfloat16)
+  leaves = [x, *lin.parameters()]
+  run = lambda f: [out := act(f(x)), *torch.autograd.grad(out, leaves, g)]
+  # Each side rounds float32 sums to bf16 (2^-9) at most twice along the way.
+  for a, b in zip(run(lambda t: mha.linear(lin, t)), run(lin)):
+    assert a.shape == b.shape and float((a.double() - b.double()).norm() / b.double().norm()) <= 2.0 ** -7
