@@ -77,7 +77,10 @@ class _Linear(torch.autograd.Function):
 
   @staticmethod
   def forward(ctx, x, weight, bias):
-    ctx.save_for_backward(x, weight)
+    # Each is kept only for the gradient that reads it, as F.linear does: a frozen weight holds no x, and
+    # may be written where x needs no gradient.
+    need_x, need_w, _ = ctx.needs_input_grad
+    ctx.save_for_backward(x if need_w else None, weight if need_x else None)
     ctx.has_bias = bias is not None
     return linear_rows(x, weight, bias)
 

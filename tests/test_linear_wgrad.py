@@ -126,3 +126,18 @@ def test_in_place_activation_after_linear(monkeypatch, act):
   # Each side rounds float32 sums to bf16 (2^-9) at most twice along the way.
   for a, b in zip(run(lambda t: mha.linear(lin, t)), run(lin)):
     assert a.shape == b.shape and float((a.double() - b.double()).norm() / b.double().norm()) <= 2.0 ** -7
+
+
+@pytest.mark.parametrize("need_x,need_w", [(True, True), (True, False), (False, True), (False, False)])
+def test_saves_what_its_gradients_read(need_x, need_w):
+  """x is kept for the weight's gradient and the weight for x's, as the module keeps them: not a frozen
+  weight's input, and a weight whose input needs no gradient may be written before the backward."""
+  lin = torch.nn.Linear(64, 128, dtype=torch.bfloat16)
+  lin.weight.requires_grad_(need_w)
+  x = torch.randn(6, 64).to(torch.bfloat16).requires_grad_(need_x)
+  kept = []
+  with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(t.data_ptr()) or t, lambda t: t):
+    mha._Linear.apply(x, lin.weight, lin.bias)
+    own, kept = kept, []
+    lin(x)
+  assert sorted(own) == sorted(kept) == sorted([x.data_ptr()] * need_w + [lin.weight.data_ptr()] * need_x)
