@@ -275,12 +275,12 @@ class _AddNorm(torch.autograd.Function):
 
 def residual_norm(x, y, *, mul, add, eps=1e-5):
   """(x + y, layer_norm_affine(x + y)) with gradients: one pass forward and one backward where x and
-  y share dtype and layout, else torch's add and the norm's own pass."""
+  y are contiguous, aligned and of one dtype, else torch's add and the norm's own pass."""
   same = (x.dtype == y.dtype and x.shape == y.shape and x.is_contiguous() and y.is_contiguous() and
           x.data_ptr() % 16 == 0 and y.data_ptr() % 16 == 0)
   if same and x.is_cuda and x.dim() == 3 and x.dtype in _DTYPES:
     return _AddNorm.apply(x, y, mul, add, float(eps))
-  s = x + y
+  s = (x + y).contiguous()  # torch's add keeps a dense operand's strides
   return s, layer_norm_affine(s, mul=mul, add=add, eps=eps)
 
 

@@ -35,3 +35,14 @@ def test_linear_rows_split_rows_are_the_unsplit_rows():
   got = linear_rows(x, w)
   for r in (0, ROW_QUANTUM - 1, ROW_QUANTUM, ROW_QUANTUM + 2):
     torch.testing.assert_close(got[r], x[r] @ w.t(), rtol=1e-12, atol=1e-12)
+
+
+def test_residual_norm_hands_a_contiguous_sum_to_the_norm(monkeypatch):
+  """torch's add keeps a dense operand's strides; the norm's pass takes contiguous rows only."""
+  from faster_weathernext_amd import rows
+  seen = []
+  monkeypatch.setattr(rows, "layer_norm_affine", lambda s, **kw: seen.append(s) or s)
+  x, y = torch.randn(2, 5, 8), torch.randn(2, 5, 8)
+  for xx in (x, x.transpose(0, 1).contiguous().transpose(0, 1), x.permute(2, 0, 1).contiguous().permute(1, 2, 0)):
+    s, _ = rows.residual_norm(xx, y, mul=None, add=None)
+    assert s.is_contiguous() and seen[-1] is s and torch.equal(s, x + y)

@@ -95,12 +95,15 @@ def test_missing_strided_and_offset_gradients():
   assert torch.equal(grad(affine(), off), grad(affine(), g1))
   # residual_norm takes any layout and mixed dtypes, as torch's add does
   s0, o0 = rows.residual_norm(x, y, mul=mul, add=add)
-  for xx, yy in ((off.copy_(x), y), (x.transpose(0, 1).contiguous().transpose(0, 1), y), (x, y[:, :1].expand(b, n, c))):
-    s, o = rows.residual_norm(xx, yy, mul=mul, add=add) if xx.is_contiguous() else (None, None)
-    if s is not None and yy is y:
-      assert torch.equal(s, s0) and torch.equal(o, o0)
-    elif s is not None:
-      assert torch.equal(s, x + yy)
+  flipped = x.transpose(0, 1).contiguous().transpose(0, 1)
+  assert not flipped.is_contiguous() and not (flipped + y).is_contiguous()
+  for xx in (off.copy_(x), flipped, x.permute(2, 0, 1).contiguous().permute(1, 2, 0)):
+    s, o = rows.residual_norm(xx, y, mul=mul, add=add)
+    assert torch.equal(s, s0) and torch.equal(o, o0)
+  same = y[:, :1].expand(b, n, c)
+  s, o = rows.residual_norm(x, same, mul=mul, add=add)
+  s1, o1 = rows.residual_norm(x, same.contiguous(), mul=mul, add=add)
+  assert torch.equal(s, s1) and torch.equal(o, o1)
   s, o = rows.residual_norm(x, y.to(torch.bfloat16), mul=mul, add=add)
   assert s.dtype == torch.float32 and torch.equal(s, x + y.to(torch.bfloat16))
 
