@@ -82,9 +82,10 @@ class NormConditioning(torch.nn.Module):
 
   def plain(self, cond):
     """Whether ``affine`` is the linear map as built, on parameters the conditioning kernel reads: no
-    subclass, hook, parametrization or autocast that would see or change the call."""
+    replaced method, hook, parametrization or autocast that would see or change the call. Asked of
+    norms of this very class only (``affines_f32``)."""
     lin = self.linear
-    return (type(self) is NormConditioning and not torch.is_autocast_enabled("cuda")
+    return (not vars(self).keys() & {"affine", "add_norm"} and not torch.is_autocast_enabled("cuda")
             and is_plain(lin, torch.nn.Linear) and cond.dim() == 2 and cond.is_cuda
             and cond.dtype in (torch.float32, torch.bfloat16) and cond.is_contiguous() and cond.numel() > 0
             and all(type(t) is torch.nn.Parameter and t.dtype == cond.dtype and t.device == cond.device and
@@ -102,11 +103,21 @@ COND_WORK = 1 << 12
 
 def affines_f32(norms, cond):
   """``affine_f32(cond)`` of each norm, without autograd, in one launch; None for each where a norm is
-  not ``plain`` or the projections are large enough for a GEMM each."""
-  if (cond.numel() <= COND_WORK and all(norm.plain(cond) for norm in norms) and
+  not a ``plain`` one or the projections are large enough for a GEMM each."""
+  if (cond.numel() <= COND_WORK and all(type(norm) is NormConditioning and norm.plain(cond) for norm in norms) and
       len({norm.linear.weight.shape for norm in norms}) == 1):
     return cond_affine(cond, [norm.linear.weight for norm in norms], [norm.linear.bias for norm in norms])
   return [None] * len(norms)
+
+
+def _is_own(obj, cls, name):
+  """Whether obj.name is cls's method: of a class or object of the program's own, its methods are called
+  as they have always been."""
+  return getattr(type(obj), name, None) is getattr(cls, name) and name not in vars(obj)
+
+
+def _add_norm(norm, x, y, cond, eps, affine):
+  return norm.add_norm(x, y, cond, eps) if affine is None else norm.add_norm(x, y, cond, eps, affine)
 
 
 class MeshBlock(torch.nn.Module):
@@ -139,7 +150,12 @@ class MeshBlock(torch.nn.Module):
     """`normed` is layernorm(x) when the caller has it already (block 0 gets it from the fused
     gather). Otherwise each conditioned layer norm is one fused pass (``layer_norm_affine``)."""
     h = self.norm_mha(normed, cond) if normed is not None else self.norm_mha.norm(x, cond, self.eps)
-    x, h = self.norm_ffw.residual_norm(x, self.mha(h), cond, self.eps)
+    y = self.mha(h)
+    if _is_own(self.norm_ffw, NormConditioning, "norm"):
+      x, h = self.norm_ffw.residual_norm(x, y, cond, self.eps)
+    else:
+      x = x + y
+      h = self.norm_ffw.norm(x, cond, self.eps)
     return x + self.feed_forward(h)
 
   def forward_fused(self, x, h, cond, next_norm=None, affines=(None, None)):
@@ -147,11 +163,11 @@ class MeshBlock(torch.nn.Module):
     add runs in one pass with the conditioned layer norm that reads it (``add_layer_norm_affine``),
     the feed-forward's own and, when `next_norm` is given, the next block's. `affines` are the two
     norms' ``affine_f32(cond)`` where the caller has them. Returns (x, the next block's h or None)."""
-    x, h = self.norm_ffw.add_norm(x, self.mha(h), cond, self.eps, affines[0])
+    x, h = _add_norm(self.norm_ffw, x, self.mha(h), cond, self.eps, affines[0])
     f = self.feed_forward(h)
     if next_norm is None:
       return x + f, None
-    return next_norm.add_norm(x, f, cond, self.eps, affines[1])
+    return _add_norm(next_norm, x, f, cond, self.eps, affines[1])
 
 
 class MeshTransformer(torch.nn.Module):
@@ -213,17 +229,19 @@ class MeshTransformer(torch.nn.Module):
       # Without autograd the residual adds are fused into the conditioned layer norms after them, and
       # every norm's conditioning is evaluated up front in one launch.
       nexts = [block.norm_mha for block in self.blocks[1:]] + [None]
-      norms = [block.norm_ffw for block in self.blocks] + nexts[:-1] + [self.final_norm]
-      affines = affines_f32(norms, cond)
-      ffw, final = affines[:len(self.blocks)], affines[-1]
+      affines = [None]
+      if all(_is_own(block, MeshBlock, "forward_fused") for block in self.blocks):
+        affines = affines_f32([block.norm_ffw for block in self.blocks] + nexts[:-1] + [self.final_norm], cond)
+      final = affines[-1]
       h = self.blocks[0].norm_mha(normed, cond)
       for i, block in enumerate(self.blocks):
-        x, h = block.forward_fused(x, h, cond, nexts[i], (ffw[i], affines[len(self.blocks) + i]))
+        given = () if final is None else ((affines[i], affines[len(self.blocks) + i]),)
+        x, h = block.forward_fused(x, h, cond, nexts[i], *given)
     else:
       for i, block in enumerate(self.blocks):
         x = block(x, cond, normed if i == 0 else None)
     if self.perm is not None:
-      mul, add = final or self.final_norm.affine_f32(cond)
-      return layer_norm_scatter(x, self.perm, mul=mul, add=add, eps=self.eps)
+      mul, add = final or self.final_norm.affine(cond)
+      return layer_norm_scatter(x, self.perm, mul=mul.float().contiguous(), add=add.float().contiguous(), eps=self.eps)
     mul, add = self.final_norm.affine(cond)
     return F.layer_norm(x, (d,), eps=self.eps) * mul[:, None, :] + add[:, None, :]
