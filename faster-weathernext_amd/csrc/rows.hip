@@ -389,8 +389,9 @@ __global__ void __launch_bounds__(64 * kSumGroups) sums_kernel(RowBwdArgs a) {
 // The conditioning of several norms in one launch: one thread per output column, its weight row read
 // straight from memory (64 bytes at 32 bf16 conditioning features; read once for 4 batch members).
 // Bound by launches, not by bytes: each norm's own GEMM, add and two casts are four or five launches.
-// The 49 norms of a 24-layer transformer of 768 channels, issued back to back: 1.7 to 2.0 ms norm by
-// norm, 58 us here (most of it the host's); its whole refinement-6 forward 30.04 -> 29.84 ms.
+// 49 norms of 768 channels, issued back to back: 1.7 to 2.0 ms norm by norm, 58 us here (most of it
+// the host's); the refinement-6 forward of a 24-layer transformer, which has 48 of its 49 norms in the
+// launch (block 0's first is projected by itself), 30.04 -> 29.84 ms.
 template <typename T>
 __device__ __forceinline__ float load_one(const void* p, size_t i) {
   if constexpr (sizeof(T) == 4) {

@@ -227,16 +227,22 @@ class MeshTransformer(torch.nn.Module):
       normed = F.layer_norm(x, (d,), eps=self.eps)
     if len(self.blocks) and not needs_grad(x, self):
       # Without autograd the residual adds are fused into the conditioned layer norms after them, and
-      # every norm's conditioning is evaluated up front in one launch.
-      nexts = [block.norm_mha for block in self.blocks[1:]] + [None]
+      # the conditioning of all norms that HIP passes apply (all but block 0's first and, without the
+      # scatter, the final one) is evaluated up front in one launch.
+      nexts = [block.norm_mha for block in self.blocks[1:]]
       affines = [None]
       if all(_is_own(block, MeshBlock, "forward_fused") for block in self.blocks):
-        affines = affines_f32([block.norm_ffw for block in self.blocks] + nexts[:-1] + [self.final_norm], cond)
-      final = affines[-1]
+        norms = [block.norm_ffw for block in self.blocks] + nexts
+        affines = affines_f32(norms if self.perm is None else norms + [self.final_norm], cond)
       h = self.blocks[0].norm_mha(normed, cond)
-      for i, block in enumerate(self.blocks):
-        given = () if final is None else ((affines[i], affines[len(self.blocks) + i]),)
-        x, h = block.forward_fused(x, h, cond, nexts[i], *given)
+      if affines[0] is None:
+        for block, after in zip(self.blocks, nexts + [None]):
+          x, h = block.forward_fused(x, h, cond, after)
+      else:
+        ffw, mha = affines[:len(self.blocks)], affines[len(self.blocks):]
+        final = None if self.perm is None else mha.pop()
+        for block, after, own, other in zip(self.blocks, nexts + [None], ffw, mha + [None]):
+          x, h = block.forward_fused(x, h, cond, after, (own, other))
     else:
       for i, block in enumerate(self.blocks):
         x = block(x, cond, normed if i == 0 else None)

@@ -123,3 +123,35 @@ def test_own_final_norm(monkeypatch, reorder, grad):
   with torch.set_grad_enabled(grad):
     got = model(x, cond)
   torch.testing.assert_close(got.float(), _expected(model, x, cond).float(), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("taken", [True, False])
+@pytest.mark.parametrize("reorder", [True, False])
+def test_conditioning_launch_holds_the_norms_that_use_it(monkeypatch, reorder, taken):
+  """All norms but block 0's first and, where no scatter pass applies it, the final one; each gets its
+  own affine."""
+  torch.manual_seed(1)
+  model = fwn.MeshTransformer(refinement=1, k_hop=1, num_layers=3, d_model=D, num_heads=1, key_size=32, ffw_hidden=32,
+                              cond_size=COND, reorder=False, device="cpu", dtype=torch.float32).requires_grad_(False)
+  for mod in model.modules():
+    if isinstance(mod, transformer.NormConditioning):
+      torch.nn.init.normal_(mod.linear.weight, std=0.3)
+  for block in model.blocks:
+    block.mha, block.ffw[1] = Scaled(), torch.nn.ReLU()
+  seen = []
+  monkeypatch.setattr(transformer, "affines_f32", lambda norms, cond: seen.extend(norms) or
+                      [norm.affine_f32(cond) if taken else None for norm in norms])
+  monkeypatch.setattr(transformer.MeshBlock, "feed_forward", lambda self, h: self.ffw(h))
+  norm = lambda x, mul, add, eps: F.layer_norm(x, (D,), eps=eps) * mul[:, None] + add[:, None]
+  monkeypatch.setattr(transformer, "add_layer_norm_affine",
+                      lambda x, y, mul, add, eps: (x + y, norm(x + y, mul, add, eps)))
+  monkeypatch.setattr(transformer, "layer_norm_affine", lambda x, mul, add, eps: norm(x, mul, add, eps))
+  if reorder:
+    model.perm = torch.arange(model.n)
+    monkeypatch.setattr(transformer, "gather_layer_norm", lambda x, perm, eps: (x, F.layer_norm(x, (D,), eps=eps)))
+    monkeypatch.setattr(transformer, "layer_norm_scatter", lambda x, perm, mul, add, eps: norm(x, mul, add, eps))
+  x, cond = torch.randn(2, model.n, D), torch.randn(2, COND)
+  got = model(x, cond)
+  want = [b.norm_ffw for b in model.blocks] + [b.norm_mha for b in model.blocks[1:]] + [model.final_norm] * reorder
+  assert len(seen) == len(want) and all(a is b for a, b in zip(seen, want))
+  torch.testing.assert_close(got, _expected(model, x, cond), rtol=1e-5, atol=1e-5)
