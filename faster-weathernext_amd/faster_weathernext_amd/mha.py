@@ -117,8 +117,9 @@ WGRAD_ENTRIES = 128 * 256 * 256
 
 
 def is_plain(module, kind):
-  """Whether calling `module` is calling kind.forward: no subclass, hook, parametrization or wrapper."""
-  return (type(module) is kind and "forward" not in module.__dict__ and
+  """Whether calling `module` is calling kind.forward: no subclass, hook, parametrization, wrapper or
+  compiled call (``Module.compile``)."""
+  return (type(module) is kind and "forward" not in module.__dict__ and module._compiled_call_impl is None and
           not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or
                module._backward_pre_hooks) and not torch.nn.modules.module._has_any_global_hook())
 

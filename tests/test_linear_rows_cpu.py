@@ -46,3 +46,16 @@ def test_residual_norm_hands_a_contiguous_sum_to_the_norm(monkeypatch):
   for xx in (x, x.transpose(0, 1).contiguous().transpose(0, 1), x.permute(2, 0, 1).contiguous().permute(1, 2, 0)):
     s, _ = rows.residual_norm(xx, y, mul=None, add=None)
     assert s.is_contiguous() and seen[-1] is s and torch.equal(s, x + y)
+
+
+def test_plain_modules_are_those_whose_call_is_their_forward():
+  from faster_weathernext_amd.mha import is_plain
+  make = lambda: torch.nn.Linear(4, 4)
+  assert is_plain(make(), torch.nn.Linear) and not is_plain(make(), torch.nn.Sequential)
+  hooked, replaced, compiled = make(), make(), make()
+  hooked.register_forward_pre_hook(lambda mod, args: None)
+  replaced.forward = lambda x: x
+  compiled._compiled_call_impl = lambda x: x  # what Module.compile() sets and a call then runs
+  assert torch.equal(compiled(torch.ones(4)), torch.ones(4))
+  for lin in (hooked, replaced, compiled, torch.nn.utils.parametrizations.weight_norm(make())):
+    assert not is_plain(lin, torch.nn.Linear)
