@@ -443,6 +443,12 @@ class TileList:
     return float(bits) / (16 * self.n_tiles)
 
 
+# Most tiles of a list in its own node order, of the given list's: each is 2 KB on the host, and an order
+# that spreads the mask over every pair of blocks would take n^2 / 8 bytes. Meshes have 0.27 to 0.87,
+# random entries 1.0, the 8-hop mesh with 20 to 60 rows that reach everywhere 1.4 to 1.8.
+PERMUTED_TILES = 2
+
+
 class _Arrays:
   """Canonical tile arrays on the host (tile_ptr, column blocks, bits) of an n x n mask."""
 
@@ -451,10 +457,13 @@ class _Arrays:
     self.args = (n, nat.ptr(ptr), nat.ptr(col), nat.ptr(bits))
 
   def permuted(self, perm):
-    """The arrays of mask[perm][:, perm]."""
+    """The arrays of mask[perm][:, perm], or None where they would hold more than PERMUTED_TILES times
+    as many tiles."""
     L = nat.lib()
     ptr = np.zeros_like(self.ptr)
     nat.check(L.fwn_tiles_permute_count(*self.args, nat.ptr(perm), nat.ptr(ptr)))
+    if int(ptr[-1]) > PERMUTED_TILES * int(self.ptr[-1]):
+      return None
     col, bits = np.empty(int(ptr[-1]), np.int32), np.empty((int(ptr[-1]), nat.BLOCK, nat.BLOCK // 32), np.uint32)
     nat.check(L.fwn_tiles_permute_fill(*self.args, nat.ptr(perm), nat.ptr(ptr), nat.ptr(col), nat.ptr(bits)))
     return _Arrays(self.n, ptr, col, bits)
@@ -572,11 +581,11 @@ class _Layout:
     nat.check(nat.lib().fwn_tiles_node_order(*given.args, nat.ptr(perm)))
     # The packed list of the mask in its own order or, if that does not pay and costs more, in the given one.
     arrays = given.permuted(perm)
-    packed = _Packed(arrays, 1)
-    if not packed.pays(tl, LAID_OUT_GAIN):
-      cost, arrays, perm = packed.cost, given, np.arange(n, dtype=np.int64)
+    packed = arrays and _Packed(arrays, 1)
+    if not packed or not packed.pays(tl, LAID_OUT_GAIN):
+      cost, arrays, perm = packed and packed.cost, given, np.arange(n, dtype=np.int64)
       packed = _Packed(arrays, 1)
-      if packed.cost >= cost or not packed.pays(tl, LAID_OUT_GAIN):
+      if (cost is not None and packed.cost >= cost) or not packed.pays(tl, LAID_OUT_GAIN):
         return None
     return cls(arrays, perm, tl.device, tl._fixed_cap, packed)
 
@@ -591,9 +600,9 @@ class _Layout:
       arrays_t = self.arrays if own else _Arrays(self.arrays.n, tiles_t._tile_ptr, tiles_t._tile_col,
                                                  tiles_t._tile_bits).permuted(self.perm)
       dq = _Packed(self.arrays, unit_keys, window=window)
-      kv = _Packed(arrays_t, 32, nat.PARTS_PAIRS16)
+      kv = arrays_t and _Packed(arrays_t, 32, nat.PARTS_PAIRS16)
       made, gain = None, _exchange_gain(products)
-      if dq.pays(tl, gain) and kv.pays(tiles_t, gain):
+      if dq.pays(tl, gain) and kv and kv.pays(tiles_t, gain):
         dq, kv = self._list(dq), self._list(kv)
         dmap = DsMap.of_packed(dq, kv, unit_keys)
         made = (dq, kv, dmap) if dmap.n_units <= gain * given.n_units else None

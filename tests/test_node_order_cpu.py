@@ -3,6 +3,7 @@ numbering of packed pairs (``fwn_tiles_node_order``, ``fwn_tiles_permute_*``, ``
 ``fwn_tiles_unit_map``): the order is a permutation for any mask, the permuted list is the one built
 from the permuted mask, a packed list holds the mask's entries, and every dS unit has one number."""
 import collections
+import ctypes
 import gc
 import threading
 import time
@@ -336,3 +337,30 @@ def test_a_list_in_the_making_holds_up_no_other_call(monkeypatch):
     for t in threads:
       t.join()
   assert len(made) == 3 and made[1] is made[2] is hip_attn._as_tiles(first, 162, cpu)
+
+
+def test_an_order_that_spreads_the_mask_is_not_laid_out(monkeypatch):
+  """A list in its own node order takes 2 KB of host memory a tile: where it has more than PERMUTED_TILES
+  times the given list's, its tiles are never filled and the given order is packed, or kept."""
+  mask, _, _, perm = fwn.mesh_mask(4, 4, reorder=True)
+  tl = fwn.TileList.from_mask(mask, perm, device="cpu")
+  n, given = mask.shape[0], hip_attn._Arrays(tl.n_cols, tl._tile_ptr, tl._tile_col, tl._tile_bits)
+  shuffle = np.random.default_rng(0).permutation(n)
+  assert _arrays(mask[perm][:, perm][shuffle][:, shuffle].tocsr())[0][-1] > 2 * tl.n_tiles
+
+  def spread(n, ptr, col, bits, out):
+    np.ctypeslib.as_array((ctypes.c_int64 * n).from_address(out))[:] = shuffle
+    return nat.OK
+
+  class Lib:
+    fwn_tiles_node_order = staticmethod(spread)
+
+    def __getattr__(self, name):
+      assert name != "fwn_tiles_permute_fill"
+      return getattr(real, name)
+
+  real = nat.lib()
+  monkeypatch.setattr(nat, "lib", Lib)
+  assert given.permuted(shuffle) is None
+  layout = hip_attn._Layout.choose(tl)
+  assert np.array_equal(layout.perm, np.arange(n)) and layout.forward.cost <= 0.95 * tl.cost
