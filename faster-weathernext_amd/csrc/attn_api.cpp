@@ -138,7 +138,7 @@ int check_tiles(const fwn_attn_desc* d, const fwn_tiles* t, const char* name) {
   if (t->flags & FWN_TILES_NODES) {
     if (!t->row_node || (t->n_tiles > 0 && !t->col_node)) return fail(FWN_ERR_TILES, "%s: null node table", name);
     if (!aligned16(t->col_node)) return fail(FWN_ERR_INVALID_ARG, "%s: col_node is not 16-byte aligned", name);
-    if ((int64_t)t->n_tiles * FWN_BLOCK * 4 >= (int64_t)1 << 31)
+    if (t->n_tiles >= FWN_TILES_NODES_MAX)
       return fail(FWN_ERR_INVALID_ARG, "%s: too many tiles for a node table (%d)", name, t->n_tiles);
     // The kernels form row offsets as 24-bit products of the node and the row stride. The stride
     // is below 2^24 bytes for lists of two or more blocks (a slice spans less than 2 GiB).

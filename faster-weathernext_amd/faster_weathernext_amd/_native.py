@@ -56,6 +56,7 @@ class Tiles(ctypes.Structure):
 
 
 TILES_NODES = 1  # FWN_TILES_NODES: the list is laid out in an order of its own (Tiles.row_node, col_node)
+TILES_NODES_MAX = 1 << 22  # FWN_TILES_NODES_MAX: such a list has fewer tiles
 
 
 class DsMap(ctypes.Structure):

@@ -490,8 +490,9 @@ class _Packed:
     self.cost = _cost(self.n_tiles, int(np.count_nonzero(words & 0xffff) + np.count_nonzero(words >> 16)))
 
   def pays(self, tl, gain):
-    """Whether this list has at most `gain` of TileList `tl`'s tiles and of their cost."""
-    return self.n_tiles <= gain * tl.n_tiles and self.cost <= gain * tl.cost
+    """Whether this list has at most `gain` of TileList `tl`'s tiles and of their cost, and no more tiles
+    than a node table holds."""
+    return self.n_tiles < nat.TILES_NODES_MAX and self.n_tiles <= gain * tl.n_tiles and self.cost <= gain * tl.cost
 
 
 class _PackedList(TileList):

@@ -364,3 +364,23 @@ def test_an_order_that_spreads_the_mask_is_not_laid_out(monkeypatch):
   assert given.permuted(shuffle) is None
   layout = hip_attn._Layout.choose(tl)
   assert np.array_equal(layout.perm, np.arange(n)) and layout.forward.cost <= 0.95 * tl.cost
+
+
+def test_lists_past_the_node_table_keep_the_given_ones(monkeypatch):
+  """The launchers refuse lists with node tables of 2^22 tiles and more, so a mask that would have
+  them is walked as given, and so is the exchange where only its lists would."""
+  F = 1 << 20
+  size, desc = np.zeros(1, np.uint64), nat.AttnDesc(1, 256, 1, 32, nat.F32, 1.0, 32 * 256, 32, 32)
+  status = lambda tiles: nat.lib().fwn_attn_workspace_size(
+      desc, nat.Tiles(2, tiles, F, F, F, F, 2, 0, 0, 0, F, None, None, None, 0, nat.TILES_NODES, F, F), nat.ptr(size))
+  assert status((1 << 22) - 1) == nat.OK and status(1 << 22) == nat.ERR_INVALID_ARG
+  mask, _, _, perm = fwn.mesh_mask(4, 4, reorder=True)
+  tl = fwn.TileList.from_mask(mask, perm, device="cpu")
+  layout = hip_attn._Layout.choose(tl)
+  tiles = [layout.forward.n_tiles, *(hip_attn._Packed(layout.arrays, g, p).n_tiles for g, p in ((16, 0), (32, 1)))]
+  assert tiles == sorted(tiles) and tiles[0] < tiles[1]
+  for most, forward in ((tiles[0], False), (tiles[0] + 1, True)):
+    monkeypatch.setattr(nat, "TILES_NODES_MAX", most)
+    tl._layout = hip_attn._Layout.choose(tl)
+    assert (tl._layout is not None) == forward
+    assert tl.exchange_lists(tl, "bf16")[:2] == tl.exchange_lists(tl, "f32")[:2] == (tl, tl)
