@@ -289,6 +289,9 @@ int check_ds(const fwn_attn_desc* d, const fwn_ds_map* m, const void* ds, uint64
   // without tiles, whose per-tile arrays are empty and may be null.
   if (m->n_units > 0 && ((need_ubase && !m->ubase) || (need_tmap && !m->tmap)))
     return fail(FWN_ERR_INVALID_ARG, "ds map: null arrays");
+  // The kernels copy a tile's 36 words in 16-byte pieces.
+  if (need_tmap && m->table && !aligned16(m->tmap))
+    return fail(FWN_ERR_INVALID_ARG, "ds map: tmap is not 16-byte aligned");
   if (!ds) return fail(FWN_ERR_INVALID_ARG, "ds is null");
   if (((uintptr_t)ds & 255u) != 0) return fail(FWN_ERR_INVALID_ARG, "ds is not 256-byte aligned");
   const uint64_t need = (uint64_t)d->batch * (uint64_t)d->heads * (uint64_t)(m->n_units * ds_unit_bytes(m));

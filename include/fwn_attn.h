@@ -358,8 +358,8 @@ typedef struct fwn_ds_map {
                             bits word (as int32: halves for 16, groups for 32) of the same tile of
                             the forward list */
   int32_t unit_keys;     /* 16 (bf16 calls) or 32 (float32 calls) */
-  int32_t table;         /* 0, or 1: tmap is [tiles_t->n_tiles][9][4] (fwn_tiles_unit_map), as lists with
-                            FWN_TILES_NODES need */
+  int32_t table;         /* 0, or 1: tmap is [tiles_t->n_tiles][9][4], 16-byte aligned (fwn_tiles_unit_map), as
+                            lists with FWN_TILES_NODES need */
 } fwn_ds_map;
 
 /* Builds the unit numbering (host arrays) from the canonical arrays of both lists (tile_ptr,

@@ -384,3 +384,19 @@ def test_lists_past_the_node_table_keep_the_given_ones(monkeypatch):
     tl._layout = hip_attn._Layout.choose(tl)
     assert (tl._layout is not None) == forward
     assert tl.exchange_lists(tl, "bf16")[:2] == tl.exchange_lists(tl, "f32")[:2] == (tl, tl)
+
+
+def test_launchers_check_the_unit_table():
+  """Refused on the host: a unit table that the kernels' 16-byte copies cannot read, or one that does not
+  go with the list. (The tensors are null, so that no call gets further than their check.)"""
+  F = 1 << 20
+  desc = nat.AttnDesc(1, 256, 1, 32, nat.BF16, 1.0, 32 * 256, 32, 32)
+  def message(flags, table, tmap):
+    t = nat.Tiles(2, 1, F, F, F, F, 2, 0, 0, 0, F, None, None, None, 0, flags, F, F)
+    m = nat.DsMap(4, F, tmap, 16, table)
+    assert nat.lib().fwn_attn_bwd_dkv_ds_launch(desc, *[None] * 6, t, m, None, None, F, 1 << 20, None, 0, None) == nat.ERR_INVALID_ARG
+    return nat.lib().fwn_last_error().decode()
+  assert "q is null" in message(nat.TILES_NODES, 1, F) and "q is null" in message(0, 0, F + 8)
+  for offset in (4, 8, 12):
+    assert "tmap" in message(nat.TILES_NODES, 1, F + offset)
+  assert "table" in message(nat.TILES_NODES, 0, F) and "table" in message(0, 1, F)
