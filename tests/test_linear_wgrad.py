@@ -13,32 +13,85 @@ from faster_weathernext_amd import mha
 DEV = "cuda"
 
 
-def _framed(rows, cols, g):
-  """A [rows, cols] tensor inside NaNs: a read outside it shows."""
+SIZES = [(1, 64, 64), (31, 64, 256), (32, 256, 64), (33, 256, 256), (127, 192, 320), (128, 320, 192), (129, 512, 256),
+         (257, 768, 2304), (1000, 128, 384), (4097, 256, 256), (70001, 64, 128), (9001, 1536, 384)]
+
+
+def _framed(t):
+  """A copy of t [rows, cols] on the GPU inside NaNs: a read outside it shows."""
+  rows, cols = t.shape
   buf = torch.full(((rows + 8) * cols,), float("nan"), device=DEV, dtype=torch.bfloat16)
-  t = buf[4 * cols:(rows + 4) * cols].view(rows, cols)
-  t.copy_(torch.randn(rows, cols, device=DEV, generator=g))
-  return t
+  return buf[4 * cols:(rows + 4) * cols].view(rows, cols).copy_(t)
+
+
+def _random(rows, outs, ins):
+  gen = torch.Generator().manual_seed(rows + outs)
+  return [torch.randn(rows, cols, generator=gen).to(torch.bfloat16) for cols in (outs, ins)]
+
+
+def _integers(rows, outs, ins):
+  gen = torch.Generator().manual_seed(rows + ins)
+  return [torch.randint(-2, 3, (rows, cols), generator=gen).to(torch.bfloat16) for cols in (outs, ins)]
+
+
+def _gradients(g, x):
+  """(weight gradient, bias gradient) in float64."""
+  return g.double().t() @ x.double(), g.double().sum(0)
+
+
+def _bounds(g, x, dw, db):
+  """How far a float32 sum of the rows in any order, rounded to bf16 once, is from the float64 sums. The
+  rounding: half an ulp of 8 significant bits, at most 2^-8 of the value. The sum: each of `rows`
+  additions rounds by 2^-24 of a partial sum, and the partial sums of k random terms grow as sqrt(k)
+  times a term's deviation, together at most (2 / 3) sqrt(rows) 2^-24 |g| |x| (norms over the rows);
+  twelve times that for partial sums several deviations large."""
+  rows, gn, xn = g.shape[0], g.double().norm(dim=0), x.double().norm(dim=0)
+  sums = 8 * rows ** 0.5 * 2.0 ** -24
+  return 2.0 ** -8 * dw.abs() + sums * gn[:, None] * xn, 2.0 ** -8 * db.abs() + sums * gn * rows ** 0.5
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,outs,ins", [(1, 64, 64), (31, 64, 256), (32, 256, 64), (33, 256, 256), (127, 192, 320),
-                                           (128, 320, 192), (129, 512, 256), (257, 768, 2304), (1000, 128, 384),
-                                           (4097, 256, 256), (70001, 64, 128), (9001, 1536, 384)])
+@pytest.mark.parametrize("rows,outs,ins", SIZES)
 @pytest.mark.parametrize("bias", [True, False])
 def test_wgrad_matches_float64(rows, outs, ins, bias):
-  gen = torch.Generator(device=DEV).manual_seed(rows + outs)
-  g, x = _framed(rows, outs, gen), _framed(rows, ins, gen)
-  dw, db = mha.linear_wgrad(g, x, bias)
-  # float32 sums of `rows` terms in some order, then one rounding to bf16 (8 significant bits: half
-  # an ulp is at most 2^-8 of the value).
-  want, terms = g.double().t() @ x.double(), g.double().abs().t() @ x.double().abs()
-  assert bool(((dw.double() - want).abs() <= 2.0 ** -8 * want.abs() + rows * 2.0 ** -23 * terms).all())
-  if bias:
-    want, terms = g.double().sum(0), g.double().abs().sum(0)
-    assert bool(((db.double() - want).abs() <= 2.0 ** -8 * want.abs() + rows * 2.0 ** -23 * terms).all())
-  else:
-    assert db is None
+  g, x = _random(rows, outs, ins)
+  dw, db = mha.linear_wgrad(_framed(g), _framed(x), bias)
+  want = _gradients(g, x)
+  assert (db is None) == (not bias)
+  for got, ref, bound in zip((dw, db), want, _bounds(g, x, *want)):
+    if got is not None:
+      assert bool(((got.double().cpu() - ref).abs() <= bound).all())
+      # One rounding to bf16 leaves 1.7e-3 of the norm.
+      assert float((got.double().cpu() - ref).norm() / ref.norm()) <= 3e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,outs,ins", SIZES)
+def test_wgrad_of_integers_is_exact(rows, outs, ins):
+  """Entries from -2 to 2: every partial sum is a whole number below 2^24, so the float32 sums are exact
+  in any order and the results are the true sums rounded to bf16, to the bit."""
+  g, x = _integers(rows, outs, ins)
+  for got, ref in zip(mha.linear_wgrad(_framed(g), _framed(x), True), _gradients(g, x)):
+    assert torch.equal(got.cpu(), ref.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("rows,outs,ins", [s for s in SIZES if s[0] > 32])
+def test_a_left_out_stage_would_show(rows, outs, ins):
+  """The two tests above fail for results that miss rows (on the CPU, the rows taken out of the sums):
+  any one 32-row stage for both, and with whole numbers a single row."""
+  for make, spans in ((_random, (32,)), (_integers, (1, 32))):
+    g, x = make(rows, outs, ins)
+    want = _gradients(g, x)
+    bounds = _bounds(g, x, *want)
+    for span in spans:
+      for lo in {0, rows // 2 // 32 * 32, (rows - 1) // 32 * 32 if span == 1 else rows - span}:
+        part = _gradients(g[lo:lo + span], x[lo:lo + span])
+        for ref, miss, bound in zip(want, part, bounds):
+          off = ref - miss
+          if make is _integers:
+            assert not torch.equal(off.to(torch.bfloat16), ref.to(torch.bfloat16))
+          else:
+            assert bool(((off - ref).abs() > bound).any()) or float((off - ref).norm() / ref.norm()) > 3e-3
 
 
 def test_invalid_arguments_are_refused():
