@@ -10,9 +10,9 @@
 // (66 MB), the pipeline's fill and the LDS reads.
 //
 // A workgroup is 8 waves on one 256 x 256 tile, a wave 128 x 64 of it (8 accumulators of 32x32, 128
-// registers): per 16 rows it reads 6 KB of LDS for 8 MFMAs, 384 of the CU's LDS clocks for 512 of its
-// matrix clocks, where 128 x 128 over 4 waves would leave one wave a SIMD and 64 x 64 over 16 would be
-// bound by LDS. Both operands are row-major in the contracted dimension, so both are transpose reads
+// registers): per 16 rows it reads 6 KB of LDS for 8 MFMAs, so the CU reads 48 KB (about 250 clocks at
+// the 198 bytes a clock that transpose reads reach) in 512 of its matrix clocks, where 128 x 128 over 4
+// waves would leave one wave a SIMD and 64 x 64 over 16 would read 64 KB for 512. Both operands are row-major in the contracted dimension, so both are transpose reads
 // (ds_read_b64_tr_b16) of [32 rows][128 columns] tiles in the swizzled layout of the attention
 // kernels. Four 32 KB stages of 32 rows (128 KB of the 160): the copies of two stages are in flight
 // while one stage is read and the next has landed.

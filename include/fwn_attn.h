@@ -141,8 +141,8 @@ typedef struct fwn_tiles {
 /* fwn_tiles.flags: the list is laid out in an order of its own (fwn_tiles_node_order,
  * fwn_tiles_permute_*), its tiles' columns gathered per block (fwn_tiles_compact_*). The tensors stay
  * in node order and the kernels address their rows through the two tables. Every node below n must
- * be the row of one position; the launchers check n < 2^24, not the entries (an entry of n or
- * more reads zeros and stores nothing). Such a list has fewer than FWN_TILES_NODES_MAX tiles (the
+ * be the row of one position; the launchers check n < 2^24, not the entries (an entry of n reads
+ * zeros and stores nothing; any other that is not a node's reads or writes within the tensors). Such a list has fewer than FWN_TILES_NODES_MAX tiles (the
  * kernels' offsets into col_node have 32 bits). Without the flag the structure may end before them. */
 #define FWN_TILES_NODES 1
 #define FWN_TILES_NODES_MAX (1 << 22)
