@@ -117,3 +117,33 @@ def test_order_is_kept_only_where_it_pays():
   assert fwn.TileList.from_mask(dense, device=DEV)._layout is None
   noise = (sparse.random(600, 600, 0.2, random_state=1) + sparse.identity(600)).astype(bool).tocsr()
   assert fwn.TileList.from_mask(noise, device=DEV)._layout is None
+
+
+@pytest.mark.parametrize("case", sorted(CASES))
+@pytest.mark.parametrize("directed,exchange", [(False, True), (True, True), (False, False)])
+def test_given_exchange_under_a_laid_out_forward(case, directed, exchange, monkeypatch):
+  """A few rows and columns that reach everywhere spoil the order for whole groups: the forward walks the
+  list laid out for it and the backward the given pair, on the same statistics."""
+  print(f"mixed lists {case} directed={directed} exchange={exchange}", flush=True)
+  monkeypatch.setattr(hip_attn, "DS_EXCHANGE", exchange)
+  mesh, _, _, perm = fwn.mesh_mask(3, 1, reorder=True)
+  mask, n = mesh[perm][:, perm].tolil(), mesh.shape[0]
+  for r in np.random.default_rng(0).choice(n, 6 if directed else 3, replace=False):
+    mask[r, :] = True
+    mask[:, r] = True
+  mask = mask.tocoo()
+  keep = (mask.row >= mask.col) | ((mask.row + mask.col) % 3 > 0) | (not directed)
+  mask = sparse.csr_matrix((mask.data[keep], (mask.row[keep], mask.col[keep])), shape=(n, n))
+  assert ((mask != mask.T).nnz > n) == directed
+  tiles = fwn.TileList.from_mask(mask, device=DEV)
+  tiles_t = fwn.TileList.from_mask(mask.T.tocsr(), device=DEV) if directed else None
+  assert tiles.launch_list() is not tiles
+  assert tiles.exchange_lists(tiles_t or tiles, case)[:2] == (tiles, tiles_t or tiles)
+  rng = np.random.default_rng(n)
+  b, h, d = 2, 2, 64
+  q, k, v, do = (rounded(rng.standard_normal((b, n, h, d)), CASES[case][0]) for _ in range(4))
+  got = _run(case, q, k, v, do, tiles, tiles_t, d ** -0.5)
+  dense = mask.toarray()
+  refs = [A.dense_attention(q, k, v, dense, d ** -0.5), *A.dense_grads(q, k, v, do, dense, d ** -0.5)]
+  for name, g, r in zip(("out", "dq", "dk", "dv"), got, refs):
+    _check(g, r, case, name)
