@@ -64,17 +64,30 @@ struct Vec<uint16_t> {  // bfloat16 bits
 
 // A row is read once by a pass: its loads are non-temporal, so that they do not push other rows out of
 // the caches. Outputs are what the program's next kernel reads: they are stored through the caches
-// while a tensor stays in the 256 MB memory-side cache, and non-temporally (`stream`) from
-// kStreamBytes up. Gather + scatter, float32, us, with plain loads and non-temporal stores / non-temporal
-// loads and plain stores / both non-temporal: forward and backward of [1, 40962, 768] (126 MB a tensor)
-// 362 / 337 / 350, [2, 40962, 768] (252 MB) 700 / 719 / 683, [4, 40962, 1280] 2872 / 2929 / 2827; forward of
-// [1, 40962, 768] 124 / 118 / 119. Below 64 MB all three are within 3%. A choice by pass only moves
-// the time to the next one.
-constexpr uint64_t kStreamBytes = 192ull << 20;
+// while what a pass writes stays in the 256 MB memory-side cache, and non-temporally (NT) above. NT is a
+// template parameter: of two stores in the branches of a run-time choice the compiler makes one, without
+// the hint. Producer, pass and consumer of [1, n, 768], us for the pass and the consumer, plain stores
+// / non-temporal:
+//   gather (two outputs), a tensor of 96 MB: float32 102 / 106, bf16 113 / 125; 126 MB 148 / 148, 155 / 144;
+//     160 MB 197 / 180, 204 / 189; 240 MB 288 / 266, 286 / 267; 480 MB 571 / 553, 547 / 514
+//   scatter (one output): 126 MB 91 / 98, 109 / 120; 176 MB 128 / 128, 158 / 160; 240 MB 186 / 171, 223 / 210
+//   residual add and norm (two outputs): 126 MB 135 / 144, 149 / 154; 160 MB 184 / 172, 199 / 188
+//   gather's gradient: 240 MB 264 / 273, 287 / 296; 320 MB 363 / 363, 397 / 398; 480 MB 563 / 547, 613 / 599
+//   scatter's gradient: 160 MB 148 / 158, 192 / 198; 240 MB 228 / 227, 280 / 280; 320 MB 306 / 296, 373 / 363.
+// With plain loads scatter and the gradients are 5 to 15% slower from 126 MB up. The float32 gather with
+// non-temporal stores takes them: up to 200 MB it is faster so (144 MB 166 for 174, 160 MB 180 for 184; at
+// 320 MB 361 for 355).
+constexpr uint64_t kStreamBytes = 256ull << 20;      // bytes written from which a pass stores non-temporally
+constexpr uint64_t kStreamOneBytes = 192ull << 20;   // the same of a forward pass with one output
 
-__device__ __forceinline__ u32x4 load16(const void* p) { return __builtin_nontemporal_load((const u32x4*)p); }
-__device__ __forceinline__ void store16(void* p, const u32x4& v, bool stream) {
-  if (stream)
+template <bool NT = true>
+__device__ __forceinline__ u32x4 load16(const void* p) {
+  if constexpr (NT) return __builtin_nontemporal_load((const u32x4*)p);
+  return *(const u32x4*)p;
+}
+template <bool NT>
+__device__ __forceinline__ void store16(void* p, const u32x4& v) {
+  if constexpr (NT)
     __builtin_nontemporal_store(v, (u32x4*)p);
   else
     *(u32x4*)p = v;
@@ -89,7 +102,7 @@ __device__ __forceinline__ float wave_sum(float x) {
 // Loads one row (VPL vectors per lane, vector lane + 64k) and returns its mean and 1/std. With
 // `row2`, the row is row + row2, added in float32 and rounded once to T (as a separate
 // elementwise add would store it); v then holds that sum and the statistics are the sum's.
-template <typename T, int VPL>
+template <typename T, int VPL, bool NT = true>
 __device__ __forceinline__ void load_row(const T* row, bool ok, int nv, int channels, float eps, int lane,
                                          u32x4 (&v)[VPL], float (&f)[VPL][Vec<T>::E], float& mean, float& rstd,
                                          const T* row2 = nullptr) {
@@ -99,11 +112,11 @@ __device__ __forceinline__ void load_row(const T* row, bool ok, int nv, int chan
   for (int k = 0; k < VPL; ++k) {
     const int idx = lane + 64 * k;
     v[k] = u32x4{0u, 0u, 0u, 0u};
-    if (ok && idx < nv) v[k] = load16(row + (size_t)idx * E);
+    if (ok && idx < nv) v[k] = load16<NT>(row + (size_t)idx * E);
     Vec<T>::unpack(v[k], f[k]);
     if (row2) {
       u32x4 w = u32x4{0u, 0u, 0u, 0u};
-      if (ok && idx < nv) w = load16(row2 + (size_t)idx * E);
+      if (ok && idx < nv) w = load16<NT>(row2 + (size_t)idx * E);
       float g[E];
       Vec<T>::unpack(w, g);
 #pragma unroll
@@ -129,7 +142,7 @@ __device__ __forceinline__ void load_row(const T* row, bool ok, int nv, int chan
   rstd = __builtin_amdgcn_rsqf(var + eps);
 }
 
-template <typename T, int VPL>
+template <typename T, int VPL, bool NT>
 __global__ void __launch_bounds__(64 * kWaves) gather_norm_kernel(RowArgs a) {
   constexpr int E = Vec<T>::E;
   const int lane = threadIdx.x & 63;
@@ -143,27 +156,28 @@ __global__ void __launch_bounds__(64 * kWaves) gather_norm_kernel(RowArgs a) {
   u32x4 v[VPL];
   float f[VPL][E];
   float mean, rstd;
-  load_row<T, VPL>((const T*)a.x + (size_t)(b * a.n + (ok ? src : 0)) * c, ok, nv, a.channels, a.eps, lane, v, f,
-                   mean, rstd);
+  constexpr bool NTL = !(NT && sizeof(T) == 4);
+  load_row<T, VPL, NTL>((const T*)a.x + (size_t)(b * a.n + (ok ? src : 0)) * c, ok, nv, a.channels, a.eps, lane, v, f,
+                        mean, rstd);
   T* xo = (T*)a.x_out + (size_t)row * c;
   T* no = a.norm_out ? (T*)a.norm_out + (size_t)row * c : nullptr;
 #pragma unroll
   for (int k = 0; k < VPL; ++k) {
     const int idx = lane + 64 * k;
     if (idx >= nv) continue;
-    store16(xo + (size_t)idx * E, v[k], a.stream);
+    store16<NT>(xo + (size_t)idx * E, v[k]);
     if (no) {
       float y[E];
 #pragma unroll
       for (int e = 0; e < E; ++e) y[e] = (f[k][e] - mean) * rstd;
-      store16(no + (size_t)idx * E, Vec<T>::pack(y), a.stream);
+      store16<NT>(no + (size_t)idx * E, Vec<T>::pack(y));
     }
   }
 }
 
 // ADD: a.addend is added to x first and the sum written to a.x_out (a compile-time switch, so
 // the plain pass carries no test for it).
-template <typename T, int VPL, bool ADD>
+template <typename T, int VPL, bool ADD, bool NT>
 __global__ void __launch_bounds__(64 * kWaves) norm_scatter_kernel(RowArgs a) {
   constexpr int E = Vec<T>::E;
   const int lane = threadIdx.x & 63;
@@ -183,7 +197,7 @@ __global__ void __launch_bounds__(64 * kWaves) norm_scatter_kernel(RowArgs a) {
     T* so = (T*)a.x_out + (size_t)row * c;
 #pragma unroll
     for (int k = 0; k < VPL; ++k)
-      if (lane + 64 * k < nv) store16(so + (size_t)(lane + 64 * k) * E, v[k], a.stream);
+      if (lane + 64 * k < nv) store16<NT>(so + (size_t)(lane + 64 * k) * E, v[k]);
   }
   T* o = (T*)a.out + (size_t)(b * a.n + dst) * c;
   const float* mul = a.mul ? a.mul + (size_t)b * c : nullptr;
@@ -211,21 +225,26 @@ __global__ void __launch_bounds__(64 * kWaves) norm_scatter_kernel(RowArgs a) {
         for (int e = 0; e < 4; ++e) y[4 * q + e] += as_float(m[e]);
       }
     }
-    store16(o + (size_t)idx * E, Vec<T>::pack(y), a.stream);
+    store16<NT>(o + (size_t)idx * E, Vec<T>::pack(y));
   }
+}
+
+template <typename T, int VPL, bool NT>
+hipError_t launch_tvn(RowPass pass, const RowArgs& a, hipStream_t stream) {
+  const int64_t rows = (int64_t)a.batch * a.n;
+  const dim3 grid((unsigned)((rows + kWaves - 1) / kWaves)), block(64 * kWaves);
+  if (pass == RowPass::kGatherNorm)
+    hipLaunchKernelGGL((gather_norm_kernel<T, VPL, NT>), grid, block, 0, stream, a);
+  else if (a.addend)
+    hipLaunchKernelGGL((norm_scatter_kernel<T, VPL, true, NT>), grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL((norm_scatter_kernel<T, VPL, false, NT>), grid, block, 0, stream, a);
+  return hipGetLastError();
 }
 
 template <typename T, int VPL>
 hipError_t launch_tv(RowPass pass, const RowArgs& a, hipStream_t stream) {
-  const int64_t rows = (int64_t)a.batch * a.n;
-  const dim3 grid((unsigned)((rows + kWaves - 1) / kWaves)), block(64 * kWaves);
-  if (pass == RowPass::kGatherNorm)
-    hipLaunchKernelGGL((gather_norm_kernel<T, VPL>), grid, block, 0, stream, a);
-  else if (a.addend)
-    hipLaunchKernelGGL((norm_scatter_kernel<T, VPL, true>), grid, block, 0, stream, a);
-  else
-    hipLaunchKernelGGL((norm_scatter_kernel<T, VPL, false>), grid, block, 0, stream, a);
-  return hipGetLastError();
+  return a.stream ? launch_tvn<T, VPL, true>(pass, a, stream) : launch_tvn<T, VPL, false>(pass, a, stream);
 }
 
 template <typename T>
@@ -262,7 +281,7 @@ __device__ __forceinline__ void wave_sum2(float& x, float& y) {
   }
 }
 
-template <typename T, int VPL, bool SUMS>
+template <typename T, int VPL, bool SUMS, bool NT>
 __global__ void __launch_bounds__(64 * kWaves) norm_bwd_kernel(RowBwdArgs a) {
   constexpr int E = Vec<T>::E;
   extern __shared__ float sums[];  // SUMS: [2][channels]
@@ -336,7 +355,7 @@ __global__ void __launch_bounds__(64 * kWaves) norm_bwd_kernel(RowBwdArgs a) {
       Vec<T>::unpack(rv[k], r);
 #pragma unroll
       for (int e = 0; e < E; ++e) y[e] = fmaf(rstd, g[k][e] - m1 - f[k][e] * m2, r[e]);
-      store16(out + (size_t)idx * E, Vec<T>::pack(y), a.stream);
+      store16<NT>(out + (size_t)idx * E, Vec<T>::pack(y));
     }
   }
   if constexpr (SUMS) {
@@ -426,18 +445,23 @@ __global__ void __launch_bounds__(256) cond_kernel(CondArgs a) {
   }
 }
 
-template <typename T, int VPL>
-hipError_t launch_bwd_tv(const RowBwdArgs& a, hipStream_t stream) {
+template <typename T, int VPL, bool NT>
+hipError_t launch_bwd_tvn(const RowBwdArgs& a, hipStream_t stream) {
   const dim3 grid((unsigned)a.blocks * (unsigned)a.batch), block(64 * kWaves);
   if (!a.part) {
-    hipLaunchKernelGGL((norm_bwd_kernel<T, VPL, false>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((norm_bwd_kernel<T, VPL, false, NT>), grid, block, 0, stream, a);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL((norm_bwd_kernel<T, VPL, true>), grid, block, 2 * (unsigned)a.channels * sizeof(float), stream, a);
+  hipLaunchKernelGGL((norm_bwd_kernel<T, VPL, true, NT>), grid, block, 2 * (unsigned)a.channels * sizeof(float), stream, a);
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   const unsigned per = (2u * (unsigned)a.channels + 63u) / 64u;
   hipLaunchKernelGGL(sums_kernel, dim3(per * (unsigned)a.batch), dim3(64 * kSumGroups), 0, stream, a);
   return hipGetLastError();
+}
+
+template <typename T, int VPL>
+hipError_t launch_bwd_tv(const RowBwdArgs& a, hipStream_t stream) {
+  return a.stream ? launch_bwd_tvn<T, VPL, true>(a, stream) : launch_bwd_tvn<T, VPL, false>(a, stream);
 }
 
 template <typename T>
@@ -452,9 +476,9 @@ hipError_t launch_bwd_t(const RowBwdArgs& a, hipStream_t stream) {
   return hipErrorInvalidValue;
 }
 
-// Whether a pass streams its outputs past the caches (kStreamBytes).
-bool streams(int dtype, int64_t batch, int64_t n, int64_t channels) {
-  return (uint64_t)(batch * n) * (uint64_t)(channels * (dtype == FWN_F32 ? 4 : 2)) >= kStreamBytes;
+// Bytes of one [batch, n, channels] tensor.
+uint64_t tensor_bytes(int dtype, int64_t batch, int64_t n, int64_t channels) {
+  return (uint64_t)(batch * n) * (uint64_t)(channels * (dtype == FWN_F32 ? 4 : 2));
 }
 
 }  // namespace
@@ -462,7 +486,9 @@ bool streams(int dtype, int64_t batch, int64_t n, int64_t channels) {
 hipError_t launch_rows(RowPass pass, int dtype, const RowArgs& args, hipStream_t stream) {
   RowArgs a = args;
   if ((int64_t)a.batch * a.n == 0) return hipSuccess;
-  a.stream = streams(dtype, a.batch, a.n, a.channels);
+  const uint64_t bytes = tensor_bytes(dtype, a.batch, a.n, a.channels);
+  const bool two = pass == RowPass::kGatherNorm ? a.norm_out != nullptr : a.addend != nullptr;
+  a.stream = two ? 2 * bytes >= kStreamBytes : bytes >= kStreamOneBytes;
   return dtype == FWN_F32 ? launch_t<float>(pass, a, stream) : launch_t<uint16_t>(pass, a, stream);
 }
 
@@ -486,7 +512,7 @@ hipError_t launch_cond(int dtype, const CondArgs& a, hipStream_t stream) {
 
 hipError_t launch_rows_bwd(int dtype, const RowBwdArgs& args, hipStream_t stream) {
   RowBwdArgs a = args;
-  a.stream = streams(dtype, a.batch, a.n, a.channels);
+  a.stream = tensor_bytes(dtype, a.batch, a.n, a.channels) >= kStreamBytes;
   return dtype == FWN_F32 ? launch_bwd_t<float>(a, stream) : launch_bwd_t<uint16_t>(a, stream);
 }
 

@@ -19,7 +19,7 @@ struct RowArgs {
   const void* addend;  // scatter: added to x before the norm (the sum goes to x_out, required then), or null
   int32_t batch, n, channels;
   float eps;
-  bool stream;  // set by launch_rows: outputs stored non-temporally
+  bool stream;  // set by launch_rows: the kernel whose stores are non-temporal
 };
 
 enum class RowPass { kGatherNorm, kNormScatter };
@@ -51,7 +51,7 @@ struct RowBwdArgs {
   float* g_add;
   int32_t batch, n, channels, blocks;  // blocks: workgroups per batch member
   float eps;
-  bool stream;  // set by launch_rows_bwd: gx stored non-temporally
+  bool stream;  // set by launch_rows_bwd: the kernel whose stores are non-temporal
 };
 
 // Workgroups per batch member of the backward pass.
