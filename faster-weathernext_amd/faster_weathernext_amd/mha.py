@@ -106,9 +106,16 @@ class _Linear(torch.autograd.Function):
     return dx, dw, db
 
 
-# Rows from which a Linear's training pass runs as ``_Linear``. The two gradients at 8,192 rows, GEMM
-# and column sum against ``linear_wgrad``: 57 and 16 us (64 x 64), 67 and 24 (384 x 384), 77 and 39
-# (2,048 x 512); at 2,562 rows of 768 x 768 40 and 25, which the Function's host time takes back.
+# Rows from which a Linear's training pass runs as ``_Linear``, where the smaller side of its weight is 800
+# wide; with a narrower weight as many entries on that side, or 8 times as many rows. Its two gradients are
+# always quicker on the GPU (8,192 rows, GEMM and column sum against ``linear_wgrad``: 57 and 16 us at 64 x
+# 64, 67 and 24 at 384 x 384, 77 and 39 at 2,048 x 512), but the Function costs about 60 us of host time a
+# layer, and a training pass of a MeshBlock launched from Python is bound by the host below the line. Whole
+# passes, us, modules against ``_Linear`` (rows x d_model, ffw_hidden = 4 d_model): below, 10,242 x 256 1222
+# and 1457, x 512 1171 and 1429, 20,484 x 256 1182 and 1417, 30,726 x 192 1217 and 1445, 40,962 x 128 1184 and
+# 1405; about the line and with the host's pace, 10,242 x 768 1307 to 1363 and 1231 to 1449, 20,484 x 384 1257 to
+# 1285 and 1191 to 1449, 81,924 x 64 1374 to 1396 and 1165 to 1482; above, 10,242 x 1,024 1598 and 1443, 20,484 x
+# 512 1582 and 1370, 30,726 x 384 1690 and 1372, 40,962 x 192 1507 and 1218, x 768 4156 and 3185.
 WGRAD_ROWS = 8192
 # Largest weight whose gradient is ``linear_wgrad``: half of the 256 CUs' 256 x 256 tiles. Above it a
 # GEMM's own tiles fill the chip (20,484 rows: 4,096 x 1,024 299 and 175 us, 8,192 x 2,048 645 and
@@ -124,11 +131,17 @@ def is_plain(module, kind):
                module._backward_pre_hooks) and not torch.nn.modules.module._has_any_global_hook())
 
 
+def rows_enough(rows, outs, ins):
+  """Whether a Linear of that weight over `rows` rows is past the line of WGRAD_ROWS."""
+  return rows >= WGRAD_ROWS and (rows * min(outs, ins) >= 800 * WGRAD_ROWS or rows >= 8 * WGRAD_ROWS)
+
+
 def linear(lin, x):
   """lin(x) with gradients: as ``_Linear`` where x and lin's parameters are plain bfloat16 tensors on one
   GPU, sizes are whole 64s and there are rows enough; else the module as it is."""
-  if (x.dtype == torch.bfloat16 and x.is_cuda and x.numel() >= WGRAD_ROWS * x.shape[-1] > 0 and is_plain(lin, torch.nn.Linear)
-      and type(x) in (torch.Tensor, torch.nn.Parameter) and type(lin.weight) is torch.nn.Parameter and
+  if (x.dtype == torch.bfloat16 and x.is_cuda and x.numel() > 0 and is_plain(lin, torch.nn.Linear) and
+      rows_enough(x.numel() // x.shape[-1], *lin.weight.shape) and
+      type(x) in (torch.Tensor, torch.nn.Parameter) and type(lin.weight) is torch.nn.Parameter and
       lin.weight.dtype == x.dtype and lin.weight.device == x.device and lin.weight.is_contiguous() and
       x.shape[-1] == lin.weight.shape[1] and
       all(s % 64 == 0 and 0 < s <= 16384 for s in lin.weight.shape) and lin.weight.numel() <= WGRAD_ENTRIES and

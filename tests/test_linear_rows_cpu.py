@@ -59,3 +59,14 @@ def test_plain_modules_are_those_whose_call_is_their_forward():
   assert torch.equal(compiled(torch.ones(4)), torch.ones(4))
   for lin in (hooked, replaced, compiled, torch.nn.utils.parametrizations.weight_norm(make())):
     assert not is_plain(lin, torch.nn.Linear)
+
+
+def test_rows_from_which_training_takes_the_split_gradients():
+  """As many entries as WGRAD_ROWS rows have at 800 wide, whichever side of the weight is the smaller;
+  always from eight times as many rows, never below them."""
+  from faster_weathernext_amd.mha import rows_enough
+  for rows, d, past in ((10242, 512, False), (20484, 256, False), (40962, 128, False), (8191, 4096, False), (65535, 64, False),
+                        (8192, 832, True), (10242, 768, True), (20484, 384, True), (30726, 256, True), (40962, 192, True),
+                        (65536, 64, True), (40962, 768, True)):
+    for outs, ins in ((d, d), (3 * d, d), (d, 4 * d)):
+      assert rows_enough(rows, outs, ins) == past
