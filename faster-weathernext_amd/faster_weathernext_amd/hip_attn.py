@@ -236,7 +236,7 @@ LAID_OUT_GAIN = 0.95
 def _exchange_gain(products):
   """The most tiles, cost and dS units the lists laid out for the exchange may have, of the given pair's.
 
-  They pack whole groups and not single columns, so they are judged apart from the forward's: a few
+  They pack whole groups and not single columns, so they are weighed apart from the forward's: a few
   rows that reach everywhere leave the forward's list 0.79 of the cost and these 2.1 times of it, with
   3.8 times the units (8-hop refinement-6 mesh with 20 such rows). Backward of 4 heads x 128 on MI355X, us,
   given -> packed pair:

@@ -269,7 +269,7 @@ def test_an_exchange_keeps_no_list_alive():
 
 @pytest.mark.parametrize("name", ["mesh", "hilbert", "global rows", "directed global rows", "random", "coarse"])
 def test_exchange_lists_are_no_costlier_than_the_given_ones(name):
-  """The lists of the dS exchange are judged by themselves: where a few rows and columns that reach
+  """The lists of the dS exchange are weighed by themselves: where a few rows and columns that reach
   everywhere spoil the order, or the mask has no locality, the forward's list pays and the given two are
   walked in the backward; in any case neither their tiles, nor their cost, nor the dS buffer grow."""
   coarse, wide = name == "coarse", "global" in name
